@@ -11,9 +11,11 @@
 //                         partial last round of tiles over the CUs is cut into 128-row half tiles.
 //   gemm_nt_kernel        128 x 128 x 128 tiles, 4 waves, loads through registers; small shapes and
 //                         operands beyond the 2 GiB reach of a buffer descriptor's 32-bit offsets.
-//   gemm_nt_naive_kernel  any K / alignment, one output per thread.
+//   gemm_any_kernel       (gemm_any.h) any K and alignment: 64- or 128-wide tiles, fp8 widened to bf16 on its way to
+//                         the matrix cores.
 #include "gemm_common.h"
 #include "gemm_big.h"
+#include "gemm_any.h"
 
 namespace ntfp8 {
 
@@ -122,57 +124,15 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __
     }
 }
 
-// Any K / alignment: one output element per thread, table-free decode through the hardware
-// fp8 -> fp32 conversion.  Only meant for tiny or odd shapes.
-template <int FA, int FB, int DT, bool kAcc>
-__global__ void gemm_nt_naive_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, void* __restrict__ Dv,
-                                     const float* __restrict__ scale_a, const float* __restrict__ scale_b, int M, int N,
-                                     int K, Fp8Out fp8, GemmExtras ex) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = idx < (int64_t)M * N;
-    if (!live && !(DT == NTFP8_OUT_E4M3 || DT == NTFP8_OUT_E5M2)) return;
-    const int m = live ? (int)(idx / N) : 0, n = live ? (int)(idx % N) : 0;
-    float acc = 0.0f;
-    for (int k = 0; live && k < K; ++k) {
-        const float a = FA == kE4M3 ? __builtin_amdgcn_cvt_f32_fp8((int)A[(int64_t)m * K + k], 0)
-                                    : __builtin_amdgcn_cvt_f32_bf8((int)A[(int64_t)m * K + k], 0);
-        const float b = FB == kE4M3 ? __builtin_amdgcn_cvt_f32_fp8((int)B[(int64_t)n * K + k], 0)
-                                    : __builtin_amdgcn_cvt_f32_bf8((int)B[(int64_t)n * K + k], 0);
-        acc += a * b;
-    }
-    float v = acc * descale_factor(scale_a, scale_b, ex.scale_inv);
-    if (ex.bias && live) v = v + bias_at(ex.bias, ex.bias_dtype, n);
-    if constexpr (DT == NTFP8_OUT_E4M3 || DT == NTFP8_OUT_E5M2) {
-        // whole waves get here (the amax reduction runs over all 64 lanes); lanes past the end hold zeros
-        constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
-        uint32_t amax = 0;
-        const uint32_t w = quant4<F>(v, 0.0f, 0.0f, 0.0f, *fp8.scale, true, amax);
-        if (live) {
-            static_cast<uint8_t*>(Dv)[idx] = (uint8_t)w;
-            if (fp8.Dt) fp8.Dt[(int64_t)n * M + m] = (uint8_t)w;
-        }
-        publish_amax(amax, fp8.ws);
-    } else {
-        typedef typename OutT<DT>::type O;
-        O* D = static_cast<O*>(Dv);
-        if constexpr (DT == NTFP8_F32) {
-            if constexpr (kAcc) v = v + D[idx];
-            D[idx] = v;
-        } else {
-            D[idx] = OutT<DT>::cvt(v);
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------------------------
-enum GemmPath { kPathNone = -1, kPathNaive = 0, kPathSmall = 1, kPathBig = 2 };
+enum GemmPath { kPathNone = -1, kPathAny = 0, kPathSmall = 1, kPathBig = 2 };
 
 // which kernel serves a problem
 static int path_of(const GemmDesc& g) {
     const bool aligned16 = (g.K % 16 == 0) &&
                            ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 &&
                            (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
-    if (!aligned16) return g.tb ? kPathNone : kPathNaive;
+    if (!aligned16) return g.tb ? kPathNone : kPathAny;
     // the big kernel addresses its operands with 32-bit buffer offsets and wants enough tiles to matter
     const bool fits32 = (int64_t)(g.M + 256) * g.K < (1LL << 31) && (int64_t)(g.N + kBigN) * g.K < (1LL << 31);
     const bool worth = g.M > kBM && g.N > kBN && g.K >= 2 * kBK;
@@ -248,9 +208,18 @@ static int launch_small(const GemmDesc& g, int path, hipStream_t st) {
         hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, DT, kAcc>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa,
                            g.sb, g.M, g.N, g.K, tm, tn, fp8, ex);
     } else {
-        const int64_t blocks = ((int64_t)g.M * g.N + 255) / 256;
-        hipLaunchKernelGGL((gemm_nt_naive_kernel<FA, FB, DT, kAcc>), dim3((int)blocks), dim3(256), 0, st, a, b, g.D, g.sa,
-                           g.sb, g.M, g.N, g.K, fp8, ex);
+        const int d_vec = (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
+        const int64_t t2m = ((int64_t)g.M + 127) / 128, t2n = ((int64_t)g.N + 127) / 128;
+        // 128-wide tiles once there is one for every CU, 64-wide below (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles
+        // of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6; 4096 x 4096 x 4095 262 / 179)
+        if (t2m * t2n >= cu_count()) {
+            hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 2>), dim3((int)(t2m * t2n)), dim3(kAnyThreads), 0, st, a, b,
+                               g.D, g.sa, g.sb, g.M, g.N, g.K, (int)t2m, (int)t2n, d_vec, fp8, ex);
+        } else {
+            const int tm = (g.M + 63) / 64, tn = (g.N + 63) / 64;
+            hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 1>), dim3(tm * tn), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa,
+                               g.sb, g.M, g.N, g.K, tm, tn, d_vec, fp8, ex);
+        }
     }
     return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
 }

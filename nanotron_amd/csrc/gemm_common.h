@@ -168,10 +168,11 @@ __device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int& pid
 }
 
 // Epilogue of one wave: MI x NJ accumulator blocks of 32 x 32, block (i, j) at rows m_base + 32 i,
-// columns n_base + 32 j.  Descale, optional fp32 accumulate, one rounding, store.
+// columns n_base + 32 j.  Descale, optional fp32 accumulate, one rounding, store.  `d_aligned`: D starts on a 16-byte
+// boundary (otherwise every element is stored by itself).
 template <int DT, bool kAcc, int MI, int NJ>
 __device__ __forceinline__ void store_wave_tile(const v16f (&acc)[MI][NJ], void* __restrict__ Dv, float alpha, int M,
-                                                int N, int m_base, int n_base, int lane) {
+                                                int N, int m_base, int n_base, int lane, bool d_aligned = true) {
     typedef typename OutT<DT>::type O;
     O* D = static_cast<O*>(Dv);
     if constexpr (DT != NTFP8_F32) {
@@ -179,7 +180,7 @@ __device__ __forceinline__ void store_wave_tile(const v16f (&acc)[MI][NJ], void*
         // wave hold adjacent groups of 4.  Swapping registers between the halves gives every lane 8
         // consecutive n (16 bytes), and lanes l / l + 32 together a full 32-byte sector per row, which
         // is what the memory side writes without read-modify-write traffic.
-        if ((N & 7) == 0) {
+        if ((N & 7) == 0 && d_aligned) {
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
                 const int m = m_base + i * 32 + (lane & 31);
@@ -205,7 +206,7 @@ __device__ __forceinline__ void store_wave_tile(const v16f (&acc)[MI][NJ], void*
             return;
         }
     }
-    const bool vec_ok = (N & 3) == 0;
+    const bool vec_ok = (N & 3) == 0 && d_aligned;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 32 + (lane & 31);
@@ -325,9 +326,10 @@ __device__ __forceinline__ void publish_amax(uint32_t lane_bits, Workspace* ws) 
 template <int F, int MI, int NJ>
 __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ], uint8_t* __restrict__ D,
                                                         uint8_t* __restrict__ Dt, float alpha, float scale_d, bool slow,
-                                                        int M, int N, int m_base, int n_base, int lane) {
+                                                        int M, int N, int m_base, int n_base, int lane,
+                                                        bool d_aligned = true) {
     uint32_t amax = 0;
-    const bool d_vec = (N & 3) == 0;   // rows of D start 4-byte aligned (the launcher checks D itself)
+    const bool d_vec = (N & 3) == 0 && d_aligned;   // rows of D start 4-byte aligned
     const bool t_vec = (M & 3) == 0 && (reinterpret_cast<uintptr_t>(Dt) & 3) == 0;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
