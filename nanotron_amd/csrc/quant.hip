@@ -520,29 +520,87 @@ __device__ __forceinline__ float decode1(uint32_t b) {
     else return __builtin_amdgcn_cvt_f32_bf8((int)b, 0);
 }
 
+// fp32 value -> one output element of type OUT, as dequantised.  The fp32 product is kept a value of its own: folded into
+// a mixed-precision fma (x*y + 0) the conversion would turn -0 into +0.
+template <int OUT>
+__device__ __forceinline__ void store_dequant1(void* __restrict__ out, int64_t j, float v) {
+    asm volatile("" : "+v"(v));
+    if constexpr (OUT == NTFP8_F32) ((float*)out)[j] = v;
+    else if constexpr (OUT == NTFP8_F16) ((__half*)out)[j] = __float2half_rn(v);
+    else {
+        // bf16 round-to-nearest-even with NaN kept quiet
+        uint32_t u = __float_as_uint(v);
+        uint16_t r;
+        if ((u & 0x7fffffffu) > kInfBits) r = (uint16_t)((u >> 16) | 0x40u);
+        else r = (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+        ((uint16_t*)out)[j] = r;
+    }
+}
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2bf));
+}
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    asm volatile("" : "+v"(a), "+v"(b));   // (no mixed-precision fma, as above)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2h));
+}
+// the two low or the two high fp8 codes of a word -> fp32
+template <int F, bool kHigh>
+__device__ __forceinline__ void decode2(uint32_t w, float& a, float& b) {
+    if constexpr (F == kE4M3) {
+        const auto p = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, kHigh);
+        a = p[0], b = p[1];
+    } else {
+        const auto p = __builtin_amdgcn_cvt_pk_f32_bf8((int)w, kHigh);
+        a = p[0], b = p[1];
+    }
+}
+
+// HBM-bound.  A lane writes 16 bytes per group (8 16-bit or 4 fp32 elements, read as 8 or 4 bytes), so that a wave's
+// loads and stores each cover one contiguous piece, and has kDqUnroll groups in flight.  Loads go through the caches (the
+// bytes were usually written by the kernel before), stores are streaming.  bf16, 4096 x 4096 (50.3 MB): 15.5 us with one
+// byte per lane and trip, 8.1 us (6.2 TB/s) now; streaming loads as well 9.4 us, ordinary stores 9.0 us, one group per
+// trip 9.3 us.
 // `is_inverse`: scale_ptr holds 1 / scale already (the form tex.cast_from_fp8 is handed, src/nanotron/fp8/tensor.py:74)
+constexpr int kDqUnroll = 4;
 template <int F, int OUT>
-__global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __restrict__ in, int64_t n,
+__global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __restrict__ in, int64_t n_vec, int64_t n,
                                                            const float* __restrict__ scale_ptr, void* __restrict__ out,
                                                            int is_inverse) {
+    constexpr int kE = OUT == NTFP8_F32 ? 4 : 8;   // elements per group
+    typedef uint32_t win __attribute__((ext_vector_type(kE / 4)));
+    typedef win win_any __attribute__((aligned(1)));   // the input may start anywhere
     const float inv = is_inverse ? *scale_ptr : 1.0f / *scale_ptr;
-    const int64_t stride = (int64_t)gridDim.x * kThreads;
-    for (int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x; j < n; j += stride) {
-        float v = decode1<F>(in[j]) * inv;
-        // keep the fp32 product a value of its own: folded into a mixed-precision fma (x*y + 0) the
-        // conversion would turn -0 into +0
-        asm volatile("" : "+v"(v));
-        if constexpr (OUT == NTFP8_F32) ((float*)out)[j] = v;
-        else if constexpr (OUT == NTFP8_F16) ((__half*)out)[j] = __float2half_rn(v);
-        else {
-            // bf16 round-to-nearest-even with NaN kept quiet
-            uint32_t u = __float_as_uint(v);
-            uint16_t r;
-            if ((u & 0x7fffffffu) > kInfBits) r = (uint16_t)((u >> 16) | 0x40u);
-            else r = (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-            ((uint16_t*)out)[j] = r;
+    const int64_t stride = (int64_t)gridDim.x * (kThreads * kDqUnroll);
+    for (int64_t i = (int64_t)blockIdx.x * (kThreads * kDqUnroll) + threadIdx.x; i < n_vec; i += stride) {
+        win w[kDqUnroll];
+#pragma unroll
+        for (int u = 0; u < kDqUnroll; ++u)
+            if (i + u * kThreads < n_vec) w[u] = *reinterpret_cast<const win_any*>(in + (i + u * kThreads) * kE);
+#pragma unroll
+        for (int u = 0; u < kDqUnroll; ++u) {
+            if (i + u * kThreads >= n_vec) break;
+            float v[kE];
+#pragma unroll
+            for (int h = 0; h < kE / 4; ++h) {
+                decode2<F, false>(w[u][h], v[4 * h], v[4 * h + 1]);
+                decode2<F, true>(w[u][h], v[4 * h + 2], v[4 * h + 3]);
+            }
+#pragma unroll
+            for (int e = 0; e < kE; ++e) v[e] *= inv;
+            u4 o;
+            if constexpr (OUT == NTFP8_F32) o = (u4){__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+            else if constexpr (OUT == NTFP8_F16) o = (u4){pack_f16(v[0], v[1]), pack_f16(v[2], v[3]), pack_f16(v[4], v[5]), pack_f16(v[6], v[7])};
+            else o = (u4){pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+            __builtin_nontemporal_store(o, reinterpret_cast<u4*>(out) + i + u * kThreads);
         }
     }
+    // elements past the last group (all of them when the output is not 16-byte aligned)
+    for (int64_t j = n_vec * kE + (int64_t)blockIdx.x * kThreads + threadIdx.x; j < n; j += (int64_t)gridDim.x * kThreads)
+        store_dequant1<OUT>(out, j, decode1<F>(in[j]) * inv);
 }
 
 // Byte transpose through a 64x64 LDS tile (pitch 65 breaks the bank pattern); any shape.
@@ -822,9 +880,10 @@ int run_quant_delayed_batch_static(QuantDesc* q, int count, hipStream_t st) {
 int run_dequant(const void* in, int fmt, const float* scale, int is_inverse, int64_t n, void* out, int out_dtype,
                 hipStream_t st) {
     clear_stale_error();
-    const int grid = grid_for(n);
+    const int64_t n_vec = aligned(out, 16) ? n / (out_dtype == NTFP8_F32 ? 4 : 8) : 0;
+    const int grid = grid_for(n_vec > 0 ? (n_vec + kDqUnroll - 1) / kDqUnroll : n, kThreads, 32);
     const uint8_t* p = static_cast<const uint8_t*>(in);
-#define NT_DQ(F, O) hipLaunchKernelGGL((dequant_kernel<F, O>), dim3(grid), dim3(kThreads), 0, st, p, n, scale, out, is_inverse)
+#define NT_DQ(F, O) hipLaunchKernelGGL((dequant_kernel<F, O>), dim3(grid), dim3(kThreads), 0, st, p, n_vec, n, scale, out, is_inverse)
     if (fmt == kE4M3) {
         if (out_dtype == NTFP8_F32) NT_DQ(kE4M3, NTFP8_F32);
         else if (out_dtype == NTFP8_F16) NT_DQ(kE4M3, NTFP8_F16);
