@@ -16,7 +16,7 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 
 // ---------------------------------------------------------------------------------------------
-// 16-element loads.  `m16` receives max|x| of the 16 elements as a comparable unsigned pattern in
+// Loads of E = 4 or 16 elements.  `mx` receives max|x| of them as a comparable unsigned pattern in
 // the *source* format (fp32 bits for float, 16-bit patterns for half / bf16).
 // kStream: the load is marked streaming and leaves no line behind in the memory-side cache.  Passes that read their
 // tensor once (delayed scaling) use it: in a training step they run behind a GEMM whose output fills that cache, and an
@@ -24,10 +24,11 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 // activations 18.6 against 20.0, although back to back on a rested cache ordinary loads are the faster ones, 11.4
 // against 13.5 us for 4096 x 4096).  Where a second pass follows (current scaling: amax, then cast) both use ordinary
 // loads, and the second finds what the first has read: fp32 11008 x 4096 with transposed copy 119 -> 78 us for the two.
-template <bool kStream, typename V>
-__device__ __forceinline__ V load_vec(const V* p) {
-    if constexpr (kStream) return __builtin_nontemporal_load(p);
-    else return *p;
+template <bool kStream, int kAlign, typename V>
+__device__ __forceinline__ V load_vec(const void* p) {   // p: kAlign-byte aligned
+    typedef V VA __attribute__((aligned(kAlign)));
+    if constexpr (kStream) return __builtin_nontemporal_load(static_cast<const VA*>(p));
+    else return *static_cast<const VA*>(p);
 }
 template <typename T>
 struct Src;
@@ -35,21 +36,20 @@ struct Src;
 template <>
 struct Src<float> {
     static constexpr int kDtype = NTFP8_F32;
-    template <bool kStream>
-    __device__ static __forceinline__ void load16(const float* p, float (&v)[16], uint32_t& m16) {
-        const f4* q = reinterpret_cast<const f4*>(p);
+    template <int E, bool kStream>
+    __device__ static __forceinline__ void load(const float* p, float (&v)[E], uint32_t& mx) {
         uint32_t m = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const f4 t = load_vec<kStream>(q + i);
+        for (int i = 0; i < E / 4; ++i) {
+            const f4 t = load_vec<kStream, 4, f4>(p + 4 * i);
             v[4 * i + 0] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        for (int i = 0; i < E; ++i) {
             const uint32_t a = __float_as_uint(v[i]) & 0x7fffffffu;
             m = a > m ? a : m;
         }
-        m16 = m;
+        mx = m;
     }
     __device__ static __forceinline__ float load1(const float* p, uint32_t& m) {
         const float x = *p;
@@ -66,16 +66,24 @@ struct Src16 {
         if constexpr (kBf16) return bf16_bits_to_float(h);
         else return half_bits_to_float(h);
     }
-    template <bool kStream>
-    __device__ static __forceinline__ void load16(const uint16_t* p, float (&v)[16], uint32_t& m16) {
-        const u4* q = reinterpret_cast<const u4*>(p);
-        const u4 a = load_vec<kStream>(q);
-        const u4 b = load_vec<kStream>(q + 1);
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    template <int E, bool kStream>
+    __device__ static __forceinline__ void load(const uint16_t* p, float (&v)[E], uint32_t& mx) {
+        uint32_t w[E / 2];
+        if constexpr (E == 4) {
+            typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+            const u2 a = load_vec<kStream, 2, u2>(p);
+            w[0] = a.x, w[1] = a.y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < E / 8; ++i) {
+                const u4 a = load_vec<kStream, 2, u4>(p + 8 * i);
+                w[4 * i] = a.x, w[4 * i + 1] = a.y, w[4 * i + 2] = a.z, w[4 * i + 3] = a.w;
+            }
+        }
         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
         us2 m = {0, 0};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < E / 2; ++i) {
             if constexpr (kBf16) {
                 v[2 * i] = __uint_as_float(w[i] << 16);
                 v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
@@ -88,7 +96,7 @@ struct Src16 {
             __builtin_memcpy(&t, &ab, 4);
             m = __builtin_elementwise_max(m, t);
         }
-        m16 = m.x > m.y ? m.x : m.y;
+        mx = m.x > m.y ? m.x : m.y;
     }
     __device__ static __forceinline__ float load1(const uint16_t* p, uint32_t& m) {
         const uint32_t h = *p;
@@ -120,21 +128,25 @@ struct ElemOf<float> {
     typedef float type;
 };
 
-// 16 scaled values -> 16 fp8 bytes.  `slow` = this group may contain a NaN (NaN input or a
+// E scaled values -> E fp8 bytes.  `slow` = this group may contain a NaN (NaN input or a
 // degenerate scale): patch the NaN bytes to sign|0x7F.
-template <int F>
-__device__ __forceinline__ u4 encode16(const float (&v)[16], float scale, bool slow) {
-    float y[16];
+template <int F, int E>
+__device__ __forceinline__ void encode(const float (&v)[E], float scale, bool slow, uint32_t (&w)[E / 4]) {
+    float y[E];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) y[i] = v[i] * scale;
-    uint32_t w[4];
+    for (int i = 0; i < E; ++i) y[i] = v[i] * scale;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < E / 4; ++i)
         w[i] = cvt4<F>(sat<F>(y[4 * i]), sat<F>(y[4 * i + 1]), sat<F>(y[4 * i + 2]), sat<F>(y[4 * i + 3]));
     if (slow) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) w[i >> 2] = patch_nan(w[i >> 2], i & 3, y[i]);
+        for (int i = 0; i < E; ++i) w[i >> 2] = patch_nan(w[i >> 2], i & 3, y[i]);
     }
+}
+template <int F>
+__device__ __forceinline__ u4 encode16(const float (&v)[16], float scale, bool slow) {
+    uint32_t w[4];
+    encode<F, 16>(v, scale, slow, w);
     return (u4){w[0], w[1], w[2], w[3]};
 }
 
@@ -325,8 +337,8 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     for (; i + stride < n_vec; i += 2 * stride) {
         float v0[16], v1[16];
         uint32_t m0, m1;
-        L::template load16<MODE == kModeDelayed>(x + i * kVec, v0, m0);
-        L::template load16<MODE == kModeDelayed>(x + (i + stride) * kVec, v1, m1);
+        L::template load<16, MODE == kModeDelayed>(x + i * kVec, v0, m0);
+        L::template load<16, MODE == kModeDelayed>(x + (i + stride) * kVec, v1, m1);
         if constexpr (kAmax) {
             m_run = m0 > m_run ? m0 : m_run;
             m_run = m1 > m_run ? m1 : m_run;
@@ -341,7 +353,7 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     if (i < n_vec) {
         float v0[16];
         uint32_t m0;
-        L::template load16<MODE == kModeDelayed>(x + i * kVec, v0, m0);
+        L::template load<16, MODE == kModeDelayed>(x + i * kVec, v0, m0);
         if constexpr (kAmax) m_run = m0 > m_run ? m0 : m_run;
         if constexpr (kCast) {
             const u4 q0 = encode16<F>(v0, scale, degen || L::has_nan(m0));
@@ -385,8 +397,8 @@ __global__ __launch_bounds__(kFlatThreads) void quant_flat_dual_kernel(const typ
     for (; i + stride < n_vec; i += 2 * stride) {
         float v0[16], v1[16];
         uint32_t m0, m1;
-        L::template load16<true>(x + i * kVec, v0, m0);
-        L::template load16<true>(x + (i + stride) * kVec, v1, m1);
+        L::template load<16, true>(x + i * kVec, v0, m0);
+        L::template load<16, true>(x + (i + stride) * kVec, v1, m1);
         m_run = m0 > m_run ? m0 : m_run;
         m_run = m1 > m_run ? m1 : m_run;
         const bool n0 = L::has_nan(m0), n1 = L::has_nan(m1);
@@ -398,7 +410,7 @@ __global__ __launch_bounds__(kFlatThreads) void quant_flat_dual_kernel(const typ
     if (i < n_vec) {
         float v0[16];
         uint32_t m0;
-        L::template load16<true>(x + i * kVec, v0, m0);
+        L::template load<16, true>(x + i * kVec, v0, m0);
         m_run = m0 > m_run ? m0 : m_run;
         const bool n0 = L::has_nan(m0);
         __builtin_nontemporal_store(encode16<kE4M3>(v0, s0, d0 || n0), reinterpret_cast<u4*>(out0 + i * kVec));
@@ -442,13 +454,111 @@ __global__ __launch_bounds__(kFlatThreads) void quant_flat_multi_kernel(const Mu
 }
 
 // ---------------------------------------------------------------------------------------------
-// Cast (+ optional amax) that also writes the transposed bytes.  One 128x128 tile per block, staged
-// through 16 KB of LDS.  LDS holds the tile transposed, [col][row], the 16-byte row chunks of each
-// column XOR-swizzled with the column's 16-wide chunk index so that both the byte stores of phase 1
-// and the 128-bit loads of phase 2 are bank-conflict free.
-constexpr int kTile = 128;
+// Byte tiles turned around in LDS: the cast that also writes the transposed bytes, and the transpose of fp8 bytes.
+//
+// A workgroup of 256 threads takes a tile of kT x kT bytes; a thread holds 4 rows x E columns of it (E = 16: kT = 128,
+// E = 4: kT = 64).  Four v_perm pairs turn each 4 x 4 block of bytes around, so LDS receives whole words, [column][row]:
+// a quarter of the stores that single bytes would need.  The 16-byte row chunks of a column are XORed with the
+// column's group (E = 16) or the columns are one word apart from a multiple of the banks (E = 4), which spreads both the
+// stores and the reads over the banks.  Global accesses are 16 bytes wide whatever the alignment of a row (gfx950
+// serves misaligned ones).  At the edges of the matrix loads are clamped to its last row and column (the copies reach
+// neither a stored byte nor change a maximum) and the last bytes of a row are stored 8, 4, 2, 1 at a time.
+//
+// Bound by HBM on large tensors, by the latency of one tile on small ones.  128-wide tiles from one tile per CU on,
+// 64-wide ones below: see the measurements at tile_edge().  Against 64-wide tiles of single bytes (transpose), byte
+// stores into LDS (cast) and one element per thread (any shape that is no multiple of 128), us before / now: transpose
+// 4096 x 4096 19.7 / 6.0 (5.5 TB/s), 2048 x 2048 6.5 / 3.0; fp32 cast with copy 4096 x 4096 26.6 / 16.9, 11008 x 4096
+// 68 / 54 (5.0 TB/s), 4095 x 4097 143 / 27; bf16 delayed step with copy 1021 x 1024 13.5 / 7.1, 1021 x 2304 19.7 / 9.1.
+template <int E>
+struct Tile {
+    static constexpr int kT = E == 16 ? 128 : 64;
+    static constexpr int kPitch = E == 16 ? 32 : 17;   // words between columns in LDS
+    static constexpr int kChunks = kT / 16;            // 16-byte row chunks per column
+};
+typedef u4 u4_any __attribute__((aligned(1)));
 
-template <typename S, int F, bool kAmax>
+// the first n (1 .. 15) bytes of q
+__device__ __forceinline__ void store_head(uint8_t* __restrict__ p, u4 q, int n) {
+    typedef uint64_t u64_any __attribute__((aligned(1)));
+    typedef uint32_t u32_any __attribute__((aligned(1)));
+    typedef uint16_t u16_any __attribute__((aligned(1)));
+    uint64_t lo = q.x | ((uint64_t)q.y << 32);
+    if (n & 8) {
+        *reinterpret_cast<u64_any*>(p) = lo;
+        lo = q.z | ((uint64_t)q.w << 32);
+        p += 8;
+    }
+    if (n & 4) {
+        *reinterpret_cast<u32_any*>(p) = (uint32_t)lo;
+        lo >>= 32;
+        p += 4;
+    }
+    if (n & 2) {
+        *reinterpret_cast<u16_any*>(p) = (uint16_t)lo;
+        lo >>= 16;
+        p += 2;
+    }
+    if (n & 1) *p = (uint8_t)lo;
+}
+
+// w[r][q] = bytes 4 q .. 4 q + 3 of row r of the thread's block -> LDS
+template <int E>
+__device__ __forceinline__ void deposit_block(uint32_t* __restrict__ tile, const uint32_t (&w)[4][E / 4], int cgrp, int rgrp) {
+    const int pos = E == 16 ? ((((rgrp >> 2) ^ cgrp) & 7) << 2) | (rgrp & 3) : rgrp;
+#pragma unroll
+    for (int q = 0; q < E / 4; ++q) {
+        const uint32_t a = __builtin_amdgcn_perm(w[1][q], w[0][q], 0x05010400u), b = __builtin_amdgcn_perm(w[3][q], w[2][q], 0x05010400u);
+        const uint32_t c = __builtin_amdgcn_perm(w[1][q], w[0][q], 0x07030602u), d = __builtin_amdgcn_perm(w[3][q], w[2][q], 0x07030602u);
+        uint32_t* t = tile + (cgrp * E + 4 * q) * Tile<E>::kPitch + pos;
+        t[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        t[Tile<E>::kPitch] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        t[2 * Tile<E>::kPitch] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+        t[3 * Tile<E>::kPitch] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+    }
+}
+
+// the tile's columns as rows of out_t [cols, rows]
+template <int E>
+__device__ __forceinline__ void emit_columns(const uint32_t* __restrict__ tile, uint8_t* __restrict__ out_t, int64_t rows,
+                                             int64_t cols, int64_t row0, int64_t col0) {
+    typedef Tile<E> T;
+#pragma unroll
+    for (int it = 0; it < T::kT * T::kChunks / kTileThreads; ++it) {
+        const int idx = threadIdx.x + kTileThreads * it;
+        const int c = idx / T::kChunks, ch = idx % T::kChunks;
+        u4 q;
+        if constexpr (E == 16) {
+            q = *reinterpret_cast<const u4*>(tile + c * T::kPitch + (((ch ^ (c >> 4)) & 7) << 2));
+        } else {
+            const uint32_t* t = tile + c * T::kPitch + 4 * ch;
+            q = (u4){t[0], t[1], t[2], t[3]};
+        }
+        const int64_t r = row0 + ch * 16;
+        if (col0 + c >= cols || r >= rows) continue;
+        uint8_t* p = out_t + (col0 + c) * rows + r;
+        if (r + 16 <= rows) {
+            __builtin_nontemporal_store(q, reinterpret_cast<u4_any*>(p));
+        } else {
+            store_head(p, q, (int)(rows - r));
+        }
+    }
+}
+
+// one row of the thread's block: `inside` of its bytes lie inside the matrix
+template <int E>
+__device__ __forceinline__ void store_row_bytes(uint8_t* __restrict__ p, const uint32_t (&w)[E / 4], int64_t inside) {
+    typedef uint32_t u32_any __attribute__((aligned(1)));
+    if constexpr (E == 16) {
+        const u4 q = {w[0], w[1], w[2], w[3]};
+        if (inside >= 16) __builtin_nontemporal_store(q, reinterpret_cast<u4_any*>(p));
+        else store_head(p, q, (int)inside);
+    } else {
+        if (inside >= 4) *reinterpret_cast<u32_any*>(p) = w[0];
+        else store_head(p, (u4){w[0], 0u, 0u, 0u}, (int)inside);
+    }
+}
+
+template <typename S, int F, bool kAmax, int E>
 __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typename ElemOf<S>::type* __restrict__ x,
                                                                    int64_t rows, int64_t cols,
                                                                    uint8_t* __restrict__ out,
@@ -456,73 +566,97 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
                                                                    const float* __restrict__ scale_ptr,
                                                                    Workspace* ws, ScalarIO io) {
     typedef Src<S> L;
-    __shared__ __attribute__((aligned(16))) uint8_t tile[kTile * kTile];
+    typedef Tile<E> T;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[T::kT * T::kPitch];
     const float scale = *scale_ptr;
     const bool degen = degenerate_scale(scale);
-    const int64_t tiles_c = cols / kTile;
-    const int64_t tiles = (rows / kTile) * tiles_c;
-    const int t = threadIdx.x;
-    const int cchunk = t & 7;   // 16-column chunk inside the tile
-    const int rsub = t >> 3;    // 0..31
-    const int rchunk = t & 7;
+    const int64_t tiles_c = (cols + T::kT - 1) / T::kT;
+    const int64_t tiles = ((rows + T::kT - 1) / T::kT) * tiles_c;
+    const int cgrp = threadIdx.x % (T::kT / E), rgrp = threadIdx.x / (T::kT / E);
     EpiloguePrefetch pre = {0.0f, 1.0f};
     if constexpr (kAmax) pre = prefetch_epilogue(io, kModeDelayed);
     uint32_t m_run = 0;
-    // persistent over tiles: the number of blocks (and so of reduction atomics) stays ~2 per CU
+    // persistent over tiles: the number of blocks (and so of reduction atomics) stays small
     for (int64_t tile_id = blockIdx.x; tile_id < tiles; tile_id += gridDim.x) {
-    const int64_t row0 = (tile_id / tiles_c) * kTile, col0 = (tile_id % tiles_c) * kTile;
+        const int64_t row0 = (tile_id / tiles_c) * T::kT, col0 = (tile_id % tiles_c) * T::kT;
+        const int64_t c = col0 + cgrp * E;
+        float v[4][E];
+        uint32_t m[4];
+        if (c + E <= cols) {
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int r = rsub + 32 * it;
-        const int64_t g = (row0 + r) * cols + col0 + cchunk * 16;
-        float v[16];
-        uint32_t m16;
-        L::template load16<kAmax>(x + g, v, m16);
-        if constexpr (kAmax) m_run = m16 > m_run ? m16 : m_run;
-        const u4 q = encode16<F>(v, scale, degen || L::has_nan(m16));
-        if (out) __builtin_nontemporal_store(q, reinterpret_cast<u4*>(out + g));
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        const int rsw = r ^ (cchunk << 4);  // swizzled row position inside a column
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = row0 + rgrp * 4 + r;
+                L::template load<E, kAmax>(x + (row < rows ? row : rows - 1) * cols + c, v[r], m[r]);
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
-            tile[(cchunk * 16 + j) * kTile + rsw] = (uint8_t)(w[j >> 2] >> (8 * (j & 3)));
-    }
-    __syncthreads();
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = row0 + rgrp * 4 + r;
+                const typename ElemOf<S>::type* p = x + (row < rows ? row : rows - 1) * cols;
+                m[r] = 0;
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int c = rsub + 32 * it;
-        const int pos = (rchunk ^ (c >> 4)) << 4;
-        const u4 q = *reinterpret_cast<const u4*>(&tile[c * kTile + pos]);
-        __builtin_nontemporal_store(q, reinterpret_cast<u4*>(out_t + (col0 + c) * rows + row0 + rchunk * 16));
-    }
-    __syncthreads();  // the tile buffer is reused by the next trip
+                for (int e = 0; e < E; ++e) {
+                    uint32_t me;
+                    v[r][e] = L::load1(p + (c + e < cols ? c + e : cols - 1), me);
+                    m[r] = me > m[r] ? me : m[r];
+                }
+            }
+        }
+        uint32_t w[4][E / 4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t row = row0 + rgrp * 4 + r;
+            if constexpr (kAmax) m_run = m[r] > m_run ? m[r] : m_run;
+            encode<F, E>(v[r], scale, degen || L::has_nan(m[r]), w[r]);
+            if (out && row < rows && c < cols) store_row_bytes<E>(out + row * cols + c, w[r], cols - c);
+        }
+        deposit_block<E>(tile, w, cgrp, rgrp);
+        __syncthreads();
+        emit_columns<E>(tile, out_t, rows, cols, row0, col0);
+        __syncthreads();  // the tile buffer is reused by the next trip
     }
     if constexpr (kAmax) publish_and_finalize<kTileThreads>(L::to_f32_bits(m_run), ws, io, kModeDelayed, pre);
 }
 
-// Any shape: one element per thread step, transposed store.  Used when the tile kernel's
-// 128-multiples / alignment requirements are not met.
-template <typename S, int F, bool kAmax>
-__global__ __launch_bounds__(kThreads) void quant_transpose_scalar_kernel(
-    const typename ElemOf<S>::type* __restrict__ x, int64_t rows, int64_t cols, uint8_t* __restrict__ out,
-    uint8_t* __restrict__ out_t, const float* __restrict__ scale_ptr, Workspace* ws, ScalarIO io) {
-    typedef Src<S> L;
-    const float scale = *scale_ptr;
-    const int64_t n = rows * cols;
-    const int64_t stride = (int64_t)gridDim.x * kThreads;
-    EpiloguePrefetch pre = {0.0f, 1.0f};
-    if constexpr (kAmax) pre = prefetch_epilogue(io, kModeDelayed);
-    uint32_t m_run = 0;
-    for (int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x; j < n; j += stride) {
-        uint32_t m;
-        const float xv = L::load1(x + j, m);
-        if constexpr (kAmax) m_run = m > m_run ? m : m_run;
-        const uint8_t b = encode1<F>(xv, scale);
-        if (out) out[j] = b;
-        const int64_t r = j / cols, c = j % cols;
-        out_t[c * rows + r] = b;
+// [rows, cols] bytes -> [cols, rows]
+template <int E>
+__global__ __launch_bounds__(kTileThreads) void transpose_kernel(const uint8_t* __restrict__ in, int64_t rows, int64_t cols,
+                                                                 uint8_t* __restrict__ out) {
+    typedef Tile<E> T;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[T::kT * T::kPitch];
+    const int64_t tiles_c = (cols + T::kT - 1) / T::kT;
+    const int64_t tiles = ((rows + T::kT - 1) / T::kT) * tiles_c;
+    const int cgrp = threadIdx.x % (T::kT / E), rgrp = threadIdx.x / (T::kT / E);
+    for (int64_t tile_id = blockIdx.x; tile_id < tiles; tile_id += gridDim.x) {
+        const int64_t row0 = (tile_id / tiles_c) * T::kT, col0 = (tile_id % tiles_c) * T::kT;
+        const int64_t c = col0 + cgrp * E;
+        uint32_t w[4][E / 4];
+        typedef uint32_t win __attribute__((ext_vector_type(E / 4)));
+        typedef win win_any __attribute__((aligned(1)));
+        if (c + E <= cols) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = row0 + rgrp * 4 + r;
+                const win v = *reinterpret_cast<const win_any*>(in + (row < rows ? row : rows - 1) * cols + c);
+#pragma unroll
+                for (int q = 0; q < E / 4; ++q) w[r][q] = v[q];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = row0 + rgrp * 4 + r;
+                const uint8_t* p = in + (row < rows ? row : rows - 1) * cols;
+#pragma unroll
+                for (int q = 0; q < E / 4; ++q) w[r][q] = 0;
+#pragma unroll
+                for (int e = 0; e < E; ++e) w[r][e >> 2] |= (uint32_t)p[c + e < cols ? c + e : cols - 1] << (8 * (e & 3));
+            }
+        }
+        deposit_block<E>(tile, w, cgrp, rgrp);
+        __syncthreads();
+        emit_columns<E>(tile, out, rows, cols, row0, col0);
+        __syncthreads();
     }
-    if constexpr (kAmax) publish_and_finalize<kThreads>(L::to_f32_bits(m_run), ws, io, kModeDelayed, pre);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -616,20 +750,6 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __rest
         store_dequant1<OUT>(out, j, decode1<F>(in[j]) * inv);
 }
 
-// Byte transpose through a 64x64 LDS tile (pitch 65 breaks the bank pattern); any shape.
-__global__ __launch_bounds__(kThreads) void transpose_kernel(const uint8_t* __restrict__ in, int64_t rows, int64_t cols,
-                                                             uint8_t* __restrict__ out) {
-    __shared__ uint8_t tile[64][65];
-    const int64_t tiles_c = (cols + 63) / 64;
-    const int64_t r0 = (blockIdx.x / tiles_c) * 64, c0 = (blockIdx.x % tiles_c) * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4)
-        if (r0 + r < rows && c0 + tx < cols) tile[r][tx] = in[(r0 + r) * cols + c0 + tx];
-    __syncthreads();
-    for (int c = ty; c < 64; c += 4)
-        if (c0 + c < cols && r0 + tx < rows) out[(c0 + c) * rows + r0 + tx] = tile[tx][c];
-}
-
 // ---------------------------------------------------------------------------------------------
 // Bandwidth yardsticks: the access pattern of the flat quantise kernel (one 1024-thread workgroup per CU, two
 // 16-element groups per lane and trip, 128-bit non-temporal accesses) with the arithmetic and the reduction taken
@@ -703,30 +823,35 @@ static int launch_flat(int mode, const void* x, int64_t n, bool vec_ok, uint8_t*
     return check_launch();
 }
 
-template <typename S, int F>
-static int launch_transpose(bool with_amax, const void* x, int64_t rows, int64_t cols, bool tile_ok, uint8_t* out,
-                            uint8_t* out_t, const float* scale_ptr, Workspace* ws, const ScalarIO& io, hipStream_t st) {
+// Columns per thread (16: 128-wide tiles, 4: 64-wide) of the kernels that turn tiles around, and their tile count.
+// 128-wide from one tile per CU on.  us, 128 / 64 wide: bf16 delayed step with transposed copy 2048 x 2048 (256 tiles)
+// 8.7 / 10.6, 4096 x 4096 18 / 34; transpose of 4096 x 4096 bytes 6.0 / 9.2; below one tile per CU fp32 cast of
+// 1021 x 1024 9.7 / 4.6, 1536 x 1584 7.2 / 5.4.
+static int tile_edge(int64_t rows, int64_t cols, int64_t* tiles) {
+    const int64_t t128 = ((rows + 127) / 128) * ((cols + 127) / 128);
+    if (t128 >= cu_count()) {
+        *tiles = t128;
+        return 16;
+    }
+    *tiles = ((rows + 63) / 64) * ((cols + 63) / 64);
+    return 4;
+}
+
+template <typename S, int F, bool kAmax>
+static int launch_transpose(const void* x, int64_t rows, int64_t cols, uint8_t* out, uint8_t* out_t, const float* scale_ptr,
+                            Workspace* ws, const ScalarIO& io, hipStream_t st) {
     typedef typename ElemOf<S>::type E;
     const E* xp = static_cast<const E*>(x);
-    if (tile_ok) {
-        const int64_t tiles = (rows / kTile) * (cols / kTile);
-        const int64_t cap = (int64_t)cu_count() * (with_amax ? 2 : 8);
-        const int tgrid = (int)(tiles < cap ? tiles : cap);
-        if (with_amax)
-            hipLaunchKernelGGL((quant_transpose_kernel<S, F, true>), dim3(tgrid), dim3(kTileThreads), 0, st, xp, rows,
-                               cols, out, out_t, scale_ptr, ws, io);
-        else
-            hipLaunchKernelGGL((quant_transpose_kernel<S, F, false>), dim3(tgrid), dim3(kTileThreads), 0, st, xp, rows,
-                               cols, out, out_t, scale_ptr, ws, io);
-    } else {
-        const int grid = grid_for(rows * cols);
-        if (with_amax)
-            hipLaunchKernelGGL((quant_transpose_scalar_kernel<S, F, true>), dim3(grid), dim3(kThreads), 0, st, xp, rows,
-                               cols, out, out_t, scale_ptr, ws, io);
-        else
-            hipLaunchKernelGGL((quant_transpose_scalar_kernel<S, F, false>), dim3(grid), dim3(kThreads), 0, st, xp, rows,
-                               cols, out, out_t, scale_ptr, ws, io);
-    }
+    int64_t tiles;
+    const int e = tile_edge(rows, cols, &tiles);
+    const int64_t cap = (int64_t)cu_count() * (kAmax ? 3 : 8);   // (kAmax: every block is an atomic at the end)
+    const int grid = (int)(tiles < cap ? tiles : cap);
+    if (e == 16)
+        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
+                           out_t, scale_ptr, ws, io);
+    else
+        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 4>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
+                           out_t, scale_ptr, ws, io);
     return check_launch();
 }
 
@@ -738,11 +863,13 @@ static int dispatch_fmt_flat(int fmt, int mode, const void* x, int64_t n, bool v
 }
 
 template <typename S>
-static int dispatch_fmt_tr(int fmt, bool with_amax, const void* x, int64_t rows, int64_t cols, bool tile_ok,
-                           uint8_t* out, uint8_t* out_t, const float* scale_ptr, Workspace* ws, const ScalarIO& io,
-                           hipStream_t st) {
-    return fmt == kE4M3 ? launch_transpose<S, kE4M3>(with_amax, x, rows, cols, tile_ok, out, out_t, scale_ptr, ws, io, st)
-                        : launch_transpose<S, kE5M2>(with_amax, x, rows, cols, tile_ok, out, out_t, scale_ptr, ws, io, st);
+static int dispatch_fmt_tr(int fmt, bool with_amax, const void* x, int64_t rows, int64_t cols, uint8_t* out, uint8_t* out_t,
+                           const float* scale_ptr, Workspace* ws, const ScalarIO& io, hipStream_t st) {
+    if (fmt == kE4M3)
+        return with_amax ? launch_transpose<S, kE4M3, true>(x, rows, cols, out, out_t, scale_ptr, ws, io, st)
+                         : launch_transpose<S, kE4M3, false>(x, rows, cols, out, out_t, scale_ptr, ws, io, st);
+    return with_amax ? launch_transpose<S, kE5M2, true>(x, rows, cols, out, out_t, scale_ptr, ws, io, st)
+                     : launch_transpose<S, kE5M2, false>(x, rows, cols, out, out_t, scale_ptr, ws, io, st);
 }
 
 static bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
@@ -753,13 +880,11 @@ int run_quant(int mode, const void* x, int x_dtype, int64_t rows, int64_t cols, 
     clear_stale_error();
     const int64_t n = rows * cols;
     if (mode != kModeAmaxOnly && out_t != nullptr) {
-        const bool tile_ok = rows % kTile == 0 && cols % kTile == 0 && aligned(x, 16) && aligned(out_t, 16) &&
-                             (out == nullptr || aligned(out, 16));
         const bool with_amax = mode == kModeDelayed;
         switch (x_dtype) {
-            case NTFP8_F32: return dispatch_fmt_tr<float>(fmt, with_amax, x, rows, cols, tile_ok, out, out_t, scale_ptr, ws, io, st);
-            case NTFP8_F16: return dispatch_fmt_tr<f16_tag>(fmt, with_amax, x, rows, cols, tile_ok, out, out_t, scale_ptr, ws, io, st);
-            default: return dispatch_fmt_tr<bf16_tag>(fmt, with_amax, x, rows, cols, tile_ok, out, out_t, scale_ptr, ws, io, st);
+            case NTFP8_F32: return dispatch_fmt_tr<float>(fmt, with_amax, x, rows, cols, out, out_t, scale_ptr, ws, io, st);
+            case NTFP8_F16: return dispatch_fmt_tr<f16_tag>(fmt, with_amax, x, rows, cols, out, out_t, scale_ptr, ws, io, st);
+            default: return dispatch_fmt_tr<bf16_tag>(fmt, with_amax, x, rows, cols, out, out_t, scale_ptr, ws, io, st);
         }
     }
     const bool vec_ok = aligned(x, 16) && (mode == kModeAmaxOnly || aligned(out, 16));
@@ -912,10 +1037,14 @@ int run_dequant(const void* in, int fmt, const float* scale, int is_inverse, int
 
 int run_transpose(const void* in, int64_t rows, int64_t cols, void* out, hipStream_t st) {
     clear_stale_error();
-    const int64_t tiles = ((rows + 63) / 64) * ((cols + 63) / 64);
-    if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
-    hipLaunchKernelGGL(transpose_kernel, dim3((int)tiles), dim3(kThreads), 0, st, static_cast<const uint8_t*>(in), rows,
-                       cols, static_cast<uint8_t*>(out));
+    int64_t tiles;
+    const int e = tile_edge(rows, cols, &tiles);
+    const int64_t cap = (int64_t)cu_count() * 8;
+    const int grid = (int)(tiles < cap ? tiles : cap);
+    const uint8_t* p = static_cast<const uint8_t*>(in);
+    uint8_t* o = static_cast<uint8_t*>(out);
+    if (e == 16) hipLaunchKernelGGL((transpose_kernel<16>), dim3(grid), dim3(kTileThreads), 0, st, p, rows, cols, o);
+    else hipLaunchKernelGGL((transpose_kernel<4>), dim3(grid), dim3(kTileThreads), 0, st, p, rows, cols, o);
     return check_launch();
 }
 
