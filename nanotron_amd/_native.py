@@ -82,6 +82,13 @@ for _name, (_res, _args) in SIGNATURES.items():
 
 lib = _lib
 
+# the host side of the hot calls (csrc/hostcall.cpp): allocation, descriptors and the C-ABI call in one step
+try:
+    from nanotron_amd import _hostcall as host
+except ImportError as e:
+    raise ImportError(f"nanotron_amd/_hostcall.so is missing or does not match this torch ({e}): build it first "
+                      "(python -m nanotron_amd.build)") from e
+
 
 def strerror(code: int) -> str:
     return _lib.ntfp8_strerror(code).decode()
@@ -95,6 +102,9 @@ def check(code: int, what: str) -> None:
             _workspaces.clear()
             _pools.clear()
         raise RuntimeError(f"{what} failed: {strerror(code)} (code {code})")
+
+
+host.set_check(check)
 
 
 def version() -> int:

@@ -6,6 +6,8 @@
 The libraries are built in-tree so that they travel with the source tree to the GPU box; nothing is
 JIT-compiled at import time.
 
+nanotron_amd/_hostcall.so is a CPython extension on top of libntfp8.so: the host side of the hot calls.
+
 Profiling libraries (nanotron_amd/profiling/, loaded by nothing but the benchmark's wg-timeline workload):
 libntfp8_stamps.so is the product library with per-workgroup time stamps compiled into the GEMM kernel
 (-DNTFP8_STAMPS); the libntfp8_<experiment>.so beside it carry the same stamps and one timing experiment each on the
@@ -21,6 +23,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libntfp8.so")
+HOSTCALL = os.path.join(HERE, "_hostcall.so")
 PROFILING_DIR = os.path.join(HERE, "profiling")
 LIB_STAMPS = os.path.join(PROFILING_DIR, "libntfp8_stamps.so")
 SOURCES = ["quant.hip", "gemm.hip", "capi.hip"]
@@ -69,6 +72,25 @@ def _link(out: str, objs) -> None:
     subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *objs])
 
 
+def _build_hostcall() -> str:
+    """The host extension: plain C++ against torch's headers, linked to the libntfp8.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    inc = [f"-I{p}" for p in [*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]]
+    libs = [f"-L{p}" for p in library_paths()]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "hostcall.cpp"),
+           "-o", HOSTCALL, *libs, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python", f"-L{HERE}", "-l:libntfp8.so",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for hostcall.cpp:\n{r.stderr}")
+    return HOSTCALL
+
+
 def build(verbose: bool = True, profiling: bool = False) -> str:
     jobs = [(s, [], "") for s in SOURCES]
     if profiling:
@@ -79,7 +101,7 @@ def build(verbose: bool = True, profiling: bool = False) -> str:
         objs = list(ex.map(_compile, jobs))
     plain = objs[:len(SOURCES)]
     _link(LIB, plain)
-    built = [LIB]
+    built = [LIB, _build_hostcall()]
     if profiling:
         os.makedirs(PROFILING_DIR, exist_ok=True)
         for obj, out in zip(objs[len(SOURCES):], [LIB_STAMPS] + [experiment_lib(n) for n in EXPERIMENTS]):

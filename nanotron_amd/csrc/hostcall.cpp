@@ -1,0 +1,356 @@
+// Host side of the hot calls: output allocation, descriptors and the C-ABI call in one step.
+//
+// A small layer's training step is bound by the host, not by the GPU (128 x 128 x 128: 39 us of kernels in a step of
+// 340 us), and most of that is Python: every attribute of an FP8Tensor passes through __torch_function__ (1.1 us, the
+// shape 2.4 us), every allocation and every view is a Python call, a descriptor is filled field by field.  The
+// functions below take tensors as they are (subclasses unwrapped without dispatch), allocate below autograd, and call
+// libntfp8.so's C entry points.  They are thin: no arithmetic and no kernel lives here.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <unordered_map>
+
+#include "../../include/ntfp8.h"
+
+namespace {
+
+PyObject* g_check = nullptr;   // nanotron_amd._native.check: raises RuntimeError, drops the workspaces after a failed launch
+
+struct Stop {};   // a Python error is set
+
+[[noreturn]] void stop(PyObject* type, const char* msg) {
+    PyErr_SetString(type, msg);
+    throw Stop{};
+}
+void require(bool ok, const char* msg) {
+    if (!ok) stop(PyExc_AssertionError, msg);
+}
+
+// Reduction workspaces, one per (device, stream), zero between launches.  Guarded by the GIL; the table is never
+// destroyed (its tensors must not outlive the runtime's teardown).
+using Key = std::pair<int, void*>;
+struct KeyHash {
+    size_t operator()(const Key& k) const { return reinterpret_cast<size_t>(k.second) * 31u + (size_t)k.first; }
+};
+std::unordered_map<Key, at::Tensor, KeyHash>& workspaces() {
+    static auto* m = new std::unordered_map<Key, at::Tensor, KeyHash>();
+    return *m;
+}
+
+void call(int rc, const char* what) {
+    if (rc == NTFP8_OK) return;
+    if (rc == NTFP8_ERR_LAUNCH) workspaces().clear();
+    PyObject* r = PyObject_CallFunction(g_check, "is", rc, what);
+    Py_XDECREF(r);
+    if (r != nullptr) stop(PyExc_RuntimeError, what);
+    throw Stop{};
+}
+
+const at::Tensor& tensor(PyObject* o) {
+    if (!THPVariable_Check(o)) stop(PyExc_TypeError, "a tensor is expected");
+    return THPVariable_Unpack(o);
+}
+bool none(PyObject* o) { return o == Py_None || o == nullptr; }
+long number(PyObject* o) {
+    const long v = PyLong_AsLong(o);
+    if (v == -1 && PyErr_Occurred()) throw Stop{};
+    return v;
+}
+bool truth(PyObject* o) {
+    if (o == Py_True) return true;
+    if (o == Py_False || o == Py_None) return false;
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw Stop{};
+    return v != 0;
+}
+PyObject* wrap(at::Tensor t) {
+    PyObject* o = THPVariable_Wrap(std::move(t));
+    if (o == nullptr) throw Stop{};
+    return o;
+}
+PyObject* wrap_or_none(at::Tensor t) {
+    if (t.defined()) return wrap(std::move(t));
+    Py_RETURN_NONE;
+}
+
+void* stream_of(const at::Tensor& t) {
+    return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream());
+}
+void* workspace_of(const at::Tensor& t, void* stream) {
+    at::Tensor& w = workspaces()[Key{(int)t.get_device(), stream}];
+    if (!w.defined()) w = at::zeros({NTFP8_WORKSPACE_BYTES / 4}, t.options().dtype(at::kInt));
+    return w.data_ptr();
+}
+
+int code_of(at::ScalarType t) {   // NTFP8_F32 / F16 / BF16, or -1
+    return t == at::kFloat ? NTFP8_F32 : t == at::kHalf ? NTFP8_F16 : t == at::kBFloat16 ? NTFP8_BF16 : -1;
+}
+at::ScalarType type_of(long code) {
+    return code == NTFP8_F32 ? at::kFloat : code == NTFP8_F16 ? at::kHalf : code == NTFP8_BF16 ? at::kBFloat16 : at::kByte;
+}
+at::Tensor bytes_like(const at::Tensor& x, at::IntArrayRef sizes) {
+    return at::empty(sizes, at::TensorOptions().dtype(at::kByte).device(x.device()));
+}
+at::Tensor dense(const at::Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+
+// [amax, scale used] of a quantisation: one allocation, and its two elements as 0-dim tensors
+struct Scalars {
+    at::Tensor both;
+    float* p;
+    explicit Scalars(const at::Tensor& like)
+        : both(at::empty({2}, at::TensorOptions().dtype(at::kFloat).device(like.device()))), p(static_cast<float*>(both.data_ptr())) {}
+    at::Tensor element(int64_t i) const {
+        at::Tensor v = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(both.storage()), both.key_set(), both.dtype());
+        v.unsafeGetTensorImpl()->set_sizes_and_strides(c10::IntArrayRef{}, c10::IntArrayRef{}, i);
+        return v;
+    }
+};
+
+void rows_cols(const at::Tensor& x, int64_t* rows, int64_t* cols) {
+    *cols = x.dim() >= 2 ? x.size(-1) : x.numel();
+    *rows = *cols ? x.numel() / *cols : 0;
+}
+
+PyObject* quantised(at::Tensor out, at::Tensor out_t, const Scalars& s) {
+    return Py_BuildValue("(NNNN)", wrap(std::move(out)), wrap_or_none(std::move(out_t)), wrap(s.element(0)), wrap(s.element(1)));
+}
+
+// quantize(x, fmt, margin, state | None, flag | None, history_len, with_transpose) -> (bytes, bytes^T | None, amax, scale)
+// state None: current scaling; flag given: the role may not hold a scale yet; otherwise the fused delayed-scaling step
+PyObject* quantize(PyObject* const* a) {
+    const at::Tensor x = dense(tensor(a[0]));
+    const int fmt = (int)number(a[1]), margin = (int)number(a[2]), hist = (int)number(a[5]);
+    const bool with_t = truth(a[6]);
+    int64_t rows, cols;
+    rows_cols(x, &rows, &cols);
+    require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    at::Tensor out = bytes_like(x, x.sizes()), out_t;
+    if (with_t) out_t = bytes_like(x, {cols, rows});
+    const Scalars s(x);
+    void* st = stream_of(x);
+    void* ws = workspace_of(x, st);
+    void* tp = with_t ? out_t.data_ptr() : nullptr;
+    const int xd = code_of(x.scalar_type());
+    if (none(a[3])) {
+        call(ntfp8_quantize_current(x.data_ptr(), xd, rows, cols, fmt, margin, s.p, s.p + 1, out.data_ptr(), tp, nullptr, 0, nullptr, ws, st),
+             "ntfp8_quantize_current");
+    } else {
+        float* buf = static_cast<float*>(tensor(a[3]).data_ptr());   // [scale, hist[0..H-1]]
+        if (!none(a[4]))
+            call(ntfp8_quantize_first_use(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist,
+                                          static_cast<float*>(tensor(a[4]).data_ptr()), s.p, s.p + 1, out.data_ptr(), tp, ws, st),
+                 "ntfp8_quantize_first_use");
+        else
+            call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
+                 "ntfp8_quantize_delayed");
+    }
+    return quantised(std::move(out), std::move(out_t), s);
+}
+
+// One GEMM problem: (a, fmt_a, scale_a, b, fmt_b, scale_b, out_code, accumulate_into | None, b_transposed, bias | None,
+// a_transposed); fills the descriptor, keeps what it points to alive, returns the output
+constexpr int kProblem = 11;
+struct Problem {
+    at::Tensor a, b, bias, out;
+};
+void fill(PyObject* const* p, ntfp8_gemm_desc* d, Problem* k, bool fp8_out = false) {
+    k->a = dense(tensor(p[0]));
+    k->b = dense(tensor(p[3]));
+    const bool bt = truth(p[8]), at_ = truth(p[10]);
+    require(k->a.dim() == 2 && k->b.dim() == 2 && k->a.size(at_ ? 0 : 1) == k->b.size(bt ? 0 : 1), "GEMM operands do not fit together");
+    require(k->a.is_cuda() && k->a.device() == k->b.device(), "GEMM operands must be on one CUDA device");
+    const int64_t M = k->a.size(at_ ? 1 : 0), K = k->a.size(at_ ? 0 : 1), N = k->b.size(bt ? 1 : 0);
+    const long code = number(p[6]);
+    d->accumulate = 0;
+    if (!none(p[7])) {
+        k->out = tensor(p[7]);
+        require(k->out.scalar_type() == at::kFloat && k->out.dim() == 2 && k->out.size(0) == M && k->out.size(1) == N &&
+                    k->out.is_contiguous() && k->out.device() == k->a.device(),
+                "accumulate_into must be a contiguous fp32 tensor of the result's shape");
+        d->accumulate = 1;
+    } else {
+        k->out = at::empty({M, N}, at::TensorOptions().dtype(type_of(code)).device(k->a.device()));
+    }
+    if (!none(p[9])) {
+        k->bias = dense(tensor(p[9]));
+        require(k->bias.dim() == 1 && k->bias.size(0) == N && k->bias.device() == k->a.device(), "bias must hold one value per output column");
+        const int bc = code_of(k->bias.scalar_type());
+        require(bc >= 0, "unsupported bias dtype");
+        require(!fp8_out || !bt, "no bias together with a transposed B operand");
+        d->bias = k->bias.data_ptr();
+        d->bias_dtype = bc;
+    }
+    d->A = k->a.data_ptr();
+    d->B = k->b.data_ptr();
+    d->D = k->out.data_ptr();
+    d->fmt_a = (int)number(p[1]);
+    d->fmt_b = (int)number(p[4]);
+    d->scale_a = static_cast<const float*>(tensor(p[2]).data_ptr());
+    d->scale_b = static_cast<const float*>(tensor(p[5]).data_ptr());
+    d->d_dtype = d->accumulate ? NTFP8_F32 : (int)code;
+    d->M = M;
+    d->N = N;
+    d->K = K;
+    d->b_transposed = bt;
+    d->a_transposed = at_;
+}
+
+// gemm(problem fields...) -> output
+PyObject* gemm(PyObject* const* p) {
+    ntfp8_gemm_desc d = {};
+    Problem k;
+    fill(p, &d, &k);
+    call(ntfp8_gemm_batch(&d, 1, stream_of(k.a)), "ntfp8_gemm_batch");
+    return wrap(std::move(k.out));
+}
+
+// gemm_batch([problem, ...]) -> [output, ...], one library call
+PyObject* gemm_batch(PyObject* const* args) {
+    PyObject* const list = args[0];
+    if (!PyList_Check(list)) stop(PyExc_TypeError, "a list of problems is expected");
+    const Py_ssize_t n = PyList_GET_SIZE(list);
+    require(n >= 1 && n <= NTFP8_MAX_BATCH, "between 1 and 64 problems");
+    std::vector<ntfp8_gemm_desc> d(n);
+    std::vector<Problem> k(n);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        PyObject* t = PyList_GET_ITEM(list, i);
+        if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != kProblem) stop(PyExc_TypeError, "a problem is a tuple of 11");
+        d[i] = {};
+        fill(&PyTuple_GET_ITEM(t, 0), &d[i], &k[i]);
+        require(k[i].a.device() == k[0].a.device(), "all problems of a batch are on one device");
+    }
+    call(ntfp8_gemm_batch(d.data(), (int)n, stream_of(k[0].a)), "ntfp8_gemm_batch");
+    PyObject* out = PyList_New(n);
+    if (out == nullptr) throw Stop{};
+    for (Py_ssize_t i = 0; i < n; ++i) PyList_SET_ITEM(out, i, wrap(std::move(k[i].out)));
+    return out;
+}
+
+// gemm_fp8(problem fields..., state, history_len, margin, fmt, with_transpose) -> (bytes, bytes^T | None, amax, scale):
+// the epilogue casts with the held scale, a one-wave kernel behind it does the bookkeeping
+PyObject* gemm_fp8(PyObject* const* p) {
+    ntfp8_gemm_desc d = {};
+    Problem k;
+    fill(p, &d, &k, true);
+    const at::Tensor& state = tensor(p[kProblem]);
+    const int hist = (int)number(p[kProblem + 1]), margin = (int)number(p[kProblem + 2]), fmt = (int)number(p[kProblem + 3]);
+    require(state.device() == k.a.device(), "delayed-scaling state on another device");
+    at::Tensor out_t;
+    if (truth(p[kProblem + 4])) out_t = bytes_like(k.a, {d.N, d.M});
+    const Scalars s(k.a);
+    void* st = stream_of(k.a);
+    void* ws = workspace_of(k.a, st);
+    float* buf = static_cast<float*>(state.data_ptr());
+    d.scale_d = buf;
+    d.D_t = out_t.defined() ? out_t.data_ptr() : nullptr;
+    d.amax_workspace = ws;
+    call(ntfp8_gemm_batch(&d, 1, st), "ntfp8_gemm_batch");
+    call(ntfp8_amax_finalize(ws, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, st), "ntfp8_amax_finalize");
+    return quantised(std::move(k.out), std::move(out_t), s);
+}
+
+// cast(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None)
+PyObject* cast(PyObject* const* a) {
+    const at::Tensor x = dense(tensor(a[0]));
+    const int fmt = (int)number(a[2]);
+    int64_t rows, cols;
+    rows_cols(x, &rows, &cols);
+    at::Tensor out = bytes_like(x, x.sizes()), out_t;
+    const bool with_t = truth(a[3]);
+    require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    if (with_t) out_t = bytes_like(x, {cols, rows});
+    call(ntfp8_cast_to_fp8(x.data_ptr(), code_of(x.scalar_type()), rows, cols, static_cast<const float*>(tensor(a[1]).data_ptr()), fmt,
+                           out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
+         "ntfp8_cast_to_fp8");
+    return Py_BuildValue("(NN)", wrap(std::move(out)), wrap_or_none(std::move(out_t)));
+}
+
+// dequantize(bytes, fmt, scale, out_code, inverse) -> tensor
+PyObject* dequantize(PyObject* const* a) {
+    const at::Tensor q = dense(tensor(a[0]));
+    const int fmt = (int)number(a[1]);
+    const float* scale = static_cast<const float*>(tensor(a[2]).data_ptr());
+    const long code = number(a[3]);
+    at::Tensor out = at::empty(q.sizes(), at::TensorOptions().dtype(type_of(code)).device(q.device()));
+    if (q.numel()) {
+        if (truth(a[4])) call(ntfp8_cast_from_fp8_scale_inv(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "cast_from_fp8");
+        else call(ntfp8_cast_from_fp8(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "ntfp8_cast_from_fp8");
+    }
+    return wrap(std::move(out));
+}
+
+// transpose([rows, cols] bytes) -> contiguous [cols, rows] bytes
+PyObject* transpose(PyObject* const* a) {
+    const at::Tensor q = dense(tensor(a[0]));
+    require(q.dim() == 2, "a 2-D tensor is expected");
+    at::Tensor out = bytes_like(q, {q.size(1), q.size(0)});
+    if (q.numel()) call(ntfp8_transpose(q.data_ptr(), q.size(0), q.size(1), out.data_ptr(), stream_of(q)), "ntfp8_transpose");
+    return wrap(std::move(out));
+}
+
+// Whether the library reads B [K, N] (and, in the second form, A [K, M] as well) from its transpose: include/ntfp8.h
+bool reads_b(int64_t M, int64_t N, int64_t K) {
+    return N % 16 == 0 && K % 16 == 0 && M > 128 && N > 128 && K >= 256 && (M + 256) * K < (1LL << 31) && (N + 256) * K < (1LL << 31);
+}
+PyObject* b_transposed_supported(PyObject* const* a) { return PyBool_FromLong(reads_b(number(a[0]), number(a[1]), number(a[2]))); }
+
+// operand_form(mat_a, a_has_copy, transpose_a, mat_b, b_has_copy, transpose_b, accumulate_into | None, allow_bt, read_b,
+// read_a) -> bits: 1 the library's A is mat_b's transposed copy, 2 its B is mat_a's transposed copy, 4 B read as its
+// transpose, 8 A read as its transpose
+PyObject* operand_form(PyObject* const* p) {
+    const at::Tensor &a = tensor(p[0]), &b = tensor(p[3]);
+    require(a.is_cuda() && b.is_cuda(), "The tensors must be on a CUDA device in order to use the FP8 kernel!!");
+    const bool ta = truth(p[2]), tb = truth(p[5]);
+    if (ta) return PyLong_FromLong(tb ? 1 : 0);
+    const bool read_b = truth(p[7]) && truth(p[8]), read_a = truth(p[9]);
+    auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };   // 16-byte loads / stores
+    const bool plain_a = read_b && !truth(p[1]) && a.dim() == 2 && a.is_contiguous() && aligned(a) && aligned(b) && (none(p[6]) || aligned(tensor(p[6])));
+    if (tb) {
+        // D[cols of mat_b, cols of mat_a], reduction over the rows of both
+        if (plain_a && read_a && !truth(p[4]) && b.dim() == 2 && b.is_contiguous() && b.size(1) % 16 == 0 && reads_b(b.size(1), a.size(1), a.size(0)))
+            return PyLong_FromLong(4 | 8);
+        // mat_b's copy is a fresh allocation or was one: aligned
+        if (plain_a && b.dim() == 2 && reads_b(b.size(1), a.size(1), a.size(0))) return PyLong_FromLong(1 | 4);
+        return PyLong_FromLong(1 | 2);
+    }
+    if (plain_a && b.dim() == 2 && reads_b(b.size(0), a.size(1), a.size(0))) return PyLong_FromLong(4);
+    return PyLong_FromLong(2);
+}
+
+PyObject* set_check(PyObject* const* a) {
+    Py_INCREF(a[0]);
+    Py_XSETREF(g_check, a[0]);
+    Py_RETURN_NONE;
+}
+
+// The common frame: argument count, autograd left out, C++ errors turned into Python ones
+template <PyObject* (*F)(PyObject* const*), int N>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "%d arguments are expected, got %zd", N, n);
+        return nullptr;
+    }
+    at::AutoDispatchBelowADInplaceOrView guard;
+    try {
+        return F(args);
+    } catch (const Stop&) {
+        return nullptr;
+    }
+    END_HANDLE_TH_ERRORS
+}
+
+#define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 5),
+                         NT_METHOD(cast, 4), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
+                         NT_METHOD(operand_form, 10), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__hostcall(void) { return PyModule_Create(&module); }

@@ -188,8 +188,9 @@ class FP8Linear(nn.Linear):
 
     def forward(self, input: Union[FP8Tensor, torch.Tensor]) -> torch.Tensor:
         # fp8 kernels only when both input and weight are on the GPU (linear.py:53-54)
-        if input.device == torch.device("cpu") or self.weight.device == torch.device("cpu"):
-            return F.linear(input, self.weight, self.bias)
+        weight = self.weight
+        if not input.is_cuda or not weight.is_cuda:
+            return F.linear(input, weight, self.bias)
 
         if self._weight_ready is not None:  # weight re-quantisation queued on another stream
             torch.cuda.current_stream(input.device).wait_event(self._weight_ready)
@@ -212,7 +213,7 @@ class FP8Linear(nn.Linear):
             box = getattr(handle, "_grad_box", None)
             if box is not None:
                 box.consumers += 1
-        output, aux = _FP8Matmul.apply(input, self.weight, self.fp8_meta, phony, self, self.bias, handle)
+        output, aux = _FP8Matmul.apply(input, weight, self.fp8_meta, phony, self, self.bias, handle)
         if isinstance(self.out_dtype, DTypes):
             output._grad_handle = aux
             aux._grad_box = self._grad_box   # made by this forward: where a consuming layer leaves an fp8 gradient
@@ -238,18 +239,21 @@ class _FP8Matmul(torch.autograd.Function):
     for.  So a chain FP8Linear(out_dtype=E4M3) -> FP8Linear trains without the activation ever leaving fp8."""
 
     @staticmethod
-    @torch.no_grad()
     def forward(ctx, input, weight, fp8_meta, phony: torch.Tensor, module: Optional["FP8Linear"] = None,
                 bias: Optional[torch.Tensor] = None, input_handle: Optional[torch.Tensor] = None):
         scaling = module.scaling if module is not None else None
         update = module.training if module is not None else True   # evaluation passes leave the scaling state alone
         needs_wgrad = weight.requires_grad
-        ctx.in_dtype = input.dtype if type(input) == torch.Tensor else (input_handle.dtype if input_handle is not None else None)
-        ctx.in_shape = input.shape
+        # (attributes of an FP8Tensor are read through its plain tensor: the subclass dispatches every one of them)
+        plain = type(input) is torch.Tensor
+        raw = input if plain else input.as_subclass(torch.Tensor)
+        ctx.in_dtype = input.dtype if plain else (input_handle.dtype if input_handle is not None else None)
+        ctx.in_shape = in_shape = raw.shape
+        ctx.set_materialize_grads(False)   # a missing gradient arrives as None, not as a tensor filled with zeros
         ctx.has_handle = input_handle is not None
         ctx.input_box = getattr(input_handle, "_grad_box", None) if input_handle is not None else None
-        if type(input) == torch.Tensor:
-            x2d = input.reshape(-1, input.shape[-1])
+        if plain:
+            x2d = input if len(in_shape) == 2 else input.reshape(-1, in_shape[-1])
             input = FP8Tensor(x2d, dtype=DTypes.FP8E4M3, state=scaling["input"] if scaling else None,
                               with_transpose=needs_wgrad and needs_transposed_copy(x2d.shape[0], x2d.shape[1], weight.shape[0]),
                               update_state=update)
@@ -280,13 +284,19 @@ class _FP8Matmul(torch.autograd.Function):
             mat_a=weight.data, transpose_a=True, mat_b=input, transpose_b=False, use_split_accumulator=False,
             out_dtype=out_dtype, bias=gemm_bias,
         )
-        if len(ctx.in_shape) != 2:
-            output = output.reshape(*ctx.in_shape[:-1], output.shape[-1])
+        if len(in_shape) != 2:
+            output = output.reshape(*in_shape[:-1], output.shape[-1])
         return output, phony
 
     @staticmethod
-    @torch.no_grad()
     def backward(ctx, grad_output: torch.Tensor, grad_aux: torch.Tensor):
+        if torch.is_grad_enabled():   # create_graph: the fp8 kernels are not differentiated again
+            with torch.no_grad():
+                return _FP8Matmul._backward(ctx, grad_output, grad_aux)
+        return _FP8Matmul._backward(ctx, grad_output, grad_aux)
+
+    @staticmethod
+    def _backward(ctx, grad_output, grad_aux):
         input, weight, bias = ctx.saved_tensors
         module = ctx.module
         scaling = module.scaling if module is not None else None
@@ -310,19 +320,19 @@ class _FP8Matmul(torch.autograd.Function):
         if bias is not None and ctx.needs_input_grad[5]:
             # what autograd does for `output + bias` (linear.py:65): the gradient summed over the tokens (in fp32)
             g_hp = grad_output
-            if type(g_hp) != torch.Tensor:
+            if type(g_hp) is not torch.Tensor:
                 from nanotron_amd.fp8.tensor import convert_tensor_from_fp8
 
                 g_hp = convert_tensor_from_fp8(g_hp, g_hp.fp8_meta, bias.dtype)
             grad_bias = g_hp.reshape(-1, g_hp.shape[-1]).sum(0, dtype=torch.float32).to(bias.dtype)
 
-        if type(grad_output) == torch.Tensor:
-            g2d = grad_output.reshape(-1, grad_output.shape[-1]).contiguous()
+        if type(grad_output) is torch.Tensor:
+            g2d = grad_output if grad_output.dim() == 2 else grad_output.reshape(-1, grad_output.shape[-1])
             # wgrad reduces over the rows of dY: it needs the transposed bytes (kernel.py:44) unless the library reads
             # dY as it is, next to an input it also reads as it is
             x_plain = getattr(input, "_transposed", None) is None
             with_t = weight.requires_grad and not (
-                x_plain and a_transposed_supported(g2d.shape[1], input.shape[1], g2d.shape[0]))
+                x_plain and a_transposed_supported(g2d.shape[1], weight.shape[1], g2d.shape[0]))
             grad_output = FP8Tensor(g2d, dtype=DTypes.FP8E5M2, state=scaling["output_grad"] if scaling else None,
                                     with_transpose=with_t)
         if module is not None and module.keep_quantised_grad:
