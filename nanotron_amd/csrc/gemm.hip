@@ -5,14 +5,17 @@
 // operand), operand tiles staged in XOR-swizzled LDS, descale + one rounding in the epilogue to fp32
 // (optionally added to what is there), bf16, fp16 or fp8 bytes.
 //
-// Three kernels:
+// Kernels:
 //   gemm_nt_big_kernel    (gemm_big.h) 256 x 256 x 128 tiles, 4 waves of 128 x 128 with 16x16x128 MFMAs,
 //                         loads staged through registers, two LDS stages, one barrier per K-tile.  The
 //                         partial last round of tiles over the CUs is cut into 128-row half tiles.
-//   gemm_nt_kernel        128 x 128 x 128 tiles, 4 waves, loads through registers; small shapes and
-//                         operands beyond the 2 GiB reach of a buffer descriptor's 32-bit offsets.
+//   gemm_mid_kernel       (gemm_mid.h) 128 x 128 and 64 x 64 tiles of the same instruction, loads straight into four LDS
+//                         stages: shapes that have too few 256-wide tiles, and operands beyond the 2 GiB reach of a
+//                         buffer descriptor's 32-bit offsets.
 //   gemm_any_kernel       (gemm_any.h) any K and alignment: 64- or 128-wide tiles, fp8 widened to bf16 on its way to
 //                         the matrix cores.
+//   gemm_nt_kernel        128 x 128 x 128 tiles, loads through registers: fp8 outputs whose rows or columns do not come in
+//                         whole words (the other kernels' fp8 epilogue stores nothing smaller).
 #include "gemm_common.h"
 #include "gemm_big.h"
 #include "gemm_any.h"
@@ -24,7 +27,7 @@ namespace ntfp8 {
 constexpr int kBM = 128, kBN = 128;
 constexpr int kGemmThreads = 256;
 
-template <int FA, int FB, int DT, bool kAcc>
+template <int FA, int FB, int DT>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                                void* __restrict__ Dv, const float* __restrict__ scale_a,
                                                                const float* __restrict__ scale_b, int M, int N, int K,
@@ -113,45 +116,87 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __
         add_bias32<2, 2>(acc, alpha, ex.bias, ex.bias_dtype, N, n0 + wn, lane);
         alpha = 1.0f;
     }
-    if constexpr (DT == NTFP8_OUT_E4M3 || DT == NTFP8_OUT_E5M2) {
-        constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
-        const float scale_d = *fp8.scale;
-        const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
-                                                           scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane);
-        publish_amax(amax, fp8.ws);
-    } else {
-        store_wave_tile<DT, kAcc, 2, 2>(acc, Dv, alpha, M, N, m0 + wm, n0 + wn, lane);
-    }
+    constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
+    const float scale_d = *fp8.scale;
+    const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
+                                                       scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane);
+    publish_amax(amax, fp8.ws);
 }
 
 // ---------------------------------------------------------------------------------------------
-enum GemmPath { kPathNone = -1, kPathAny = 0, kPathSmall = 1, kPathBig = 2 };
+enum GemmPath { kPathNone = -1, kPathAny = 0, kPathWords = 1, kPathTiles = 2 };
 
-// which kernel serves a problem
+int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
+
+// operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
+static bool fits32(const GemmDesc& g) {
+    return (int64_t)(g.M + 256) * g.K < (1LL << 31) && (int64_t)(g.N + kBigN) * g.K < (1LL << 31);
+}
+// the 256-wide tiles' pipeline starts with two K-tiles
+static bool big_ok(const GemmDesc& g) { return fits32(g) && g.K >= 2 * kBK; }
+
+// which kernels serve a problem
 static int path_of(const GemmDesc& g) {
     const bool aligned16 = (g.K % 16 == 0) &&
                            ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 &&
                            (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
     if (!aligned16) return g.tb ? kPathNone : kPathAny;
-    // the big kernel addresses its operands with 32-bit buffer offsets and wants enough tiles to matter
-    const bool fits32 = (int64_t)(g.M + 256) * g.K < (1LL << 31) && (int64_t)(g.N + kBigN) * g.K < (1LL << 31);
-    const bool worth = g.M > kBM && g.N > kBN && g.K >= 2 * kBK;
-    // its fp8 epilogue stores whole words through 32-bit buffer offsets
+    // the tiles' fp8 epilogue stores whole words through 32-bit buffer offsets
     const bool fp8_ok = !is_fp8_out(g.d_dtype) ||
                         (g.N % 16 == 0 && g.M % 4 == 0 && (int64_t)g.M * g.N < (1LL << 32) - 16 &&
                          (reinterpret_cast<uintptr_t>(g.Dt) & 15) == 0);
-    // an operand given as its transpose, [K, N] or [K, M], is loaded in 16-byte pieces of its rows; only the big
-    // kernel reads it, and a transposed A only next to a transposed B (the wgrad form)
+    // an operand given as its transpose, [K, N] or [K, M], is loaded in 16-byte pieces of its rows; a transposed A is
+    // read only next to a transposed B (the wgrad form)
     if (g.ta && (!g.tb || g.M % 16 != 0)) return kPathNone;
-    if (g.tb) return (g.N % 16 == 0 && fits32 && worth && fp8_ok) ? kPathBig : kPathNone;
-    return (fits32 && worth && fp8_ok) ? kPathBig : kPathSmall;
+    if (g.tb) return (g.N % 16 == 0 && fits32(g) && g.M > kBM && g.N > kBN && g.K >= 2 * kBK && fp8_ok) ? kPathTiles : kPathNone;
+    if (!fp8_ok) return kPathWords;
+    return (int64_t)g.K * 128 < (1LL << 31) ? kPathTiles : kPathAny;   // (a tile's rows within reach of 32-bit offsets)
 }
 
-// One launch (plus one for the half-tile tail) of the big kernel over up to kBigMaxProblems problems of the
-// same operand formats.  Tiles are listed problem by problem, longest K first: the long tiles start together and
-// the shorter ones fill the rounds behind them.
-template <int FA, int FB, bool kFp8Out, bool kBT>
-static int launch_big(const GemmDesc* const* g, int n, hipStream_t st) {
+// What a launch of `n` problems takes in tiles of edge 256, 128 or 64, in nanoseconds: rounds of workgroups times what a
+// workgroup takes for its K-tiles and for everything else.  The constants are fits to launches of one problem with
+// bf16 output (plain / B transposed / both transposed), warm operands; what matters is where the lines cross.
+//   us, 256 / 128 / 64 wide:  1024 x 1024 x 1024  10.1 / 7.5 / 4.8     2048 x 1024 x 4096  26.5 / 16.3 / 15.3
+//   2048 x 2048 x 2048  16.7 / 11.8 / 16.9      both transposed  19.6 / 12.6 / 24.3
+//   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101      16 x 6144 x 4096  - / 13.8 / 8.3
+static int64_t launch_cost(const GemmDesc* const* g, int n, int edge) {
+    const int64_t cus = cu_count();
+    int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
+    int form = 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t t = (((int64_t)g[i]->M + edge - 1) / edge) * (((int64_t)g[i]->N + edge - 1) / edge);
+        tiles += t;
+        kt += t * ((g[i]->K + kBK - 1) / kBK);
+        form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
+    }
+    const int64_t k = kt / tiles;   // K-tiles of an average tile
+    if (edge == 256) {
+        const int64_t rem = tiles % cus, full = tiles / cus;
+        return full * (1400 * k + 7000) + (rem == 0 ? 0 : 2 * rem <= cus ? 700 * k + 7000 : 1400 * k + 7000);
+    }
+    if (edge == 128) return ((tiles + cus - 1) / cus) * (390 * k + 5200);
+    // two workgroups per CU
+    static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
+    const int64_t rem = tiles % (2 * cus), full = tiles / (2 * cus);
+    return full * (kPair[form] * k + 3500) + (rem == 0 ? 0 : rem <= cus ? kAlone[form] * k + 3000 : kPair[form] * k + 3500);
+}
+
+// One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
+// tiles: one more launch for a half-tile tail).  Tiles are listed problem by problem, longest K first: the long tiles
+// start together and the shorter ones fill the rounds behind them.
+template <int FA, int FB>
+static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
+    int edge = 128;
+    {
+        bool big = true;
+        for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
+        int64_t best = launch_cost(g, n, 128);
+        for (const int e : {64, 256}) {
+            if (e == 256 && !big) continue;
+            const int64_t c = launch_cost(g, n, e);
+            if (c < best) best = c, edge = e;
+        }
+    }
     int order[kBigMaxProblems];
     for (int i = 0; i < n; ++i) order[i] = i;
     for (int i = 1; i < n; ++i)   // insertion sort, stable, K descending
@@ -162,7 +207,7 @@ static int launch_big(const GemmDesc* const* g, int n, hipStream_t st) {
         }
     BigLaunch L = {};
     L.count = n;
-    int tiles = 0;
+    int64_t tiles = 0;
     for (int i = 0; i < n; ++i) {
         const GemmDesc& d = *g[order[i]];
         BigProblem& p = L.p[i];
@@ -174,72 +219,95 @@ static int launch_big(const GemmDesc* const* g, int n, hipStream_t st) {
         p.M = d.M;
         p.N = d.N;
         p.K = d.K;
-        p.tiles_m = (d.M + 255) / 256;
-        p.tiles_n = (d.N + kBigN - 1) / kBigN;
-        p.tile_begin = tiles;
+        p.tiles_m = (d.M - 1) / edge + 1;
+        p.tiles_n = (d.N - 1) / edge + 1;
+        p.tile_begin = (int)tiles;
         p.d_dtype = d.d_dtype;
         p.accumulate = d.accumulate;
         p.fp8 = Fp8Out{d.sd, static_cast<uint8_t*>(d.Dt), static_cast<Workspace*>(d.ws)};
         p.ex = GemmExtras{d.bias, d.bias_dtype, d.scale_inv};
         p.at = d.ta;
-        tiles += p.tiles_m * p.tiles_n;
+        p.bt = d.tb;
+        tiles += (int64_t)p.tiles_m * p.tiles_n;
     }
-    const int rem = tiles % cu_count();
+    if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
+    const bool fp8_out = is_fp8_out(g[0]->d_dtype);
+    L.round_size = cu_count() * (edge == 64 ? 2 : 1);
+    if (edge != 256) return launch_mid(L, FA, FB, edge, fp8_out, (int)tiles, st);
+    const int rem = (int)(tiles % cu_count());
     L.tail_tiles = (rem != 0 && 2 * rem <= cu_count()) ? rem : 0;
-    L.full_blocks = tiles - L.tail_tiles;
-    L.round_size = cu_count();
+    L.full_blocks = (int)tiles - L.tail_tiles;
     (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
-    if (L.full_blocks > 0)
-        hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 8, kFp8Out, kBT>), dim3(L.full_blocks), dim3(kBigThreads), 0, st, L);
-    if (L.tail_tiles > 0)
-        hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 4, kFp8Out, kBT>), dim3(2 * L.tail_tiles), dim3(kBigThreads), 0, st, L);
+    auto go = [&](auto fp8_tag, auto bt_tag) {
+        constexpr bool kFp8Out = decltype(fp8_tag)::value, kBT = decltype(bt_tag)::value;
+        if (L.full_blocks > 0)
+            hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 8, kFp8Out, kBT>), dim3(L.full_blocks), dim3(kBigThreads), 0, st, L);
+        if (L.tail_tiles > 0)
+            hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 4, kFp8Out, kBT>), dim3(2 * L.tail_tiles), dim3(kBigThreads), 0, st, L);
+    };
+#ifdef NTFP8_PROFILE_NARROW
+    go(std::false_type{}, std::false_type{});
+#else
+    if (g[0]->tb) {
+        if (fp8_out) go(std::true_type{}, std::true_type{});
+        else go(std::false_type{}, std::true_type{});
+    } else {
+        if (fp8_out) go(std::true_type{}, std::false_type{});
+        else go(std::false_type{}, std::false_type{});
+    }
+#endif
     return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
 }
 
 template <int FA, int FB, int DT, bool kAcc>
-static int launch_small(const GemmDesc& g, int path, hipStream_t st) {
+static int launch_any(const GemmDesc& g, hipStream_t st) {
     const uint8_t* a = static_cast<const uint8_t*>(g.A);
     const uint8_t* b = static_cast<const uint8_t*>(g.B);
     const Fp8Out fp8 = {g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)};
     const GemmExtras ex = {g.bias, g.bias_dtype, g.scale_inv};
     (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
-    if (path == kPathSmall) {
-        const int tm = (g.M + kBM - 1) / kBM, tn = (g.N + kBN - 1) / kBN;
-        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, DT, kAcc>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa,
-                           g.sb, g.M, g.N, g.K, tm, tn, fp8, ex);
+    const int d_vec = (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
+    const int64_t t2m = ((int64_t)g.M + 127) / 128, t2n = ((int64_t)g.N + 127) / 128;
+    // 128-wide tiles once there is one for every CU, 64-wide below (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles
+    // of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6; 4096 x 4096 x 4095 262 / 179)
+    if (t2m * t2n >= cu_count()) {
+        hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 2>), dim3((int)(t2m * t2n)), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa,
+                           g.sb, g.M, g.N, g.K, (int)t2m, (int)t2n, d_vec, fp8, ex);
     } else {
-        const int d_vec = (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
-        const int64_t t2m = ((int64_t)g.M + 127) / 128, t2n = ((int64_t)g.N + 127) / 128;
-        // 128-wide tiles once there is one for every CU, 64-wide below (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles
-        // of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6; 4096 x 4096 x 4095 262 / 179)
-        if (t2m * t2n >= cu_count()) {
-            hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 2>), dim3((int)(t2m * t2n)), dim3(kAnyThreads), 0, st, a, b,
-                               g.D, g.sa, g.sb, g.M, g.N, g.K, (int)t2m, (int)t2n, d_vec, fp8, ex);
-        } else {
-            const int tm = (g.M + 63) / 64, tn = (g.N + 63) / 64;
-            hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 1>), dim3(tm * tn), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa,
-                               g.sb, g.M, g.N, g.K, tm, tn, d_vec, fp8, ex);
-        }
+        const int tm = (g.M + 63) / 64, tn = (g.N + 63) / 64;
+        hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 1>), dim3(tm * tn), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa, g.sb,
+                           g.M, g.N, g.K, tm, tn, d_vec, fp8, ex);
     }
+    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+}
+
+template <int FA, int FB, int DT>
+static int launch_words(const GemmDesc& g, hipStream_t st) {
+    const int tm = (g.M + kBM - 1) / kBM, tn = (g.N + kBN - 1) / kBN;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, DT>), dim3(tm * tn), dim3(kGemmThreads), 0, st, static_cast<const uint8_t*>(g.A),
+                       static_cast<const uint8_t*>(g.B), g.D, g.sa, g.sb, g.M, g.N, g.K, tm, tn,
+                       Fp8Out{g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)}, GemmExtras{g.bias, g.bias_dtype, g.scale_inv});
     return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
 }
 
 template <int FA, int FB>
 static int dispatch_fmt(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     if (path == kPathNone) return NTFP8_ERR_UNSUPPORTED;
-    if (path == kPathBig) {
-        if (g[0]->tb)
-            return is_fp8_out(g[0]->d_dtype) ? launch_big<FA, FB, true, true>(g, n, st) : launch_big<FA, FB, false, true>(g, n, st);
-        return is_fp8_out(g[0]->d_dtype) ? launch_big<FA, FB, true, false>(g, n, st) : launch_big<FA, FB, false, false>(g, n, st);
-    }
-    const GemmDesc& d = *g[0];   // the small kernels take one problem
+    if (path == kPathTiles) return launch_tiles<FA, FB>(g, n, st);
+#ifdef NTFP8_PROFILE_NARROW
+    return NTFP8_ERR_UNSUPPORTED;
+#else
+    const GemmDesc& d = *g[0];   // the other kernels take one problem
+    if (path == kPathWords)
+        return d.d_dtype == NTFP8_OUT_E4M3 ? launch_words<FA, FB, NTFP8_OUT_E4M3>(d, st) : launch_words<FA, FB, NTFP8_OUT_E5M2>(d, st);
     if (d.d_dtype == NTFP8_F32)
-        return d.accumulate ? launch_small<FA, FB, NTFP8_F32, true>(d, path, st)
-                            : launch_small<FA, FB, NTFP8_F32, false>(d, path, st);
-    if (d.d_dtype == NTFP8_BF16) return launch_small<FA, FB, NTFP8_BF16, false>(d, path, st);
-    if (d.d_dtype == NTFP8_OUT_E4M3) return launch_small<FA, FB, NTFP8_OUT_E4M3, false>(d, path, st);
-    if (d.d_dtype == NTFP8_OUT_E5M2) return launch_small<FA, FB, NTFP8_OUT_E5M2, false>(d, path, st);
-    return launch_small<FA, FB, NTFP8_F16, false>(d, path, st);
+        return d.accumulate ? launch_any<FA, FB, NTFP8_F32, true>(d, st) : launch_any<FA, FB, NTFP8_F32, false>(d, st);
+    if (d.d_dtype == NTFP8_BF16) return launch_any<FA, FB, NTFP8_BF16, false>(d, st);
+    if (d.d_dtype == NTFP8_OUT_E4M3) return launch_any<FA, FB, NTFP8_OUT_E4M3, false>(d, st);
+    if (d.d_dtype == NTFP8_OUT_E5M2) return launch_any<FA, FB, NTFP8_OUT_E5M2, false>(d, st);
+    return launch_any<FA, FB, NTFP8_F16, false>(d, st);
+#endif
 }
 
 static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
@@ -247,8 +315,8 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
 #ifdef NTFP8_PROFILE_NARROW
     // experiment builds of the profiling library carry one instantiation only: e4m3 x e4m3, K-contiguous operands,
     // 16-bit or fp32 output (what the loop experiments launch); everything else is refused
-    if (fa != kE4M3 || fb != kE4M3 || path != kPathBig || g[0]->tb || is_fp8_out(g[0]->d_dtype)) return NTFP8_ERR_UNSUPPORTED;
-    return launch_big<kE4M3, kE4M3, false, false>(g, n, st);
+    if (fa != kE4M3 || fb != kE4M3 || path != kPathTiles || g[0]->tb || is_fp8_out(g[0]->d_dtype)) return NTFP8_ERR_UNSUPPORTED;
+    return launch_tiles<kE4M3, kE4M3>(g, n, st);
 #else
     if (fa == kE4M3) return fb == kE4M3 ? dispatch_fmt<kE4M3, kE4M3>(g, n, path, st) : dispatch_fmt<kE4M3, kE5M2>(g, n, path, st);
     return fb == kE4M3 ? dispatch_fmt<kE5M2, kE4M3>(g, n, path, st) : dispatch_fmt<kE5M2, kE5M2>(g, n, path, st);
@@ -260,8 +328,7 @@ int run_gemm(const GemmDesc& g, hipStream_t st) {
     return dispatch(one, 1, path_of(g), st);
 }
 
-// Independent problems (no output of one is an operand of another).  Problems that qualify for the big kernel
-// and share their operand formats go out together, up to kBigMaxProblems per launch; the rest one by one.
+// Independent problems (no output of one is an operand of another).  Problems that go to the tile kernels and share their operand formats go out together, up to kBigMaxProblems per launch; the rest one by one.
 int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
     bool done[64] = {false};
     if (n > 64) return NTFP8_ERR_SIZE;
@@ -275,9 +342,9 @@ int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
         const int path = path_of(g[i]);
         group[cnt++] = &g[i];
         done[i] = true;
-        if (path == kPathBig) {
+        if (path == kPathTiles) {
             for (int j = i + 1; j < n && cnt < kBigMaxProblems; ++j)
-                if (!done[j] && g[j].fmt_a == g[i].fmt_a && g[j].fmt_b == g[i].fmt_b && path_of(g[j]) == kPathBig &&
+                if (!done[j] && g[j].fmt_a == g[i].fmt_a && g[j].fmt_b == g[i].fmt_b && path_of(g[j]) == kPathTiles &&
                     is_fp8_out(g[j].d_dtype) == is_fp8_out(g[i].d_dtype) && g[j].tb == g[i].tb) {
                     group[cnt++] = &g[j];
                     done[j] = true;

@@ -300,7 +300,8 @@ struct BigProblem {
     int accumulate;         // fp32 outputs only: D += result
     Fp8Out fp8;             // fp8 outputs only
     GemmExtras ex;          // bias, inverse-scale flag
-    int at;                 // A is given as [K, M] row-major (its transpose); kBT launches only
+    int at;                 // A is given as [K, M] row-major (its transpose); only together with bt
+    int bt;                 // B is given as [K, N] row-major (its transpose)
 };
 constexpr int kBigMaxProblems = 4;
 struct BigLaunch {
