@@ -18,115 +18,16 @@
 //                         whole words (the other kernels' fp8 epilogue stores nothing smaller).
 #include "gemm_common.h"
 #include "gemm_big.h"
-#include "gemm_any.h"
 
 namespace ntfp8 {
 
 // ---------------------------------------------------------------------------------------------
-// 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.
-constexpr int kBM = 128, kBN = 128;
-constexpr int kGemmThreads = 256;
-
-template <int FA, int FB, int DT>
-__global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
-                                                               void* __restrict__ Dv, const float* __restrict__ scale_a,
-                                                               const float* __restrict__ scale_b, int M, int N, int K,
-                                                               int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex) {
-    __shared__ __attribute__((aligned(16))) uint8_t sA[kBM * kBK];
-    __shared__ __attribute__((aligned(16))) uint8_t sB[kBN * kBK];
-
-    int pid_m, pid_n;
-    tile_of_block(tiles_m, tiles_n, pid_m, pid_n);
-    const int m0 = pid_m * kBM, n0 = pid_n * kBN;
-
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-
-    // global -> LDS assignment: 1024 16-byte chunks per operand tile, 4 per thread
-    int ld_row[4], ld_kc[4];
-    const uint8_t* a_ptr[4];
-    const uint8_t* b_ptr[4];
-    bool a_ok[4], b_ok[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int c = t + kGemmThreads * i;
-        ld_row[i] = c >> 3;
-        ld_kc[i] = c & 7;
-        a_ok[i] = m0 + ld_row[i] < M;
-        b_ok[i] = n0 + ld_row[i] < N;
-        a_ptr[i] = A + (int64_t)(a_ok[i] ? m0 + ld_row[i] : 0) * K + ld_kc[i] * 16;
-        b_ptr[i] = B + (int64_t)(b_ok[i] ? n0 + ld_row[i] : 0) * K + ld_kc[i] * 16;
-    }
-
-    v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    v4i ra[4], rb[4];
-    const v4i zero = {0, 0, 0, 0};
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool kin = k0 + ld_kc[i] * 16 < K;
-            ra[i] = (a_ok[i] && kin) ? *reinterpret_cast<const v4i*>(a_ptr[i] + k0) : zero;
-            rb[i] = (b_ok[i] && kin) ? *reinterpret_cast<const v4i*>(b_ptr[i] + k0) : zero;
-        }
-    };
-
-    const int frow = lane & 31;
-    const int fk = (lane >> 5) * 2;
-
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += kBK) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            *reinterpret_cast<v4i*>(&sA[lds_off(ld_row[i], ld_kc[i])]) = ra[i];
-            *reinterpret_cast<v4i*>(&sB[lds_off(ld_row[i], ld_kc[i])]) = rb[i];
-        }
-        __syncthreads();
-        if (k0 + kBK < K) fetch(k0 + kBK);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            v8i fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int ra_row = wm + i * 32 + frow, rb_row = wn + i * 32 + frow;
-                const v4i a0 = *reinterpret_cast<const v4i*>(&sA[lds_off(ra_row, ks * 4 + fk)]);
-                const v4i a1 = *reinterpret_cast<const v4i*>(&sA[lds_off(ra_row, ks * 4 + fk + 1)]);
-                const v4i b0 = *reinterpret_cast<const v4i*>(&sB[lds_off(rb_row, ks * 4 + fk)]);
-                const v4i b1 = *reinterpret_cast<const v4i*>(&sB[lds_off(rb_row, ks * 4 + fk + 1)]);
-                fa[i] = (v8i){a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-                fb[i] = (v8i){b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x64<FA, FB>(fb[j], fa[i], acc[i][j]);
-        }
-    }
-
-    float alpha = descale_factor(scale_a, scale_b, ex.scale_inv);
-    if (ex.bias) {   // uniform
-        add_bias32<2, 2>(acc, alpha, ex.bias, ex.bias_dtype, N, n0 + wn, lane);
-        alpha = 1.0f;
-    }
-    constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
-    const float scale_d = *fp8.scale;
-    const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
-                                                       scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane);
-    publish_amax(amax, fp8.ws);
-}
-
-// ---------------------------------------------------------------------------------------------
+constexpr int kMinTransposed = 128;   // rows and columns of a result whose B is given as its transpose: more than this
 enum GemmPath { kPathNone = -1, kPathAny = 0, kPathWords = 1, kPathTiles = 2 };
 
 int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
+int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
+int launch_words(const GemmDesc& g, hipStream_t st);
 
 // operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
 static bool fits32(const GemmDesc& g) {
@@ -148,7 +49,7 @@ static int path_of(const GemmDesc& g) {
     // an operand given as its transpose, [K, N] or [K, M], is loaded in 16-byte pieces of its rows; a transposed A is
     // read only next to a transposed B (the wgrad form)
     if (g.ta && (!g.tb || g.M % 16 != 0)) return kPathNone;
-    if (g.tb) return (g.N % 16 == 0 && fits32(g) && g.M > kBM && g.N > kBN && g.K >= 2 * kBK && fp8_ok) ? kPathTiles : kPathNone;
+    if (g.tb) return (g.N % 16 == 0 && fits32(g) && g.M > kMinTransposed && g.N > kMinTransposed && g.K >= 2 * kBK && fp8_ok) ? kPathTiles : kPathNone;
     if (!fp8_ok) return kPathWords;
     return (int64_t)g.K * 128 < (1LL << 31) ? kPathTiles : kPathAny;   // (a tile's rows within reach of 32-bit offsets)
 }
@@ -181,22 +82,9 @@ static int64_t launch_cost(const GemmDesc* const* g, int n, int edge) {
     return full * (kPair[form] * k + 3500) + (rem == 0 ? 0 : rem <= cus ? kAlone[form] * k + 3000 : kPair[form] * k + 3500);
 }
 
-// One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
-// tiles: one more launch for a half-tile tail).  Tiles are listed problem by problem, longest K first: the long tiles
-// start together and the shorter ones fill the rounds behind them.
-template <int FA, int FB>
-static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
-    int edge = 128;
-    {
-        bool big = true;
-        for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
-        int64_t best = launch_cost(g, n, 128);
-        for (const int e : {64, 256}) {
-            if (e == 256 && !big) continue;
-            const int64_t c = launch_cost(g, n, e);
-            if (c < best) best = c, edge = e;
-        }
-    }
+// The tile list of a launch, problem by problem, longest K first: the long tiles start together and the shorter ones fill
+// the rounds behind them.  Returns the number of tiles.
+static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* L) {
     int order[kBigMaxProblems];
     for (int i = 0; i < n; ++i) order[i] = i;
     for (int i = 1; i < n; ++i)   // insertion sort, stable, K descending
@@ -205,12 +93,12 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
             order[j] = order[j - 1];
             order[j - 1] = t;
         }
-    BigLaunch L = {};
-    L.count = n;
+    *L = {};
+    L->count = n;
     int64_t tiles = 0;
     for (int i = 0; i < n; ++i) {
         const GemmDesc& d = *g[order[i]];
-        BigProblem& p = L.p[i];
+        BigProblem& p = L->p[i];
         p.A = static_cast<const uint8_t*>(d.A);
         p.B = static_cast<const uint8_t*>(d.B);
         p.D = d.D;
@@ -230,6 +118,26 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
         p.bt = d.tb;
         tiles += (int64_t)p.tiles_m * p.tiles_n;
     }
+    return tiles;
+}
+
+// One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
+// tiles: one more launch for a half-tile tail).
+template <int FA, int FB>
+static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
+    int edge = 128;
+    {
+        bool big = true;
+        for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
+        int64_t best = launch_cost(g, n, 128);
+        for (const int e : {64, 256}) {
+            if (e == 256 && !big) continue;
+            const int64_t c = launch_cost(g, n, e);
+            if (c < best) best = c, edge = e;
+        }
+    }
+    BigLaunch L;
+    const int64_t tiles = list_tiles(g, n, edge, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     const bool fp8_out = is_fp8_out(g[0]->d_dtype);
     L.round_size = cu_count() * (edge == 64 ? 2 : 1);
@@ -259,67 +167,31 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
 }
 
-template <int FA, int FB, int DT, bool kAcc>
-static int launch_any(const GemmDesc& g, hipStream_t st) {
-    const uint8_t* a = static_cast<const uint8_t*>(g.A);
-    const uint8_t* b = static_cast<const uint8_t*>(g.B);
-    const Fp8Out fp8 = {g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)};
-    const GemmExtras ex = {g.bias, g.bias_dtype, g.scale_inv};
-    (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
-    const int d_vec = (reinterpret_cast<uintptr_t>(g.D) & 15) == 0;
-    const int64_t t2m = ((int64_t)g.M + 127) / 128, t2n = ((int64_t)g.N + 127) / 128;
-    // 128-wide tiles once there is one for every CU, 64-wide below (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles
-    // of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6; 4096 x 4096 x 4095 262 / 179)
-    if (t2m * t2n >= cu_count()) {
-        hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 2>), dim3((int)(t2m * t2n)), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa,
-                           g.sb, g.M, g.N, g.K, (int)t2m, (int)t2n, d_vec, fp8, ex);
-    } else {
-        const int tm = (g.M + 63) / 64, tn = (g.N + 63) / 64;
-        hipLaunchKernelGGL((gemm_any_kernel<FA, FB, DT, kAcc, 1>), dim3(tm * tn), dim3(kAnyThreads), 0, st, a, b, g.D, g.sa, g.sb,
-                           g.M, g.N, g.K, tm, tn, d_vec, fp8, ex);
-    }
-    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
-}
-
-template <int FA, int FB, int DT>
-static int launch_words(const GemmDesc& g, hipStream_t st) {
-    const int tm = (g.M + kBM - 1) / kBM, tn = (g.N + kBN - 1) / kBN;
-    (void)hipGetLastError();
-    hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, DT>), dim3(tm * tn), dim3(kGemmThreads), 0, st, static_cast<const uint8_t*>(g.A),
-                       static_cast<const uint8_t*>(g.B), g.D, g.sa, g.sb, g.M, g.N, g.K, tm, tn,
-                       Fp8Out{g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)}, GemmExtras{g.bias, g.bias_dtype, g.scale_inv});
-    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
-}
-
-template <int FA, int FB>
-static int dispatch_fmt(const GemmDesc* const* g, int n, int path, hipStream_t st) {
-    if (path == kPathNone) return NTFP8_ERR_UNSUPPORTED;
-    if (path == kPathTiles) return launch_tiles<FA, FB>(g, n, st);
-#ifdef NTFP8_PROFILE_NARROW
-    return NTFP8_ERR_UNSUPPORTED;
-#else
-    const GemmDesc& d = *g[0];   // the other kernels take one problem
-    if (path == kPathWords)
-        return d.d_dtype == NTFP8_OUT_E4M3 ? launch_words<FA, FB, NTFP8_OUT_E4M3>(d, st) : launch_words<FA, FB, NTFP8_OUT_E5M2>(d, st);
-    if (d.d_dtype == NTFP8_F32)
-        return d.accumulate ? launch_any<FA, FB, NTFP8_F32, true>(d, st) : launch_any<FA, FB, NTFP8_F32, false>(d, st);
-    if (d.d_dtype == NTFP8_BF16) return launch_any<FA, FB, NTFP8_BF16, false>(d, st);
-    if (d.d_dtype == NTFP8_OUT_E4M3) return launch_any<FA, FB, NTFP8_OUT_E4M3, false>(d, st);
-    if (d.d_dtype == NTFP8_OUT_E5M2) return launch_any<FA, FB, NTFP8_OUT_E5M2, false>(d, st);
-    return launch_any<FA, FB, NTFP8_F16, false>(d, st);
-#endif
+// Problems no 16-byte chunk of which lies in one piece: 128-wide tiles once there is one for every CU, 64-wide below
+// (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6;
+// 4096 x 4096 x 4095 262 / 179)
+static int launch_any_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
+    BigLaunch L;
+    int edge = 128;
+    int64_t tiles = list_tiles(g, n, edge, &L);
+    if (tiles < cu_count()) tiles = list_tiles(g, n, edge = 64, &L);
+    if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
+    return launch_any(L, g[0]->fmt_a, g[0]->fmt_b, edge, is_fp8_out(g[0]->d_dtype), (int)tiles, st);
 }
 
 static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     const int fa = g[0]->fmt_a, fb = g[0]->fmt_b;
+    if (path == kPathNone) return NTFP8_ERR_UNSUPPORTED;
 #ifdef NTFP8_PROFILE_NARROW
     // experiment builds of the profiling library carry one instantiation only: e4m3 x e4m3, K-contiguous operands,
     // 16-bit or fp32 output (what the loop experiments launch); everything else is refused
     if (fa != kE4M3 || fb != kE4M3 || path != kPathTiles || g[0]->tb || is_fp8_out(g[0]->d_dtype)) return NTFP8_ERR_UNSUPPORTED;
     return launch_tiles<kE4M3, kE4M3>(g, n, st);
 #else
-    if (fa == kE4M3) return fb == kE4M3 ? dispatch_fmt<kE4M3, kE4M3>(g, n, path, st) : dispatch_fmt<kE4M3, kE5M2>(g, n, path, st);
-    return fb == kE4M3 ? dispatch_fmt<kE5M2, kE4M3>(g, n, path, st) : dispatch_fmt<kE5M2, kE5M2>(g, n, path, st);
+    if (path == kPathAny) return launch_any_tiles(g, n, st);
+    if (path == kPathWords) return launch_words(*g[0], st);
+    if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, st) : launch_tiles<kE4M3, kE5M2>(g, n, st);
+    return fb == kE4M3 ? launch_tiles<kE5M2, kE4M3>(g, n, st) : launch_tiles<kE5M2, kE5M2>(g, n, st);
 #endif
 }
 
@@ -328,7 +200,7 @@ int run_gemm(const GemmDesc& g, hipStream_t st) {
     return dispatch(one, 1, path_of(g), st);
 }
 
-// Independent problems (no output of one is an operand of another).  Problems that go to the tile kernels and share their operand formats go out together, up to kBigMaxProblems per launch; the rest one by one.
+// Independent problems (no output of one is an operand of another).  Problems that go to the same tile kernel and share their operand formats go out together, up to kBigMaxProblems per launch; the rest one by one.
 int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
     bool done[64] = {false};
     if (n > 64) return NTFP8_ERR_SIZE;
@@ -342,9 +214,9 @@ int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
         const int path = path_of(g[i]);
         group[cnt++] = &g[i];
         done[i] = true;
-        if (path == kPathTiles) {
+        if (path != kPathWords) {
             for (int j = i + 1; j < n && cnt < kBigMaxProblems; ++j)
-                if (!done[j] && g[j].fmt_a == g[i].fmt_a && g[j].fmt_b == g[i].fmt_b && path_of(g[j]) == kPathTiles &&
+                if (!done[j] && g[j].fmt_a == g[i].fmt_a && g[j].fmt_b == g[i].fmt_b && path_of(g[j]) == path &&
                     is_fp8_out(g[j].d_dtype) == is_fp8_out(g[i].d_dtype) && g[j].tb == g[i].tb) {
                     group[cnt++] = &g[j];
                     done[j] = true;

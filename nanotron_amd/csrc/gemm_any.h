@@ -1,4 +1,4 @@
-// FP8 GEMM for any K and any pointer alignment (gfx950); included by gemm.hip.
+// FP8 GEMM for any K and any pointer alignment (gfx950); included by gemm_any.hip.
 //
 // What the other kernels do not take: rows of A and B that start on no 16-byte boundary, because K is not a multiple
 // of 16 (a weight gradient reduces over the tokens of the batch, and those are a multiple of nothing) or because a
@@ -66,18 +66,29 @@ __device__ __forceinline__ v4i any_chunk(const uint8_t* __restrict__ P, int64_t 
     return v;
 }
 
-template <int FA, int FB, int DT, bool kAcc, int MB>
-__global__ __launch_bounds__(kAnyThreads) void gemm_any_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
-                                                               void* __restrict__ Dv, const float* __restrict__ scale_a,
-                                                               const float* __restrict__ scale_b, int M, int N, int K,
-                                                               int tiles_m, int tiles_n, int d_vec, Fp8Out fp8, GemmExtras ex) {
+// Output type and accumulation are run-time properties of a problem and a launch takes up to kBigMaxProblems of the same
+// operand formats, as in the other tile kernels (BigLaunch, gemm_big.h): the two GEMMs of a small layer's backward share
+// one launch.
+template <int FA, int FB, int MB, bool kFp8Out>
+__global__ __launch_bounds__(kAnyThreads) void gemm_any_kernel(const BigLaunch L) {
     constexpr int kT = 64 * MB;             // tile edge
     constexpr int kC = kT * 8 / kAnyThreads;   // 16-byte chunks per operand and thread
     __shared__ __attribute__((aligned(16))) uint8_t sA[2][kT * kBK];
     __shared__ __attribute__((aligned(16))) uint8_t sB[2][kT * kBK];
 
+    int pid = blockIdx.x;
+    if (gridDim.x % kXcds == 0) pid = (pid % kXcds) * (gridDim.x / kXcds) + pid / kXcds;   // an XCD works on a run of tiles
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kBigMaxProblems; ++i)
+        if (i < L.count && pid >= L.p[i].tile_begin) which = i;
+    const BigProblem& P = L.p[which];
+    const uint8_t* __restrict__ A = P.A;
+    const uint8_t* __restrict__ B = P.B;
+    const int M = P.M, N = P.N, K = P.K;
+    pid -= P.tile_begin;
     int pid_m, pid_n;
-    tile_of_block(tiles_m, tiles_n, pid_m, pid_n);
+    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
     const int m0 = pid_m * kT, n0 = pid_n * kT;
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
@@ -140,19 +151,29 @@ __global__ __launch_bounds__(kAnyThreads) void gemm_any_kernel(const uint8_t* __
         }
     }
 
-    float alpha = descale_factor(scale_a, scale_b, ex.scale_inv);
-    if (ex.bias) {   // uniform
-        add_bias32<MB, MB>(acc, alpha, ex.bias, ex.bias_dtype, N, n0 + wn, lane);
+    float alpha = descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);
+    if (P.ex.bias) {   // uniform
+        add_bias32<MB, MB>(acc, alpha, P.ex.bias, P.ex.bias_dtype, N, n0 + wn, lane);
         alpha = 1.0f;
     }
-    if constexpr (DT == NTFP8_OUT_E4M3 || DT == NTFP8_OUT_E5M2) {
-        constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
-        const float scale_d = *fp8.scale;
-        const uint32_t amax = store_wave_tile_fp8<F, MB, MB>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
-                                                             scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane, d_vec != 0);
-        publish_amax(amax, fp8.ws);
+    const bool d_aligned = (reinterpret_cast<uintptr_t>(P.D) & 15) == 0;
+    const int mb = m0 + wm, nb = n0 + wn;
+    if constexpr (kFp8Out) {
+        const float scale_d = *P.fp8.scale;
+        const bool slow = scale_is_degenerate(scale_d);
+        uint8_t* D = static_cast<uint8_t*>(P.D);
+        const uint32_t amax = P.d_dtype == NTFP8_OUT_E4M3
+                                  ? store_wave_tile_fp8<kE4M3, MB, MB>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, d_aligned)
+                                  : store_wave_tile_fp8<kE5M2, MB, MB>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, d_aligned);
+        publish_amax(amax, P.fp8.ws);
+    } else if (P.d_dtype == NTFP8_BF16) {
+        store_wave_tile<NTFP8_BF16, false, MB, MB>(acc, P.D, alpha, M, N, mb, nb, lane, d_aligned);
+    } else if (P.d_dtype == NTFP8_F16) {
+        store_wave_tile<NTFP8_F16, false, MB, MB>(acc, P.D, alpha, M, N, mb, nb, lane, d_aligned);
+    } else if (P.accumulate) {
+        store_wave_tile<NTFP8_F32, true, MB, MB>(acc, P.D, alpha, M, N, mb, nb, lane, d_aligned);
     } else {
-        store_wave_tile<DT, kAcc, MB, MB>(acc, Dv, alpha, M, N, m0 + wm, n0 + wn, lane, d_vec != 0);
+        store_wave_tile<NTFP8_F32, false, MB, MB>(acc, P.D, alpha, M, N, mb, nb, lane, d_aligned);
     }
 }
 

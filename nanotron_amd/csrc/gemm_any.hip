@@ -1,0 +1,156 @@
+// Instantiations and launchers of the GEMM kernels off the main path: any K and alignment (gemm_any.h), and fp8 outputs
+// whose rows or columns do not come in whole words.  The choice is made in gemm.hip.
+#include "gemm_common.h"
+#include "gemm_big.h"
+#include "gemm_any.h"
+
+namespace ntfp8 {
+
+template <int FA, int FB>
+static int launch_fmt(const BigLaunch& L, int tile, bool fp8_out, int tiles, hipStream_t st) {
+    (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
+    if (tile == 128) {
+        if (fp8_out) hipLaunchKernelGGL((gemm_any_kernel<FA, FB, 2, true>), dim3(tiles), dim3(kAnyThreads), 0, st, L);
+        else hipLaunchKernelGGL((gemm_any_kernel<FA, FB, 2, false>), dim3(tiles), dim3(kAnyThreads), 0, st, L);
+    } else {
+        if (fp8_out) hipLaunchKernelGGL((gemm_any_kernel<FA, FB, 1, true>), dim3(tiles), dim3(kAnyThreads), 0, st, L);
+        else hipLaunchKernelGGL((gemm_any_kernel<FA, FB, 1, false>), dim3(tiles), dim3(kAnyThreads), 0, st, L);
+    }
+    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+}
+
+int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st) {
+    if (fa == kE4M3)
+        return fb == kE4M3 ? launch_fmt<kE4M3, kE4M3>(L, tile, fp8_out, tiles, st) : launch_fmt<kE4M3, kE5M2>(L, tile, fp8_out, tiles, st);
+    return fb == kE4M3 ? launch_fmt<kE5M2, kE4M3>(L, tile, fp8_out, tiles, st) : launch_fmt<kE5M2, kE5M2>(L, tile, fp8_out, tiles, st);
+}
+
+// ---------------------------------------------------------------------------------------------
+// 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.
+constexpr int kBM = 128, kBN = 128;
+constexpr int kGemmThreads = 256;
+
+template <int FA, int FB, int DT>
+__global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
+                                                               void* __restrict__ Dv, const float* __restrict__ scale_a,
+                                                               const float* __restrict__ scale_b, int M, int N, int K,
+                                                               int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex) {
+    __shared__ __attribute__((aligned(16))) uint8_t sA[kBM * kBK];
+    __shared__ __attribute__((aligned(16))) uint8_t sB[kBN * kBK];
+
+    int pid_m, pid_n;
+    tile_of_block(tiles_m, tiles_n, pid_m, pid_n);
+    const int m0 = pid_m * kBM, n0 = pid_n * kBN;
+
+    const int t = threadIdx.x;
+    const int lane = t & 63, wave = t >> 6;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+
+    // global -> LDS assignment: 1024 16-byte chunks per operand tile, 4 per thread
+    int ld_row[4], ld_kc[4];
+    const uint8_t* a_ptr[4];
+    const uint8_t* b_ptr[4];
+    bool a_ok[4], b_ok[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int c = t + kGemmThreads * i;
+        ld_row[i] = c >> 3;
+        ld_kc[i] = c & 7;
+        a_ok[i] = m0 + ld_row[i] < M;
+        b_ok[i] = n0 + ld_row[i] < N;
+        a_ptr[i] = A + (int64_t)(a_ok[i] ? m0 + ld_row[i] : 0) * K + ld_kc[i] * 16;
+        b_ptr[i] = B + (int64_t)(b_ok[i] ? n0 + ld_row[i] : 0) * K + ld_kc[i] * 16;
+    }
+
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    v4i ra[4], rb[4];
+    const v4i zero = {0, 0, 0, 0};
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool kin = k0 + ld_kc[i] * 16 < K;
+            ra[i] = (a_ok[i] && kin) ? *reinterpret_cast<const v4i*>(a_ptr[i] + k0) : zero;
+            rb[i] = (b_ok[i] && kin) ? *reinterpret_cast<const v4i*>(b_ptr[i] + k0) : zero;
+        }
+    };
+
+    const int frow = lane & 31;
+    const int fk = (lane >> 5) * 2;
+
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += kBK) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            *reinterpret_cast<v4i*>(&sA[lds_off(ld_row[i], ld_kc[i])]) = ra[i];
+            *reinterpret_cast<v4i*>(&sB[lds_off(ld_row[i], ld_kc[i])]) = rb[i];
+        }
+        __syncthreads();
+        if (k0 + kBK < K) fetch(k0 + kBK);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            v8i fa[2], fb[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int ra_row = wm + i * 32 + frow, rb_row = wn + i * 32 + frow;
+                const v4i a0 = *reinterpret_cast<const v4i*>(&sA[lds_off(ra_row, ks * 4 + fk)]);
+                const v4i a1 = *reinterpret_cast<const v4i*>(&sA[lds_off(ra_row, ks * 4 + fk + 1)]);
+                const v4i b0 = *reinterpret_cast<const v4i*>(&sB[lds_off(rb_row, ks * 4 + fk)]);
+                const v4i b1 = *reinterpret_cast<const v4i*>(&sB[lds_off(rb_row, ks * 4 + fk + 1)]);
+                fa[i] = (v8i){a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+                fb[i] = (v8i){b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x64<FA, FB>(fb[j], fa[i], acc[i][j]);
+        }
+    }
+
+    float alpha = descale_factor(scale_a, scale_b, ex.scale_inv);
+    if (ex.bias) {   // uniform
+        add_bias32<2, 2>(acc, alpha, ex.bias, ex.bias_dtype, N, n0 + wn, lane);
+        alpha = 1.0f;
+    }
+    constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
+    const float scale_d = *fp8.scale;
+    const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
+                                                       scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane);
+    publish_amax(amax, fp8.ws);
+}
+
+template <int FA, int FB>
+static void launch_words_fmt(const GemmDesc& g, hipStream_t st) {
+    const int tm = (g.M + kBM - 1) / kBM, tn = (g.N + kBN - 1) / kBN;
+    const uint8_t* a = static_cast<const uint8_t*>(g.A);
+    const uint8_t* b = static_cast<const uint8_t*>(g.B);
+    const Fp8Out fp8 = {g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)};
+    const GemmExtras ex = {g.bias, g.bias_dtype, g.scale_inv};
+    if (g.d_dtype == NTFP8_OUT_E4M3)
+        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, NTFP8_OUT_E4M3>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb, g.M,
+                           g.N, g.K, tm, tn, fp8, ex);
+    else
+        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, NTFP8_OUT_E5M2>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb, g.M,
+                           g.N, g.K, tm, tn, fp8, ex);
+}
+
+int launch_words(const GemmDesc& g, hipStream_t st) {
+    (void)hipGetLastError();
+    if (g.fmt_a == kE4M3) {
+        if (g.fmt_b == kE4M3) launch_words_fmt<kE4M3, kE4M3>(g, st);
+        else launch_words_fmt<kE4M3, kE5M2>(g, st);
+    } else {
+        if (g.fmt_b == kE4M3) launch_words_fmt<kE5M2, kE4M3>(g, st);
+        else launch_words_fmt<kE5M2, kE5M2>(g, st);
+    }
+    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+}
+
+}  // namespace ntfp8

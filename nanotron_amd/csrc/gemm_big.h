@@ -370,14 +370,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     const int M = P.M, N = P.N, K = P.K;
     pid -= P.tile_begin;
     int pid_m, pid_n;
-    {
-        const int in_group = kGroupM * P.tiles_n;
-        const int group = pid / in_group;
-        const int first_m = group * kGroupM;
-        const int gsz = min(P.tiles_m - first_m, kGroupM);
-        pid_m = first_m + (pid % in_group) % gsz;
-        pid_n = (pid % in_group) / gsz;
-    }
+    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
     const int n0 = pid_n * kBigN;
     const int m0 = pid_m * 256 + half * 128;
     if (m0 >= M) return;   // second half of a bottom-edge tile with nothing in it (uniform for the workgroup)

@@ -154,17 +154,21 @@ struct GemmExtras {
     int scale_inv;      // the scale pointers hold inverse scales
 };
 
-// tile order: XCD-contiguous, then kGroupM row-tiles swept before moving along N
-__device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int& pid_m, int& pid_n) {
-    int pid = blockIdx.x;
-    const int nwg = gridDim.x;
-    if (nwg % kXcds == 0) pid = (pid % kXcds) * (nwg / kXcds) + pid / kXcds;
+// tile `pid` of a problem: kGroupM row-tiles are swept before moving along N
+__device__ __forceinline__ void tile_in_group(int pid, int tiles_m, int tiles_n, int& pid_m, int& pid_n) {
     const int in_group = kGroupM * tiles_n;
     const int group = pid / in_group;
     const int first_m = group * kGroupM;
     const int gsz = min(tiles_m - first_m, kGroupM);
     pid_m = first_m + (pid % in_group) % gsz;
     pid_n = (pid % in_group) / gsz;
+}
+// the same with the workgroups of an XCD on a contiguous run of tiles
+__device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int& pid_m, int& pid_n) {
+    int pid = blockIdx.x;
+    const int nwg = gridDim.x;
+    if (nwg % kXcds == 0) pid = (pid % kXcds) * (nwg / kXcds) + pid / kXcds;
+    tile_in_group(pid, tiles_m, tiles_n, pid_m, pid_n);
 }
 
 // Epilogue of one wave: MI x NJ accumulator blocks of 32 x 32, block (i, j) at rows m_base + 32 i,

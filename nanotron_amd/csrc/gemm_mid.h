@@ -43,14 +43,7 @@ __global__ __launch_bounds__(kBigThreads, T == 128 ? 1 : 2) void gemm_mid_kernel
     const int M = P.M, N = P.N, K = P.K;
     pid -= P.tile_begin;
     int pid_m, pid_n;
-    {
-        const int in_group = kGroupM * P.tiles_n;
-        const int group = pid / in_group;
-        const int first_m = group * kGroupM;
-        const int gsz = min(P.tiles_m - first_m, kGroupM);
-        pid_m = first_m + (pid % in_group) % gsz;
-        pid_n = (pid % in_group) / gsz;
-    }
+    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
     const int m0 = pid_m * T, n0 = pid_n * T;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
