@@ -79,6 +79,12 @@ float ntfp8_update_scaling_factor_host(float amax, float old_scale, int fmt, int
 int ntfp8_cast_to_fp8(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale,
                       int fmt, void* out, void* out_t, void* stream);
 
+/* ntfp8_cast_to_fp8 that also leaves what an FP8Tensor carries beside its bytes: *scale_used_out = *scale (a copy, so that
+ * the bytes keep their scale when the caller's moves on) and *amax_out = 0 (none was taken).  What an evaluation pass
+ * does with the scale a role holds; no counterpart in the reference. */
+int ntfp8_cast_with_scale(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, int fmt, float* amax_out,
+                          float* scale_used_out, void* out, void* out_t, void* stream);
+
 /* tex.cast_to_fp8(input, scale, amax, scale_inv, otype) with all of its effects (src/nanotron/fp8/tensor.py:65; the
  * arithmetic lives in Transformer Engine, which the reference does not vendor: the effects below are its published
  * behaviour): out = saturating_rne_fp8(fp32(x) * *scale); *amax_inout = max(*amax_inout, max|x|) (a NaN on either
@@ -173,6 +179,13 @@ int ntfp8_cast_from_fp8(const void* in, int fmt, const float* scale, int64_t n, 
  * src/nanotron/fp8/tensor.py:74: out = out_dtype(fp32(fp8) * *scale_inv). */
 int ntfp8_cast_from_fp8_scale_inv(const void* in, int fmt, const float* scale_inv, int64_t n, void* out, int out_dtype,
                                   void* stream);
+
+/* out[c] = out_dtype(sum over r of x[r, c]), summed in fp32 in an order that depends on the shape alone: the gradient of
+ * the bias that src/nanotron/fp8/linear.py:65 adds.  `scratch` is ntfp8_column_sum_scratch(rows, cols) bytes of device
+ * memory (may be NULL where that is 0); `workspace` as everywhere. */
+int64_t ntfp8_column_sum_scratch(int64_t rows, int64_t cols);
+int ntfp8_column_sum(const void* x, int x_dtype, int64_t rows, int64_t cols, void* out, int out_dtype, void* scratch,
+                     void* workspace, void* stream);
 
 /* Byte transpose [rows, cols] -> [cols, rows].  Replaces tex.fp8_transpose
  * (src/nanotron/fp8/kernel.py:43-44). */

@@ -6,6 +6,10 @@ namespace ntfp8 {
 
 int run_quant(int mode, const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, uint8_t* out, uint8_t* out_t,
               const float* scale_ptr, Workspace* ws, const ScalarIO& io, hipStream_t st);
+int run_quant_current(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, uint8_t* out, uint8_t* out_t, Workspace* ws,
+                      const ScalarIO& io, hipStream_t st);
+int column_sum_runs(int64_t rows, int64_t cols);
+int run_column_sum(const void* x, int x_dtype, int64_t rows, int64_t cols, void* out, int out_dtype, float* partial, void* ws, hipStream_t st);
 int run_dequant(const void* in, int fmt, const float* scale, int is_inverse, int64_t n, void* out, int out_dtype,
                 hipStream_t st);
 int run_quant_dual(const void* x, int x_dtype, int64_t n, uint8_t* out_e4m3, uint8_t* out_e5m2, Workspace* ws,
@@ -168,6 +172,20 @@ int ntfp8_cast_to_fp8(const void* x, int x_dtype, int64_t rows, int64_t cols, co
                      scale, nullptr, io, static_cast<hipStream_t>(stream));
 }
 
+int ntfp8_cast_with_scale(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, int fmt, float* amax_out,
+                          float* scale_used_out, void* out, void* out_t, void* stream) {
+    int64_t n;
+    if (!scale || !amax_out || !scale_used_out || (!out && !out_t)) return NTFP8_ERR_NULL;
+    int rc = check_quant_common(x, x_dtype, rows, cols, fmt, 0, &n);
+    if (rc) return rc;
+    if (!is_aligned(scale, 4) || !is_aligned(amax_out, 4) || !is_aligned(scale_used_out, 4)) return NTFP8_ERR_ALIGN;
+    rc = check_outputs(x, x_dtype, n, out, out_t);
+    if (rc) return rc;
+    ScalarIO io = {nullptr, amax_out, scale_used_out, nullptr, nullptr, 0, fmt, 0};
+    return run_quant(kModeCastOnly, x, x_dtype, rows, cols, fmt, static_cast<uint8_t*>(out), static_cast<uint8_t*>(out_t),
+                     scale, nullptr, io, static_cast<hipStream_t>(stream));
+}
+
 int ntfp8_quantize_current(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, int margin, float* amax_out,
                            float* scale_used_out, void* out, void* out_t, float* amax_history, int history_len,
                            float* scale_state, void* workspace, void* stream) {
@@ -186,12 +204,8 @@ int ntfp8_quantize_current(const void* x, int x_dtype, int64_t rows, int64_t col
     hipStream_t st = static_cast<hipStream_t>(stream);
     ScalarIO io = {nullptr, amax_out, scale_used_out, amax_history ? scale_state : nullptr, amax_history,
                    amax_history ? history_len : 0, fmt, margin};
-    rc = run_quant(kModeAmaxOnly, x, x_dtype, n, 1, fmt, nullptr, nullptr, nullptr, static_cast<Workspace*>(workspace), io,
-                   st);
-    if (rc) return rc;
-    ScalarIO none = {nullptr, nullptr, nullptr, nullptr, nullptr, 0, fmt, 0};
-    return run_quant(kModeCastOnly, x, x_dtype, rows, cols, fmt, static_cast<uint8_t*>(out), static_cast<uint8_t*>(out_t),
-                     scale_used_out, nullptr, none, st);
+    return run_quant_current(x, x_dtype, rows, cols, fmt, static_cast<uint8_t*>(out), static_cast<uint8_t*>(out_t),
+                             static_cast<Workspace*>(workspace), io, st);
 }
 
 int ntfp8_quantize_first_use(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, int margin, float* scale_state,
@@ -209,16 +223,11 @@ int ntfp8_quantize_first_use(const void* x, int x_dtype, int64_t rows, int64_t c
     rc = check_outputs(x, x_dtype, n, out, out_t);
     if (rc) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // launch 1: amax, the decision between this tensor's scale and the held one, history roll, next scale
+    // amax, the decision between this tensor's scale and the held one, history roll, next scale, cast
     ScalarIO io = {nullptr, amax_out, scale_used_out, scale_state, amax_history, history_len, fmt, margin, nullptr, nullptr,
                    initialised};
-    rc = run_quant(kModeAmaxOnly, x, x_dtype, n, 1, fmt, nullptr, nullptr, nullptr, static_cast<Workspace*>(workspace), io,
-                   st);
-    if (rc) return rc;
-    // launch 2: the cast with the scale launch 1 chose
-    ScalarIO none = {nullptr, nullptr, nullptr, nullptr, nullptr, 0, fmt, 0};
-    return run_quant(kModeCastOnly, x, x_dtype, rows, cols, fmt, static_cast<uint8_t*>(out), static_cast<uint8_t*>(out_t),
-                     scale_used_out, nullptr, none, st);
+    return run_quant_current(x, x_dtype, rows, cols, fmt, static_cast<uint8_t*>(out), static_cast<uint8_t*>(out_t),
+                             static_cast<Workspace*>(workspace), io, st);
 }
 
 int ntfp8_quantize_delayed(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, int margin,
@@ -357,6 +366,30 @@ int ntfp8_cast_from_fp8_scale_inv(const void* in, int fmt, const float* scale_in
     if (!is_aligned(scale_inv, 4) || !is_aligned(out, dtype_size(out_dtype))) return NTFP8_ERR_ALIGN;
     if (overlap(in, (size_t)n, out, (size_t)n * dtype_size(out_dtype))) return NTFP8_ERR_ALIAS;
     return run_dequant(in, fmt, scale_inv, 1, n, out, out_dtype, static_cast<hipStream_t>(stream));
+}
+
+int64_t ntfp8_column_sum_scratch(int64_t rows, int64_t cols) {
+    int64_t n;
+    if (!numel(rows, cols, &n)) return 0;
+    const int runs = column_sum_runs(rows, cols);
+    return runs > 1 ? runs * cols * (int64_t)sizeof(float) : 0;
+}
+
+int ntfp8_column_sum(const void* x, int x_dtype, int64_t rows, int64_t cols, void* out, int out_dtype, void* scratch, void* workspace,
+                     void* stream) {
+    int64_t n;
+    if (!x || !out || !workspace) return NTFP8_ERR_NULL;
+    if (!dtype_ok(x_dtype) || !dtype_ok(out_dtype)) return NTFP8_ERR_ENUM;
+    if (!numel(rows, cols, &n)) return NTFP8_ERR_SIZE;
+    const int64_t need = ntfp8_column_sum_scratch(rows, cols);
+    if (need > 0 && !scratch) return NTFP8_ERR_NULL;
+    if (!is_aligned(x, dtype_size(x_dtype)) || !is_aligned(out, dtype_size(out_dtype)) || !is_aligned(workspace, 4) ||
+        (scratch && !is_aligned(scratch, 4)))
+        return NTFP8_ERR_ALIGN;
+    const size_t xb = (size_t)n * dtype_size(x_dtype), ob = (size_t)cols * dtype_size(out_dtype);
+    if (overlap(x, xb, out, ob) || (need > 0 && (overlap(x, xb, scratch, (size_t)need) || overlap(out, ob, scratch, (size_t)need))))
+        return NTFP8_ERR_ALIAS;
+    return run_column_sum(x, x_dtype, rows, cols, out, out_dtype, static_cast<float*>(scratch), workspace, static_cast<hipStream_t>(stream));
 }
 
 int ntfp8_transpose(const void* in, int64_t rows, int64_t cols, void* out, void* stream) {

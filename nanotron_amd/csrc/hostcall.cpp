@@ -254,6 +254,39 @@ PyObject* gemm_fp8(PyObject* const* p) {
     return quantised(std::move(k.out), std::move(out_t), s);
 }
 
+// cast_with_scale(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None, amax = 0, scale)
+PyObject* cast_with_scale(PyObject* const* a) {
+    const at::Tensor x = dense(tensor(a[0]));
+    const int fmt = (int)number(a[2]);
+    const bool with_t = truth(a[3]);
+    int64_t rows, cols;
+    rows_cols(x, &rows, &cols);
+    require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    at::Tensor out = bytes_like(x, x.sizes()), out_t;
+    if (with_t) out_t = bytes_like(x, {cols, rows});
+    const Scalars s(x);
+    call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, static_cast<const float*>(tensor(a[1]).data_ptr()), fmt,
+                               s.p, s.p + 1, out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
+         "ntfp8_cast_with_scale");
+    return quantised(std::move(out), std::move(out_t), s);
+}
+
+// column_sum([rows, cols], out_code) -> [cols]
+PyObject* column_sum(PyObject* const* a) {
+    const at::Tensor x = dense(tensor(a[0]));
+    require(x.dim() == 2, "a 2-D tensor is expected");
+    const long code = number(a[1]);
+    const auto opt = at::TensorOptions().device(x.device());
+    at::Tensor out = at::empty({x.size(1)}, opt.dtype(type_of(code))), scratch;
+    const int64_t need = ntfp8_column_sum_scratch(x.size(0), x.size(1));
+    if (need > 0) scratch = at::empty({need / 4}, opt.dtype(at::kFloat));
+    void* st = stream_of(x);
+    call(ntfp8_column_sum(x.data_ptr(), code_of(x.scalar_type()), x.size(0), x.size(1), out.data_ptr(), (int)code,
+                          need > 0 ? scratch.data_ptr() : nullptr, workspace_of(x, st), st),
+         "ntfp8_column_sum");
+    return wrap(std::move(out));
+}
+
 // cast(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None)
 PyObject* cast(PyObject* const* a) {
     const at::Tensor x = dense(tensor(a[0]));
@@ -347,7 +380,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 5),
-                         NT_METHOD(cast, 4), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
+                         NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
                          NT_METHOD(operand_form, 10), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -197,8 +197,8 @@ __device__ inline uint32_t collect_amax(Workspace* ws) {
     return bits;
 }
 
-// bookkeep: what one tensor role learns from the amax `bits` of this launch.
-__device__ inline void bookkeep(uint32_t bits, const ScalarIO& io, int mode, const EpiloguePrefetch& pre) {
+// bookkeep: what one tensor role learns from the amax `bits` of this launch.  Returns the scale in force.
+__device__ inline float bookkeep(uint32_t bits, const ScalarIO& io, int mode, const EpiloguePrefetch& pre) {
     const int lane = threadIdx.x;
     const float a = __uint_as_float(bits);
     float used;
@@ -244,6 +244,7 @@ __device__ inline void bookkeep(uint32_t bits, const ScalarIO& io, int mode, con
         if (io.hist) *io.scale_state = update_scale(__uint_as_float(hm), used, io.fmt, io.margin);
         if (io.init_flag && bits != 0u && bits < kInfBits) *io.init_flag = 1.0f;
     }
+    return used;
 }
 
 __device__ inline void clear_workspace(Workspace* ws) {
@@ -313,6 +314,14 @@ __device__ __forceinline__ bool degenerate_scale(float s) {
     return b == 0u || b >= kInfBits;
 }
 
+// Cast-only launches: the scale the bytes were made with, beside an amax of zero (none was taken).
+__device__ __forceinline__ void record_cast_scale(const ScalarIO& io, float scale, uint32_t bid) {
+    if (io.scale_out && bid == 0 && threadIdx.x == 0) {
+        *io.scale_out = scale;
+        *io.amax_out = 0.0f;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Flat (no transpose) kernel: amax only, cast only, or both (delayed scaling).
 template <typename S, int F, int MODE>
@@ -328,6 +337,7 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
         scale = *scale_ptr;
         degen = degenerate_scale(scale);
     }
+    if constexpr (!kAmax) record_cast_scale(io, scale, bid);
     EpiloguePrefetch pre = {0.0f, 1.0f};
     if constexpr (kAmax) pre = prefetch_epilogue(io, MODE);
     uint32_t m_run = 0;  // in source-format bits
@@ -575,6 +585,7 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
     const int cgrp = threadIdx.x % (T::kT / E), rgrp = threadIdx.x / (T::kT / E);
     EpiloguePrefetch pre = {0.0f, 1.0f};
     if constexpr (kAmax) pre = prefetch_epilogue(io, kModeDelayed);
+    else record_cast_scale(io, scale, blockIdx.x);
     uint32_t m_run = 0;
     // persistent over tiles: the number of blocks (and so of reduction atomics) stays small
     for (int64_t tile_id = blockIdx.x; tile_id < tiles; tile_id += gridDim.x) {
@@ -657,6 +668,151 @@ __global__ __launch_bounds__(kTileThreads) void transpose_kernel(const uint8_t* 
         emit_columns<E>(tile, out, rows, cols, row0, col0);
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Current scaling of a small tensor in one launch: one workgroup holds all of it in registers, takes the amax, decides
+// on the scale (with everything the amax-only launch books: history, first use) and casts.  The two launches this
+// replaces cost their latency twice (fp32 128 x 128 with its transposed copy 4.9 + 3.7 us, and another 3 us of host
+// time); one workgroup is slower than the chip from about kOnceMax elements on.  With a transposed copy the bytes pass
+// through LDS, one word of padding per row, and leave as words of four rows.
+constexpr int kOnceGroups = 4;
+constexpr int64_t kOnceMax = (int64_t)kOnceGroups * kFlatThreads * kVec;   // 65536 elements
+template <typename S, int F, bool kT>
+__global__ __launch_bounds__(kFlatThreads) void quant_once_kernel(const typename ElemOf<S>::type* __restrict__ x, int rows, int cols,
+                                                              uint8_t* __restrict__ out, uint8_t* __restrict__ out_t, ScalarIO io) {
+    typedef Src<S> L;
+    __shared__ uint32_t s_part[kFlatThreads / 64];
+    __shared__ float s_scale;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[kT ? kOnceMax / 4 + kOnceMax / 16 : 1];
+    const int n = rows * cols, n_vec = n / kVec, t = threadIdx.x;
+    const EpiloguePrefetch pre = prefetch_epilogue(io, kModeAmaxOnly);
+    float v[kOnceGroups][kVec];
+    uint32_t m[kOnceGroups] = {0, 0, 0, 0}, mt = 0;
+    float tail = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kOnceGroups; ++i)
+        if (t + i * kFlatThreads < n_vec) L::template load<kVec, false>(x + (t + i * kFlatThreads) * kVec, v[i], m[i]);
+    const int j = n_vec * kVec + t;
+    if (j < n) tail = L::load1(x + j, mt);
+    uint32_t mr = mt;
+#pragma unroll
+    for (int i = 0; i < kOnceGroups; ++i) mr = m[i] > mr ? m[i] : mr;
+    const uint32_t wm = wave_max_u32(mr);
+    if ((t & 63) == 0) s_part[t >> 6] = wm;
+    __syncthreads();
+    if (t < 64) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < kFlatThreads / 64; ++i) bits = s_part[i] > bits ? s_part[i] : bits;
+        bits = L::to_f32_bits(bits);
+        if (bits > kInfBits) bits = kNanBits;
+        const float used = bookkeep(bits, io, kModeAmaxOnly, pre);
+        if (t == 0) s_scale = used;
+    }
+    __syncthreads();
+    const float scale = s_scale;
+    const bool degen = degenerate_scale(scale);
+    const int pitch = cols / 4 + 1;   // words
+#pragma unroll
+    for (int i = 0; i < kOnceGroups; ++i) {
+        const int g = t + i * kFlatThreads;
+        if (g >= n_vec) break;
+        const u4 q = encode16<F>(v[i], scale, degen || L::has_nan(m[i]));
+        if (out) *reinterpret_cast<u4*>(out + g * kVec) = q;
+        if constexpr (kT) {   // (cols is a multiple of 16: a group lies in one row)
+            const int r = g * kVec / cols, c = g * kVec % cols;
+            uint32_t* p = tile + r * pitch + c / 4;
+            p[0] = q.x, p[1] = q.y, p[2] = q.z, p[3] = q.w;
+        }
+    }
+    if (j < n) out[j] = encode1<F>(tail, scale);
+    if constexpr (kT) {
+        __syncthreads();
+        const int quads = rows / 4;   // rows is a multiple of 4
+        for (int b = t; b < quads * (cols / 4); b += kFlatThreads) {
+            const int r = b % quads, c = b / quads;
+            const uint32_t* p = tile + 4 * r * pitch + c;
+            const uint32_t w0 = p[0], w1 = p[pitch], w2 = p[2 * pitch], w3 = p[3 * pitch];
+            const uint32_t lo01 = __builtin_amdgcn_perm(w1, w0, 0x05010400u), lo23 = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
+            const uint32_t hi01 = __builtin_amdgcn_perm(w1, w0, 0x07030602u), hi23 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+            uint32_t* o = reinterpret_cast<uint32_t*>(out_t) + c * 4 * quads + r;
+            o[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+            o[quads] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+            o[2 * quads] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+            o[3 * quads] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Column sums in fp32 (the bias gradient: the output gradient summed over the tokens), rounded once to the output type.
+// HBM-bound on large tensors, latency-bound on small ones.  A workgroup sums a run of rows of 64 columns, 16 threads of
+// 4 columns side by side and 16 rows of them; the runs of one column block are put together by the workgroup that
+// arrives last, in order, so the result does not depend on timing.  Partial sums and tickets go through device-scope
+// accesses, as the reductions above.
+template <int OUT>
+__device__ __forceinline__ void store_dequant1(void* __restrict__ out, int64_t j, float v);
+constexpr int kSumCols = 64, kSumTickets = NTFP8_WORKSPACE_BYTES / 4;
+template <typename S, bool kVec4>
+__global__ __launch_bounds__(kThreads) void column_sum_kernel(const typename ElemOf<S>::type* __restrict__ x, int64_t rows, int64_t cols,
+                                                          int64_t run, void* __restrict__ out, int out_dtype,
+                                                          float* __restrict__ partial, uint32_t* __restrict__ tickets) {
+    typedef Src<S> L;
+    __shared__ float part[16][kSumCols];
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int64_t c = (int64_t)blockIdx.x * kSumCols + tx * 4;
+    const int64_t r0 = blockIdx.y * run, r1 = min(r0 + run, rows);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    auto row = [&](int64_t r, float (&v)[4]) {
+        uint32_t m;
+        if constexpr (kVec4) {
+            if (c < cols) L::template load<4, false>(x + r * cols + c, v, m);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = L::load1(x + r * cols + (c + e < cols ? c + e : cols - 1), m);
+        }
+    };
+    int64_t r = r0 + ty;
+    for (; r + 48 < r1; r += 64) {
+        float v[4][4] = {};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) row(r + 16 * u, v[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += v[u][e];
+    }
+    for (; r < r1; r += 16) {
+        float v[4] = {};
+        row(r, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[ty][tx * 4 + e] = s[e];
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    float total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) total += part[i][threadIdx.x];
+    const int64_t col = (int64_t)blockIdx.x * kSumCols + threadIdx.x;
+    if (gridDim.y > 1) {
+        if (col < cols) __hip_atomic_store(partial + blockIdx.y * cols + col, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's sums are in place before its ticket is drawn
+        uint32_t ticket = 0;
+        if (threadIdx.x == 0) ticket = __hip_atomic_fetch_add(tickets + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(ticket) != gridDim.y - 1) return;
+        if (threadIdx.x == 0) __hip_atomic_store(tickets + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        total = 0.0f;
+        if (col < cols)
+            for (uint32_t y = 0; y < gridDim.y; ++y)
+                total += __hip_atomic_load(partial + y * cols + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (col >= cols) return;
+    if (out_dtype == NTFP8_F32) store_dequant1<NTFP8_F32>(out, col, total);
+    else if (out_dtype == NTFP8_F16) store_dequant1<NTFP8_F16>(out, col, total);
+    else store_dequant1<NTFP8_BF16>(out, col, total);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -873,6 +1029,71 @@ static int dispatch_fmt_tr(int fmt, bool with_amax, const void* x, int64_t rows,
 }
 
 static bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+
+int run_quant(int mode, const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, uint8_t* out, uint8_t* out_t,
+              const float* scale_ptr, Workspace* ws, const ScalarIO& io, hipStream_t st);
+
+template <typename S>
+static void launch_once(int fmt, const void* x, int rows, int cols, uint8_t* out, uint8_t* out_t, const ScalarIO& io, hipStream_t st) {
+    const typename ElemOf<S>::type* xp = static_cast<const typename ElemOf<S>::type*>(x);
+#define NT_ONCE(F, T) hipLaunchKernelGGL((quant_once_kernel<S, F, T>), dim3(1), dim3(kFlatThreads), 0, st, xp, rows, cols, out, out_t, io)
+    if (fmt == kE4M3) {
+        if (out_t) NT_ONCE(kE4M3, true);
+        else NT_ONCE(kE4M3, false);
+    } else {
+        if (out_t) NT_ONCE(kE5M2, true);
+        else NT_ONCE(kE5M2, false);
+    }
+#undef NT_ONCE
+}
+
+// Current scaling (or a role's first use): amax, scale, cast.  One launch of one workgroup for small tensors, two launches
+// otherwise.
+int run_quant_current(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, uint8_t* out, uint8_t* out_t, Workspace* ws,
+                      const ScalarIO& io, hipStream_t st) {
+    const int64_t n = rows * cols;
+    if (n <= kOnceMax && out && aligned(x, 16) && aligned(out, 16) &&
+        (!out_t || (cols % kVec == 0 && rows % 4 == 0 && aligned(out_t, 4)))) {
+        clear_stale_error();
+        switch (x_dtype) {
+            case NTFP8_F32: launch_once<float>(fmt, x, (int)rows, (int)cols, out, out_t, io, st); break;
+            case NTFP8_F16: launch_once<f16_tag>(fmt, x, (int)rows, (int)cols, out, out_t, io, st); break;
+            default: launch_once<bf16_tag>(fmt, x, (int)rows, (int)cols, out, out_t, io, st); break;
+        }
+        return check_launch();
+    }
+    const int rc = run_quant(kModeAmaxOnly, x, x_dtype, n, 1, fmt, nullptr, nullptr, nullptr, ws, io, st);
+    if (rc != NTFP8_OK) return rc;
+    const ScalarIO none = {nullptr, nullptr, nullptr, nullptr, nullptr, 0, fmt, 0};
+    return run_quant(kModeCastOnly, x, x_dtype, rows, cols, fmt, out, out_t, io.scale_out, nullptr, none, st);
+}
+
+// row runs of a column sum: about two workgroups per CU, no run shorter than 64 rows
+int column_sum_runs(int64_t rows, int64_t cols) {
+    const int64_t blocks = (cols + kSumCols - 1) / kSumCols;
+    if (blocks > kSumTickets) return 1;
+    int64_t runs = 2 * (int64_t)cu_count() / blocks;
+    if (runs > (rows + 63) / 64) runs = (rows + 63) / 64;
+    return (int)(runs < 1 ? 1 : runs > 64 ? 64 : runs);
+}
+
+int run_column_sum(const void* x, int x_dtype, int64_t rows, int64_t cols, void* out, int out_dtype, float* partial, void* ws, hipStream_t st) {
+    clear_stale_error();
+    const int runs = column_sum_runs(rows, cols);
+    const int64_t blocks = (cols + kSumCols - 1) / kSumCols;
+    if (blocks > 0x7fffffff) return NTFP8_ERR_SIZE;
+    const int64_t run = ((rows + runs - 1) / runs + 15) / 16 * 16;
+    const dim3 grid((unsigned)blocks, (unsigned)((rows + run - 1) / run));
+    uint32_t* tk = static_cast<uint32_t*>(ws);
+#define NT_SUM(S) \
+    if (cols % 4 == 0) hipLaunchKernelGGL((column_sum_kernel<S, true>), grid, dim3(kThreads), 0, st, static_cast<const ElemOf<S>::type*>(x), rows, cols, run, out, out_dtype, partial, tk); \
+    else hipLaunchKernelGGL((column_sum_kernel<S, false>), grid, dim3(kThreads), 0, st, static_cast<const ElemOf<S>::type*>(x), rows, cols, run, out, out_dtype, partial, tk)
+    if (x_dtype == NTFP8_F32) { NT_SUM(float); }
+    else if (x_dtype == NTFP8_F16) { NT_SUM(f16_tag); }
+    else { NT_SUM(bf16_tag); }
+#undef NT_SUM
+    return check_launch();
+}
 
 // mode: kModeAmaxOnly / kModeCastOnly / kModeDelayed.  out_t may be NULL.
 int run_quant(int mode, const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, uint8_t* out, uint8_t* out_t,

@@ -4,6 +4,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from nanotron_amd import _native as nt
 from nanotron_amd.fp8.constants import INITIAL_AMAX, INITIAL_SCALING_FACTOR
 from nanotron_amd.fp8.dtypes import DTypes
 from nanotron_amd.fp8.kernel import a_transposed_supported, fp8_matmul_kernel, fp8_matmul_pair, needs_transposed_copy
@@ -324,7 +325,11 @@ class _FP8Matmul(torch.autograd.Function):
                 from nanotron_amd.fp8.tensor import convert_tensor_from_fp8
 
                 g_hp = convert_tensor_from_fp8(g_hp, g_hp.fp8_meta, bias.dtype)
-            grad_bias = g_hp.reshape(-1, g_hp.shape[-1]).sum(0, dtype=torch.float32).to(bias.dtype)
+            g_hp = g_hp if g_hp.dim() == 2 else g_hp.reshape(-1, g_hp.shape[-1])
+            if g_hp.numel() and g_hp.dtype in nt.TORCH_TO_NT and bias.dtype in nt.TORCH_TO_NT:
+                grad_bias = nt.host.column_sum(g_hp, nt.TORCH_TO_NT[bias.dtype])
+            else:
+                grad_bias = g_hp.sum(0, dtype=torch.float32).to(bias.dtype)
 
         if type(grad_output) is torch.Tensor:
             g2d = grad_output if grad_output.dim() == 2 else grad_output.reshape(-1, grad_output.shape[-1])

@@ -230,10 +230,10 @@ def cast_with_scale(tensor: torch.Tensor, scale: torch.Tensor, dtype: DTypes, wi
     x = tensor.detach()
     dev = x.device
     assert dev.type != "cpu", "cast_with_scale only supports CUDA tensors"
-    scalars = torch.zeros(2, dtype=torch.float32, device=dev)  # [amax (not computed), scale]
-    scalars[1].copy_(scale.reshape(()).to(device=dev, dtype=torch.float32))
-    out, out_t = nt.host.cast(x, scalars[1], _FMT[dtype], with_transpose)
-    return _assemble(FP8Tensor, dtype, out, out_t, scalars[0], scalars[1])
+    scale = scale.reshape(())
+    if scale.device != dev or scale.dtype != torch.float32:
+        scale = scale.to(device=dev, dtype=torch.float32)
+    return _assemble(FP8Tensor, dtype, *nt.host.cast_with_scale(x, scale, _FMT[dtype], with_transpose))
 
 
 def convert_torch_dtype_to_te_dtype(dtype) -> DType:
