@@ -265,6 +265,12 @@ int ntfp8_gemm_batch(const ntfp8_gemm_desc* problems, int count, void* stream);
 int ntfp8_amax_finalize(void* workspace, int fmt, int margin, float* scale_state, float* amax_history,
                         int history_len, float* amax_out, float* scale_used_out, void* stream);
 
+/* A GEMM with an fp8 output and the bookkeeping of its role in one call: ntfp8_gemm_batch on `problem` (d_dtype
+ * NTFP8_OUT_*, amax_workspace given), then ntfp8_amax_finalize, same results; the bookkeeping is done by the workgroup
+ * that finishes last wherever the kernel serving the shape can. */
+int ntfp8_gemm_fp8(const ntfp8_gemm_desc* problem, int margin, float* scale_state, float* amax_history, int history_len,
+                   float* amax_out, float* scale_used_out, void* stream);
+
 /* Bandwidth yardstick: a kernel with the access pattern of the flat quantise kernels (same workgroup size, same grid,
  * 128-bit streaming loads and stores) and none of their arithmetic, so that a quantise figure can be set against what
  * the memory system gives that pattern on the same GPU in the same run.  It has no counterpart in the reference; it is

@@ -442,6 +442,24 @@ int ntfp8_gemm_batch(const ntfp8_gemm_desc* problems, int count, void* stream) {
     return run_gemm_batch(g, count, static_cast<hipStream_t>(stream));
 }
 
+int ntfp8_gemm_fp8(const ntfp8_gemm_desc* problem, int margin, float* scale_state, float* amax_history, int history_len,
+                   float* amax_out, float* scale_used_out, void* stream) {
+    if (!problem || !problem->amax_workspace || !scale_state || !amax_out) return NTFP8_ERR_NULL;
+    if (!is_fp8_out(problem->d_dtype)) return NTFP8_ERR_ENUM;
+    if (margin < -kMaxMargin || margin > kMaxMargin) return NTFP8_ERR_SIZE;
+    if (amax_history ? (history_len < 1 || history_len > kMaxHistory) : history_len != 0) return NTFP8_ERR_SIZE;
+    if (!is_aligned(scale_state, 4) || !is_aligned(amax_out, 4) || (amax_history && !is_aligned(amax_history, 4)) ||
+        (scale_used_out && !is_aligned(scale_used_out, 4)))
+        return NTFP8_ERR_ALIGN;
+    GemmDesc g;
+    const int rc = check_gemm(*problem, &g);
+    if (rc) return rc;
+    const ScalarIO io = {nullptr, amax_out, scale_used_out, scale_state, amax_history, history_len,
+                         problem->d_dtype == NTFP8_OUT_E4M3 ? NTFP8_E4M3 : NTFP8_E5M2, margin};
+    g.fin = &io;
+    return run_gemm_batch(&g, 1, static_cast<hipStream_t>(stream));
+}
+
 int ntfp8_amax_finalize(void* workspace, int fmt, int margin, float* scale_state, float* amax_history, int history_len,
                         float* amax_out, float* scale_used_out, void* stream) {
     if (!workspace || !scale_state || !amax_out) return NTFP8_ERR_NULL;

@@ -28,6 +28,7 @@ enum GemmPath { kPathNone = -1, kPathAny = 0, kPathWords = 1, kPathTiles = 2 };
 int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_words(const GemmDesc& g, hipStream_t st);
+int run_amax_finalize(Workspace* ws, const ScalarIO& io, hipStream_t st);
 
 // operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
 static bool fits32(const GemmDesc& g) {
@@ -141,10 +142,15 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     const bool fp8_out = is_fp8_out(g[0]->d_dtype);
     L.round_size = cu_count() * (edge == 64 ? 2 : 1);
+    if (n == 1 && g[0]->fin) {
+        L.fin = *g[0]->fin;
+        L.fin_blocks = (int)tiles;
+    }
     if (edge != 256) return launch_mid(L, FA, FB, edge, fp8_out, (int)tiles, st);
     const int rem = (int)(tiles % cu_count());
     L.tail_tiles = (rem != 0 && 2 * rem <= cu_count()) ? rem : 0;
     L.full_blocks = (int)tiles - L.tail_tiles;
+    if (L.fin_blocks) L.fin_blocks = L.full_blocks + 2 * L.tail_tiles;
     (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
     auto go = [&](auto fp8_tag, auto bt_tag) {
         constexpr bool kFp8Out = decltype(fp8_tag)::value, kBT = decltype(bt_tag)::value;
@@ -176,6 +182,10 @@ static int launch_any_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     int64_t tiles = list_tiles(g, n, edge, &L);
     if (tiles < cu_count()) tiles = list_tiles(g, n, edge = 64, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
+    if (n == 1 && g[0]->fin) {
+        L.fin = *g[0]->fin;
+        L.fin_blocks = (int)tiles;
+    }
     return launch_any(L, g[0]->fmt_a, g[0]->fmt_b, edge, is_fp8_out(g[0]->d_dtype), (int)tiles, st);
 }
 
@@ -189,7 +199,10 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     return launch_tiles<kE4M3, kE4M3>(g, n, st);
 #else
     if (path == kPathAny) return launch_any_tiles(g, n, st);
-    if (path == kPathWords) return launch_words(*g[0], st);
+    if (path == kPathWords) {
+        const int rc = launch_words(*g[0], st);
+        return rc == NTFP8_OK && g[0]->fin ? run_amax_finalize(static_cast<Workspace*>(g[0]->ws), *g[0]->fin, st) : rc;
+    }
     if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, st) : launch_tiles<kE4M3, kE5M2>(g, n, st);
     return fb == kE4M3 ? launch_tiles<kE5M2, kE4M3>(g, n, st) : launch_tiles<kE5M2, kE5M2>(g, n, st);
 #endif

@@ -166,6 +166,7 @@ __global__ __launch_bounds__(kAnyThreads) void gemm_any_kernel(const BigLaunch L
                                   ? store_wave_tile_fp8<kE4M3, MB, MB>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, d_aligned)
                                   : store_wave_tile_fp8<kE5M2, MB, MB>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, d_aligned);
         publish_amax(amax, P.fp8.ws);
+        finish_fp8(L, P.fp8.ws, blockIdx.x);
     } else if (P.d_dtype == NTFP8_BF16) {
         store_wave_tile<NTFP8_BF16, false, MB, MB>(acc, P.D, alpha, M, N, mb, nb, lane, d_aligned);
     } else if (P.d_dtype == NTFP8_F16) {

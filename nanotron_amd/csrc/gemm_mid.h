@@ -212,6 +212,7 @@ __global__ __launch_bounds__(kBigThreads, T == 128 ? 1 : 2) void gemm_mid_kernel
                                       ? store_wave_tile16_fp8<kE4M3, MI, NJ, kBias, true>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv, P.at)
                                       : store_wave_tile16_fp8<kE5M2, MI, NJ, kBias, true>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv, P.at);
             publish_amax(amax, P.fp8.ws);
+            finish_fp8(L, P.fp8.ws, blockIdx.x);
         } else if (P.d_dtype == NTFP8_BF16) {
             store_wave_tile16<NTFP8_BF16, false, MI, NJ, kBias>(acc, P.D, alpha, M, N, mb, nb, lane, bv);
         } else if (P.d_dtype == NTFP8_F16) {

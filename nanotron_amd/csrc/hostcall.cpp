@@ -231,17 +231,17 @@ PyObject* gemm_batch(PyObject* const* args) {
     return out;
 }
 
-// gemm_fp8(problem fields..., state, history_len, margin, fmt, with_transpose) -> (bytes, bytes^T | None, amax, scale):
-// the epilogue casts with the held scale, a one-wave kernel behind it does the bookkeeping
+// gemm_fp8(problem fields..., state, history_len, margin, with_transpose) -> (bytes, bytes^T | None, amax, scale):
+// the epilogue casts with the held scale, the workgroup that finishes last does the bookkeeping
 PyObject* gemm_fp8(PyObject* const* p) {
     ntfp8_gemm_desc d = {};
     Problem k;
     fill(p, &d, &k, true);
     const at::Tensor& state = tensor(p[kProblem]);
-    const int hist = (int)number(p[kProblem + 1]), margin = (int)number(p[kProblem + 2]), fmt = (int)number(p[kProblem + 3]);
+    const int hist = (int)number(p[kProblem + 1]), margin = (int)number(p[kProblem + 2]);
     require(state.device() == k.a.device(), "delayed-scaling state on another device");
     at::Tensor out_t;
-    if (truth(p[kProblem + 4])) out_t = bytes_like(k.a, {d.N, d.M});
+    if (truth(p[kProblem + 3])) out_t = bytes_like(k.a, {d.N, d.M});
     const Scalars s(k.a);
     void* st = stream_of(k.a);
     void* ws = workspace_of(k.a, st);
@@ -249,8 +249,7 @@ PyObject* gemm_fp8(PyObject* const* p) {
     d.scale_d = buf;
     d.D_t = out_t.defined() ? out_t.data_ptr() : nullptr;
     d.amax_workspace = ws;
-    call(ntfp8_gemm_batch(&d, 1, st), "ntfp8_gemm_batch");
-    call(ntfp8_amax_finalize(ws, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, st), "ntfp8_amax_finalize");
+    call(ntfp8_gemm_fp8(&d, margin, buf, buf + 1, hist, s.p, s.p + 1, st), "ntfp8_gemm_fp8");
     return quantised(std::move(k.out), std::move(out_t), s);
 }
 
@@ -379,7 +378,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 5),
+PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
                          NT_METHOD(operand_form, 10), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

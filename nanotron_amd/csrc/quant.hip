@@ -3,6 +3,7 @@
 // over the input with 128-bit loads and stores, a wavefront reduction for the amax, one atomic per
 // block and a last-block epilogue that finishes the scalar bookkeeping in the same launch.
 #include "common.h"
+#include "reduce.h"
 
 namespace ntfp8 {
 
@@ -159,151 +160,7 @@ __device__ __forceinline__ uint8_t encode1(float x, float scale) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Block reduction of the partial max, publication, and the last-block epilogue.
-//
-// Inter-block traffic uses relaxed device-scope atomics only (they execute at the level where all
-// XCDs agree) and orders them with the wave's own memory counter: the partial max is folded in with
-// a returning atomic, the wave waits for it, then takes a ticket.  A release fence here would write
-// back the whole L2 once per block, which costs more than the streaming pass itself.
-// What the last block's epilogue will read, requested by the first wave of every block while the
-// tensor is still streaming: the history entry that moves into this lane's slot and the scale in
-// force.  It takes one round trip out of the dependent chain at the end of the kernel.
-struct EpiloguePrefetch {
-    float hist_prev;  // hist[lane - 1] (lanes 1 .. hist_len-1; histories of up to 64 entries)
-    float scale;      // *scale_state; amax-only mode: *old_scale (1.0 if there is none)
-};
-__device__ __forceinline__ EpiloguePrefetch prefetch_epilogue(const ScalarIO& io, int mode) {
-    EpiloguePrefetch p = {0.0f, 1.0f};
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        if (io.hist && io.hist_len <= 64 && lane >= 1 && lane < io.hist_len) p.hist_prev = io.hist[lane - 1];
-        if (mode != kModeAmaxOnly) p.scale = *io.scale_state;
-        else if (io.old_scale) p.scale = *io.old_scale;
-    }
-    return p;
-}
-
-// Bookkeeping of one launch, run by one wave (lanes 0..63 of a workgroup) once every workgroup's maximum is in
-// the slots: amax, history roll, next scale; leaves the workspace zeroed.  Every global access is one round
-// trip for the whole wave instead of one per history entry.
-//
-// collect_amax: the maximum over the slots as a bit pattern (NaN patterns normalised to the quiet NaN).
-__device__ inline uint32_t collect_amax(Workspace* ws) {
-    const int lane = threadIdx.x;
-    uint32_t bits = 0;
-    if (lane < kMaxSlots) bits = __hip_atomic_load(&ws->slot[lane].bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    bits = wave_max_u32(bits);
-    if (bits > kInfBits) bits = kNanBits;
-    return bits;
-}
-
-// bookkeep: what one tensor role learns from the amax `bits` of this launch.  Returns the scale in force.
-__device__ inline float bookkeep(uint32_t bits, const ScalarIO& io, int mode, const EpiloguePrefetch& pre) {
-    const int lane = threadIdx.x;
-    const float a = __uint_as_float(bits);
-    float used;
-    if (mode == kModeAmaxOnly) {
-        // (the flag and the held scale are read here, before lane 0 writes either below)
-        if (io.init_flag && *io.init_flag != 0.0f) used = *io.scale_state;
-        else used = update_scale(a, pre.scale, io.fmt, io.margin);
-    } else {
-        used = pre.scale;
-    }
-    uint32_t hm = bits;
-    if (io.hist && io.hist_len <= 64) {
-        const bool ok = lane < io.hist_len;
-        const float h = lane == 0 ? a : pre.hist_prev;
-        if (ok) io.hist[lane] = h;
-        const uint32_t hb = wave_max_u32(ok ? (__float_as_uint(h) & 0x7fffffffu) : 0u);
-        hm = hb > hm ? hb : hm;
-        if (hm > kInfBits) hm = kNanBits;
-    } else if (io.hist) {
-        // hist[i] <- hist[i-1], hist[0] <- a; 64 entries per trip, highest chunk first so that an entry is
-        // read before the chunk below overwrites it
-        for (int base = ((io.hist_len - 1) / 64) * 64; base >= 0; base -= 64) {
-            const int i = base + lane;
-            const bool ok = i < io.hist_len;
-            float h = 0.0f;
-            if (ok) h = (i == 0) ? a : io.hist[i - 1];
-            if (ok) io.hist[i] = h;
-            const uint32_t hb = wave_max_u32(ok ? (__float_as_uint(h) & 0x7fffffffu) : 0u);
-            hm = hb > hm ? hb : hm;
-        }
-        if (hm > kInfBits) hm = kNanBits;
-    }
-    if (lane == 0) {
-        uint32_t out_bits = bits;
-        if (io.amax_in) {   // running maximum kept by the caller (NaN patterns compare above everything)
-            uint32_t prev = __float_as_uint(*io.amax_in) & 0x7fffffffu;
-            if (prev > kInfBits) prev = kNanBits;
-            out_bits = prev > out_bits ? prev : out_bits;
-        }
-        if (io.amax_out) *io.amax_out = __uint_as_float(out_bits);
-        if (io.scale_out) *io.scale_out = used;
-        if (io.scale_inv_out) *io.scale_inv_out = 1.0f / used;
-        if (io.hist) *io.scale_state = update_scale(__uint_as_float(hm), used, io.fmt, io.margin);
-        if (io.init_flag && bits != 0u && bits < kInfBits) *io.init_flag = 1.0f;
-    }
-    return used;
-}
-
-__device__ inline void clear_workspace(Workspace* ws) {
-    const int lane = threadIdx.x;
-    if (lane == 0) __hip_atomic_store(&ws->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (lane < kMaxSlots) {
-        __hip_atomic_store(&ws->slot[lane].bits, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&ws->slot[lane].ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// `io2` / `pre2`: a second tensor role fed by the same amax (one source tensor quantised to both formats).
-__device__ inline void finalize_wave(Workspace* ws, const ScalarIO& io, int mode, const EpiloguePrefetch& pre,
-                                     const ScalarIO* io2 = nullptr, const EpiloguePrefetch* pre2 = nullptr) {
-    const uint32_t bits = collect_amax(ws);
-    bookkeep(bits, io, mode, pre);
-    if (io2) bookkeep(bits, *io2, mode, *pre2);
-    clear_workspace(ws);
-}
-
-// `bid` of `nblocks`: this workgroup's place among the workgroups that reduce the same tensor (the whole grid,
-// except in a launch that carries several tensors).
-template <int THREADS>
-__device__ inline void publish_and_finalize(uint32_t m_f32bits, Workspace* ws, const ScalarIO& io, int mode,
-                                            const EpiloguePrefetch& pre, uint32_t bid = blockIdx.x,
-                                            uint32_t nblocks = gridDim.x, const ScalarIO* io2 = nullptr,
-                                            const EpiloguePrefetch* pre2 = nullptr) {
-    __shared__ uint32_t s_part[THREADS / 64];
-    __shared__ bool s_last;
-    const uint32_t wm = wave_max_u32(m_f32bits);
-    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = wm;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t bm = 0;
-#pragma unroll
-        for (int i = 0; i < THREADS / 64; ++i) bm = s_part[i] > bm ? s_part[i] : bm;
-        // Two-level arrival count: a block publishes into the slot of its group and draws a ticket there; the
-        // last block of a group draws a ticket of the launch.  All blocks finish at about the same time, and
-        // their atomics on one address would queue one behind the other.
-        const uint32_t grp = bid % kMaxSlots;
-        const uint32_t old = __hip_atomic_fetch_max(&ws->slot[grp].bits, bm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::"v"(old) : "memory");   // the max is in place before the ticket is drawn
-        const uint32_t in_group = (nblocks - grp + kMaxSlots - 1) / kMaxSlots;
-        const uint32_t t = __hip_atomic_fetch_add(&ws->slot[grp].ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bool last = false;
-        if (t == in_group - 1) {
-            const uint32_t groups = nblocks < (uint32_t)kMaxSlots ? nblocks : (uint32_t)kMaxSlots;
-            const uint32_t t2 = __hip_atomic_fetch_add(&ws->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last = (t2 == groups - 1);
-        }
-        s_last = last;
-    }
-    __syncthreads();
-    // the epilogue runs on the first wave of the block that drew the last ticket
-    if (!s_last || threadIdx.x >= 64) return;
-    finalize_wave(ws, io, mode, pre, io2, pre2);
-}
-
-// The same bookkeeping for maxima that another kernel (the fp8-output GEMM epilogue) left in the slots.
+// The bookkeeping of reduce.h for maxima that another kernel (the fp8-output GEMM epilogue) left in the slots.
 __global__ __launch_bounds__(64) void amax_finalize_kernel(Workspace* ws, ScalarIO io) {
     const EpiloguePrefetch pre = prefetch_epilogue(io, kModeDelayed);
     finalize_wave(ws, io, kModeDelayed, pre);
@@ -805,9 +662,16 @@ __global__ __launch_bounds__(kThreads) void column_sum_kernel(const typename Ele
         if (__builtin_amdgcn_readfirstlane(ticket) != gridDim.y - 1) return;
         if (threadIdx.x == 0) __hip_atomic_store(tickets + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         total = 0.0f;
-        if (col < cols)
-            for (uint32_t y = 0; y < gridDim.y; ++y)
-                total += __hip_atomic_load(partial + y * cols + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int64_t at = col < cols ? col : cols - 1;
+        for (uint32_t y0 = 0; y0 < gridDim.y; y0 += 16) {   // 16 requested before the first is needed
+            float p[16];
+#pragma unroll
+            for (uint32_t y = 0; y < 16; ++y)
+                p[y] = __hip_atomic_load(partial + min(y0 + y, gridDim.y - 1) * cols + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (uint32_t y = 0; y < 16; ++y)
+                if (y0 + y < gridDim.y) total += p[y];
+        }
     }
     if (col >= cols) return;
     if (out_dtype == NTFP8_F32) store_dequant1<NTFP8_F32>(out, col, total);

@@ -28,8 +28,8 @@ def _gemm_nt(a: FP8Tensor, b: FP8Tensor, out_dtype: torch.dtype, accumulate_into
 def _gemm_nt_fp8(a: FP8Tensor, b: FP8Tensor, dtype: DTypes, state: Optional[DelayedScaling],
                  with_transpose: bool, bias: Optional[torch.Tensor] = None, bt: bool = False, at: bool = False) -> FP8Tensor:
     """FP8Tensor(_gemm_nt(a, b, float32), dtype, state=state, with_transpose=with_transpose), bit for bit, with the
-    fp32 result never written to memory: the GEMM epilogue casts with the scale `state` holds from earlier steps,
-    leaves max|result| behind, and a one-wave kernel turns that into amax, history roll and next scale.
+    fp32 result never written to memory: the GEMM epilogue casts with the scale `state` holds from earlier steps, and
+    the workgroup that finishes last turns max|result| into amax, history roll and next scale.
 
     The amax of a GEMM result is not known before the GEMM has run, so a step without a held scale (no `state`, or
     one that has not seen a usable amax yet) goes the long way: fp32 result, then the ordinary quantisation."""
@@ -41,7 +41,7 @@ def _gemm_nt_fp8(a: FP8Tensor, b: FP8Tensor, dtype: DTypes, state: Optional[Dela
     assert state.dtype == dtype, "delayed-scaling state was created for another format"
     assert not at or bt, "a transposed A operand is only read next to a transposed B operand"
     return _assemble(FP8Tensor, dtype, *nt.host.gemm_fp8(
-        *_problem(a, b, _OUT_FMT[dtype], None, bt, bias, at), state._buf, state.history_len, state.margin, _FMT[dtype], with_transpose))
+        *_problem(a, b, _OUT_FMT[dtype], None, bt, bias, at), state._buf, state.history_len, state.margin, with_transpose))
 
 
 # Module switch: False makes every GEMM use materialised transposed copies (the reference's way, kernel.py:43-44).

@@ -75,6 +75,7 @@ class FP8Linear(nn.Linear):
         self.fp8_grad_input = True
         self.fp8_grad_inputs_sent = 0   # backward passes of this layer that did so
         self._grad_box = None
+        self._zero_element = None
         self.scaling = None
         self._weight_ready = None
         if self.weight.device != torch.device("cpu"):
@@ -105,6 +106,16 @@ class FP8Linear(nn.Linear):
                 }
                 if isinstance(out_dtype, DTypes):
                     self.scaling["output"] = DelayedScaling(out_dtype, amax_history_len, margin, dev)
+
+    def _zero(self, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+        """A zero that stands for a whole tensor once expanded (the gradient handles, of which nothing is ever read).  The
+        layer keeps it, since filling one costs a launch; memory of a graph capture is not kept beyond it."""
+        z = self._zero_element
+        if z is None or z.dtype != dtype or z.device != device:
+            z = torch.zeros(1, dtype=dtype, device=device)
+            if not torch.cuda.is_current_stream_capturing():
+                self._zero_element = z
+        return z
 
     @torch.no_grad()
     def requantize_weight(self, stream: Optional[torch.cuda.Stream] = None) -> None:
@@ -277,7 +288,8 @@ class _FP8Matmul(torch.autograd.Function):
             ctx.mark_non_differentiable(output)
             ctx.grad_box = module._grad_box = _GradBox(scaling["output_grad"] if scaling else None)
             hp = weight.dtype if weight.dtype in (torch.float32, torch.float16, torch.bfloat16) else torch.float32
-            handle = torch.zeros(1, dtype=hp, device=output.device).expand(output.shape)
+            out_shape = output.as_subclass(torch.Tensor).shape
+            handle = module._zero(hp, weight.device).expand(out_shape)
             ctx.fp8_out = True
             return output, handle
         ctx.fp8_out = False
@@ -373,7 +385,7 @@ class _FP8Matmul(torch.autograd.Function):
             # the rounding to the high-precision type in between); autograd carries a placeholder without memory
             box.fp8_grad = fp8_matmul_kernel(mat_a=weight.data, transpose_a=False, mat_b=grad_output, transpose_b=False,
                                              use_split_accumulator=True, out_dtype=DTypes.FP8E5M2, out_state=box.state)
-            grad_input = torch.zeros(1, dtype=ctx.in_dtype or torch.float32, device=grad_output.device).expand(ctx.in_shape)
+            grad_input = module._zero(ctx.in_dtype or torch.float32, weight.device).expand(ctx.in_shape)
             module.fp8_grad_inputs_sent += 1
             if wgrad is not None:
                 grad_weight = fp8_matmul_kernel(**wgrad)
