@@ -152,6 +152,68 @@ PyObject* quantize(PyObject* const* a) {
     return quantised(std::move(out), std::move(out_t), s);
 }
 
+// [>= count] workspaces for the tensors of a batched call, one table entry per (device, stream)
+at::Tensor workspace_pool(const at::Tensor& t, void* stream, int64_t count) {
+    at::Tensor& w = workspaces()[Key{(int)t.get_device() + 1024, stream}];
+    if (!w.defined() || w.size(0) < count)
+        w = at::zeros({count < 16 ? 16 : count, NTFP8_WORKSPACE_BYTES / 4}, t.options().dtype(at::kInt));
+    return w;
+}
+
+// quantize_batch([(x, state, history_len, margin, with_transpose), ...], fmt) -> [(bytes, bytes^T | None, amax, scale), ...]:
+// the fused delayed-scaling step of several tensors, one library call
+PyObject* quantize_batch(PyObject* const* args) {
+    PyObject* const list = args[0];
+    const int fmt = (int)number(args[1]);
+    if (!PyList_Check(list)) stop(PyExc_TypeError, "a list of tensors is expected");
+    const Py_ssize_t n = PyList_GET_SIZE(list);
+    require(n >= 1 && n <= NTFP8_MAX_BATCH, "between 1 and 64 tensors");
+    std::vector<ntfp8_quant_desc> d(n);
+    std::vector<at::Tensor> x(n), out(n), out_t(n);
+    std::vector<Scalars> s;
+    s.reserve(n);
+    void* st = nullptr;
+    at::Tensor pool;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        PyObject* t = PyList_GET_ITEM(list, i);
+        if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 5) stop(PyExc_TypeError, "a tensor comes as a tuple of 5");
+        PyObject* const* f = &PyTuple_GET_ITEM(t, 0);
+        x[i] = dense(tensor(f[0]));
+        const at::Tensor& state = tensor(f[1]);
+        require(x[i].is_cuda() && x[i].device() == x[0].device() && state.device() == x[0].device(), "all tensors of a batch are on one device");
+        require(x[i].numel() > 0, "cannot quantise an empty tensor");
+        const bool with_t = truth(f[4]);
+        require(!with_t || x[i].dim() == 2, "with_transpose needs a 2-D tensor");
+        if (i == 0) {
+            st = stream_of(x[0]);
+            pool = workspace_pool(x[0], st, n);
+        }
+        ntfp8_quant_desc& q = d[i];
+        q = {};
+        rows_cols(x[i], &q.rows, &q.cols);
+        out[i] = bytes_like(x[i], x[i].sizes());
+        if (with_t) out_t[i] = bytes_like(x[i], {q.cols, q.rows});
+        s.emplace_back(x[i]);
+        q.x = x[i].data_ptr();
+        q.x_dtype = code_of(x[i].scalar_type());
+        q.fmt = fmt;
+        q.history_len = (int)number(f[2]);
+        q.margin = (int)number(f[3]);
+        q.scale_state = static_cast<float*>(state.data_ptr());
+        q.amax_history = q.scale_state + 1;
+        q.amax_out = s[i].p;
+        q.scale_used_out = s[i].p + 1;
+        q.out = out[i].data_ptr();
+        q.out_t = with_t ? out_t[i].data_ptr() : nullptr;
+        q.workspace = static_cast<char*>(pool.data_ptr()) + i * NTFP8_WORKSPACE_BYTES;
+    }
+    call(ntfp8_quantize_delayed_batch(d.data(), (int)n, st), "ntfp8_quantize_delayed_batch");
+    PyObject* res = PyList_New(n);
+    if (res == nullptr) throw Stop{};
+    for (Py_ssize_t i = 0; i < n; ++i) PyList_SET_ITEM(res, i, quantised(std::move(out[i]), std::move(out_t[i]), s[i]));
+    return res;
+}
+
 // One GEMM problem: (a, fmt_a, scale_a, b, fmt_b, scale_b, out_code, accumulate_into | None, b_transposed, bias | None,
 // a_transposed); fills the descriptor, keeps what it points to alive, returns the output
 constexpr int kProblem = 11;
@@ -378,7 +440,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
+PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
                          NT_METHOD(operand_form, 10), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

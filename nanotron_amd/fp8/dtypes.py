@@ -9,6 +9,12 @@ class DTypes(Enum):
     KFLOAT16 = auto()
 
 
+# The native library's codes of a format (storage, and as a GEMM's output type), as plain attributes: a dictionary keyed by
+# enum members hashes in Python on every look-up.  KFLOAT16 is no FP8 format.
+for _member, _code, _out_code in ((DTypes.FP8E4M3, 0, 3), (DTypes.FP8E5M2, 1, 4), (DTypes.KFLOAT16, None, None)):
+    _member.code, _member.out_code = _code, _out_code
+
+
 class DType(IntEnum):
     """Element types understood by the native library; member names follow tex.DType
     (used at src/nanotron/fp8/tensor.py:39-55)."""

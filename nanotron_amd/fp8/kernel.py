@@ -6,15 +6,12 @@ from nanotron_amd import _native as nt
 from nanotron_amd.fp8.dtypes import DTypes
 from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, _assemble
 
-_FMT = {DTypes.FP8E4M3: nt.E4M3, DTypes.FP8E5M2: nt.E5M2}
-_OUT_FMT = {DTypes.FP8E4M3: nt.OUT_E4M3, DTypes.FP8E5M2: nt.OUT_E5M2}
-
 
 def _problem(a: FP8Tensor, b: FP8Tensor, out_code: int, accumulate_into=None, bt: bool = False, bias=None, at: bool = False):
     """The fields of one GEMM as csrc/hostcall.cpp takes them.  (A meta is a Python attribute of the FP8Tensor object; a
     copy made of a view does not carry it, so it is read here and the extension makes the copy.)"""
     ma, mb = a.fp8_meta, b.fp8_meta
-    return (a, _FMT[ma.dtype], ma.scale, b, _FMT[mb.dtype], mb.scale, out_code, accumulate_into, bt, bias, at)
+    return (a, ma.dtype.code, ma.scale, b, mb.dtype.code, mb.scale, out_code, accumulate_into, bt, bias, at)
 
 
 def _gemm_nt(a: FP8Tensor, b: FP8Tensor, out_dtype: torch.dtype, accumulate_into: Optional[torch.Tensor],
@@ -33,7 +30,7 @@ def _gemm_nt_fp8(a: FP8Tensor, b: FP8Tensor, dtype: DTypes, state: Optional[Dela
 
     The amax of a GEMM result is not known before the GEMM has run, so a step without a held scale (no `state`, or
     one that has not seen a usable amax yet) goes the long way: fp32 result, then the ordinary quantisation."""
-    assert dtype in _OUT_FMT, f"{dtype} is not an FP8 format"
+    assert dtype.out_code is not None, f"{dtype} is not an FP8 format"
     if state is None or not state.known_initialised:
         hp = (_gemm_nt_batch([(a, b, torch.float32, None, True, None, at)])[0] if bt
               else _gemm_nt(a, b, torch.float32, None, bias))
@@ -41,7 +38,7 @@ def _gemm_nt_fp8(a: FP8Tensor, b: FP8Tensor, dtype: DTypes, state: Optional[Dela
     assert state.dtype == dtype, "delayed-scaling state was created for another format"
     assert not at or bt, "a transposed A operand is only read next to a transposed B operand"
     return _assemble(FP8Tensor, dtype, *nt.host.gemm_fp8(
-        *_problem(a, b, _OUT_FMT[dtype], None, bt, bias, at), state._buf, state.history_len, state.margin, with_transpose))
+        *_problem(a, b, dtype.out_code, None, bt, bias, at), state._buf, state.history_len, state.margin, with_transpose))
 
 
 # Module switch: False makes every GEMM use materialised transposed copies (the reference's way, kernel.py:43-44).
@@ -110,7 +107,7 @@ def fp8_matmul_pair(first: dict, second: dict):
     for kw in (first, second):
         acc = kw.get("accumulate_into")
         A, B, bt, at = _operands(kw["mat_a"], kw["transpose_a"], kw["mat_b"], kw["transpose_b"], acc)
-        probs.append((A, B, (kw.get("out_dtype") or torch.float32) if acc is None else torch.float32, acc, bt, None, at))
+        probs.append((A, B, torch.float32 if acc is not None else kw.get("out_dtype") or torch.float32, acc, bt, None, at))
     return _gemm_nt_batch(probs)
 
 

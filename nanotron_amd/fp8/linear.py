@@ -391,9 +391,7 @@ class _FP8Matmul(torch.autograd.Function):
                 grad_weight = fp8_matmul_kernel(**wgrad)
         elif wants_dx and wgrad is not None:
             # the two GEMMs are independent: issued together they share kernel launches
-            grad_input, grad_weight = fp8_matmul_pair(
-                {k: v for k, v in dgrad.items() if k != "use_split_accumulator"},
-                {k: v for k, v in wgrad.items() if k != "use_split_accumulator"})
+            grad_input, grad_weight = fp8_matmul_pair(dgrad, wgrad)
         elif wants_dx:
             grad_input = fp8_matmul_kernel(**dgrad)
         elif wgrad is not None:

@@ -21,7 +21,7 @@ def fp8_linears(module_or_modules: Union[nn.Module, Iterable[nn.Module]]):
     mods = [module_or_modules] if isinstance(module_or_modules, nn.Module) else list(module_or_modules)
     seen = set()
     for root in mods:
-        for m in root.modules():
+        for m in (root.modules() if root._modules else (root,)):
             if isinstance(m, FP8Linear) and id(m) not in seen:
                 seen.add(id(m))
                 yield m
@@ -31,17 +31,19 @@ def fp8_linears(module_or_modules: Union[nn.Module, Iterable[nn.Module]]):
 def requantize_fp8_weights(module_or_modules, stream: Optional[torch.cuda.Stream] = None) -> int:
     """Re-quantise the weight of every FP8Linear from its master copy (one delayed-scaling step for the
     weight role where delayed scaling is on).  Returns the number of layers refreshed."""
-    layers = [lin for lin in fp8_linears(module_or_modules) if lin.weight.device.type != "cpu"]
+    layers = [lin for lin in fp8_linears(module_or_modules) if lin.weight.is_cuda]
     rest = layers
-    if stream is None:
+    if stream is None and len(layers) > 1:
         # weights whose delayed-scaling role already holds a scale go through one batched library call per device
-        ready = [lin for lin in layers if lin.scaling is not None and lin.scaling["weight"].known_initialised]
-        by_device = {}
-        for lin in ready:
-            by_device.setdefault(lin.weight.device, []).append(lin)
-        batched = set()
+        by_device, rest = {}, []
+        for lin in layers:
+            if lin.scaling is not None and lin.scaling["weight"].known_initialised:
+                by_device.setdefault(lin.weight.device, []).append(lin)
+            else:
+                rest.append(lin)
         for dev, lins in by_device.items():
             if len(lins) < 2:
+                rest += lins
                 continue
             with torch.cuda.device(dev):
                 hp = [lin.weight.as_subclass(torch.Tensor) for lin in lins]
@@ -50,8 +52,6 @@ def requantize_fp8_weights(module_or_modules, stream: Optional[torch.cuda.Stream
             for lin, q in zip(lins, qs):
                 lin.weight.data = q
                 lin._weight_ready = None
-                batched.add(id(lin))
-        rest = [lin for lin in layers if id(lin) not in batched]
     for lin in rest:
         lin.requantize_weight(stream=stream)
     return len(layers)

@@ -20,8 +20,6 @@ from nanotron_amd.fp8.constants import (
 from nanotron_amd.fp8.dtypes import DType, DTypes
 from nanotron_amd.fp8.meta import FP8Meta
 
-_FMT = {DTypes.FP8E4M3: nt.E4M3, DTypes.FP8E5M2: nt.E5M2}
-
 
 def _int_margin(margin) -> int:
     m = float(margin)
@@ -46,7 +44,7 @@ class DelayedScaling:
 
     def __init__(self, dtype: DTypes, history_len: int = DEFAULT_AMAX_HISTORY_LEN, margin: int = DEFAULT_MARGIN,
                  device: Union[str, torch.device] = "cuda"):
-        assert isinstance(dtype, DTypes) and dtype in _FMT
+        assert isinstance(dtype, DTypes) and dtype.code is not None
         assert history_len >= 1
         self.dtype = dtype
         self.margin = _int_margin(margin)
@@ -146,13 +144,13 @@ class FP8Tensor(torch.Tensor):
 
 def _quantize(cls, tensor: torch.Tensor, dtype: DTypes, state: Optional[DelayedScaling], with_transpose: bool,
               margin: int = 0) -> FP8Tensor:
-    if dtype not in _FMT:
+    fmt = dtype.code
+    if fmt is None:
         raise ValueError(f"{dtype} is not an FP8 format")
     if tensor.dtype not in nt.TORCH_TO_NT:
         raise TypeError(f"cannot quantise a {tensor.dtype} tensor to FP8 (float32 / float16 / bfloat16 only)")
     if tensor.numel() == 0:
         raise RuntimeError("cannot quantise an empty tensor (amax of an empty tensor is undefined)")
-    fmt = _FMT[dtype]
     if state is None:
         parts = nt.host.quantize(tensor, fmt, _int_margin(margin), None, None, 0, with_transpose)
     else:
@@ -189,38 +187,12 @@ def quantize_delayed_batch(tensors, dtype: DTypes, states, with_transpose) -> li
     beginning of the next.  Same results as the separate constructions, bit for bit."""
     tensors, states, with_transpose = list(tensors), list(states), list(with_transpose)
     assert len(tensors) == len(states) == len(with_transpose) and tensors
-    dev = tensors[0].device
-    fmt = _FMT[dtype]
-    results = []
-    for lo in range(0, len(tensors), 64):
-        chunk = range(lo, min(lo + 64, len(tensors)))
-        pool, st = nt.workspace_pool(dev, len(chunk))
-        descs = (nt.QuantDesc * len(chunk))()
-        keep = []
-        for d, i in zip(descs, chunk):
-            x, state = tensors[i].detach(), states[i]
-            assert state.known_initialised and state.dtype == dtype and state._buf.device == dev and x.device == dev
-            assert x.dtype in nt.TORCH_TO_NT and x.numel() > 0
-            if not x.is_contiguous():
-                x = x.contiguous()
-            cols = x.shape[-1] if x.dim() >= 2 else x.numel()
-            rows = x.numel() // cols
-            out = torch.empty(x.shape, dtype=torch.uint8, device=dev)
-            out_t = None
-            if with_transpose[i]:
-                assert x.dim() == 2, "with_transpose needs a 2-D tensor"
-                out_t = torch.empty((cols, rows), dtype=torch.uint8, device=dev)
-            scalars = torch.empty(2, dtype=torch.float32, device=dev)  # [amax, scale used]
-            state_p = state._buf.data_ptr()
-            d.x, d.x_dtype, d.fmt, d.margin, d.history_len = x.data_ptr(), nt.TORCH_TO_NT[x.dtype], fmt, state.margin, state.history_len
-            d.rows, d.cols = rows, cols
-            d.scale_state, d.amax_history = state_p, state_p + 4
-            d.amax_out, d.scale_used_out = scalars.data_ptr(), scalars.data_ptr() + 4
-            d.out, d.out_t, d.workspace = out.data_ptr(), nt.ptr(out_t), pool[i - lo].data_ptr()
-            keep.append((x, out, out_t, scalars))
-        nt.check(nt.lib.ntfp8_quantize_delayed_batch(descs, len(chunk), st), "ntfp8_quantize_delayed_batch")
-        results += [_assemble(FP8Tensor, dtype, out, out_t, scalars[0], scalars[1]) for x, out, out_t, scalars in keep]
-    return results
+    for t, state in zip(tensors, states):
+        assert state.known_initialised and state.dtype == dtype
+        assert t.dtype in nt.TORCH_TO_NT
+    problems = [(t, s._buf, s.history_len, s.margin, w) for t, s, w in zip(tensors, states, with_transpose)]
+    return [_assemble(FP8Tensor, dtype, *parts) for lo in range(0, len(problems), 64)
+            for parts in nt.host.quantize_batch(problems[lo:lo + 64], dtype.code)]
 
 
 def cast_with_scale(tensor: torch.Tensor, scale: torch.Tensor, dtype: DTypes, with_transpose: bool = False) -> FP8Tensor:
@@ -233,7 +205,7 @@ def cast_with_scale(tensor: torch.Tensor, scale: torch.Tensor, dtype: DTypes, wi
     scale = scale.reshape(())
     if scale.device != dev or scale.dtype != torch.float32:
         scale = scale.to(device=dev, dtype=torch.float32)
-    return _assemble(FP8Tensor, dtype, *nt.host.cast_with_scale(x, scale, _FMT[dtype], with_transpose))
+    return _assemble(FP8Tensor, dtype, *nt.host.cast_with_scale(x, scale, dtype.code, with_transpose))
 
 
 def convert_torch_dtype_to_te_dtype(dtype) -> DType:
@@ -260,7 +232,7 @@ def convert_tensor_to_fp8(tensor: torch.Tensor, meta) -> torch.Tensor:
     scale = meta.scale
     if not (isinstance(scale, torch.Tensor) and scale.device == dev and scale.dtype == torch.float32):
         scale = torch.as_tensor(scale, dtype=torch.float32).to(dev)
-    return nt.host.cast(x, scale.reshape(()), _FMT[meta.dtype], False)[0]
+    return nt.host.cast(x, scale.reshape(()), meta.dtype.code, False)[0]
 
 
 def convert_tensor_from_fp8(tensor: torch.Tensor, meta, dtype: torch.dtype) -> torch.Tensor:
@@ -275,7 +247,7 @@ def convert_tensor_from_fp8(tensor: torch.Tensor, meta, dtype: torch.dtype) -> t
     scale = meta.scale
     if not (isinstance(scale, torch.Tensor) and scale.device == dev and scale.dtype == torch.float32):
         scale = torch.as_tensor(scale, dtype=torch.float32).to(dev)
-    return nt.host.dequantize(q, _FMT[meta.dtype], scale, nt.TORCH_TO_NT[dtype], False)
+    return nt.host.dequantize(q, meta.dtype.code, scale, nt.TORCH_TO_NT[dtype], False)
 
 
 def update_scaling_factor(amax: torch.Tensor, scaling_factor: torch.Tensor, dtype: DTypes,
@@ -287,7 +259,7 @@ def update_scaling_factor(amax: torch.Tensor, scaling_factor: torch.Tensor, dtyp
     native library evaluates the same function on the host."""
     assert amax.dtype == torch.float32
     assert scaling_factor.dtype == torch.float32
-    fmt = _FMT[dtype]
+    fmt = dtype.code
     m = _int_margin(margin)
     if not amax.is_cuda and not scaling_factor.is_cuda:
         a, s = torch.broadcast_tensors(amax, scaling_factor)
