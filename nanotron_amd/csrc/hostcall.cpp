@@ -97,6 +97,12 @@ at::Tensor bytes_like(const at::Tensor& x, at::IntArrayRef sizes) {
     return at::empty(sizes, at::TensorOptions().dtype(at::kByte).device(x.device()));
 }
 at::Tensor dense(const at::Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+// the same of an operand that a kernel is about to read: an address of host memory would fault the GPU
+at::Tensor operand(PyObject* o) {
+    const at::Tensor& t = tensor(o);
+    require(t.is_cuda(), "a tensor on a CUDA device is expected");
+    return dense(t);
+}
 
 // [amax, scale used] of a quantisation: one allocation, and its two elements as 0-dim tensors
 struct Scalars {
@@ -123,7 +129,7 @@ PyObject* quantised(at::Tensor out, at::Tensor out_t, const Scalars& s) {
 // quantize(x, fmt, margin, state | None, flag | None, history_len, with_transpose) -> (bytes, bytes^T | None, amax, scale)
 // state None: current scaling; flag given: the role may not hold a scale yet; otherwise the fused delayed-scaling step
 PyObject* quantize(PyObject* const* a) {
-    const at::Tensor x = dense(tensor(a[0]));
+    const at::Tensor x = operand(a[0]);
     const int fmt = (int)number(a[1]), margin = (int)number(a[2]), hist = (int)number(a[5]);
     const bool with_t = truth(a[6]);
     int64_t rows, cols;
@@ -317,7 +323,7 @@ PyObject* gemm_fp8(PyObject* const* p) {
 
 // cast_with_scale(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None, amax = 0, scale)
 PyObject* cast_with_scale(PyObject* const* a) {
-    const at::Tensor x = dense(tensor(a[0]));
+    const at::Tensor x = operand(a[0]);
     const int fmt = (int)number(a[2]);
     const bool with_t = truth(a[3]);
     int64_t rows, cols;
@@ -334,7 +340,7 @@ PyObject* cast_with_scale(PyObject* const* a) {
 
 // column_sum([rows, cols], out_code) -> [cols]
 PyObject* column_sum(PyObject* const* a) {
-    const at::Tensor x = dense(tensor(a[0]));
+    const at::Tensor x = operand(a[0]);
     require(x.dim() == 2, "a 2-D tensor is expected");
     const long code = number(a[1]);
     const auto opt = at::TensorOptions().device(x.device());
@@ -350,7 +356,7 @@ PyObject* column_sum(PyObject* const* a) {
 
 // cast(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None)
 PyObject* cast(PyObject* const* a) {
-    const at::Tensor x = dense(tensor(a[0]));
+    const at::Tensor x = operand(a[0]);
     const int fmt = (int)number(a[2]);
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
@@ -366,7 +372,7 @@ PyObject* cast(PyObject* const* a) {
 
 // dequantize(bytes, fmt, scale, out_code, inverse) -> tensor
 PyObject* dequantize(PyObject* const* a) {
-    const at::Tensor q = dense(tensor(a[0]));
+    const at::Tensor q = operand(a[0]);
     const int fmt = (int)number(a[1]);
     const float* scale = static_cast<const float*>(tensor(a[2]).data_ptr());
     const long code = number(a[3]);
@@ -380,7 +386,7 @@ PyObject* dequantize(PyObject* const* a) {
 
 // transpose([rows, cols] bytes) -> contiguous [cols, rows] bytes
 PyObject* transpose(PyObject* const* a) {
-    const at::Tensor q = dense(tensor(a[0]));
+    const at::Tensor q = operand(a[0]);
     require(q.dim() == 2, "a 2-D tensor is expected");
     at::Tensor out = bytes_like(q, {q.size(1), q.size(0)});
     if (q.numel()) call(ntfp8_transpose(q.data_ptr(), q.size(0), q.size(1), out.data_ptr(), stream_of(q)), "ntfp8_transpose");

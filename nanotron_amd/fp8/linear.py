@@ -52,6 +52,8 @@ class FP8Linear(nn.Linear):
     The bias is added inside the GEMM epilogue (the TODO at linear.py:62).  In evaluation mode (`module.eval()`)
     tensors are quantised with the scales the delayed-scaling roles hold and the roles are left untouched."""
 
+    _zero_element = None   # see _zero (on the class: a module pickled without it has one too)
+
     def __init__(self, in_features: int, out_features: int, bias: bool = True, device: Optional[torch.device] = None,
                  *, dtype: Optional[torch.dtype] = None, out_dtype: Union[torch.dtype, DTypes, None] = None,
                  delayed_scaling: bool = False, amax_history_len: int = 16, margin: int = 0,
@@ -75,7 +77,6 @@ class FP8Linear(nn.Linear):
         self.fp8_grad_input = True
         self.fp8_grad_inputs_sent = 0   # backward passes of this layer that did so
         self._grad_box = None
-        self._zero_element = None
         self.scaling = None
         self._weight_ready = None
         if self.weight.device != torch.device("cpu"):
@@ -291,6 +292,7 @@ class _FP8Matmul(torch.autograd.Function):
             out_shape = output.as_subclass(torch.Tensor).shape
             handle = module._zero(hp, weight.device).expand(out_shape)
             ctx.fp8_out = True
+            ctx.out_shape, ctx.out_dtype = out_shape, hp
             return output, handle
         ctx.fp8_out = False
         output = fp8_matmul_kernel(
@@ -299,6 +301,7 @@ class _FP8Matmul(torch.autograd.Function):
         )
         if len(in_shape) != 2:
             output = output.reshape(*in_shape[:-1], output.shape[-1])
+        ctx.out_shape, ctx.out_dtype = output.shape, out_dtype
         return output, phony
 
     @staticmethod
@@ -313,7 +316,6 @@ class _FP8Matmul(torch.autograd.Function):
         input, weight, bias = ctx.saved_tensors
         module = ctx.module
         scaling = module.scaling if module is not None else None
-        none = (None,) * 7
         if ctx.fp8_out:
             grad_output = grad_aux   # the gradient of the fp8 output arrives through its handle ...
             box = ctx.grad_box
@@ -326,8 +328,8 @@ class _FP8Matmul(torch.autograd.Function):
                                        "on the consuming FP8Linear (high-precision gradients, summed by autograd), or give "
                                        "the producing layer a high-precision out_dtype")
                 grad_output = fp8_grad   # ... or beside it, already quantised by the consumer's dgrad epilogue
-        if grad_output is None:
-            return none
+        if grad_output is None:   # a consumer's backward produced no gradient: a gradient of zeros
+            grad_output = torch.zeros(ctx.out_shape, dtype=ctx.out_dtype, device=weight.device)
 
         grad_bias = None
         if bias is not None and ctx.needs_input_grad[5]:
