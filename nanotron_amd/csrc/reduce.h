@@ -6,13 +6,14 @@
 namespace ntfp8 {
 
 // ---------------------------------------------------------------------------------------------
-// Block reduction of the partial max, publication, and the last-block epilogue.
+// Block reduction of the partial max, publication, and the bookkeeping epilogue of one block.
 //
 // Inter-block traffic uses relaxed device-scope atomics only (they execute at the level where all
-// XCDs agree) and orders them with the wave's own memory counter: the partial max is folded in with
-// a returning atomic, the wave waits for it, then takes a ticket.  A release fence here would write
-// back the whole L2 once per block, which costs more than the streaming pass itself.
-// What the last block's epilogue will read, requested by the first wave of every block while the
+// XCDs agree).  Either a block's maximum is one word that says by itself that it has arrived (publish_and_finalize), or
+// the wave's own memory counter orders two of them: the partial max is folded in with a returning atomic, the wave waits
+// for it, then takes a ticket.  A release fence here would write back the whole L2 once per block, which costs more than
+// the streaming pass itself.
+// What the bookkeeping block's epilogue will read, requested by the first wave of every block while the
 // tensor is still streaming: the history entry that moves into this lane's slot and the scale in
 // force.  It takes one round trip out of the dependent chain at the end of the kernel.
 struct EpiloguePrefetch {
@@ -124,6 +125,40 @@ __device__ __forceinline__ bool draw_ticket(Workspace* ws, uint32_t bid, uint32_
     return __hip_atomic_fetch_add(&ws->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
 }
 
+// Up to kCells workgroups: the workspace as one word per workgroup.  A workgroup stores its maximum, marked as present, and
+// is done; the one with the highest number (dispatched last) reads the words until all are there.  That is one store and
+// one read behind the last maximum, where the ticket protocol needs four dependent round trips to the memory side
+// (maximum, ticket of the group, ticket of the launch, slots).  Bound by that latency on small tensors: delayed step of
+// bf16 2048 x 2048 8.8 -> 7.3 us, 4096 x 4096 12.0 -> 10.8 us alone and 14.9 -> 13.4 us inside a training step.  Beyond
+// kCells (transposed copies of more than two tiles per CU) the ticket protocol serves.  Nobody waits for the reading wave, so every word arrives;
+// the trip limit (many seconds) only keeps a workspace that two overlapping launches share against the rules from
+// holding the GPU.
+constexpr uint32_t kCells = NTFP8_WORKSPACE_BYTES / 4, kPresent = 0x80000000u;
+__device__ inline uint32_t collect_cells(uint32_t own, Workspace* ws, uint32_t others) {
+    uint32_t* cell = reinterpret_cast<uint32_t*>(ws);
+    uint32_t best = own, trips = 1u << 25;
+    for (uint32_t base = threadIdx.x; base - threadIdx.x < others; base += 256) {
+        uint32_t v[4];
+        for (;;) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                v[j] = kPresent;
+                if (base + 64 * j < others) v[j] = __hip_atomic_load(cell + base + 64 * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (__all((v[0] & v[1] & v[2] & v[3] & kPresent) != 0u) || --trips == 0u) break;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t m = v[j] & ~kPresent;
+            best = m > best ? m : best;
+            if (base + 64 * j < others) __hip_atomic_store(cell + base + 64 * j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (trips == 0u) trips = 1u;
+    }
+    best = wave_max_u32(best);
+    return best > kInfBits ? kNanBits : best;
+}
+
 // `bid` of `nblocks`: this workgroup's place among the workgroups that reduce the same tensor (the whole grid,
 // except in a launch that carries several tensors).
 template <int THREADS>
@@ -132,23 +167,33 @@ __device__ inline void publish_and_finalize(uint32_t m_f32bits, Workspace* ws, c
                                             uint32_t nblocks = gridDim.x, const ScalarIO* io2 = nullptr,
                                             const EpiloguePrefetch* pre2 = nullptr) {
     __shared__ uint32_t s_part[THREADS / 64];
-    __shared__ bool s_last;
     const uint32_t wm = wave_max_u32(m_f32bits);
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = wm;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t bm = 0;
+    if (threadIdx.x >= 64) return;   // the rest is the first wave's
+    uint32_t bm = 0;
 #pragma unroll
-        for (int i = 0; i < THREADS / 64; ++i) bm = s_part[i] > bm ? s_part[i] : bm;
+    for (int i = 0; i < THREADS / 64; ++i) bm = s_part[i] > bm ? s_part[i] : bm;
+    if (nblocks <= kCells) {
+        if (bid != nblocks - 1) {
+            if (threadIdx.x == 0)
+                __hip_atomic_store(reinterpret_cast<uint32_t*>(ws) + bid, bm | kPresent, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+        const uint32_t bits = collect_cells(bm, ws, nblocks - 1);
+        bookkeep(bits, io, mode, pre);
+        if (io2) bookkeep(bits, *io2, mode, *pre2);
+        return;
+    }
+    uint32_t last = 0;
+    if (threadIdx.x == 0) {
         const uint32_t grp = bid % kMaxSlots;
         const uint32_t old = __hip_atomic_fetch_max(&ws->slot[grp].bits, bm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::"v"(old) : "memory");   // the max is in place before the ticket is drawn
-        s_last = draw_ticket(ws, bid, nblocks);
+        last = draw_ticket(ws, bid, nblocks) ? 1u : 0u;
     }
-    __syncthreads();
-    // the epilogue runs on the first wave of the block that drew the last ticket
-    if (!s_last || threadIdx.x >= 64) return;
-    finalize_wave(ws, io, mode, pre, io2, pre2);
+    // the bookkeeping is the work of the block that drew the last ticket
+    if (__builtin_amdgcn_readfirstlane(last)) finalize_wave(ws, io, mode, pre, io2, pre2);
 }
 
 }  // namespace ntfp8
