@@ -26,7 +26,7 @@ LIB = os.path.join(HERE, "libntfp8.so")
 HOSTCALL = os.path.join(HERE, "_hostcall.so")
 PROFILING_DIR = os.path.join(HERE, "profiling")
 LIB_STAMPS = os.path.join(PROFILING_DIR, "libntfp8_stamps.so")
-SOURCES = ["quant.hip", "gemm.hip", "gemm_mid.hip", "gemm_any.hip", "capi.hip"]
+SOURCES = ["quant.hip", "gemm.hip", "gemm_mid.hip", "gemm_few.hip", "gemm_any.hip", "capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -12,6 +12,8 @@
 //   gemm_mid_kernel       (gemm_mid.h) 128 x 128 and 64 x 64 tiles of the same instruction, loads straight into four LDS
 //                         stages: shapes that have too few 256-wide tiles, and operands beyond the 2 GiB reach of a
 //                         buffer descriptor's 32-bit offsets.
+//   gemm_few_kernel       (gemm_few.h) up to 32 rows against a full-size weight: 16 or 32 columns per workgroup, K
+//                         split over its waves.
 //   gemm_any_kernel       (gemm_any.h) any K and alignment: 64- or 128-wide tiles, fp8 widened to bf16 on its way to
 //                         the matrix cores.
 //   gemm_nt_kernel        128 x 128 x 128 tiles, loads through registers: fp8 outputs whose rows or columns do not come in
@@ -26,6 +28,7 @@ constexpr int kMinTransposed = 128;   // rows and columns of a result whose B is
 enum GemmPath { kPathNone = -1, kPathAny = 0, kPathWords = 1, kPathTiles = 2 };
 
 int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
+int launch_few(const BigProblem& p, int fa, int fb, hipStream_t st);
 int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_words(const GemmDesc& g, hipStream_t st);
 int run_amax_finalize(Workspace* ws, const ScalarIO& io, hipStream_t st);
@@ -122,6 +125,17 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* 
     return tiles;
 }
 
+// A few rows against a weight whose columns the 64-wide tiles spread over few CUs (gemm_few.h).  The lines, us in 64-wide
+// tiles / there, weights not in a cache:
+//   16 rows, N x K:  4096 x 1024 4.7 / 4.9     1024 x 2048 5.8 / 5.4     4096 x 2048 7.5 / 6.0     5120 x 2048 7.7 / 7.7
+//                    6144 x 3072 9.7 / 9.3     8192 x 4096 13.6 / 12.2   14336 x 4096 15.3 / 16.8 (in 64 columns)
+//   32 rows:         1024 x 4096 8.3 / 8.9     2048 x 6144 15.7 / 13.4   4096 x 14336 31.9 / 24.3   5120 x 5120 14.8 / 17.2
+static bool few_rows(const GemmDesc& g) {
+    if (g.tb || is_fp8_out(g.d_dtype)) return false;
+    if (g.M <= 16) return g.K >= 2048 && g.N <= 32 * cu_count();
+    return g.M <= 32 && g.K >= 6144 && g.N <= 16 * cu_count();
+}
+
 // One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
 // tiles: one more launch for a half-tile tail).
 template <int FA, int FB>
@@ -202,6 +216,11 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     if (path == kPathWords) {
         const int rc = launch_words(*g[0], st);
         return rc == NTFP8_OK && g[0]->fin ? run_amax_finalize(static_cast<Workspace*>(g[0]->ws), *g[0]->fin, st) : rc;
+    }
+    if (n == 1 && few_rows(*g[0])) {
+        BigLaunch L;
+        list_tiles(g, 1, 64, &L);
+        return launch_few(L.p[0], fa, fb, st);
     }
     if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, st) : launch_tiles<kE4M3, kE5M2>(g, n, st);
     return fb == kE4M3 ? launch_tiles<kE5M2, kE4M3>(g, n, st) : launch_tiles<kE5M2, kE5M2>(g, n, st);
