@@ -221,15 +221,15 @@ __device__ __forceinline__ void reg_store4(__amdgpu_buffer_rsrc_t r, uint32_t vo
 // All stores go through buffer descriptors of M N bytes: rows past the end fall outside and are dropped, columns
 // past the end get an offset that does; nothing is predicated, which keeps the scalar registers of the epilogue
 // (and with them the register budget of the K loop before it) small.
-// kMask: accumulator blocks past N (and past M if `mask_rows`: A given as its transpose) hold arbitrary values,
-// because an operand read through the transposing loads wraps into its next row there instead of reading zeros, and
-// must stay out of the amax.  N (and M, with a transposed A) is a multiple of 16 then, so whole blocks are in or
-// out, uniformly for the wave.  Rows past M of an ordinary A operand read as zeros and need no mask.
-template <int F, int MI, int NJ, bool kBias = false, bool kMask = false>
+// Accumulators past M and past N stay out of the amax: they hold zeros times whatever the other operand holds (NaN
+// against an infinite code), plus the bias, or, where an operand is read through the transposing loads and wraps
+// into its next row, arbitrary values.  N is a multiple of 16, so a block's columns are in or out together, uniformly
+// for the wave; rows are masked lane by lane.
+template <int F, int MI, int NJ, bool kBias = false>
 __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][NJ], uint8_t* __restrict__ D,
                                                           uint8_t* __restrict__ Dt, float alpha, float scale_d, bool slow,
                                                           int M, int N, int m_base, int n_base, int lane,
-                                                          const float (*bv)[4] = nullptr, bool mask_rows = false) {
+                                                          const float (*bv)[4] = nullptr) {
     auto val = [&](int i, int j, int e) -> float {
         if constexpr (kBias) return acc[i][j][e] * alpha + bv[j][e];
         else return acc[i][j][e] * alpha;
@@ -245,16 +245,13 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 16 + mrow;
         const int mq = m & ~3;
+        const uint32_t inside = m < M ? ~0u : 0u;
         uint32_t w[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if constexpr (kMask) {
-                uint32_t a = amax;
-                w[j] = quant4<F>(val(i, j, 0), val(i, j, 1), val(i, j, 2), val(i, j, 3), scale_d, slow, a);
-                if ((!mask_rows || m_base + i * 16 < M) && n_base + j * 16 < N) amax = a;
-            } else {
-                w[j] = quant4<F>(val(i, j, 0), val(i, j, 1), val(i, j, 2), val(i, j, 3), scale_d, slow, amax);
-            }
+            uint32_t a = 0;
+            w[j] = quant4<F>(val(i, j, 0), val(i, j, 1), val(i, j, 2), val(i, j, 3), scale_d, slow, a);
+            if (n_base + j * 16 < N) amax = max(amax, a & inside);
         }
         if (Dt) {   // uniform
 #pragma unroll
@@ -826,10 +823,10 @@ void gemm_nt_big_kernel(const BigLaunch L) {
                 const bool slow = scale_is_degenerate(scale_d);
                 const uint32_t amax =
                     P.d_dtype == NTFP8_OUT_E4M3
-                        ? store_wave_tile16_fp8<kE4M3, MI, kBigNJ, kBias, kBT>(acc, static_cast<uint8_t*>(Dv), P.fp8.Dt, alpha, scale_d,
-                                                                          slow, M, N, m0 + wm, n0 + wn, lane, bv, kBT && P.at)
-                        : store_wave_tile16_fp8<kE5M2, MI, kBigNJ, kBias, kBT>(acc, static_cast<uint8_t*>(Dv), P.fp8.Dt, alpha, scale_d,
-                                                                          slow, M, N, m0 + wm, n0 + wn, lane, bv, kBT && P.at);
+                        ? store_wave_tile16_fp8<kE4M3, MI, kBigNJ, kBias>(acc, static_cast<uint8_t*>(Dv), P.fp8.Dt, alpha, scale_d, slow, M,
+                                                                     N, m0 + wm, n0 + wn, lane, bv)
+                        : store_wave_tile16_fp8<kE5M2, MI, kBigNJ, kBias>(acc, static_cast<uint8_t*>(Dv), P.fp8.Dt, alpha, scale_d, slow, M,
+                                                                     N, m0 + wm, n0 + wn, lane, bv);
                 publish_amax(amax, P.fp8.ws);
                 finish_fp8(L, P.fp8.ws, bid);
             } else if (P.d_dtype == NTFP8_BF16) {

@@ -326,7 +326,8 @@ __device__ __forceinline__ void publish_amax(uint32_t lane_bits, Workspace* ws) 
         __hip_atomic_fetch_max(&ws->slot[blockIdx.x % kMaxSlots].bits, wm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// fp8 epilogue of one wave for 32 x 32 accumulator blocks (layout as store_wave_tile); returns the lane's max|r| bits
+// fp8 epilogue of one wave for 32 x 32 accumulator blocks (layout as store_wave_tile); returns the lane's max|r| bits, over
+// the elements inside the matrix only: an accumulator past its end holds the bias, or NaN (zero times an infinite code)
 template <int F, int MI, int NJ>
 __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ], uint8_t* __restrict__ D,
                                                         uint8_t* __restrict__ Dt, float alpha, float scale_d, bool slow,
@@ -344,8 +345,16 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int n = n_base + j * 32 + g * 8 + (lane >> 5) * 4;
+                uint32_t a = 0;
                 const uint32_t w = quant4<F>(acc[i][j][g * 4 + 0] * alpha, acc[i][j][g * 4 + 1] * alpha,
-                                             acc[i][j][g * 4 + 2] * alpha, acc[i][j][g * 4 + 3] * alpha, scale_d, slow, amax);
+                                             acc[i][j][g * 4 + 2] * alpha, acc[i][j][g * 4 + 3] * alpha, scale_d, slow, a);
+                if (n + 4 > N) {   // a word across the last column, or past it
+                    a = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < N) a = max(a, __float_as_uint(acc[i][j][g * 4 + e] * alpha) & 0x7fffffffu);
+                }
+                if (m < M) amax = max(amax, a);
                 if (m < M && n < N) store_bytes4(D + (int64_t)m * N + n, w, d_vec, N - n);
                 if (Dt) {   // uniform
                     const uint32_t t = quad_transpose_bytes(w, lane);

@@ -209,8 +209,8 @@ __global__ __launch_bounds__(kBigThreads, T == 128 ? 1 : 2) void gemm_mid_kernel
             const bool slow = scale_is_degenerate(scale_d);
             uint8_t* D = static_cast<uint8_t*>(P.D);
             const uint32_t amax = P.d_dtype == NTFP8_OUT_E4M3
-                                      ? store_wave_tile16_fp8<kE4M3, MI, NJ, kBias, true>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv, P.at)
-                                      : store_wave_tile16_fp8<kE5M2, MI, NJ, kBias, true>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv, P.at);
+                                      ? store_wave_tile16_fp8<kE4M3, MI, NJ, kBias>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv)
+                                      : store_wave_tile16_fp8<kE5M2, MI, NJ, kBias>(acc, D, P.fp8.Dt, alpha, scale_d, slow, M, N, mb, nb, lane, bv);
             publish_amax(amax, P.fp8.ws);
             finish_fp8(L, P.fp8.ws, blockIdx.x);
         } else if (P.d_dtype == NTFP8_BF16) {

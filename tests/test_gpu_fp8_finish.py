@@ -37,3 +37,67 @@ def test_bookkeeping_in_the_gemm(mnk, fmt):
         assert torch.equal(got.as_subclass(torch.Tensor), want.as_subclass(torch.Tensor))
         assert torch.equal(one._buf, two._buf)
         assert got.fp8_meta.amax.item() == want.fp8_meta.amax.item() and got.fp8_meta.scale.item() == want.fp8_meta.scale.item()
+
+
+# rows and columns that end inside a tile, some of them after one element: (M, N, K)
+RAGGED = [
+    (1, 1, 7), (1, 16, 515), (20, 48, 33), (130, 129, 77),          # K a multiple of nothing
+    (4, 16, 32), (20, 48, 64), (100, 80, 272), (132, 144, 128),     # 64-wide tiles
+    (2052, 2064, 768),                                              # 128-wide
+    (1124, 5136, 1024),                                             # halves of 256-wide tiles
+    (4100, 6160, 512),                                              # whole tiles and a tail
+    (1, 1, 16), (66, 100, 128), (33, 18, 64),                       # rows and columns that do not come in words
+]
+
+
+def _held(fmt):
+    """Two delayed-scaling states that hold the same scale (so that the epilogue casts)."""
+    from nanotron_amd.fp8 import DelayedScaling, FP8Tensor
+
+    states = [DelayedScaling(fmt, 3, 0, "cuda") for _ in range(2)]
+    for s in states:
+        FP8Tensor(torch.full((16,), 3.0, device="cuda"), fmt, state=s)
+        assert s.initialised
+    return states
+
+
+def _same(got, want, one, two, amax):
+    assert got.fp8_meta.amax.item() == want.fp8_meta.amax.item() == amax
+    assert torch.equal(one._buf, two._buf)
+    assert torch.equal(got.as_subclass(torch.Tensor), want.as_subclass(torch.Tensor))
+
+
+@pytest.mark.parametrize("mnk", RAGGED)
+def test_bias_of_padding_rows_stays_out_of_the_amax(mnk):
+    """Every result is K + (1/8 - K): a row that is not there would count as |1/8 - K|."""
+    from nanotron_amd.fp8 import FP8Tensor
+    from nanotron_amd.fp8.kernel import fp8_matmul_kernel
+
+    M, N, K = mnk
+    print(f"{mnk}", flush=True)
+    fmt = DTypes.FP8E4M3
+    one, two = _held(fmt)
+    x, w = (FP8Tensor(torch.ones(r, K, device="cuda"), DTypes.FP8E4M3) for r in (M, N))
+    bias = torch.full((N,), 0.125 - K, device="cuda")
+    got = fp8_matmul_kernel(w, True, x, False, False, out_dtype=fmt, out_state=one, bias=bias)
+    want = FP8Tensor(fp8_matmul_kernel(w, True, x, False, False, bias=bias), fmt, state=two)
+    _same(got, want, one, two, 0.125)
+
+
+@pytest.mark.parametrize("infinite", ["x", "w"])
+@pytest.mark.parametrize("mnk,plain_w", [(s, True) for s in RAGGED] + [((132, 144, 256), False), ((2052, 2064, 768), False)])
+def test_infinite_operand_against_padding_stays_out_of_the_amax(mnk, plain_w, infinite):
+    """An infinite code makes one row or column of the result infinite; against the zeros of padding it makes NaN, which
+    must not become the amax."""
+    from nanotron_amd.fp8 import FP8Tensor
+    from nanotron_amd.fp8.kernel import fp8_matmul_kernel
+
+    M, N, K = mnk
+    print(f"{mnk} {plain_w} {infinite}", flush=True)
+    fmt = DTypes.FP8E5M2
+    one, two = _held(fmt)
+    x, w = (FP8Tensor(torch.ones(s, device="cuda"), DTypes.FP8E5M2) for s in ((M, K), (N, K) if plain_w else (K, N)))
+    (x if infinite == "x" else w).as_subclass(torch.Tensor)[0, 0] = 0x7c   # +Inf in e5m2
+    got = fp8_matmul_kernel(w, plain_w, x, False, False, out_dtype=fmt, out_state=one)
+    want = FP8Tensor(fp8_matmul_kernel(w, plain_w, x, False, False), fmt, state=two)
+    _same(got, want, one, two, float("inf"))
