@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
-from typing import Dict, Optional, Tuple
+from typing import Optional, Tuple
 
 import torch
 
@@ -103,8 +103,7 @@ def check(code: int, what: str) -> None:
         if code == ERR_LAUNCH:
             # whatever went wrong at the launch, nothing may be assumed about the reduction workspaces any more (they
             # must be all zero between launches): drop them, the next call gets fresh zeroed ones
-            _workspaces.clear()
-            _pools.clear()
+            host.drop_workspaces()
         raise RuntimeError(f"{what} failed: {strerror(code)} (code {code})")
 
 
@@ -126,34 +125,16 @@ def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-_workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
-
-
 def workspace_and_stream(device: torch.device) -> Tuple[torch.Tensor, int]:
-    """(zero-initialised reduction workspace, stream pointer) for torch's current stream on `device`; one
-    workspace per (device, stream): kernels leave it zero."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    st = stream_ptr(device)
-    ws = _workspaces.get((idx, st))
-    if ws is None:
-        ws = torch.zeros(WORKSPACE_BYTES // 4, dtype=torch.int32, device=device)
-        _workspaces[(idx, st)] = ws
-    return ws, st
-
-
-_pools: Dict[Tuple[int, int], torch.Tensor] = {}
+    """(reduction workspace, stream pointer) for torch's current stream on `device`; one workspace per (device, stream),
+    the one that the native host calls use there: zero between launches."""
+    return host.workspace(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def workspace_pool(device: torch.device, count: int) -> Tuple[torch.Tensor, int]:
-    """([>= count, WORKSPACE_BYTES / 4] zero-initialised workspaces, stream pointer) for torch's current stream on
-    `device`: one workspace per tensor of a batched call (kernels leave them zero)."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    st = stream_ptr(device)
-    pool = _pools.get((idx, st))
-    if pool is None or pool.shape[0] < count:
-        pool = torch.zeros(max(count, 16), WORKSPACE_BYTES // 4, dtype=torch.int32, device=device)
-        _pools[(idx, st)] = pool
-    return pool, st
+    """([>= count, WORKSPACE_BYTES / 4] workspaces, stream pointer) for torch's current stream on `device`: one per tensor
+    of a batched call, shared with the native host calls as above."""
+    return host.workspace_pool(device.index if device.index is not None else torch.cuda.current_device(), count)
 
 
 def workspace(device: torch.device) -> torch.Tensor:

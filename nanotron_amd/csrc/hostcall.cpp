@@ -19,7 +19,7 @@
 
 namespace {
 
-PyObject* g_check = nullptr;   // nanotron_amd._native.check: raises RuntimeError, drops the workspaces after a failed launch
+PyObject* g_check = nullptr;   // nanotron_amd._native.check: raises RuntimeError, has the workspaces dropped after a failed launch
 
 struct Stop {};   // a Python error is set
 
@@ -31,20 +31,24 @@ void require(bool ok, const char* msg) {
     if (!ok) stop(PyExc_AssertionError, msg);
 }
 
-// Reduction workspaces, one per (device, stream), zero between launches.  Guarded by the GIL; the table is never
-// destroyed (its tensors must not outlive the runtime's teardown).
+// Reduction workspaces, zero between launches: one for calls of one tensor and a pool for batched calls, per (device,
+// stream).  The package's other callers take theirs from here too (workspace() below).  Guarded by the GIL; the table is
+// never destroyed (its tensors must not outlive the runtime's teardown).
 using Key = std::pair<int, void*>;
 struct KeyHash {
     size_t operator()(const Key& k) const { return reinterpret_cast<size_t>(k.second) * 31u + (size_t)k.first; }
 };
-std::unordered_map<Key, at::Tensor, KeyHash>& workspaces() {
-    static auto* m = new std::unordered_map<Key, at::Tensor, KeyHash>();
+struct Space {
+    at::Tensor one, many;
+};
+using Spaces = std::unordered_map<Key, Space, KeyHash>;
+Spaces& workspaces() {
+    static auto* m = new Spaces();
     return *m;
 }
 
 void call(int rc, const char* what) {
     if (rc == NTFP8_OK) return;
-    if (rc == NTFP8_ERR_LAUNCH) workspaces().clear();
     PyObject* r = PyObject_CallFunction(g_check, "is", rc, what);
     Py_XDECREF(r);
     if (r != nullptr) stop(PyExc_RuntimeError, what);
@@ -81,11 +85,22 @@ PyObject* wrap_or_none(at::Tensor t) {
 void* stream_of(const at::Tensor& t) {
     return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream());
 }
-void* workspace_of(const at::Tensor& t, void* stream) {
-    at::Tensor& w = workspaces()[Key{(int)t.get_device(), stream}];
-    if (!w.defined()) w = at::zeros({NTFP8_WORKSPACE_BYTES / 4}, t.options().dtype(at::kInt));
-    return w.data_ptr();
+Space& space_of(int device, void* stream) { return workspaces()[Key{device, stream}]; }
+at::Tensor zeroed(int device, int64_t count) {
+    return at::zeros({count, NTFP8_WORKSPACE_BYTES / 4}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA, (c10::DeviceIndex)device));
 }
+const at::Tensor& workspace_at(int device, void* stream) {
+    at::Tensor& w = space_of(device, stream).one;
+    if (!w.defined()) w = zeroed(device, 1).squeeze(0);
+    return w;
+}
+// [>= count] workspaces for the tensors of a batched call
+const at::Tensor& pool_at(int device, void* stream, int64_t count) {
+    at::Tensor& w = space_of(device, stream).many;
+    if (!w.defined() || w.size(0) < count) w = zeroed(device, count < 16 ? 16 : count);
+    return w;
+}
+void* workspace_of(const at::Tensor& t, void* stream) { return workspace_at((int)t.get_device(), stream).data_ptr(); }
 
 int code_of(at::ScalarType t) {   // NTFP8_F32 / F16 / BF16, or -1
     return t == at::kFloat ? NTFP8_F32 : t == at::kHalf ? NTFP8_F16 : t == at::kBFloat16 ? NTFP8_BF16 : -1;
@@ -158,14 +173,6 @@ PyObject* quantize(PyObject* const* a) {
     return quantised(std::move(out), std::move(out_t), s);
 }
 
-// [>= count] workspaces for the tensors of a batched call, one table entry per (device, stream)
-at::Tensor workspace_pool(const at::Tensor& t, void* stream, int64_t count) {
-    at::Tensor& w = workspaces()[Key{(int)t.get_device() + 1024, stream}];
-    if (!w.defined() || w.size(0) < count)
-        w = at::zeros({count < 16 ? 16 : count, NTFP8_WORKSPACE_BYTES / 4}, t.options().dtype(at::kInt));
-    return w;
-}
-
 // quantize_batch([(x, state, history_len, margin, with_transpose), ...], fmt) -> [(bytes, bytes^T | None, amax, scale), ...]:
 // the fused delayed-scaling step of several tensors, one library call
 PyObject* quantize_batch(PyObject* const* args) {
@@ -192,7 +199,7 @@ PyObject* quantize_batch(PyObject* const* args) {
         require(!with_t || x[i].dim() == 2, "with_transpose needs a 2-D tensor");
         if (i == 0) {
             st = stream_of(x[0]);
-            pool = workspace_pool(x[0], st, n);
+            pool = pool_at((int)x[0].get_device(), st, n);
         }
         ntfp8_quant_desc& q = d[i];
         q = {};
@@ -422,6 +429,27 @@ PyObject* operand_form(PyObject* const* p) {
     return PyLong_FromLong(2);
 }
 
+// workspace(device index) -> (workspace, stream); workspace_pool(device index, count) -> ([>= count] workspaces, stream): what
+// the calls above use on torch's current stream of that device
+PyObject* with_stream(const at::Tensor& w, void* stream) { return Py_BuildValue("(NN)", wrap(w), PyLong_FromVoidPtr(stream)); }
+void* current_stream(int device) {
+    return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA((c10::DeviceIndex)device).stream());
+}
+PyObject* workspace(PyObject* const* a) {
+    const int device = (int)number(a[0]);
+    void* st = current_stream(device);
+    return with_stream(workspace_at(device, st), st);
+}
+PyObject* workspace_pool(PyObject* const* a) {
+    const int device = (int)number(a[0]);
+    void* st = current_stream(device);
+    return with_stream(pool_at(device, st, number(a[1])), st);
+}
+PyObject* drop_workspaces(PyObject* const*) {
+    workspaces().clear();
+    Py_RETURN_NONE;
+}
+
 PyObject* set_check(PyObject* const* a) {
     Py_INCREF(a[0]);
     Py_XSETREF(g_check, a[0]);
@@ -448,7 +476,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
-                         NT_METHOD(operand_form, 10), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
+                         NT_METHOD(operand_form, 10), NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
