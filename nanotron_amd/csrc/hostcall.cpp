@@ -46,6 +46,17 @@ Spaces& workspaces() {
     static auto* m = new Spaces();
     return *m;
 }
+// Those of a stream that records a graph: made in the capture that uses them (the fill is a node of its graph, the memory
+// comes from its pool) and never seen by another capture or by eager calls, of which the graph's replays know nothing.
+// Only the table lets go of them afterwards, at the next eager call.
+struct CapturedSpace {
+    unsigned long long capture;
+    Space space;
+};
+std::unordered_map<Key, CapturedSpace, KeyHash>& captured_workspaces() {
+    static auto* m = new std::unordered_map<Key, CapturedSpace, KeyHash>();
+    return *m;
+}
 
 void call(int rc, const char* what) {
     if (rc == NTFP8_OK) return;
@@ -85,7 +96,21 @@ PyObject* wrap_or_none(at::Tensor t) {
 void* stream_of(const at::Tensor& t) {
     return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.get_device()).stream());
 }
-Space& space_of(int device, void* stream) { return workspaces()[Key{device, stream}]; }
+Space& space_of(int device, void* stream) {
+    const Key key{device, stream};
+    if (stream != nullptr) {   // (the legacy stream cannot be captured, and must not be asked while another one is)
+        hipStreamCaptureStatus status;
+        unsigned long long id = 0;
+        if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) stop(PyExc_RuntimeError, "hipStreamGetCaptureInfo failed");
+        if (status == hipStreamCaptureStatusActive) {
+            CapturedSpace& c = captured_workspaces()[key];
+            if (c.capture != id) c = CapturedSpace{id, Space{}};
+            return c.space;
+        }
+    }
+    if (!captured_workspaces().empty()) captured_workspaces().clear();
+    return workspaces()[key];
+}
 at::Tensor zeroed(int device, int64_t count) {
     return at::zeros({count, NTFP8_WORKSPACE_BYTES / 4}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA, (c10::DeviceIndex)device));
 }
@@ -447,6 +472,7 @@ PyObject* workspace_pool(PyObject* const* a) {
 }
 PyObject* drop_workspaces(PyObject* const*) {
     workspaces().clear();
+    captured_workspaces().clear();
     Py_RETURN_NONE;
 }
 
