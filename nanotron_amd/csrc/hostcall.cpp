@@ -144,6 +144,21 @@ at::Tensor operand(PyObject* o) {
     return dense(t);
 }
 
+// fp32 values in device memory that a kernel will read or write: a scale, a flag, a delayed-scaling state.  An address of host
+// memory would fault the GPU here as well, and another type would be read as something else.
+float* values(PyObject* o, c10::Device device, int64_t count = 1) {
+    const at::Tensor& t = tensor(o);
+    require(t.is_cuda() && t.device() == device, "scales and delayed-scaling states must be on the device of the operand");
+    require(t.scalar_type() == at::kFloat && t.numel() >= count && (count == 1 || t.is_contiguous()),
+            "scales and delayed-scaling states are fp32 tensors of one value, or of a scale and its history");
+    return static_cast<float*>(t.data_ptr());
+}
+// fp8 codes: one byte each
+const at::Tensor& codes(const at::Tensor& t) {
+    require(t.element_size() == 1, "fp8 codes take one byte each");
+    return t;
+}
+
 // [amax, scale used] of a quantisation: one allocation, and its two elements as 0-dim tensors
 struct Scalars {
     at::Tensor both;
@@ -175,6 +190,8 @@ PyObject* quantize(PyObject* const* a) {
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    float* const buf = none(a[3]) ? nullptr : values(a[3], x.device(), 1 + hist);   // [scale, hist[0..H-1]]
+    float* const flag = none(a[4]) ? nullptr : values(a[4], x.device());
     at::Tensor out = bytes_like(x, x.sizes()), out_t;
     if (with_t) out_t = bytes_like(x, {cols, rows});
     const Scalars s(x);
@@ -182,19 +199,15 @@ PyObject* quantize(PyObject* const* a) {
     void* ws = workspace_of(x, st);
     void* tp = with_t ? out_t.data_ptr() : nullptr;
     const int xd = code_of(x.scalar_type());
-    if (none(a[3])) {
+    if (buf == nullptr)
         call(ntfp8_quantize_current(x.data_ptr(), xd, rows, cols, fmt, margin, s.p, s.p + 1, out.data_ptr(), tp, nullptr, 0, nullptr, ws, st),
              "ntfp8_quantize_current");
-    } else {
-        float* buf = static_cast<float*>(tensor(a[3]).data_ptr());   // [scale, hist[0..H-1]]
-        if (!none(a[4]))
-            call(ntfp8_quantize_first_use(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist,
-                                          static_cast<float*>(tensor(a[4]).data_ptr()), s.p, s.p + 1, out.data_ptr(), tp, ws, st),
-                 "ntfp8_quantize_first_use");
-        else
-            call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
-                 "ntfp8_quantize_delayed");
-    }
+    else if (flag != nullptr)
+        call(ntfp8_quantize_first_use(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, flag, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
+             "ntfp8_quantize_first_use");
+    else
+        call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
+             "ntfp8_quantize_delayed");
     return quantised(std::move(out), std::move(out_t), s);
 }
 
@@ -217,17 +230,18 @@ PyObject* quantize_batch(PyObject* const* args) {
         if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 5) stop(PyExc_TypeError, "a tensor comes as a tuple of 5");
         PyObject* const* f = &PyTuple_GET_ITEM(t, 0);
         x[i] = dense(tensor(f[0]));
-        const at::Tensor& state = tensor(f[1]);
-        require(x[i].is_cuda() && x[i].device() == x[0].device() && state.device() == x[0].device(), "all tensors of a batch are on one device");
+        require(x[i].is_cuda() && x[i].device() == x[0].device(), "all tensors of a batch are on one device");
         require(x[i].numel() > 0, "cannot quantise an empty tensor");
         const bool with_t = truth(f[4]);
         require(!with_t || x[i].dim() == 2, "with_transpose needs a 2-D tensor");
+        ntfp8_quant_desc& q = d[i];
+        q = {};
+        q.history_len = (int)number(f[2]);
+        q.scale_state = values(f[1], x[0].device(), 1 + q.history_len);
         if (i == 0) {
             st = stream_of(x[0]);
             pool = pool_at((int)x[0].get_device(), st, n);
         }
-        ntfp8_quant_desc& q = d[i];
-        q = {};
         rows_cols(x[i], &q.rows, &q.cols);
         out[i] = bytes_like(x[i], x[i].sizes());
         if (with_t) out_t[i] = bytes_like(x[i], {q.cols, q.rows});
@@ -235,9 +249,7 @@ PyObject* quantize_batch(PyObject* const* args) {
         q.x = x[i].data_ptr();
         q.x_dtype = code_of(x[i].scalar_type());
         q.fmt = fmt;
-        q.history_len = (int)number(f[2]);
         q.margin = (int)number(f[3]);
-        q.scale_state = static_cast<float*>(state.data_ptr());
         q.amax_history = q.scale_state + 1;
         q.amax_out = s[i].p;
         q.scale_used_out = s[i].p + 1;
@@ -264,6 +276,9 @@ void fill(PyObject* const* p, ntfp8_gemm_desc* d, Problem* k, bool fp8_out = fal
     const bool bt = truth(p[8]), at_ = truth(p[10]);
     require(k->a.dim() == 2 && k->b.dim() == 2 && k->a.size(at_ ? 0 : 1) == k->b.size(bt ? 0 : 1), "GEMM operands do not fit together");
     require(k->a.is_cuda() && k->a.device() == k->b.device(), "GEMM operands must be on one CUDA device");
+    codes(k->a), codes(k->b);
+    d->scale_a = values(p[2], k->a.device());
+    d->scale_b = values(p[5], k->a.device());
     const int64_t M = k->a.size(at_ ? 1 : 0), K = k->a.size(at_ ? 0 : 1), N = k->b.size(bt ? 1 : 0);
     const long code = number(p[6]);
     d->accumulate = 0;
@@ -290,8 +305,6 @@ void fill(PyObject* const* p, ntfp8_gemm_desc* d, Problem* k, bool fp8_out = fal
     d->D = k->out.data_ptr();
     d->fmt_a = (int)number(p[1]);
     d->fmt_b = (int)number(p[4]);
-    d->scale_a = static_cast<const float*>(tensor(p[2]).data_ptr());
-    d->scale_b = static_cast<const float*>(tensor(p[5]).data_ptr());
     d->d_dtype = d->accumulate ? NTFP8_F32 : (int)code;
     d->M = M;
     d->N = N;
@@ -336,16 +349,14 @@ PyObject* gemm_batch(PyObject* const* args) {
 PyObject* gemm_fp8(PyObject* const* p) {
     ntfp8_gemm_desc d = {};
     Problem k;
-    fill(p, &d, &k, true);
-    const at::Tensor& state = tensor(p[kProblem]);
     const int hist = (int)number(p[kProblem + 1]), margin = (int)number(p[kProblem + 2]);
-    require(state.device() == k.a.device(), "delayed-scaling state on another device");
+    float* const buf = values(p[kProblem], tensor(p[0]).device(), 1 + hist);
+    fill(p, &d, &k, true);
     at::Tensor out_t;
     if (truth(p[kProblem + 3])) out_t = bytes_like(k.a, {d.N, d.M});
     const Scalars s(k.a);
     void* st = stream_of(k.a);
     void* ws = workspace_of(k.a, st);
-    float* buf = static_cast<float*>(state.data_ptr());
     d.scale_d = buf;
     d.D_t = out_t.defined() ? out_t.data_ptr() : nullptr;
     d.amax_workspace = ws;
@@ -361,10 +372,11 @@ PyObject* cast_with_scale(PyObject* const* a) {
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    const float* scale = values(a[1], x.device());
     at::Tensor out = bytes_like(x, x.sizes()), out_t;
     if (with_t) out_t = bytes_like(x, {cols, rows});
     const Scalars s(x);
-    call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, static_cast<const float*>(tensor(a[1]).data_ptr()), fmt,
+    call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, scale, fmt,
                                s.p, s.p + 1, out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
          "ntfp8_cast_with_scale");
     return quantised(std::move(out), std::move(out_t), s);
@@ -390,23 +402,23 @@ PyObject* column_sum(PyObject* const* a) {
 PyObject* cast(PyObject* const* a) {
     const at::Tensor x = operand(a[0]);
     const int fmt = (int)number(a[2]);
+    const float* scale = values(a[1], x.device());
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     at::Tensor out = bytes_like(x, x.sizes()), out_t;
     const bool with_t = truth(a[3]);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
     if (with_t) out_t = bytes_like(x, {cols, rows});
-    call(ntfp8_cast_to_fp8(x.data_ptr(), code_of(x.scalar_type()), rows, cols, static_cast<const float*>(tensor(a[1]).data_ptr()), fmt,
-                           out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
+    call(ntfp8_cast_to_fp8(x.data_ptr(), code_of(x.scalar_type()), rows, cols, scale, fmt, out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
          "ntfp8_cast_to_fp8");
     return Py_BuildValue("(NN)", wrap(std::move(out)), wrap_or_none(std::move(out_t)));
 }
 
 // dequantize(bytes, fmt, scale, out_code, inverse) -> tensor
 PyObject* dequantize(PyObject* const* a) {
-    const at::Tensor q = operand(a[0]);
+    const at::Tensor q = codes(operand(a[0]));
     const int fmt = (int)number(a[1]);
-    const float* scale = static_cast<const float*>(tensor(a[2]).data_ptr());
+    const float* scale = values(a[2], q.device());
     const long code = number(a[3]);
     at::Tensor out = at::empty(q.sizes(), at::TensorOptions().dtype(type_of(code)).device(q.device()));
     if (q.numel()) {
@@ -418,7 +430,7 @@ PyObject* dequantize(PyObject* const* a) {
 
 // transpose([rows, cols] bytes) -> contiguous [cols, rows] bytes
 PyObject* transpose(PyObject* const* a) {
-    const at::Tensor q = operand(a[0]);
+    const at::Tensor q = codes(operand(a[0]));
     require(q.dim() == 2, "a 2-D tensor is expected");
     at::Tensor out = bytes_like(q, {q.size(1), q.size(0)});
     if (q.numel()) call(ntfp8_transpose(q.data_ptr(), q.size(0), q.size(1), out.data_ptr(), stream_of(q)), "ntfp8_transpose");
