@@ -113,7 +113,8 @@ class FP8Linear(nn.Linear):
         layer keeps it, since filling one costs a launch; memory of a graph capture is not kept beyond it."""
         z = self._zero_element
         if z is None or z.dtype != dtype or z.device != device:
-            z = torch.zeros(1, dtype=dtype, device=device)
+            with torch.inference_mode(False):   # (kept beyond a validation pass under inference mode: training expands it)
+                z = torch.zeros(1, dtype=dtype, device=device)
             if not torch.cuda.is_current_stream_capturing():
                 self._zero_element = z
         return z
