@@ -331,6 +331,8 @@ class _FP8Matmul(torch.autograd.Function):
                 grad_output = fp8_grad   # ... or beside it, already quantised by the consumer's dgrad epilogue
         if grad_output is None:   # a consumer's backward produced no gradient: a gradient of zeros
             grad_output = torch.zeros(ctx.out_shape, dtype=ctx.out_dtype, device=weight.device)
+        if type(grad_output) is torch.Tensor and not grad_output.is_contiguous():
+            grad_output = grad_output.contiguous()   # once: the bias gradient and the quantisation both read it whole
 
         grad_bias = None
         if bias is not None and ctx.needs_input_grad[5]:
