@@ -443,8 +443,8 @@ bool reads_b(int64_t M, int64_t N, int64_t K) {
 }
 PyObject* b_transposed_supported(PyObject* const* a) { return PyBool_FromLong(reads_b(number(a[0]), number(a[1]), number(a[2]))); }
 
-// operand_form(mat_a, a_has_copy, transpose_a, mat_b, b_has_copy, transpose_b, accumulate_into | None, allow_bt, read_b,
-// read_a) -> bits: 1 the library's A is mat_b's transposed copy, 2 its B is mat_a's transposed copy, 4 B read as its
+// operand_form(mat_a, its transposed copy | None, transpose_a, mat_b, its transposed copy | None, transpose_b, accumulate_into |
+// None, allow_bt, read_b, read_a) -> bits: 1 the library's A is mat_b's transposed copy, 2 its B is mat_a's transposed copy, 4 B read as its
 // transpose, 8 A read as its transpose
 PyObject* operand_form(PyObject* const* p) {
     const at::Tensor &a = tensor(p[0]), &b = tensor(p[3]);
@@ -453,13 +453,13 @@ PyObject* operand_form(PyObject* const* p) {
     if (ta) return PyLong_FromLong(tb ? 1 : 0);
     const bool read_b = truth(p[7]) && truth(p[8]), read_a = truth(p[9]);
     auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };   // 16-byte loads / stores
-    const bool plain_a = read_b && !truth(p[1]) && a.dim() == 2 && a.is_contiguous() && aligned(a) && aligned(b) && (none(p[6]) || aligned(tensor(p[6])));
+    const bool plain_a = read_b && none(p[1]) && a.dim() == 2 && a.is_contiguous() && aligned(a) && aligned(b) && (none(p[6]) || aligned(tensor(p[6])));
     if (tb) {
         // D[cols of mat_b, cols of mat_a], reduction over the rows of both
-        if (plain_a && read_a && !truth(p[4]) && b.dim() == 2 && b.is_contiguous() && b.size(1) % 16 == 0 && reads_b(b.size(1), a.size(1), a.size(0)))
+        if (plain_a && read_a && none(p[4]) && b.dim() == 2 && b.is_contiguous() && b.size(1) % 16 == 0 && reads_b(b.size(1), a.size(1), a.size(0)))
             return PyLong_FromLong(4 | 8);
-        // mat_b's copy is a fresh allocation or was one: aligned
-        if (plain_a && b.dim() == 2 && reads_b(b.size(1), a.size(1), a.size(0))) return PyLong_FromLong(1 | 4);
+        // (a copy that has yet to be made is a fresh allocation: aligned)
+        if (plain_a && (none(p[4]) || aligned(tensor(p[4]))) && b.dim() == 2 && reads_b(b.size(1), a.size(1), a.size(0))) return PyLong_FromLong(1 | 4);
         return PyLong_FromLong(1 | 2);
     }
     if (plain_a && b.dim() == 2 && reads_b(b.size(0), a.size(1), a.size(0))) return PyLong_FromLong(4);

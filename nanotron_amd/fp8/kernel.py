@@ -92,9 +92,8 @@ def _operands(mat_a: FP8Tensor, transpose_a: bool, mat_b: FP8Tensor, transpose_b
     (`b_transposed`): that is taken when mat_a carries no transposed copy yet and the shape qualifies; otherwise the
     copy is used (and made, once, if it does not exist).  The same for mat_b (kernel.py:44, `a_transposed`), which the
     library serves next to an untransposed mat_a: the wgrad form."""
-    form = nt.host.operand_form(mat_a, getattr(mat_a, "_transposed", None) is not None, transpose_a, mat_b,
-                                getattr(mat_b, "_transposed", None) is not None, transpose_b, accumulate_into, allow_bt,
-                                READ_B_TRANSPOSED, READ_A_TRANSPOSED)
+    form = nt.host.operand_form(mat_a, getattr(mat_a, "_transposed", None), transpose_a, mat_b, getattr(mat_b, "_transposed", None),
+                                transpose_b, accumulate_into, allow_bt, READ_B_TRANSPOSED, READ_A_TRANSPOSED)
     assert hasattr(mat_a, "fp8_meta") and hasattr(mat_b, "fp8_meta"), "operands must be FP8Tensors"
     return (mat_b.transposed() if form & 1 else mat_b), (mat_a.transposed() if form & 2 else mat_a), bool(form & 4), bool(form & 8)
 
