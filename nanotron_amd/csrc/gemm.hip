@@ -64,8 +64,7 @@ static int path_of(const GemmDesc& g) {
 //   us, 256 / 128 / 64 wide:  1024 x 1024 x 1024  10.1 / 7.5 / 4.8     2048 x 1024 x 4096  26.5 / 16.3 / 15.3
 //   2048 x 2048 x 2048  16.7 / 11.8 / 16.9      both transposed  19.6 / 12.6 / 24.3
 //   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101      16 x 6144 x 4096  - / 13.8 / 8.3
-static int64_t launch_cost(const GemmDesc* const* g, int n, int edge) {
-    const int64_t cus = cu_count();
+static int64_t launch_cost(const GemmDesc* const* g, int n, int edge, int64_t cus) {
     int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
     int form = 0;
     for (int i = 0; i < n; ++i) {
@@ -131,23 +130,24 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* 
 //                    6144 x 3072 9.7 / 9.3     8192 x 4096 13.6 / 12.2   14336 x 4096 15.3 / 16.8 (in 64 columns)
 //   32 rows:         1024 x 4096 8.3 / 8.9     2048 x 6144 15.7 / 13.4   4096 x 14336 31.9 / 24.3   5120 x 5120 14.8 / 17.2
 static bool few_rows(const GemmDesc& g) {
-    if (g.tb || is_fp8_out(g.d_dtype)) return false;
+    if (g.M > 32 || g.tb || is_fp8_out(g.d_dtype)) return false;
     if (g.M <= 16) return g.K >= 2048 && g.N <= 32 * cu_count();
-    return g.M <= 32 && g.K >= 6144 && g.N <= 16 * cu_count();
+    return g.K >= 6144 && g.N <= 16 * cu_count();
 }
 
 // One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
 // tiles: one more launch for a half-tile tail).
 template <int FA, int FB>
 static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
+    const int cus = cu_count();   // (asked once: the question goes to the runtime)
     int edge = 128;
     {
         bool big = true;
         for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
-        int64_t best = launch_cost(g, n, 128);
+        int64_t best = launch_cost(g, n, 128, cus);
         for (const int e : {64, 256}) {
             if (e == 256 && !big) continue;
-            const int64_t c = launch_cost(g, n, e);
+            const int64_t c = launch_cost(g, n, e, cus);
             if (c < best) best = c, edge = e;
         }
     }
@@ -155,14 +155,14 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     const int64_t tiles = list_tiles(g, n, edge, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     const bool fp8_out = is_fp8_out(g[0]->d_dtype);
-    L.round_size = cu_count() * (edge == 64 ? 2 : 1);
+    L.round_size = cus * (edge == 64 ? 2 : 1);
     if (n == 1 && g[0]->fin) {
         L.fin = *g[0]->fin;
         L.fin_blocks = (int)tiles;
     }
     if (edge != 256) return launch_mid(L, FA, FB, edge, fp8_out, (int)tiles, st);
-    const int rem = (int)(tiles % cu_count());
-    L.tail_tiles = (rem != 0 && 2 * rem <= cu_count()) ? rem : 0;
+    const int rem = (int)(tiles % cus);
+    L.tail_tiles = (rem != 0 && 2 * rem <= cus) ? rem : 0;
     L.full_blocks = (int)tiles - L.tail_tiles;
     if (L.fin_blocks) L.fin_blocks = L.full_blocks + 2 * L.tail_tiles;
     (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's

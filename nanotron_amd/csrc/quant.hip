@@ -847,9 +847,9 @@ static int launch_flat(int mode, const void* x, int64_t n, bool vec_ok, uint8_t*
 // 128-wide from one tile per CU on.  us, 128 / 64 wide: bf16 delayed step with transposed copy 2048 x 2048 (256 tiles)
 // 8.7 / 10.6, 4096 x 4096 18 / 34; transpose of 4096 x 4096 bytes 6.0 / 9.2; below one tile per CU fp32 cast of
 // 1021 x 1024 9.7 / 4.6, 1536 x 1584 7.2 / 5.4.
-static int tile_edge(int64_t rows, int64_t cols, int64_t* tiles) {
+static int tile_edge(int64_t rows, int64_t cols, int cus, int64_t* tiles) {
     const int64_t t128 = ((rows + 127) / 128) * ((cols + 127) / 128);
-    if (t128 >= cu_count()) {
+    if (t128 >= cus) {
         *tiles = t128;
         return 16;
     }
@@ -863,8 +863,9 @@ static int launch_transpose(const void* x, int64_t rows, int64_t cols, uint8_t* 
     typedef typename ElemOf<S>::type E;
     const E* xp = static_cast<const E*>(x);
     int64_t tiles;
-    const int e = tile_edge(rows, cols, &tiles);
-    const int64_t cap = (int64_t)cu_count() * (kAmax ? 3 : 8);   // (kAmax: every block is an atomic at the end)
+    const int cus = cu_count();
+    const int e = tile_edge(rows, cols, cus, &tiles);
+    const int64_t cap = (int64_t)cus * (kAmax ? 3 : 8);   // (kAmax: every block is an atomic at the end)
     const int grid = (int)(tiles < cap ? tiles : cap);
     if (e == 16)
         hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
@@ -1123,8 +1124,9 @@ int run_dequant(const void* in, int fmt, const float* scale, int is_inverse, int
 int run_transpose(const void* in, int64_t rows, int64_t cols, void* out, hipStream_t st) {
     clear_stale_error();
     int64_t tiles;
-    const int e = tile_edge(rows, cols, &tiles);
-    const int64_t cap = (int64_t)cu_count() * 8;
+    const int cus = cu_count();
+    const int e = tile_edge(rows, cols, cus, &tiles);
+    const int64_t cap = (int64_t)cus * 8;
     const int grid = (int)(tiles < cap ? tiles : cap);
     const uint8_t* p = static_cast<const uint8_t*>(in);
     uint8_t* o = static_cast<uint8_t*>(out);
