@@ -224,7 +224,8 @@ __device__ __forceinline__ void reg_store4(__amdgpu_buffer_rsrc_t r, uint32_t vo
 // Accumulators past M and past N stay out of the amax: they hold zeros times whatever the other operand holds (NaN
 // against an infinite code), plus the bias, or, where an operand is read through the transposing loads and wraps
 // into its next row, arbitrary values.  N is a multiple of 16, so a block's columns are in or out together, uniformly
-// for the wave; rows are masked lane by lane.
+// for the wave; rows are masked lane by lane.  (By selects: with a branch per block 41 shapes of 256 to 512 256-wide tiles
+// took 65.2 us on average, with these 64.1, without a mask about the same.)
 template <int F, int MI, int NJ, bool kBias = false>
 __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][NJ], uint8_t* __restrict__ D,
                                                           uint8_t* __restrict__ Dt, float alpha, float scale_d, bool slow,
@@ -245,14 +246,14 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 16 + mrow;
         const int mq = m & ~3;
-        const uint32_t inside = m < M ? ~0u : 0u;
-        uint32_t w[NJ];
+        uint32_t w[NJ], row_max = 0;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             uint32_t a = 0;
             w[j] = quant4<F>(val(i, j, 0), val(i, j, 1), val(i, j, 2), val(i, j, 3), scale_d, slow, a);
-            if (n_base + j * 16 < N) amax = max(amax, a & inside);
+            row_max = max(row_max, a & (n_base + j * 16 < N ? ~0u : 0u));
         }
+        amax = max(amax, m < M ? row_max : 0u);
         if (Dt) {   // uniform
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {

@@ -336,6 +336,7 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
     uint32_t amax = 0;
     const bool d_vec = (N & 3) == 0 && d_aligned;   // rows of D start 4-byte aligned
     const bool t_vec = (M & 3) == 0 && (reinterpret_cast<uintptr_t>(Dt) & 3) == 0;
+    const bool n_edge = __builtin_amdgcn_readfirstlane(n_base) + NJ * 32 > N;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 32 + (lane & 31);
@@ -348,13 +349,15 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
                 uint32_t a = 0;
                 const uint32_t w = quant4<F>(acc[i][j][g * 4 + 0] * alpha, acc[i][j][g * 4 + 1] * alpha,
                                              acc[i][j][g * 4 + 2] * alpha, acc[i][j][g * 4 + 3] * alpha, scale_d, slow, a);
-                if (n + 4 > N) {   // a word across the last column, or past it
-                    a = 0;
+                if (n_edge) {   // uniform; a word across the last column, or past it
+                    if (n + 4 > N) {
+                        a = 0;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < N) a = max(a, __float_as_uint(acc[i][j][g * 4 + e] * alpha) & 0x7fffffffu);
+                        for (int e = 0; e < 4; ++e)
+                            if (n + e < N) a = max(a, __float_as_uint(acc[i][j][g * 4 + e] * alpha) & 0x7fffffffu);
+                    }
                 }
-                if (m < M) amax = max(amax, a);
+                amax = max(amax, m < M ? a : 0u);
                 if (m < M && n < N) store_bytes4(D + (int64_t)m * N + n, w, d_vec, N - n);
                 if (Dt) {   // uniform
                     const uint32_t t = quad_transpose_bytes(w, lane);
