@@ -17,7 +17,8 @@
 //   gemm_any_kernel       (gemm_any.h) any K and alignment: 64- or 128-wide tiles, fp8 widened to bf16 on its way to
 //                         the matrix cores.
 //   gemm_nt_kernel        128 x 128 x 128 tiles, loads through registers: fp8 outputs whose rows or columns do not come in
-//                         whole words (the other kernels' fp8 epilogue stores nothing smaller).
+//                         whole words (the other kernels' fp8 epilogue stores nothing smaller), and large results of
+//                         fewer than two K-tiles.
 #include "gemm_common.h"
 #include "gemm_big.h"
 
@@ -25,12 +26,12 @@ namespace ntfp8 {
 
 // ---------------------------------------------------------------------------------------------
 constexpr int kMinTransposed = 128;   // rows and columns of a result whose B is given as its transpose: more than this
-enum GemmPath { kPathNone = -1, kPathAny = 0, kPathWords = 1, kPathTiles = 2 };
+enum GemmPath { kPathNone = -1, kPathAny = 0, kPathPlain = 1, kPathTiles = 2 };
 
 int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_few(const BigProblem& p, int fa, int fb, hipStream_t st);
 int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
-int launch_words(const GemmDesc& g, hipStream_t st);
+int launch_plain(const GemmDesc& g, hipStream_t st);
 int run_amax_finalize(Workspace* ws, const ScalarIO& io, hipStream_t st);
 
 // operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
@@ -39,6 +40,22 @@ static bool fits32(const GemmDesc& g) {
 }
 // the 256-wide tiles' pipeline starts with two K-tiles
 static bool big_ok(const GemmDesc& g) { return fits32(g) && g.K >= 2 * kBK; }
+
+// A launch of one problem of fewer than two K-tiles (the 256-wide tiles cannot take it) and more 64-wide tiles than the
+// chip works on at once: nothing hides the prologue and epilogue of the one or two workgroups per CU of the smaller tiles,
+// and 16- and 32-bit rows that end inside a 64-byte piece of memory make their streaming stores partial writes (for fp8
+// only the transposed copy has any).  us, tiles of gemm_mid.h / gemm_nt_kernel, K 144 to 240:
+//   bf16, whole pieces:   513 to 1024 tiles of 64 5.7 / 6.1, 1025 to 1536 9.0 / 7.8, 3136 x 3920 25.1 / 12.1
+//   bf16, others:         up to 256 tiles 4.0 / 4.8, 257 to 512 5.7 / 5.3, 513 to 1024 8.0 / 6.1, more 18.5 / 10.1
+//   fp8:                  257 to 512 tiles 9.3 / 11.3, 513 to 1024 10.7 / 12.2, 1025 to 1536 16.0 / 13.4
+//   fp8 with its copy, N % 64 != 0:  257 to 512 11.7 / 12.5, 513 to 768 14.2 / 13.2, more 38.7 / 22.1
+static bool short_k(const GemmDesc& g) {
+    if (g.K >= 2 * kBK || g.tb) return false;
+    const int64_t tiles = (((int64_t)g.M + 63) / 64) * (((int64_t)g.N + 63) / 64);
+    const bool whole = (int64_t)g.N * (g.d_dtype == NTFP8_F32 ? 4 : is_fp8_out(g.d_dtype) ? 1 : 2) % 64 == 0;
+    const int per_cu = whole ? 4 : !is_fp8_out(g.d_dtype) ? 1 : g.Dt ? 2 : 4;
+    return tiles > per_cu * cu_count();
+}
 
 // which kernels serve a problem
 static int path_of(const GemmDesc& g) {
@@ -54,7 +71,7 @@ static int path_of(const GemmDesc& g) {
     // read only next to a transposed B (the wgrad form)
     if (g.ta && (!g.tb || g.M % 16 != 0)) return kPathNone;
     if (g.tb) return (g.N % 16 == 0 && fits32(g) && g.M > kMinTransposed && g.N > kMinTransposed && g.K >= 2 * kBK && fp8_ok) ? kPathTiles : kPathNone;
-    if (!fp8_ok) return kPathWords;
+    if (!fp8_ok) return kPathPlain;
     return (int64_t)g.K * 128 < (1LL << 31) ? kPathTiles : kPathAny;   // (a tile's rows within reach of 32-bit offsets)
 }
 
@@ -228,7 +245,7 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     return launch_tiles<kE4M3, kE4M3>(g, n, st);
 #else
     if (path == kPathAny) return launch_any_tiles(g, n, st);
-    if (path == kPathWords) return finish_behind(*g[0], launch_words(*g[0], st), st);
+    if (path == kPathPlain || (n == 1 && short_k(*g[0]))) return finish_behind(*g[0], launch_plain(*g[0], st), st);
     if (n == 1 && few_rows(*g[0])) {
         BigLaunch L;
         list_tiles(g, 1, 64, &L);
@@ -258,7 +275,7 @@ int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
         const int path = path_of(g[i]);
         group[cnt++] = &g[i];
         done[i] = true;
-        if (path != kPathWords) {
+        if (path != kPathPlain) {
             for (int j = i + 1; j < n && cnt < kBigMaxProblems; ++j)
                 if (!done[j] && g[j].fmt_a == g[i].fmt_a && g[j].fmt_b == g[i].fmt_b && path_of(g[j]) == path &&
                     is_fp8_out(g[j].d_dtype) == is_fp8_out(g[i].d_dtype) && g[j].tb == g[i].tb) {

@@ -1,5 +1,5 @@
 // Instantiations and launchers of the GEMM kernels off the main path: any K and alignment (gemm_any.h), and fp8 outputs
-// whose rows or columns do not come in whole words.  The choice is made in gemm.hip.
+// whose rows or columns do not come in whole words or large results of few K-tiles.  The choice is made in gemm.hip.
 #include "gemm_common.h"
 #include "gemm_big.h"
 #include "gemm_any.h"
@@ -26,15 +26,18 @@ int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int t
 }
 
 // ---------------------------------------------------------------------------------------------
-// 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.
+// 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.  Bound by HBM on the shapes it serves
+// (mostly output): 32 KB of LDS and 120 registers put several workgroups on a CU, whose prologues and epilogues overlap.
 constexpr int kBM = 128, kBN = 128;
 constexpr int kGemmThreads = 256;
 
+// DT: an fp8 output type, or NTFP8_F32 for every other (`d_dtype` and `accumulate` at run time).
 template <int FA, int FB, int DT>
 __global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                                void* __restrict__ Dv, const float* __restrict__ scale_a,
                                                                const float* __restrict__ scale_b, int M, int N, int K,
-                                                               int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex) {
+                                                               int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex,
+                                                               int d_dtype, int accumulate) {
     __shared__ __attribute__((aligned(16))) uint8_t sA[kBM * kBK];
     __shared__ __attribute__((aligned(16))) uint8_t sB[kBN * kBK];
 
@@ -119,36 +122,48 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __
         add_bias32<2, 2>(acc, alpha, ex.bias, ex.bias_dtype, N, n0 + wn, lane);
         alpha = 1.0f;
     }
-    constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
-    const float scale_d = *fp8.scale;
-    const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
-                                                       scale_is_degenerate(scale_d), M, N, m0 + wm, n0 + wn, lane);
-    publish_amax(amax, fp8.ws);
+    const int mb = m0 + wm, nb = n0 + wn;
+    if constexpr (DT != NTFP8_F32) {
+        constexpr int F = DT == NTFP8_OUT_E4M3 ? kE4M3 : kE5M2;
+        const float scale_d = *fp8.scale;
+        const uint32_t amax = store_wave_tile_fp8<F, 2, 2>(acc, static_cast<uint8_t*>(Dv), fp8.Dt, alpha, scale_d,
+                                                           scale_is_degenerate(scale_d), M, N, mb, nb, lane);
+        publish_amax(amax, fp8.ws);
+    } else if (d_dtype == NTFP8_BF16) {
+        store_wave_tile<NTFP8_BF16, false, 2, 2>(acc, Dv, alpha, M, N, mb, nb, lane);
+    } else if (d_dtype == NTFP8_F16) {
+        store_wave_tile<NTFP8_F16, false, 2, 2>(acc, Dv, alpha, M, N, mb, nb, lane);
+    } else if (accumulate) {
+        store_wave_tile<NTFP8_F32, true, 2, 2>(acc, Dv, alpha, M, N, mb, nb, lane);
+    } else {
+        store_wave_tile<NTFP8_F32, false, 2, 2>(acc, Dv, alpha, M, N, mb, nb, lane);
+    }
 }
 
 template <int FA, int FB>
-static void launch_words_fmt(const GemmDesc& g, hipStream_t st) {
+static void launch_plain_fmt(const GemmDesc& g, hipStream_t st) {
     const int tm = (g.M + kBM - 1) / kBM, tn = (g.N + kBN - 1) / kBN;
     const uint8_t* a = static_cast<const uint8_t*>(g.A);
     const uint8_t* b = static_cast<const uint8_t*>(g.B);
     const Fp8Out fp8 = {g.sd, static_cast<uint8_t*>(g.Dt), static_cast<Workspace*>(g.ws)};
     const GemmExtras ex = {g.bias, g.bias_dtype, g.scale_inv};
-    if (g.d_dtype == NTFP8_OUT_E4M3)
-        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, NTFP8_OUT_E4M3>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb, g.M,
-                           g.N, g.K, tm, tn, fp8, ex);
-    else
-        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, NTFP8_OUT_E5M2>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb, g.M,
-                           g.N, g.K, tm, tn, fp8, ex);
+    auto go = [&](auto dt) {
+        hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, decltype(dt)::value>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb,
+                           g.M, g.N, g.K, tm, tn, fp8, ex, g.d_dtype, g.accumulate);
+    };
+    if (g.d_dtype == NTFP8_OUT_E4M3) go(std::integral_constant<int, NTFP8_OUT_E4M3>{});
+    else if (g.d_dtype == NTFP8_OUT_E5M2) go(std::integral_constant<int, NTFP8_OUT_E5M2>{});
+    else go(std::integral_constant<int, NTFP8_F32>{});
 }
 
-int launch_words(const GemmDesc& g, hipStream_t st) {
+int launch_plain(const GemmDesc& g, hipStream_t st) {
     (void)hipGetLastError();
     if (g.fmt_a == kE4M3) {
-        if (g.fmt_b == kE4M3) launch_words_fmt<kE4M3, kE4M3>(g, st);
-        else launch_words_fmt<kE4M3, kE5M2>(g, st);
+        if (g.fmt_b == kE4M3) launch_plain_fmt<kE4M3, kE4M3>(g, st);
+        else launch_plain_fmt<kE4M3, kE5M2>(g, st);
     } else {
-        if (g.fmt_b == kE4M3) launch_words_fmt<kE5M2, kE4M3>(g, st);
-        else launch_words_fmt<kE5M2, kE5M2>(g, st);
+        if (g.fmt_b == kE4M3) launch_plain_fmt<kE5M2, kE4M3>(g, st);
+        else launch_plain_fmt<kE5M2, kE5M2>(g, st);
     }
     return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
 }

@@ -74,3 +74,13 @@ def test_problems_of_different_layout_and_depth_in_one_call():
         dx, dw = nt.host.gemm_batch([(q[0], 0, one, q[2], 0, one, nt.BF16, None, True, None, False),
                                      (q[0], 0, one, q[1], 0, one, nt.F32, None, True, None, True)])
         assert torch.equal(dx, (dy @ w).to(torch.bfloat16)) and torch.equal(dw, dy.t() @ x)
+
+
+@pytest.mark.parametrize("K", [16, 128, 240, 256])
+@pytest.mark.parametrize("mn", [(1024, 4096), (1040, 4100), (1009, 1008), (1025, 1008), (1030, 1001), (2100, 2130)])
+def test_large_results_of_few_k_tiles(mn, K):
+    """Both sides of the lines beyond which a launch of fewer than two K-tiles goes to gemm_nt_kernel."""
+    _check(*mn, K, "plain", torch.float32)
+    _check(*mn, K, "plain", torch.float32, acc=True)
+    _check(*mn, K, "plain", torch.bfloat16, bias=True)
+    _check(*mn, K, "plain", torch.float16)
