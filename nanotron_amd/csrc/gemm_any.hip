@@ -27,13 +27,13 @@ int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int t
 
 // ---------------------------------------------------------------------------------------------
 // 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.  Bound by HBM on the shapes it serves
-// (mostly output): 32 KB of LDS and 120 registers put several workgroups on a CU, whose prologues and epilogues overlap.
+// (mostly output): its prologues and epilogues overlap in the three workgroups that a CU holds (168 registers: two more and it is two).
 constexpr int kBM = 128, kBN = 128;
 constexpr int kGemmThreads = 256;
 
 // DT: an fp8 output type, or NTFP8_F32 for every other (`d_dtype` and `accumulate` at run time).
 template <int FA, int FB, int DT>
-__global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
+__global__ __launch_bounds__(kGemmThreads, 3) void gemm_nt_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                                void* __restrict__ Dv, const float* __restrict__ scale_a,
                                                                const float* __restrict__ scale_b, int M, int N, int K,
                                                                int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex,

@@ -336,11 +336,11 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
     uint32_t amax = 0;
     const bool d_vec = (N & 3) == 0 && d_aligned;   // rows of D start 4-byte aligned
     const bool t_vec = (M & 3) == 0 && (reinterpret_cast<uintptr_t>(Dt) & 3) == 0;
-    const bool n_edge = __builtin_amdgcn_readfirstlane(n_base) + NJ * 32 > N;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 32 + (lane & 31);
         const int mq = m & ~3;   // first row of this lane's quad
+        uint32_t row_max = 0;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
 #pragma unroll
@@ -349,15 +349,7 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
                 uint32_t a = 0;
                 const uint32_t w = quant4<F>(acc[i][j][g * 4 + 0] * alpha, acc[i][j][g * 4 + 1] * alpha,
                                              acc[i][j][g * 4 + 2] * alpha, acc[i][j][g * 4 + 3] * alpha, scale_d, slow, a);
-                if (n_edge) {   // uniform; a word across the last column, or past it
-                    if (n + 4 > N) {
-                        a = 0;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (n + e < N) a = max(a, __float_as_uint(acc[i][j][g * 4 + e] * alpha) & 0x7fffffffu);
-                    }
-                }
-                amax = max(amax, m < M ? a : 0u);
+                row_max = max(row_max, n + 4 <= N ? a : 0u);
                 if (m < M && n < N) store_bytes4(D + (int64_t)m * N + n, w, d_vec, N - n);
                 if (Dt) {   // uniform
                     const uint32_t t = quad_transpose_bytes(w, lane);
@@ -366,6 +358,17 @@ __device__ __forceinline__ uint32_t store_wave_tile_fp8(const v16f (&acc)[MI][NJ
                 }
             }
         }
+        amax = max(amax, m < M ? row_max : 0u);
+    }
+    if ((N & 3) != 0 && __builtin_amdgcn_readfirstlane(n_base) + NJ * 32 > N) {   // uniform: the words across the last column
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int r = 0; r < 16 * NJ; ++r) {
+                const int n = n_base + (r >> 4) * 32 + ((r >> 2) & 3) * 8 + (lane >> 5) * 4;
+                const uint32_t a = __float_as_uint(acc[i][r >> 4][r & 15] * alpha) & 0x7fffffffu;
+                amax = max(amax, n + 4 > N && n + (r & 3) < N && m_base + i * 32 + (lane & 31) < M ? a : 0u);
+            }
     }
     return amax;
 }
