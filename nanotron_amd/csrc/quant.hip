@@ -486,6 +486,29 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
     if constexpr (kAmax) publish_and_finalize<kTileThreads>(L::to_f32_bits(m_run), ws, io, kModeDelayed, pre);
 }
 
+// The same for small tensors, one element per thread: bound by the latency of one pass, which a tile's trip through LDS
+// and its code (read from memory by every CU) lengthen.  us, tiles / here: cast of 333 x 515 fp32 4.9 / 3.9, 223 x 162
+// 4.8 / 3.2, delayed step of 2^15 elements bf16 5.8 / 4.7.
+template <typename S, int F, bool kAmax>
+__global__ __launch_bounds__(kThreads) void quant_transpose_small_kernel(const typename ElemOf<S>::type* __restrict__ x, int rows, int cols,
+                                                                     uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
+                                                                     const float* __restrict__ scale_ptr, Workspace* ws, ScalarIO io) {
+    typedef Src<S> L;
+    const float scale = *scale_ptr;
+    EpiloguePrefetch pre = {0.0f, 1.0f};
+    if constexpr (kAmax) pre = prefetch_epilogue(io, kModeDelayed);
+    else record_cast_scale(io, scale, blockIdx.x);
+    const uint32_t n = (uint32_t)rows * cols;
+    uint32_t m = 0;
+    const uint32_t j = blockIdx.x * kThreads + threadIdx.x;
+    if (j < n) {
+        const uint8_t b = encode1<F>(L::load1(x + j, m), scale);
+        if (out) out[j] = b;
+        out_t[j % (uint32_t)cols * rows + j / (uint32_t)cols] = b;
+    }
+    if constexpr (kAmax) publish_and_finalize<kThreads>(L::to_f32_bits(m), ws, io, kModeDelayed, pre);
+}
+
 // [rows, cols] bytes -> [cols, rows]
 template <int E>
 __global__ __launch_bounds__(kTileThreads) void transpose_kernel(const uint8_t* __restrict__ in, int64_t rows, int64_t cols,
@@ -862,6 +885,15 @@ static int launch_transpose(const void* x, int64_t rows, int64_t cols, uint8_t* 
                             Workspace* ws, const ScalarIO& io, hipStream_t st) {
     typedef typename ElemOf<S>::type E;
     const E* xp = static_cast<const E*>(x);
+    // One element per thread up to where tiles are faster.  us, tiles / small kernel, 16-bit: cast of 2^17 to 2^17.5 elements
+    // 4.1 / 3.6, to 2^18 4.1 / 3.9, to 2^18.5 4.2 / 4.4; delayed step up to 2^17 6.1 / 5.4, beyond (more workgroups than
+    // have a word each, reduce.h) 6.1 / 7.0.
+    if (rows * cols <= (kAmax ? (int64_t)kCells * kThreads : 3 << 16)) {
+        const int grid = (int)((rows * cols + kThreads - 1) / kThreads);
+        hipLaunchKernelGGL((quant_transpose_small_kernel<S, F, kAmax>), dim3(grid), dim3(kThreads), 0, st, xp, (int)rows, (int)cols, out, out_t,
+                           scale_ptr, ws, io);
+        return check_launch();
+    }
     int64_t tiles;
     const int cus = cu_count();
     const int e = tile_edge(rows, cols, cus, &tiles);

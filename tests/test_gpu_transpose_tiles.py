@@ -9,7 +9,9 @@ pytestmark = pytest.mark.gpu
 
 # below one 128-wide tile per CU (64-wide tiles), and above it with remainders of every kind
 SHAPES = [(1, 1), (1, 70), (67, 1), (63, 65), (64, 64), (129, 3), (200, 333), (128 * 16, 128 * 16), (128 * 16 + 1, 128 * 16 + 15),
-          (128 * 16 + 14, 128 * 17 + 7)]
+          (128 * 16 + 14, 128 * 17 + 7),
+          # one element per thread up to 131072 (delayed step) and 196608 (cast) elements, 64-wide tiles beyond
+          (512, 256), (257, 511), (384, 512), (131, 1501), (449, 515), (1021, 703)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
