@@ -17,8 +17,8 @@ constexpr int kE5M2 = NTFP8_E5M2;
 constexpr uint32_t kInfBits = 0x7f800000u;
 constexpr uint32_t kNanBits = 0x7fc00000u;
 
-// Reduction scratch shared by the blocks of one launch.  All zero between launches.  Quantise launches of up to 512 blocks
-// use it as one word per block instead (reduce.h); the members below are the ticket protocol's.
+// Reduction scratch shared by the blocks of one launch.  All zero between launches.  Quantise launches use it as one word
+// per block instead (reduce.h); the members below are for GEMMs with fp8 outputs.
 // Every counter sits on its own 128-byte line: atomics on one address serialise (~10 ns each on
 // MI355X), atomics on different lines proceed in parallel.
 constexpr int kMaxSlots = 8;

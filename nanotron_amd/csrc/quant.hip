@@ -1,7 +1,7 @@
 // amax reduction, delayed-scaling history roll + scale update, saturating casts to OCP FP8,
-// dequantisation and byte transpose for gfx950.  All kernels are HBM-bandwidth bound: one pass
-// over the input with 128-bit loads and stores, a wavefront reduction for the amax, one atomic per
-// block and a last-block epilogue that finishes the scalar bookkeeping in the same launch.
+// dequantisation and byte transpose for gfx950.  All kernels are HBM-bandwidth bound on large tensors: one pass
+// over the input with 128-bit loads and stores, a wavefront reduction for the amax, one word stored per
+// block and the bookkeeping by the highest-numbered block, which waits for the words, in the same launch.
 #include "common.h"
 #include "reduce.h"
 
@@ -835,7 +835,7 @@ __global__ void update_scale_kernel(const float* amax, const float* old_scale, i
 // blocks for `work_items` thread-steps with `threads` per block, at most `per_cu_blocks` per CU
 static int grid_for(int64_t work_items, int threads = kThreads, int per_cu_blocks = 8) {
     int64_t want = (work_items + threads - 1) / threads;
-    int64_t cap = (int64_t)cu_count() * per_cu_blocks;
+    int64_t cap = (int64_t)cu_count() * per_cu_blocks;   // (one per CU for whatever takes a maximum: fewer than kCells)
     if (want < 1) want = 1;
     return (int)(want < cap ? want : cap);
 }
@@ -866,13 +866,16 @@ static int launch_flat(int mode, const void* x, int64_t n, bool vec_ok, uint8_t*
     return check_launch();
 }
 
-// Columns per thread (16: 128-wide tiles, 4: 64-wide) of the kernels that turn tiles around, and their tile count.
-// 128-wide from one tile per CU on.  us, 128 / 64 wide: bf16 delayed step with transposed copy 2048 x 2048 (256 tiles)
-// 8.7 / 10.6, 4096 x 4096 18 / 34; transpose of 4096 x 4096 bytes 6.0 / 9.2; below one tile per CU fp32 cast of
-// 1021 x 1024 9.7 / 4.6, 1536 x 1584 7.2 / 5.4.
-static int tile_edge(int64_t rows, int64_t cols, int cus, int64_t* tiles) {
+// Columns per thread (16: 128-wide tiles, 4: 64-wide) of the kernels that turn tiles around, and their tile count: 128-wide
+// from `from` of them on, in eighths of the CUs.  us, 128 / 64 wide:
+//   delayed step with copy (5 eighths: from there on 64-wide tiles are more workgroups than have a word each, reduce.h),
+//     bf16, 128 to 159 tiles 7.8 / 8.7, 160 to 191 8.2 / 9.6, 224 to 255 8.4 / 10.8; fp32 9.5 / 9.3, 9.9 / 10.4, 10.9 / 13.3
+//   cast with copy (7 eighths), bf16, 160 to 191 tiles 5.8 / 5.5, 192 to 223 5.8 / 5.9, 224 to 255 6.2 / 6.3; fp32 6.3 / 5.9,
+//     6.3 / 6.4, 6.6 / 6.9; rows of any alignment 7.3 / 6.6, 7.3 / 7.2, 7.6 / 7.8
+//   transpose (8) of 4096 x 4096 bytes 6.0 / 9.2
+static int tile_edge(int64_t rows, int64_t cols, int cus, int from, int64_t* tiles) {
     const int64_t t128 = ((rows + 127) / 128) * ((cols + 127) / 128);
-    if (t128 >= cus) {
+    if (8 * t128 >= (int64_t)from * cus) {
         *tiles = t128;
         return 16;
     }
@@ -896,8 +899,10 @@ static int launch_transpose(const void* x, int64_t rows, int64_t cols, uint8_t* 
     }
     int64_t tiles;
     const int cus = cu_count();
-    const int e = tile_edge(rows, cols, cus, &tiles);
-    const int64_t cap = (int64_t)cus * (kAmax ? 3 : 8);   // (kAmax: every block is an atomic at the end)
+    const int e = tile_edge(rows, cols, cus, kAmax ? 5 : 7, &tiles);
+    // (kAmax: no more workgroups than have a word each; with three per CU and tickets bf16 of 1024 tiles took 25.4 us
+    // instead of 24.2, fp32 of 512 24.6 instead of 23.6)
+    const int64_t cap = kAmax ? std::min<int64_t>(2 * cus, kCells) : 8 * cus;
     const int grid = (int)(tiles < cap ? tiles : cap);
     if (e == 16)
         hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
@@ -1157,7 +1162,7 @@ int run_transpose(const void* in, int64_t rows, int64_t cols, void* out, hipStre
     clear_stale_error();
     int64_t tiles;
     const int cus = cu_count();
-    const int e = tile_edge(rows, cols, cus, &tiles);
+    const int e = tile_edge(rows, cols, cus, 8, &tiles);
     const int64_t cap = (int64_t)cus * 8;
     const int grid = (int)(tiles < cap ? tiles : cap);
     const uint8_t* p = static_cast<const uint8_t*>(in);

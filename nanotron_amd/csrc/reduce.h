@@ -8,11 +8,10 @@ namespace ntfp8 {
 // ---------------------------------------------------------------------------------------------
 // Block reduction of the partial max, publication, and the bookkeeping epilogue of one block.
 //
-// Inter-block traffic uses relaxed device-scope atomics only (they execute at the level where all
-// XCDs agree).  Either a block's maximum is one word that says by itself that it has arrived (publish_and_finalize), or
-// the wave's own memory counter orders two of them: the partial max is folded in with a returning atomic, the wave waits
-// for it, then takes a ticket.  A release fence here would write back the whole L2 once per block, which costs more than
-// the streaming pass itself.
+// Inter-block traffic uses relaxed device-scope atomics only (they execute at the level where all XCDs agree).  In a
+// quantise launch a block's maximum is one word that says by itself that it has arrived (publish_and_finalize); in a GEMM
+// the wave's own memory counter orders two: the maxima of a workgroup's waves are in the slots before it draws a ticket.
+// A release fence here would write back the whole L2 once per block, which costs more than the streaming pass itself.
 // What the bookkeeping block's epilogue will read, requested by the first wave of every block while the
 // tensor is still streaming: the history entry that moves into this lane's slot and the scale in
 // force.  It takes one round trip out of the dependent chain at the end of the kernel.
@@ -104,12 +103,8 @@ __device__ inline void clear_workspace(Workspace* ws) {
     }
 }
 
-// `io2` / `pre2`: a second tensor role fed by the same amax (one source tensor quantised to both formats).
-__device__ inline void finalize_wave(Workspace* ws, const ScalarIO& io, int mode, const EpiloguePrefetch& pre,
-                                     const ScalarIO* io2 = nullptr, const EpiloguePrefetch* pre2 = nullptr) {
-    const uint32_t bits = collect_amax(ws);
-    bookkeep(bits, io, mode, pre);
-    if (io2) bookkeep(bits, *io2, mode, *pre2);
+__device__ inline void finalize_wave(Workspace* ws, const ScalarIO& io, int mode, const EpiloguePrefetch& pre) {
+    bookkeep(collect_amax(ws), io, mode, pre);
     clear_workspace(ws);
 }
 
@@ -125,14 +120,13 @@ __device__ __forceinline__ bool draw_ticket(Workspace* ws, uint32_t bid, uint32_
     return __hip_atomic_fetch_add(&ws->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
 }
 
-// Up to kCells workgroups: the workspace as one word per workgroup.  A workgroup stores its maximum, marked as present, and
-// is done; the one with the highest number (dispatched last) reads the words until all are there.  That is one store and
-// one read behind the last maximum, where the ticket protocol needs four dependent round trips to the memory side
-// (maximum, ticket of the group, ticket of the launch, slots).  Bound by that latency on small tensors: delayed step of
-// bf16 2048 x 2048 8.8 -> 7.3 us, 4096 x 4096 12.0 -> 10.8 us alone and 14.9 -> 13.4 us inside a training step.  Beyond
-// kCells (transposed copies of more than two tiles per CU) the ticket protocol serves.  Nobody waits for the reading wave, so every word arrives;
-// the trip limit (many seconds) only keeps a workspace that two overlapping launches share against the rules from
-// holding the GPU.
+// Quantise launches (at most kCells workgroups reduce one tensor): the workspace as one word per workgroup.  A workgroup
+// stores its maximum, marked as present, and is done; the one with the highest number (dispatched last) reads the words
+// until all are there.  That is one store and one read behind the last maximum, where slots and tickets need four
+// dependent round trips to the memory side (maximum, ticket of the group, ticket of the launch, slots).  Bound by that
+// latency on small tensors: delayed step of bf16 2048 x 2048 8.8 -> 7.3 us, 4096 x 4096 12.0 -> 10.8 us alone and 14.9 ->
+// 13.4 us inside a training step.  Nobody waits for the reading wave, so every word arrives; the trip limit (many seconds)
+// only keeps a workspace that two overlapping launches share against the rules from holding the GPU.
 constexpr uint32_t kCells = NTFP8_WORKSPACE_BYTES / 4, kPresent = 0x80000000u;
 __device__ inline uint32_t collect_cells(uint32_t own, Workspace* ws, uint32_t others) {
     uint32_t* cell = reinterpret_cast<uint32_t*>(ws);
@@ -159,8 +153,9 @@ __device__ inline uint32_t collect_cells(uint32_t own, Workspace* ws, uint32_t o
     return best > kInfBits ? kNanBits : best;
 }
 
-// `bid` of `nblocks`: this workgroup's place among the workgroups that reduce the same tensor (the whole grid,
-// except in a launch that carries several tensors).
+// `bid` of `nblocks` (at most kCells): this workgroup's place among the workgroups that reduce the same tensor (the whole
+// grid, except in a launch that carries several tensors).
+// `io2` / `pre2`: a second tensor role fed by the same amax (one source tensor quantised to both formats).
 template <int THREADS>
 __device__ inline void publish_and_finalize(uint32_t m_f32bits, Workspace* ws, const ScalarIO& io, int mode,
                                             const EpiloguePrefetch& pre, uint32_t bid = blockIdx.x,
@@ -174,26 +169,14 @@ __device__ inline void publish_and_finalize(uint32_t m_f32bits, Workspace* ws, c
     uint32_t bm = 0;
 #pragma unroll
     for (int i = 0; i < THREADS / 64; ++i) bm = s_part[i] > bm ? s_part[i] : bm;
-    if (nblocks <= kCells) {
-        if (bid != nblocks - 1) {
-            if (threadIdx.x == 0)
-                __hip_atomic_store(reinterpret_cast<uint32_t*>(ws) + bid, bm | kPresent, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return;
-        }
-        const uint32_t bits = collect_cells(bm, ws, nblocks - 1);
-        bookkeep(bits, io, mode, pre);
-        if (io2) bookkeep(bits, *io2, mode, *pre2);
+    if (bid != nblocks - 1) {
+        if (threadIdx.x == 0)
+            __hip_atomic_store(reinterpret_cast<uint32_t*>(ws) + bid, bm | kPresent, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    uint32_t last = 0;
-    if (threadIdx.x == 0) {
-        const uint32_t grp = bid % kMaxSlots;
-        const uint32_t old = __hip_atomic_fetch_max(&ws->slot[grp].bits, bm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::"v"(old) : "memory");   // the max is in place before the ticket is drawn
-        last = draw_ticket(ws, bid, nblocks) ? 1u : 0u;
-    }
-    // the bookkeeping is the work of the block that drew the last ticket
-    if (__builtin_amdgcn_readfirstlane(last)) finalize_wave(ws, io, mode, pre, io2, pre2);
+    const uint32_t bits = collect_cells(bm, ws, nblocks - 1);
+    bookkeep(bits, io, mode, pre);
+    if (io2) bookkeep(bits, *io2, mode, *pre2);
 }
 
 }  // namespace ntfp8

@@ -40,7 +40,7 @@ def test_one_table_of_workspaces():
 
         FP8Tensor(xs[0], DTypes.FP8E4M3, state=states[0])                                        # one word per workgroup
         assert int(ws.abs().sum()) == 0
-        FP8Tensor(torch.randn(4096, 3072, device=DEV), DTypes.FP8E4M3, state=states[0], with_transpose=True)   # tickets
+        FP8Tensor(torch.randn(4096, 3072, device=DEV), DTypes.FP8E4M3, state=states[0], with_transpose=True)   # of two per CU
         assert int(ws.abs().sum()) == 0
         nt.host.column_sum(torch.randn(4096, 256, device=DEV), nt.F32)                           # tickets of the column blocks
         assert int(ws.abs().sum()) == 0
