@@ -750,13 +750,14 @@ __device__ __forceinline__ void decode2(uint32_t w, float& a, float& b) {
 }
 
 // HBM-bound.  A lane writes 16 bytes per group (8 16-bit or 4 fp32 elements, read as 8 or 4 bytes), so that a wave's
-// loads and stores each cover one contiguous piece, and has kDqUnroll groups in flight.  Loads go through the caches (the
+// loads and stores each cover one contiguous piece, and has kUnroll groups in flight.  Loads go through the caches (the
 // bytes were usually written by the kernel before), stores are streaming.  bf16, 4096 x 4096 (50.3 MB): 15.5 us with one
 // byte per lane and trip, 8.1 us (6.2 TB/s) now; streaming loads as well 9.4 us, ordinary stores 9.0 us, one group per
-// trip 9.3 us.
+// trip 9.3 us.  kUnroll: groups a thread has in flight; one where that still is no more than eight workgroups per CU (us, one
+// / four: 16-bit of 2^18 to 2^20 elements 3.04 / 3.11, 2^21 to 2^22 3.7 / 3.8, 2^23 to 2^24 6.5 / 6.0; fp32 of 2^19 to 2^21
+// 3.55 / 3.60, 2^22 to 2^23 6.8 / 6.0).
 // `is_inverse`: scale_ptr holds 1 / scale already (the form tex.cast_from_fp8 is handed, src/nanotron/fp8/tensor.py:74)
-constexpr int kDqUnroll = 4;
-template <int F, int OUT>
+template <int F, int OUT, int kUnroll>
 __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __restrict__ in, int64_t n_vec, int64_t n,
                                                            const float* __restrict__ scale_ptr, void* __restrict__ out,
                                                            int is_inverse) {
@@ -764,14 +765,14 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __rest
     typedef uint32_t win __attribute__((ext_vector_type(kE / 4)));
     typedef win win_any __attribute__((aligned(1)));   // the input may start anywhere
     const float inv = is_inverse ? *scale_ptr : 1.0f / *scale_ptr;
-    const int64_t stride = (int64_t)gridDim.x * (kThreads * kDqUnroll);
-    for (int64_t i = (int64_t)blockIdx.x * (kThreads * kDqUnroll) + threadIdx.x; i < n_vec; i += stride) {
-        win w[kDqUnroll];
+    const int64_t stride = (int64_t)gridDim.x * (kThreads * kUnroll);
+    for (int64_t i = (int64_t)blockIdx.x * (kThreads * kUnroll) + threadIdx.x; i < n_vec; i += stride) {
+        win w[kUnroll];
 #pragma unroll
-        for (int u = 0; u < kDqUnroll; ++u)
+        for (int u = 0; u < kUnroll; ++u)
             if (i + u * kThreads < n_vec) w[u] = *reinterpret_cast<const win_any*>(in + (i + u * kThreads) * kE);
 #pragma unroll
-        for (int u = 0; u < kDqUnroll; ++u) {
+        for (int u = 0; u < kUnroll; ++u) {
             if (i + u * kThreads >= n_vec) break;
             float v[kE];
 #pragma unroll
@@ -1142,9 +1143,14 @@ int run_dequant(const void* in, int fmt, const float* scale, int is_inverse, int
                 hipStream_t st) {
     clear_stale_error();
     const int64_t n_vec = aligned(out, 16) ? n / (out_dtype == NTFP8_F32 ? 4 : 8) : 0;
-    const int grid = grid_for(n_vec > 0 ? (n_vec + kDqUnroll - 1) / kDqUnroll : n, kThreads, 32);
+    const bool one = n_vec <= (int64_t)cu_count() * 8 * kThreads;
+    const int grid = grid_for(n_vec > 0 ? (one ? n_vec : (n_vec + 3) / 4) : n, kThreads, 32);
     const uint8_t* p = static_cast<const uint8_t*>(in);
-#define NT_DQ(F, O) hipLaunchKernelGGL((dequant_kernel<F, O>), dim3(grid), dim3(kThreads), 0, st, p, n_vec, n, scale, out, is_inverse)
+#define NT_DQ(F, O) \
+    do { \
+        if (one) hipLaunchKernelGGL((dequant_kernel<F, O, 1>), dim3(grid), dim3(kThreads), 0, st, p, n_vec, n, scale, out, is_inverse); \
+        else hipLaunchKernelGGL((dequant_kernel<F, O, 4>), dim3(grid), dim3(kThreads), 0, st, p, n_vec, n, scale, out, is_inverse); \
+    } while (0)
     if (fmt == kE4M3) {
         if (out_dtype == NTFP8_F32) NT_DQ(kE4M3, NTFP8_F32);
         else if (out_dtype == NTFP8_F16) NT_DQ(kE4M3, NTFP8_F16);

@@ -15,7 +15,7 @@ def test_sizes_and_alignments(fmt, odt):
 
     dev = torch.device("cuda", 0)
     scale = torch.tensor([2.0 ** 3])
-    cases = [(n, 0, 0) for n in (1, 3, 4, 7, 8, 9, 255, 2047, 2049, 8191, 8193, 256 * 32 * 8192 + 5)] + [(4099, 1, 0), (4099, 3, 1), (4099, 0, 2), (64, 5, 0)]
+    cases = [(n, 0, 0) for n in (1, 3, 4, 7, 8, 9, 255, 2047, 2049, 8191, 8193, 2 ** 21, 2 ** 21 + 5, 2 ** 22, 2 ** 22 + 9, 256 * 32 * 8192 + 5)] + [(4099, 1, 0), (4099, 3, 1), (4099, 0, 2), (64, 5, 0)]
     for n, i_shift, o_shift in cases:
         codes = (torch.arange(n + i_shift) * 37 % 256).to(torch.uint8)
         q = codes.to(dev)[i_shift:]
