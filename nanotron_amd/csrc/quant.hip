@@ -434,6 +434,10 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
                                                                    Workspace* ws, ScalarIO io) {
     typedef Src<S> L;
     typedef Tile<E> T;
+    // (16 fp32 values are four 16-byte loads of a lane that lie 64 bytes apart across the lanes: streaming lines do not stay
+    // for the other three.  Streaming / ordinary, us: delayed step of 2^22 to 2^23 elements 12.5 / 10.2, 2^24 to 2^25 44 / 29,
+    // 2^25 to 2^26 103 / 64)
+    constexpr bool kStream = kAmax && sizeof(*x) == 2;
     __shared__ __attribute__((aligned(16))) uint32_t tile[T::kT * T::kPitch];
     const float scale = *scale_ptr;
     const bool degen = degenerate_scale(scale);
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int64_t row = row0 + rgrp * 4 + r;
-                L::template load<E, kAmax>(x + (row < rows ? row : rows - 1) * cols + c, v[r], m[r]);
+                L::template load<E, kStream>(x + (row < rows ? row : rows - 1) * cols + c, v[r], m[r]);
             }
         } else {
 #pragma unroll
