@@ -80,7 +80,11 @@ static int path_of(const GemmDesc& g) {
 // bf16 output (plain / B transposed / both transposed), warm operands; what matters is where the lines cross.
 //   us, 256 / 128 / 64 wide:  1024 x 1024 x 1024  10.1 / 7.5 / 4.8     2048 x 1024 x 4096  26.5 / 16.3 / 15.3
 //   2048 x 2048 x 2048  16.7 / 11.8 / 16.9      both transposed  19.6 / 12.6 / 24.3
-//   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101      16 x 6144 x 4096  - / 13.8 / 8.3
+//   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101
+//   at equal estimates:   3696 x 1088 x 944 (bf16) 10.6 / - / 11.8     1072 x 3600 x 320 (fp8 output) 12.5 / - / 17.6,
+//                         528 x 2528 x 1008 with its weight gradient 19.5 / - / 14.8
+// Several problems: by their average depth.  (The end of the list as the CUs work it off, longest tile first, predicts
+// single launches no better and chose worse for one pair in twenty, up to 10.7 -> 18.1 us, though 4 % better on average.)
 static int64_t launch_cost(const GemmDesc* const* g, int n, int edge, int64_t cus) {
     int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
     int form = 0;
@@ -176,7 +180,8 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
         bool big = true;
         for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
         int64_t best = launch_cost(g, n, 128, cus);
-        for (const int e : {64, 256}) {
+        // (where the lines meet, the wider tiles for one problem, the narrower for several)
+        for (const int e : {n == 1 ? 256 : 64, n == 1 ? 64 : 256}) {
             if (e == 256 && !big) continue;
             const int64_t c = launch_cost(g, n, e, cus);
             if (c < best) best = c, edge = e;

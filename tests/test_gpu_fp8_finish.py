@@ -14,6 +14,7 @@ SHAPES = [
     (1124, 5120, 1024),                               # halves of 256-wide tiles, the last row of them empty
     (4096, 6144, 512),                                # whole tiles and a tail
     (1024, 2048, 144), (1056, 2048, 144),             # 512 tiles of 64 (one round, bookkeeping inside) and more
+    (1072, 3600, 320),                                # 256- and 64-wide tiles at equal estimates
     (1024, 4096, 240), (1040, 4112, 240),             # few K-tiles, both sides of the line to gemm_nt_kernel
     (1472, 1408, 77), (1500, 1500, 77),               # the same of tiles for any K (506 and 576)
     (64, 40, 77), (200, 300, 333),                    # K a multiple of nothing
