@@ -16,6 +16,7 @@
 //                         split over its waves.
 //   gemm_any_kernel       (gemm_any.h) any K and alignment: 64- or 128-wide tiles, fp8 widened to bf16 on its way to
 //                         the matrix cores.
+//   gemm_tiny_kernel      the smallest of those, one output per thread.
 //   gemm_nt_kernel        128 x 128 x 128 tiles, loads through registers: fp8 outputs whose rows or columns do not come in
 //                         whole words (the other kernels' fp8 epilogue stores nothing smaller), and large results of
 //                         fewer than two K-tiles.
@@ -32,6 +33,7 @@ int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int t
 int launch_few(const BigProblem& p, int fa, int fb, hipStream_t st);
 int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_plain(const GemmDesc& g, hipStream_t st);
+int launch_tiny(const BigProblem& p, int fa, int fb, hipStream_t st);
 int run_amax_finalize(Workspace* ws, const ScalarIO& io, hipStream_t st);
 
 // operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
@@ -240,6 +242,14 @@ static int launch_any_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     return L.fin_blocks ? rc : finish_behind(*g[0], rc, st);
 }
 
+// One problem of any K so small that a thread per output is done before a tile has been through LDS.  us, tiles / thread per
+// output: K 16 to 31, up to 2^16 outputs 5.5 / 4.3, to 2^17 5.8 / 5.1, beyond 6.0 / 6.5; K 32 to 63 5.6 / 6.0 on average, equal
+// at 40; fp8 outputs with their bookkeeping K 16 to 31 8.8 / 7.1.
+static bool tiny(const GemmDesc& g) {
+    const int64_t out = (int64_t)g.M * g.N;
+    return g.K < 40 && out <= 1 << 17 && out * g.K <= 40 << 16;
+}
+
 static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     const int fa = g[0]->fmt_a, fb = g[0]->fmt_b;
     if (path == kPathNone) return NTFP8_ERR_UNSUPPORTED;
@@ -249,6 +259,11 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
     if (fa != kE4M3 || fb != kE4M3 || path != kPathTiles || g[0]->tb || is_fp8_out(g[0]->d_dtype)) return NTFP8_ERR_UNSUPPORTED;
     return launch_tiles<kE4M3, kE4M3>(g, n, st);
 #else
+    if (path == kPathAny && n == 1 && tiny(*g[0])) {
+        BigLaunch L;
+        list_tiles(g, 1, 64, &L);
+        return finish_behind(*g[0], launch_tiny(L.p[0], fa, fb, st), st);
+    }
     if (path == kPathAny) return launch_any_tiles(g, n, st);
     if (path == kPathPlain || (n == 1 && short_k(*g[0]))) return finish_behind(*g[0], launch_plain(*g[0], st), st);
     if (n == 1 && few_rows(*g[0])) {

@@ -26,6 +26,54 @@ int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int t
 }
 
 // ---------------------------------------------------------------------------------------------
+// One output per thread, for the smallest products (gemm.hip has the line): bound by the latency of a launch, not by the
+// K loads of each thread, while a tile's trip through LDS and its code cost 2 us more.  128 x 62 x 22 6.6 -> 4.2 us.
+constexpr int kTinyThreads = 256;
+template <int FA, int FB>
+__global__ __launch_bounds__(kTinyThreads) void gemm_tiny_kernel(const BigProblem P) {
+    const int M = P.M, N = P.N, K = P.K;
+    const uint32_t idx = blockIdx.x * kTinyThreads + threadIdx.x;
+    const bool live = idx < (uint32_t)M * N;   // (whole waves stay: the amax reduction runs over all lanes)
+    const int m = live ? idx / N : 0, n = live ? idx % N : 0;
+    float acc = 0.0f;
+    for (int k = 0; live && k < K; ++k) {
+        const int a = P.A[(int64_t)m * K + k], b = P.B[(int64_t)n * K + k];
+        acc += (FA == kE4M3 ? __builtin_amdgcn_cvt_f32_fp8(a, 0) : __builtin_amdgcn_cvt_f32_bf8(a, 0)) *
+               (FB == kE4M3 ? __builtin_amdgcn_cvt_f32_fp8(b, 0) : __builtin_amdgcn_cvt_f32_bf8(b, 0));
+    }
+    float v = acc * descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);
+    if (P.ex.bias && live) v += bias_at(P.ex.bias, P.ex.bias_dtype, n);
+    if (P.d_dtype == NTFP8_OUT_E4M3 || P.d_dtype == NTFP8_OUT_E5M2) {   // uniform
+        uint32_t amax = 0;
+        const uint32_t w = P.d_dtype == NTFP8_OUT_E4M3 ? quant4<kE4M3>(v, 0.f, 0.f, 0.f, *P.fp8.scale, true, amax)
+                                                       : quant4<kE5M2>(v, 0.f, 0.f, 0.f, *P.fp8.scale, true, amax);
+        if (live) {
+            static_cast<uint8_t*>(P.D)[idx] = (uint8_t)w;
+            if (P.fp8.Dt) P.fp8.Dt[(int64_t)n * M + m] = (uint8_t)w;
+        }
+        publish_amax(live ? amax : 0u, P.fp8.ws);
+    } else if (live) {
+        if (P.d_dtype == NTFP8_BF16) static_cast<uint16_t*>(P.D)[idx] = OutT<NTFP8_BF16>::cvt(v);
+        else if (P.d_dtype == NTFP8_F16) static_cast<uint16_t*>(P.D)[idx] = OutT<NTFP8_F16>::cvt(v);
+        else if (P.accumulate) static_cast<float*>(P.D)[idx] += v;
+        else static_cast<float*>(P.D)[idx] = v;
+    }
+}
+
+int launch_tiny(const BigProblem& p, int fa, int fb, hipStream_t st) {
+    (void)hipGetLastError();
+    const dim3 grid((unsigned)(((int64_t)p.M * p.N + kTinyThreads - 1) / kTinyThreads)), block(kTinyThreads);
+    if (fa == kE4M3) {
+        if (fb == kE4M3) hipLaunchKernelGGL((gemm_tiny_kernel<kE4M3, kE4M3>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((gemm_tiny_kernel<kE4M3, kE5M2>), grid, block, 0, st, p);
+    } else {
+        if (fb == kE4M3) hipLaunchKernelGGL((gemm_tiny_kernel<kE5M2, kE4M3>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((gemm_tiny_kernel<kE5M2, kE5M2>), grid, block, 0, st, p);
+    }
+    return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+}
+
+// ---------------------------------------------------------------------------------------------
 // 128 x 128 x 128, 4 waves (2 x 2, each 64 x 64), loads staged through registers.  Bound by HBM on the shapes it serves
 // (mostly output): its prologues and epilogues overlap in the three workgroups that a CU holds (168 registers: two more and it is two).
 constexpr int kBM = 128, kBN = 128;

@@ -62,3 +62,13 @@ def test_edges_of_the_tile(M, N, acc):
 @pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
 def test_views_that_start_anywhere(shift, d_shift, K, N, odt):
     _run(130, N, K, O.E4M3, O.E4M3, shift=shift, d_shift=d_shift, odt=odt, seed=shift)
+
+
+# (M, N, K) around the lines between one output per thread and tiles: K below 40, 2^17 outputs, 40 * 2^16 products
+@pytest.mark.parametrize("mnk", [(1, 1, 1), (255, 1, 17), (3, 86, 39), (3, 86, 41), (362, 362, 19), (363, 362, 19), (257, 255, 39), (259, 263, 39)])
+@pytest.mark.parametrize("fa,fb", [(O.E4M3, O.E4M3), (O.E5M2, O.E4M3), (O.E4M3, O.E5M2), (O.E5M2, O.E5M2)])
+def test_one_output_per_thread(mnk, fa, fb):
+    _run(*mnk, fa, fb, seed=mnk[0])
+    _run(*mnk, fa, fb, acc=True, seed=mnk[1])
+    _run(*mnk, fa, fb, odt=torch.bfloat16, d_shift=1, seed=mnk[2])
+    _run(*mnk, fa, fb, odt=torch.bfloat16, shift=1, seed=mnk[2])
