@@ -105,8 +105,11 @@ __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0
 // (nt).  An ordinary store leaves its line dirty in the XCD's L2; a tile's worth of output per CU then fills that L2,
 // and the lines are written back in one burst when the kernel ends.  Written through, the output drains while the
 // other waves still compute: 2.5 us less per round of tiles (4096^3: 58.0 -> 55.5 us; `nt` alone changes nothing).
+// The two wait states belong to the store: its data registers are still being read then, and the compiler, which keeps such
+// a distance behind stores of its own, does not see this one (without them the next block's first product overwrote a word
+// of four lanes now and then).
 __device__ __forceinline__ void store16_through(void* p, v4i v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" ::"v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // Epilogue of one wave: MI x NJ accumulator blocks of 16 x 16, block (i, j) at rows m_base + 16 i,
