@@ -603,7 +603,7 @@ __global__ __launch_bounds__(kFlatThreads) void quant_once_kernel(const typename
         const int g = t + i * kFlatThreads;
         if (g >= n_vec) break;
         const u4 q = encode16<F>(v[i], scale, degen || L::has_nan(m[i]));
-        if (out) *reinterpret_cast<u4*>(out + g * kVec) = q;
+        *reinterpret_cast<u4*>(out + g * kVec) = q;
         if constexpr (kT) {   // (cols is a multiple of 16: a group lies in one row)
             const int r = g * kVec / cols, c = g * kVec % cols;
             uint32_t* p = tile + r * pitch + c / 4;
