@@ -109,8 +109,8 @@ int ntfp8_quantize_current(const void* x, int x_dtype, int64_t rows, int64_t col
  *   *initialised == 0:  the result of ntfp8_quantize_current with the history arguments (the reference's scaling,
  *                       src/nanotron/fp8/tensor.py:25-28: the scale comes from this tensor's own amax);
  *   *initialised != 0:  the result of ntfp8_quantize_delayed, bit for bit (cast with *scale_state, history rolled,
- *                       next scale stored), from two launches instead of one (amax pass, then cast: 5 bytes per 16-bit
- *                       element instead of 3);
+ *                       next scale stored), from an amax pass and a cast (5 bytes per 16-bit element instead of 3), one
+ *                       launch up to 65536 elements and two beyond;
  * and *initialised becomes 1.0 if this tensor's amax is finite and positive.  A caller that knows the role holds a scale
  * calls ntfp8_quantize_delayed. */
 int ntfp8_quantize_first_use(const void* x, int x_dtype, int64_t rows, int64_t cols, int fmt, int margin, float* scale_state,

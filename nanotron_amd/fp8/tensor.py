@@ -160,7 +160,7 @@ def _quantize(cls, tensor: torch.Tensor, dtype: DTypes, state: Optional[DelayedS
         if state.known_initialised:
             parts = nt.host.quantize(tensor, fmt, state.margin, buf, None, state.history_len, with_transpose)
         else:
-            # two launches that decide on the device: current scaling while the role holds no scale, the held scale once
+            # decided on the device (one launch for small tensors, two otherwise): current scaling while the role holds no scale, the held scale once
             # it does (then with the results of the fused pass, bit for bit)
             parts = nt.host.quantize(tensor, fmt, state.margin, buf, state._flag, state.history_len, with_transpose)
             state._watch_flag()

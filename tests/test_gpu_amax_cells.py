@@ -1,5 +1,5 @@
 """GPU parity of the maximum that the workgroups of a quantise launch put together: one word per workgroup up to 512 of them
-(one, two, the last one short, exactly 512), tickets beyond; the largest element in the first, a middle and the last
+(one, two, the last one short, exactly 512), which work through more tiles than that beyond; the largest element in the first, a middle and the last
 workgroup; maxima that shrink from call to call, so that a word left behind by an earlier launch would show.  Exact."""
 import pytest
 import torch
@@ -9,7 +9,7 @@ from oracle import fp8_oracle as O
 pytestmark = pytest.mark.gpu
 
 FLAT = [(1, 7), (1, 32768), (1, 32769), (1, 98304), (2048, 4096)]   # 1, 1, 2, 3 and 256 workgroups of 32768 elements
-# 64-wide tiles: 1, 511, 512 and 520 of them; 128-wide ones: 512 and 768 workgroups
+# one element per thread; 64-wide tiles: 511, 512 and 520 of them; 128-wide ones: 512 and 768 (in 512 workgroups)
 TILES = [(64, 64), (4672, 448), (4096, 512), (4160, 512), (4096, 2048), (4096, 3072)]
 
 

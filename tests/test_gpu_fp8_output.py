@@ -82,7 +82,7 @@ def _check_against_two_step(A, B, fo, st, with_transpose=True):
 
 
 # shapes: big kernel whole tiles + half-tile tail, big kernel ragged edges, small kernel, small kernel ragged
-# (N not a multiple of 16 / M not of 4), naive kernel (K not a multiple of 16)
+# (N not a multiple of 16 / M not of 4), kernels of any K (K not a multiple of 16)
 SHAPES = [(512, 768, 256), (2304, 2048, 384), (260, 400, 512), (1000, 144, 272), (128, 128, 128), (64, 48, 32),
           (130, 250, 272), (131, 200, 256), (33, 17, 96), (5, 3, 7), (1, 1, 1), (200, 36, 1040)]
 
@@ -136,7 +136,7 @@ def test_random_operands_equal_cast_of_the_fp32_result(fa, fb, fo, mnk):
     assert O.rel_l2(deq, r_ref) <= (0.04 if fo == O.E4M3 else 0.08)
 
 
-@pytest.mark.parametrize("mnk", [(512, 768, 256), (96, 80, 128), (33, 17, 100)])   # big, small, naive kernel
+@pytest.mark.parametrize("mnk", [(512, 768, 256), (96, 80, 128), (33, 17, 100)])   # big, small, any K
 @pytest.mark.parametrize("fo", FMTS)
 def test_nan_inf_and_degenerate_scales(mnk, fo):
     M, N, K = mnk

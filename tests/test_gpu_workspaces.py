@@ -1,5 +1,5 @@
 """The reduction workspaces that Python hands out are the ones that the native host calls use, and every kind of launch
-leaves them zero: words and tickets of quantise launches, tickets of column sums, maxima of fp8-output GEMMs."""
+leaves them zero: words of quantise launches, tickets of column sums, maxima and tickets of fp8-output GEMMs."""
 import pytest
 import torch
 
