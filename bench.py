@@ -756,9 +756,8 @@ def _stamp_report(lib, n, k_tiles):
 
 
 def loop_experiments(device, reps=3, launches=24):
-    """What the K loop of a whole tile pays for, piece by piece, under sustained load: the experiment builds of the
-    profiling library (nanotron_amd/build.py: EXPERIMENTS; parts of the loop left out, or idle cycles put in) run the
-    one-round forward GEMMs of the O projection (K = 4096) and of the down projection (K = 14336) `launches` times
+    """The K loop of a whole tile under sustained load: the narrow builds of the profiling library
+    (nanotron_amd/build.py: EXPERIMENTS) and the vendor library's kernel run the one-round forward GEMMs of the O projection (K = 4096) and of the down projection (K = 14336) `launches` times
     back to back on rotating operand sets, alternating between the builds.  Per build: microseconds per launch (HIP
     events, best of `reps`), and from the stamps of the last launch the cycles per K-tile and the shader clock."""
     import torch

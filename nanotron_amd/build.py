@@ -10,8 +10,8 @@ nanotron_amd/_hostcall.so is a CPython extension on top of libntfp8.so: the host
 
 Profiling libraries (nanotron_amd/profiling/, loaded by nothing but the benchmark's wg-timeline workload):
 libntfp8_stamps.so is the product library with per-workgroup time stamps compiled into the GEMM kernel
-(-DNTFP8_STAMPS); the libntfp8_<experiment>.so beside it carry the same stamps and one timing experiment each on the
-K loop of the forward GEMM (parts of the loop left out, or idle cycles put in; their results are wrong by design).
+(-DNTFP8_STAMPS); the libntfp8_<name>.so beside it carry the same stamps and, for a quick build, only the instantiation
+that the forward GEMM launches.
 """
 from __future__ import annotations
 
@@ -34,21 +34,8 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
-# name -> extra defines of gemm.hip: what the K loop of a whole tile costs, piece by piece (NTFP8_KNOCKOUT bits: 1 global
-# loads, 2 deposits into LDS, 4 barrier, 8 B-fragment reads, 16 A-fragment reads), and what idle cycles cost
-EXPERIMENTS = {
-    "base": [],
-    "no_loads": ["-DNTFP8_KNOCKOUT=1"],
-    "no_loads_no_deposits": ["-DNTFP8_KNOCKOUT=3"],
-    "no_barrier": ["-DNTFP8_KNOCKOUT=4"],
-    "no_lds_reads": ["-DNTFP8_KNOCKOUT=24"],
-    "mfma_only": ["-DNTFP8_KNOCKOUT=31"],
-    "idle_256": ["-DNTFP8_IDLE=4"],
-    "idle_512": ["-DNTFP8_IDLE=8"],
-    "mfma_only_32x32x64": ["-DNTFP8_KNOCKOUT=31", "-DNTFP8_MFMA32=1"],
-    "columns_224": ["-DNTFP8_COLUMNS=7"],
-    "columns_192": ["-DNTFP8_COLUMNS=6"],
-}
+# name -> extra defines of gemm.hip
+EXPERIMENTS = {"base": []}
 
 
 def experiment_lib(name: str) -> str:

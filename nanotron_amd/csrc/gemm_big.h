@@ -35,43 +35,14 @@ namespace ntfp8 {
 constexpr int kStampSlots = 16384;
 __device__ unsigned long long g_stamps[kStampSlots * 8];
 // 1: workgroups take the tiles in launch order, i.e. every XCD gets every eighth tile and touches all operand panels
-// (an experiment on what the fetch traffic costs; set with ntfp8_debug_set_tile_order)
+// (what the fetch traffic costs; set with ntfp8_debug_set_tile_order)
 __device__ int g_plain_tile_order = 0;
 #define NTFP8_STAMP(var) var = wall_clock64()
 #define NTFP8_CYCLES(var) var = __builtin_readcyclecounter()
-// Timing experiments on the K loop of whole tiles, chosen when a profiling build is compiled (the results of such a
-// build are wrong, only its stamps mean something).  -DNTFP8_KNOCKOUT=<bits> leaves parts of the loop out: 1 the global
-// loads (the registers of the first K-tile are deposited again and again), 2 the deposits into LDS, 4 the workgroup barrier, 8 the LDS reads of the B
-// fragments, 16 those of the A fragments.  -DNTFP8_IDLE=<n> lets every wave sleep 64 n cycles behind the barrier of
-// every K-tile.  -DNTFP8_COLUMNS=<6 | 7> runs the K loop of a tile that is 192 or 224 columns wide instead of 256 (that
-// many of a wave's eight block columns, B loads and B fragments; the schedule is the same with the last front groups
-// left out): what a tile width that divides N = 6144 or 14336 into a whole number of rounds would cost per K-tile.
-// -DNTFP8_MFMA32=1 (with -DNTFP8_KNOCKOUT=31) issues 32 V_MFMA_F32_32X32X64_F8F6F4 per K-tile in place of the 64
-// 16x16x128 ones (the same FLOPs and matrix-pipe cycles, half the operand registers read per FLOP, twice the accumulator
-// registers touched): what the other instruction shape draws.
-#ifndef NTFP8_KNOCKOUT
-#define NTFP8_KNOCKOUT 0
-#endif
-#ifndef NTFP8_IDLE
-#define NTFP8_IDLE 0
-#endif
-#ifndef NTFP8_COLUMNS
-#define NTFP8_COLUMNS 8
-#endif
-#ifndef NTFP8_MFMA32
-#define NTFP8_MFMA32 0
-#endif
-constexpr int kKnockout = NTFP8_KNOCKOUT, kIdle = NTFP8_IDLE, kColumns = NTFP8_COLUMNS;
-constexpr bool kMfma32 = NTFP8_MFMA32 != 0;
 #else
 #define NTFP8_STAMP(var) (void)0
 #define NTFP8_CYCLES(var) (void)0
-constexpr int kKnockout = 0, kIdle = 0, kColumns = 8;
-constexpr bool kMfma32 = false;
 #endif
-constexpr bool kNoLoads = kKnockout & 1, kNoDeposits = kKnockout & 2, kNoBarrier = kKnockout & 4, kNoBReads = kKnockout & 8,
-               kNoAReads = kKnockout & 16;
-
 
 constexpr int kBigN = 256;
 constexpr int kBigWaves = 4, kBigThreads = kBigWaves * 64;
@@ -416,10 +387,9 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     const float alpha = descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);
 
     constexpr int LA = MI * 2 * 16 / 8 / kBigWaves;  // wave-level loads of the A tile per wave per stage
-    constexpr int NJe = MI == 8 ? kColumns : kBigNJ;   // block columns the K loop computes (8 outside experiments)
-    constexpr int LB = MI == 8 ? kBigLB - (kBigNJ - NJe) : kBigLB;
+    constexpr int LB = kBigLB;
     constexpr int NL = LA + LB;                      // loads per wave per K-tile
-    static_assert(NL % 4 == 0 || NJe != kBigNJ, "the loads are queued in four equal portions");
+    static_assert(NL % 4 == 0, "the loads are queued in four equal portions");
     const int wm = (wave >> 1) * (MI * 16), wn = (wave & 1) * 128;
 
     v4f acc[MI][kBigNJ];
@@ -427,28 +397,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < kBigNJ; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
-    // (experiment builds only: the accumulators of the 32 x 32 instruction shape)
-    [[maybe_unused]] v16f big[kMfma32 ? MI / 2 : 1][kMfma32 ? kBigNJ / 2 : 1];
-    if constexpr (kMfma32) {
-#pragma unroll
-        for (int i = 0; i < MI / 2; ++i)
-#pragma unroll
-            for (int j = 0; j < kBigNJ / 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) big[i][j][e] = 0.f;
-    }
-    // one step of the MFMA loop: block (i, j) of the wave tile; in the 32 x 32 experiment every fourth step issues the
-    // two instructions (K = 2 x 64) of the 32 x 32 block it belongs to, on whatever fragments are at hand
-    auto mma = [&](int i, int j, const v8i b, const v8i a) {
-        if constexpr (kMfma32) {
-            if (!(i & 1) && !(j & 1)) {
-                big[i >> 1][j >> 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b, a, big[i >> 1][j >> 1], FB, FA, 0, 0, 0, 0);
-                big[i >> 1][j >> 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, big[i >> 1][j >> 1], FB, FA, 0, 0, 0, 0);
-            }
-        } else {
-            acc[i][j] = mfma_16x16x128<FA, FB>(b, a, acc[i][j]);
-        }
-    };
+    auto mma = [&](int i, int j, const v8i b, const v8i a) { acc[i][j] = mfma_16x16x128<FA, FB>(b, a, acc[i][j]); };
 
     // The K loop.  kAT: the A operand is given as its transpose, a [K, M] tensor (what wgrad has of dY: its reduction
     // index, the token, is the row index).  Its K-tiles lie in LDS as they lie in memory, 128 rows of k with 256 (whole
@@ -624,21 +573,21 @@ void gemm_nt_big_kernel(const BigLaunch L) {
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
                 // fa[i] is dead after its two MFMAs; it is refilled with the fragment of the next tile one step later
-                mma(i, NJe - 2, frag(fb[(NJe - 2) & 3]), frag(fa[i]));
-                if (prefetch && !kNoAReads && i > 0) {
+                mma(i, kBigNJ - 2, frag(fb[(kBigNJ - 2) & 3]), frag(fa[i]));
+                if (prefetch && i > 0) {
                     fa[i - 1][0] = rd_a(s1, i - 1, 0);
                     fa[i - 1][1] = rd_a(s1, i - 1, 1);
                 }
                 sched_fence();
-                mma(i, NJe - 1, frag(fb[(NJe - 1) & 3]), frag(fa[i]));
+                mma(i, kBigNJ - 1, frag(fb[(kBigNJ - 1) & 3]), frag(fa[i]));
                 if constexpr (loads) {   // loads [i kBackLoads / MI, (i + 1) kBackLoads / MI) ride on this step
 #pragma unroll
                     for (int l = i * kBackLoads / MI; l < (i + 1) * kBackLoads / MI; ++l) issue(kt + NS, l);
                 }
-                if (prefetch && !kNoBReads && i < 4) fb[i >> 1][i & 1] = rd_b(s1, i >> 1, i & 1);
+                if (prefetch && i < 4) fb[i >> 1][i & 1] = rd_b(s1, i >> 1, i & 1);
                 sched_fence();
             }
-            if constexpr (prefetch && !kNoAReads) {
+            if constexpr (prefetch) {
                 fa[MI - 1][0] = rd_a(s1, MI - 1, 0);
                 fa[MI - 1][1] = rd_a(s1, MI - 1, 1);
             }
@@ -657,20 +606,10 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             // than from the memory-side cache stalled the barrier.
             v4i g[NL];
             const int wr_lane = wave * 1024 + lane * 16;   // a wave-level load covers 1 KB of a stage: 16 bytes per lane
-            auto load_now = [&](int ktile, int l) {
+            auto request = [&](int ktile, int l) {
                 g[l] = l < LA ? reg_load16(ra, a_off[l], ktile * a_step) : reg_load16(rb, b_off[l - LA], ktile * b_step);
             };
-            if constexpr (kNoLoads) {
-                // one real K-tile, deposited again and again: operand bytes of the real distribution (what the matrix
-                // cores draw depends on the data: zeros would make this build look far cheaper than it is)
-#pragma unroll
-                for (int l = 0; l < NL; ++l) load_now(0, l);
-            }
-            auto request = [&](int ktile, int l) {
-                if constexpr (!kNoLoads) load_now(ktile, l);
-            };
             auto deposit = [&](int s, int l) {
-                if constexpr (kNoDeposits) return;
                 if (l < LA) *reinterpret_cast<v4i*>(&sA[s][wr_lane + l * (kBigWaves * 1024)]) = g[l];
                 else *reinterpret_cast<v4i*>(&sB[s][wr_lane + (l - LA) * (kBigWaves * 1024)]) = g[l];
             };
@@ -683,12 +622,12 @@ void gemm_nt_big_kernel(const BigLaunch L) {
                 sched_fence();
                 int l = 0;
 #pragma unroll
-                for (int j = 0; j < NJe - 2; ++j) {
+                for (int j = 0; j < kBigNJ - 2; ++j) {
 #pragma unroll
                     for (int i = 0; i < MI; ++i) {
                         mma(i, j, frag(fb[j & 3]), frag(fa[i]));
-                        if (i == 0) { if constexpr (!kNoBReads) fb[(j + 2) & 3][0] = rd_b(s, j + 2, 0); }
-                        else if (i == 2) { if constexpr (!kNoBReads) fb[(j + 2) & 3][1] = rd_b(s, j + 2, 1); }
+                        if (i == 0) fb[(j + 2) & 3][0] = rd_b(s, j + 2, 0);
+                        else if (i == 2) fb[(j + 2) & 3][1] = rd_b(s, j + 2, 1);
                         else if (l < NL) {
                             const bool second = i == 3 || i == 5 || i == 7;   // slots 1,3 / 4,5 / 6,7 form the pairs
                             if (!second) { if (W) deposit(s ^ 1, l); }
@@ -704,8 +643,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
                     // the first front publishes tile 1, which the prologue sent straight to LDS: its loads are
                     // older than the NL requests of tile 2 queued above
                     if constexpr (!W) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L ? NL : 0) : "memory");
-                    if constexpr (!kNoBarrier) wg_barrier();
-                    if constexpr (kIdle > 0) __builtin_amdgcn_s_sleep(kIdle);
+                    wg_barrier();
                 }
             };
             // prologue: tiles 0 and 1 straight into LDS
@@ -810,14 +748,6 @@ void gemm_nt_big_kernel(const BigLaunch L) {
 
     NTFP8_STAMP(st_loop);
     NTFP8_CYCLES(cy_loop);
-    if constexpr (kMfma32) {   // the experiment's results must reach memory, or its MFMAs are dead code
-#pragma unroll
-        for (int i = 0; i < MI / 2; ++i)
-#pragma unroll
-            for (int j = 0; j < kBigNJ / 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[2 * i + (e >> 3)][2 * j + ((e >> 2) & 1)][e & 3] += big[i][j][e];
-    }
     {
         // output type, accumulation and bias are properties of the problem, not of the kernel (fp8 outputs apart)
         auto epilogue = [&](auto bias_tag, const float (*bv)[4]) {
