@@ -9,15 +9,18 @@
 // registers, and streams its 8 B fragments from LDS two MFMA groups ahead of their use.  One MFMA
 // group = the MI MFMAs that share one B fragment.
 //
-// Pipeline, two LDS stages, ONE workgroup barrier per K-tile placed after MFMA group 5:
-//   * before the barrier a wave has read every fragment of the current tile into registers, so the
-//     barrier releases the current stage for tile kt + 2 and publishes tile kt + 1 at once;
-//   * groups 6 and 7 are issued interleaved, two MFMAs per A fragment; the fragment register is dead
-//     after them and is refilled with the same fragment of tile kt + 1, so one set of A registers
-//     suffices.
-// Global loads: whole tiles (MI = 8) keep one K-tile in flight in registers and write it to LDS a
-// K-tile later, so that every load has a full K-tile of MFMA time to arrive; half tiles (MI = 4) have
-// no registers to spare and load straight into the released LDS stage.
+// Loads go straight from memory into LDS.  Whole tiles (MI = 8): two LDS stages and two workgroup barriers per K-tile.
+//   * all B fragments of a tile have registers of their own and are read during its first 24 MFMAs; the first barrier
+//     (behind MFMA 26 of 64) so releases the stage early, and the loads of tile kt + 2 have the rest of this K-tile and most
+//     of the next to arrive;
+//   * the second barrier (behind group 5) publishes tile kt + 1, whose A fragments are read during groups 6 and 7: these
+//     are issued interleaved, two MFMAs per A fragment, and the fragment register, dead after them, is refilled with the
+//     same fragment of tile kt + 1, so one set of A registers suffices.
+// Bound by the package power limit and by issue slots: 191 instructions per K-tile of 64 MFMAs became 161, and no operand
+// byte passes through a register on its way to LDS.  us, loads kept in registers for a K-tile / straight into LDS:
+// 4096 x 4096 x 4096 50.6 / 48.5, 4096 x 14336 x 4096 179 / 173, 4096 x 4096 x 14336 165 / 160; both operands transposed
+// beside dgrad, 4096 tokens: 4096 -> 4096 110 / 104, 4096 -> 14336 384 / 362, 14336 -> 4096 387 / 372.
+// Half tiles (MI = 4): three stages, one barrier behind group 5 that releases the stage of tile kt and publishes tile kt + 1.
 //
 // Instantiations beside the operand formats and MI: kFp8Out (the outputs are fp8 bytes, cast in the
 // epilogue, with an optional transposed copy and the amax of the results) and kBT (the B operands are
@@ -320,8 +323,7 @@ __device__ __forceinline__ void finish_fp8(const BigLaunch& L, Workspace* ws, ui
 template <int FA, int FB, int MI, bool kFp8Out = false, bool kBT = false>
 __global__ __launch_bounds__(MI == 8 ? kBigThreads : 2 * kBigThreads)
 void gemm_nt_big_kernel(const BigLaunch L) {
-    // whole tiles: 2 stages of 64 KB; half tiles: 3 stages of 48 KB (their loads go straight to LDS and need the
-    // extra stage to have two K-tiles of flight time, see below)
+    // whole tiles: 2 stages of 64 KB; half tiles: 3 stages of 48 KB (their K-tiles are half as long)
     constexpr int NS = MI == 8 ? 2 : 3;
     __shared__ __attribute__((aligned(1024))) uint8_t sA[NS][32 * MI * kBK];
     __shared__ __attribute__((aligned(1024))) uint8_t sB[NS][kBigN * kBK];
@@ -517,22 +519,131 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         };
         auto frag = [](const v4i (&x)[2]) -> v8i { return (v8i){x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w}; };
 
-        v4i fa[MI][2], fb[4][2];
+        v4i fa[MI][2];
 
-        // A K-tile kt lives in LDS stage kt mod NS and is computed in two parts:
-        //   front(kt): MFMA groups 0-5.  Entered with fa[] = the tile's A fragments and fb[0], fb[1] = its first
-        //              two B fragments; streams B fragments 2..7; ends with the barrier that publishes tile
-        //              kt + 1 and releases the stage of tile kt.
-        //   back(kt):  MFMA groups 6-7, interleaved per A fragment; refills fa[] / fb[0], fb[1] from tile kt + 1.
-        // The K loop runs back(kt); front(kt + 1), so that its back edge sits right behind the barrier, where no
-        // LDS read is outstanding.  With direct-to-LDS loads (half tiles) the stage released by the barrier of
-        // tile kt is refilled with tile kt + NS between that barrier and the next: half of the loads under
-        // back(kt), the rest under groups 0-1 of front(kt + 1).
+        // A K-tile kt lives in LDS stage kt mod NS and is computed in two parts, front(kt) = MFMA groups 0-5 and back(kt) =
+        // groups 6-7.  The K loop runs back(kt); front(kt + 1), so that its back edge sits right behind the barrier at
+        // the end of front(), where no LDS read is outstanding.
         //
         // An MFMA occupies the matrix pipe for 32 cycles and the wave issues in order, so whatever stands between
         // two MFMAs must issue within that time or the pipe idles.  The code below therefore puts at most one
         // memory instruction (two LDS reads at most) behind each MFMA, and a scheduling fence behind each such
         // pair keeps the compiler from regrouping them.
+        using Yes = std::true_type;
+        using No = std::false_type;
+
+        if constexpr (MI == 8) {
+            // ---- whole tiles ---------------------------------------------------------------------------
+            // Two stages.  front(f), MFMA groups 0-5 of tile f, in slots of one MFMA each (8 per group): the B
+            // fragments 2-7 are read behind every other one of the first 24, a barrier then releases the stage, and the
+            // loads of tile f + 2 go into it, one behind every third MFMA up to the end of back(f): spread out, because
+            // sixteen in a row cost more than they gain (us, 4096 x 4096 x 4096 and x 14336: behind every MFMA 51.3 and
+            // 184, every second 48.8 and 162, every third 48.5 and 160, every fourth 49.5 and 165; through registers,
+            // deposited in LDS a K-tile later, 50.6 and 165).  The barrier at the end of front(f) publishes tile f + 1,
+            // whose loads have had at least 48 MFMAs of time.
+            constexpr int kRelease = 25;              // slot of the first barrier
+            constexpr int kEvery = 3;                 // slots from load to load
+            constexpr int kFront = (MI * 6 - 1 - kRelease) / kEvery;   // loads in front(), the others in back()
+            v4i fw[kBigNJ][2];   // all B fragments of a tile
+            auto front_w = [&](auto l_tag, auto b_tag, int f) {
+                constexpr bool L = decltype(l_tag)::value, B = decltype(b_tag)::value;   // L: there is a tile f + 2; B: f + 1
+                const int s = f & 1;
+                sched_fence();
+#pragma unroll
+                for (int x = 0; x < MI * 6; ++x) {
+                    const int j = x / MI, i = x % MI;
+                    mma(i, j, frag(fw[j]), frag(fa[i]));
+                    if (x < 24 && x % 2 == 0) fw[2 + x / 4][x / 2 % 2] = rd_b(s, 2 + x / 4, x / 2 % 2);
+                    if constexpr (L) {
+                        if (x == kRelease) {
+                            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every fragment of tile f is in registers
+                            wg_barrier();
+                        }
+                        if (x > kRelease && (x - kRelease) % kEvery == 0) issue(f + 2, (x - kRelease) / kEvery - 1);
+                    }
+                    sched_fence();
+                }
+                if constexpr (B) {
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L ? kFront : 0) : "memory");   // all but tile f + 2's
+                    wg_barrier();
+                }
+            };
+            // groups 6 and 7, interleaved per A fragment, which is dead after them and refilled from tile f + 1
+            auto back_w = [&](auto l_tag, auto prefetch_tag, int f) {
+                constexpr bool L = decltype(l_tag)::value, prefetch = decltype(prefetch_tag)::value;
+                const int s1 = (f + 1) & 1;
+                sched_fence();
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    mma(i, 6, frag(fw[6]), frag(fa[i]));
+                    if (prefetch && i > 0) {
+                        fa[i - 1][0] = rd_a(s1, i - 1, 0);
+                        fa[i - 1][1] = rd_a(s1, i - 1, 1);
+                    }
+                    sched_fence();
+                    mma(i, 7, frag(fw[7]), frag(fa[i]));
+                    if (prefetch && i < 4) fw[i >> 1][i & 1] = rd_b(s1, i >> 1, i & 1);
+                    if constexpr (L) {
+#pragma unroll
+                        for (int l = kFront + i * (NL - kFront) / MI; l < kFront + (i + 1) * (NL - kFront) / MI; ++l) issue(f + 2, l);
+                    }
+                    sched_fence();
+                }
+                if constexpr (prefetch) {
+                    fa[MI - 1][0] = rd_a(s1, MI - 1, 0);
+                    fa[MI - 1][1] = rd_a(s1, MI - 1, 1);
+                }
+                sched_fence();
+            };
+            // prologue: tiles 0 and 1
+#pragma unroll
+            for (int l = 0; l < NL; ++l) issue(0, l);
+            if (KT == 2) poison_tail();
+#pragma unroll
+            for (int l = 0; l < NL; ++l) issue(1, l);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");   // tile 0 has landed, tile 1 may still be in flight
+            wg_barrier();
+            NTFP8_STAMP(st_first);
+            NTFP8_CYCLES(cy_first);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                fa[i][0] = rd_a(0, i, 0);
+                fa[i][1] = rd_a(0, i, 1);
+            }
+#pragma unroll
+            for (int h = 0; h < 4; ++h) fw[h >> 1][h & 1] = rd_b(0, h >> 1, h & 1);
+
+            // (poison_tail() runs between the loads of tile KT - 2 and those of tile KT - 1 = f + 2)
+            if (KT == 3) poison_tail();
+            if (KT > 2) front_w(Yes{}, Yes{}, 0);
+            else front_w(No{}, Yes{}, 0);
+            int f = 1;
+            for (; f + 3 < KT; ++f) {
+                back_w(Yes{}, Yes{}, f - 1);
+                front_w(Yes{}, Yes{}, f);
+            }
+            if (f + 2 < KT) {   // f = KT - 3 >= 1
+                back_w(Yes{}, Yes{}, f - 1);
+                poison_tail();
+                front_w(Yes{}, Yes{}, f);
+                ++f;
+            }
+            if (f + 1 < KT) {   // f = KT - 2 >= 1: back(f - 1) sends the rest of the last tile
+                back_w(Yes{}, Yes{}, f - 1);
+                front_w(No{}, Yes{}, f);
+                ++f;
+            }
+            back_w(No{}, Yes{}, f - 1);   // f = KT - 1
+            front_w(No{}, No{}, f);
+            back_w(No{}, No{}, f);
+        } else {
+        // ---- half tiles ------------------------------------------------------------------------------
+        //   front(kt): entered with fa[] = the tile's A fragments and fb[0], fb[1] = its first two B fragments; streams B
+        //              fragments 2..7; ends with the barrier that publishes tile kt + 1 and releases the stage of tile kt.
+        //   back(kt):  refills fa[] / fb[0], fb[1] from tile kt + 1.
+        // The stage released by the barrier of tile kt is refilled with tile kt + NS between that barrier and the next:
+        // half of the loads under back(kt), the rest under groups 0-1 of front(kt + 1).
+        v4i fb[4][2];
         constexpr int kBackLoads = NL / 2;
         constexpr int kFrontLoads = NL - kBackLoads;   // half under group 0, half under group 1
         // loads: queue the second half of tile kt + NS - 1; WAIT (>= 0): barrier, after all but the newest WAIT
@@ -593,102 +704,6 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             }
             sched_fence();
         };
-        using Yes = std::true_type;
-        using No = std::false_type;
-
-        if constexpr (MI == 8) {
-            // ---- whole tiles: loads staged through registers ------------------------------------------
-            // g[] always holds one K-tile in flight.  front(f) runs between the barriers B(f-1) and B(f); there
-            // g[l] (tile f + 1, requested one K-tile earlier) is written to the stage released by B(f-1) and
-            // at once re-requested for tile f + 2.  Every load so has a full K-tile of MFMA time to arrive
-            // whatever its position, and the requests are spread evenly over the K-tile; with direct-to-LDS
-            // loads (which can only be issued once their stage is free) operands that come from HBM rather
-            // than from the memory-side cache stalled the barrier.
-            v4i g[NL];
-            const int wr_lane = wave * 1024 + lane * 16;   // a wave-level load covers 1 KB of a stage: 16 bytes per lane
-            auto request = [&](int ktile, int l) {
-                g[l] = l < LA ? reg_load16(ra, a_off[l], ktile * a_step) : reg_load16(rb, b_off[l - LA], ktile * b_step);
-            };
-            auto deposit = [&](int s, int l) {
-                if (l < LA) *reinterpret_cast<v4i*>(&sA[s][wr_lane + l * (kBigWaves * 1024)]) = g[l];
-                else *reinterpret_cast<v4i*>(&sB[s][wr_lane + (l - LA) * (kBigWaves * 1024)]) = g[l];
-            };
-            // MFMA groups 0-5 of tile f.  W: deposit tile f + 1; L: request tile f + 2; B: barrier that publishes
-            // tile f + 1.  A group has 8 MFMA slots: two carry the LDS reads of B fragment j + 2, the other six
-            // take deposit / request pairs (three pairs in groups 0-4, the sixteenth pair in group 5).
-            auto front_st = [&](auto w_tag, auto l_tag, auto b_tag, int f) {
-                constexpr bool W = decltype(w_tag)::value, L = decltype(l_tag)::value, B = decltype(b_tag)::value;
-                const int s = f & 1;
-                sched_fence();
-                int l = 0;
-#pragma unroll
-                for (int j = 0; j < kBigNJ - 2; ++j) {
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) {
-                        mma(i, j, frag(fb[j & 3]), frag(fa[i]));
-                        if (i == 0) fb[(j + 2) & 3][0] = rd_b(s, j + 2, 0);
-                        else if (i == 2) fb[(j + 2) & 3][1] = rd_b(s, j + 2, 1);
-                        else if (l < NL) {
-                            const bool second = i == 3 || i == 5 || i == 7;   // slots 1,3 / 4,5 / 6,7 form the pairs
-                            if (!second) { if (W) deposit(s ^ 1, l); }
-                            else { if (L) request(f + 2, l); ++l; }
-                        }
-                        sched_fence();
-                    }
-                }
-                if constexpr (B) {
-                    // Every fragment of tile f is in registers (or in flight) and this wave's part of tile f + 1 is
-                    // written: after the barrier stage s may be overwritten and tile f + 1 is complete in s ^ 1.
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    // the first front publishes tile 1, which the prologue sent straight to LDS: its loads are
-                    // older than the NL requests of tile 2 queued above
-                    if constexpr (!W) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L ? NL : 0) : "memory");
-                    wg_barrier();
-                }
-            };
-            // prologue: tiles 0 and 1 straight into LDS
-#pragma unroll
-            for (int l = 0; l < NL; ++l) issue(0, l);
-            if (KT == 2) poison_tail();
-#pragma unroll
-            for (int l = 0; l < NL; ++l) issue(1, l);
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");   // tile 0 has landed, tile 1 may still be in flight
-            wg_barrier();
-            NTFP8_STAMP(st_first);
-            NTFP8_CYCLES(cy_first);
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                fa[i][0] = rd_a(0, i, 0);
-                fa[i][1] = rd_a(0, i, 1);
-            }
-#pragma unroll
-            for (int h = 0; h < 4; ++h) fb[h >> 1][h & 1] = rd_b(0, h >> 1, h & 1);
-
-            // (poison_tail() runs right before the front that requests the last tile, KT - 1 = f + 2)
-            if (KT == 3) poison_tail();
-            if (KT > 2) front_st(No{}, Yes{}, Yes{}, 0);   // nothing to deposit: tile 1 is on its way to LDS already
-            else front_st(No{}, No{}, Yes{}, 0);
-            int f = 1;
-            for (; f + 3 < KT; ++f) {
-                back(No{}, Yes{}, f - 1);
-                front_st(Yes{}, Yes{}, Yes{}, f);
-            }
-            if (f + 2 < KT) {   // f = KT - 3 >= 1
-                poison_tail();
-                back(No{}, Yes{}, f - 1);
-                front_st(Yes{}, Yes{}, Yes{}, f);
-                ++f;
-            }
-            if (f + 1 < KT) {   // f = KT - 2 >= 1: the last tile is deposited, nothing left to request
-                back(No{}, Yes{}, f - 1);
-                front_st(Yes{}, No{}, Yes{}, f);
-                ++f;
-            }
-            back(No{}, Yes{}, f - 1);   // f = KT - 1
-            front_st(No{}, No{}, No{}, f);
-            back(No{}, No{}, f);
-        } else {
-        // ---- half tiles: loads go straight into LDS (the register budget has no room for staging) --------
         // Three stages: the loads of tile t are queued while tile t - 3's stage is the one just released, i.e.
         // two K-tiles before tile t is published.  A half-tile K-tile is only 32 MFMAs (about 0.55 us): with
         // two stages the loads had half a K-tile to arrive, less than an L2 hit takes.
