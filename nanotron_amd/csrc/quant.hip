@@ -19,12 +19,11 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------------------------
 // Loads of E = 4 or 16 elements.  `mx` receives max|x| of them as a comparable unsigned pattern in
 // the *source* format (fp32 bits for float, 16-bit patterns for half / bf16).
-// kStream: the load is marked streaming and leaves no line behind in the memory-side cache.  Passes that read their
-// tensor once (delayed scaling) use it: in a training step they run behind a GEMM whose output fills that cache, and an
-// ordinary read waits for the lines it displaces (output gradients of a Llama-3-8B layer 23.3 us a tensor against 26.8,
-// activations 18.6 against 20.0, although back to back on a rested cache ordinary loads are the faster ones, 11.4
-// against 13.5 us for 4096 x 4096).  Where a second pass follows (current scaling: amax, then cast) both use ordinary
-// loads, and the second finds what the first has read: fp32 11008 x 4096 with transposed copy 119 -> 78 us for the two.
+// kStream: the load is marked streaming and leaves no line behind in the memory-side cache: for passes that read their
+// tensor once, or last.  In a training step they run behind a GEMM whose output fills that cache, and an ordinary read waits
+// for the lines it displaces.  The amax pass of current scaling, which a cast follows, uses ordinary loads: the cast finds part
+// of the tensor in the cache (bf16 4096 x 4096, amax and cast: ordinary / ordinary 15.4 us, ordinary / streaming 13.7,
+// streaming / streaming 18.2).  Streaming loads have to take whole lines, since a line is not there for a second load.
 template <bool kStream, int kAlign, typename V>
 __device__ __forceinline__ V load_vec(const void* p) {   // p: kAlign-byte aligned
     typedef V VA __attribute__((aligned(kAlign)));
@@ -37,6 +36,15 @@ struct Src;
 template <>
 struct Src<float> {
     static constexpr int kDtype = NTFP8_F32;
+    __device__ static __forceinline__ void unpack(u4 w, float (&v)[4], uint32_t& mx) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = __uint_as_float(w[i]);
+            m = max(m, w[i] & 0x7fffffffu);
+        }
+        mx = m;
+    }
     template <int E, bool kStream>
     __device__ static __forceinline__ void load(const float* p, float (&v)[E], uint32_t& mx) {
         uint32_t m = 0;
@@ -81,6 +89,14 @@ struct Src16 {
                 w[4 * i] = a.x, w[4 * i + 1] = a.y, w[4 * i + 2] = a.z, w[4 * i + 3] = a.w;
             }
         }
+        widen<E>(w, v, mx);
+    }
+    __device__ static __forceinline__ void unpack(u4 w, float (&v)[8], uint32_t& mx) {
+        const uint32_t a[4] = {w.x, w.y, w.z, w.w};
+        widen<8>(a, v, mx);
+    }
+    template <int E>
+    __device__ static __forceinline__ void widen(const uint32_t (&w)[E / 2], float (&v)[E], uint32_t& mx) {
         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
         us2 m = {0, 0};
 #pragma unroll
@@ -181,6 +197,99 @@ __device__ __forceinline__ void record_cast_scale(const ScalarIO& io, float scal
 
 // ---------------------------------------------------------------------------------------------
 // Flat (no transpose) kernel: amax only, cast only, or both (delayed scaling).
+//
+// Bound by HBM.  A lane's load is 16 bytes and the wave's 64 loads lie side by side: 1 KB of whole lines per instruction
+// (16 elements per lane in a row, as two or four loads 32 or 64 bytes apart, touch every line two or four times, which a
+// streaming load pays for; the bytes then leave 8 or 4 a lane).  A workgroup takes spans of 16384 elements, two in flight.
+// us, 16 elements per lane / side by side, 4096 x 4096 and 4096 x 14336: bf16 delayed step 12.5 and 34.0 / 12.0 and 32.6, cast
+// 10.4 and 31.4 / 9.8 and 29.9 (5.9 TB/s), current scaling 15.4 and 47.6 / 13.7 and 44.2; fp32 delayed step 24.9 and 76.6 /
+// 17.3 and 51.7, cast 16.2 and 54.3 / 15.4 and 49.9.  (Probes with two to eight workgroups of 256 or 512 threads per CU: 5 to
+// 20 % slower.  A span requested again as soon as it is done, instead of two at a time: the same, and 0.2 us more for small
+// tensors.)
+template <typename S>
+constexpr int kChunk = 16 / (int)sizeof(typename ElemOf<S>::type);   // elements of a 16-byte load
+template <typename S>
+constexpr int kSpan = kFlatThreads * (kVec / kChunk<S>);             // loads of a span
+
+template <int E>
+__device__ __forceinline__ void store_chunk(uint8_t* __restrict__ p, const uint32_t (&w)[E / 4]) {   // p: E-byte aligned
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    if constexpr (E == 8) __builtin_nontemporal_store((u2){w[0], w[1]}, reinterpret_cast<u2*>(p));
+    else __builtin_nontemporal_store(w[0], reinterpret_cast<uint32_t*>(p));
+}
+
+// Streams a tensor of n elements, n_vec whole 16-byte chunks of it as vectors: `body(v, m, index)` for every chunk,
+// `one(x, m, index)` for elements past them (all of them where a pointer is misaligned).
+template <typename S, typename Body, typename One>
+__device__ __forceinline__ void for_each_chunk(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n, uint32_t bid,
+                                               uint32_t nblocks, Body body, One one) {
+    typedef Src<S> L;
+    constexpr int E = kChunk<S>, U = kVec / E;
+    const int64_t full = n_vec / kSpan<S>;
+    int64_t g = bid;
+    auto spans = [&](auto count_tag) {
+        constexpr int G = decltype(count_tag)::value;
+        float v[G * U][E];
+        uint32_t m[G * U];
+        auto index = [&](int k) -> int64_t {
+            return ((g + (int64_t)(k / U) * nblocks) * kSpan<S> + k % U * kFlatThreads + (int)threadIdx.x) * E;
+        };
+#pragma unroll
+        for (int k = 0; k < G * U; ++k) L::template load<E, true>(x + index(k), v[k], m[k]);
+#pragma unroll
+        for (int k = 0; k < G * U; ++k) body(v[k], m[k], index(k));
+        g += (int64_t)G * nblocks;
+    };
+    while (g + nblocks < full) spans(std::integral_constant<int, 2>{});
+    if (g < full) spans(std::integral_constant<int, 1>{});
+    if (g == full) {   // what is left of the last span: one workgroup's
+        for (int64_t c = full * kSpan<S> + threadIdx.x; c < n_vec; c += kFlatThreads) {
+            float v[E];
+            uint32_t m;
+            L::template load<E, true>(x + c * E, v, m);
+            body(v, m, c * E);
+        }
+    }
+    for (int64_t j = n_vec * E + (int64_t)bid * kFlatThreads + threadIdx.x; j < n; j += (int64_t)nblocks * kFlatThreads) {
+        uint32_t m;
+        const float v = L::load1(x + j, m);
+        one(v, m, j);
+    }
+}
+
+// max|x| alone: 16 elements per lane in a row and ordinary loads (the first touches every line, the others find it in the
+// cache; and the pass that follows finds lines in the memory-side cache).  fp32 11008 x 4096, 16 elements in a row / side by
+// side: 32.2 / 33.1 us.
+template <typename S>
+__device__ __forceinline__ uint32_t flat_max(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n, uint32_t bid,
+                                             uint32_t nblocks) {
+    typedef Src<S> L;
+    uint32_t m_run = 0;
+    n_vec /= kVec / kChunk<S>;
+    const int64_t stride = (int64_t)nblocks * kFlatThreads;
+    int64_t i = (int64_t)bid * kFlatThreads + threadIdx.x;
+    for (; i + stride < n_vec; i += 2 * stride) {
+        float v0[16], v1[16];
+        uint32_t m0, m1;
+        L::template load<16, false>(x + i * kVec, v0, m0);
+        L::template load<16, false>(x + (i + stride) * kVec, v1, m1);
+        m_run = m0 > m_run ? m0 : m_run;
+        m_run = m1 > m_run ? m1 : m_run;
+    }
+    if (i < n_vec) {
+        float v0[16];
+        uint32_t m0;
+        L::template load<16, false>(x + i * kVec, v0, m0);
+        m_run = m0 > m_run ? m0 : m_run;
+    }
+    for (int64_t j = n_vec * kVec + (int64_t)bid * kFlatThreads + threadIdx.x; j < n; j += stride) {
+        uint32_t m;
+        (void)L::load1(x + j, m);
+        m_run = m > m_run ? m : m_run;
+    }
+    return m_run;
+}
+
 template <typename S, int F, int MODE>
 __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n,
                                                 uint8_t* __restrict__ out, const float* __restrict__ scale_ptr,
@@ -188,6 +297,7 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     typedef Src<S> L;
     constexpr bool kCast = MODE != kModeAmaxOnly;
     constexpr bool kAmax = MODE != kModeCastOnly;
+    constexpr int E = kChunk<S>;
     float scale = 1.0f;
     bool degen = false;
     if constexpr (kCast) {
@@ -198,41 +308,21 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     EpiloguePrefetch pre = {0.0f, 1.0f};
     if constexpr (kAmax) pre = prefetch_epilogue(io, MODE);
     uint32_t m_run = 0;  // in source-format bits
-    const int64_t stride = (int64_t)nblocks * kFlatThreads;
-    int64_t i = (int64_t)bid * kFlatThreads + threadIdx.x;
-    // two groups per trip: four (bf16) or eight (fp32) 128-bit loads in flight per lane
-    for (; i + stride < n_vec; i += 2 * stride) {
-        float v0[16], v1[16];
-        uint32_t m0, m1;
-        L::template load<16, MODE == kModeDelayed>(x + i * kVec, v0, m0);
-        L::template load<16, MODE == kModeDelayed>(x + (i + stride) * kVec, v1, m1);
-        if constexpr (kAmax) {
-            m_run = m0 > m_run ? m0 : m_run;
-            m_run = m1 > m_run ? m1 : m_run;
-        }
-        if constexpr (kCast) {
-            const u4 q0 = encode16<F>(v0, scale, degen || L::has_nan(m0));
-            const u4 q1 = encode16<F>(v1, scale, degen || L::has_nan(m1));
-            __builtin_nontemporal_store(q0, reinterpret_cast<u4*>(out + i * kVec));
-            __builtin_nontemporal_store(q1, reinterpret_cast<u4*>(out + (i + stride) * kVec));
-        }
-    }
-    if (i < n_vec) {
-        float v0[16];
-        uint32_t m0;
-        L::template load<16, MODE == kModeDelayed>(x + i * kVec, v0, m0);
-        if constexpr (kAmax) m_run = m0 > m_run ? m0 : m_run;
-        if constexpr (kCast) {
-            const u4 q0 = encode16<F>(v0, scale, degen || L::has_nan(m0));
-            __builtin_nontemporal_store(q0, reinterpret_cast<u4*>(out + i * kVec));
-        }
-    }
-    // elements the vector body does not cover (tail, or everything when a pointer is misaligned)
-    for (int64_t j = n_vec * kVec + (int64_t)bid * kFlatThreads + threadIdx.x; j < n; j += stride) {
-        uint32_t m;
-        const float xv = L::load1(x + j, m);
-        if constexpr (kAmax) m_run = m > m_run ? m : m_run;
-        if constexpr (kCast) out[j] = encode1<F>(xv, scale);
+    if constexpr (!kCast) {
+        m_run = flat_max<S>(x, n_vec, n, bid, nblocks);
+    } else {
+        for_each_chunk<S>(
+            x, n_vec, n, bid, nblocks,
+            [&](const float(&v)[E], uint32_t m, int64_t at) {
+                if constexpr (kAmax) m_run = m > m_run ? m : m_run;
+                uint32_t w[E / 4];
+                encode<F, E>(v, scale, degen || L::has_nan(m), w);
+                store_chunk<E>(out + at, w);
+            },
+            [&](float v, uint32_t m, int64_t j) {
+                if constexpr (kAmax) m_run = m > m_run ? m : m_run;
+                out[j] = encode1<F>(v, scale);
+            });
     }
     if constexpr (kAmax) publish_and_finalize<kFlatThreads>(L::to_f32_bits(m_run), ws, io, MODE, pre, bid, nblocks);
 }
@@ -259,37 +349,22 @@ __global__ __launch_bounds__(kFlatThreads) void quant_flat_dual_kernel(const typ
     const EpiloguePrefetch pre0 = prefetch_epilogue(io0, kModeDelayed);
     const EpiloguePrefetch pre1 = prefetch_epilogue(io1, kModeDelayed);
     uint32_t m_run = 0;
-    const int64_t stride = (int64_t)gridDim.x * kFlatThreads;
-    int64_t i = (int64_t)blockIdx.x * kFlatThreads + threadIdx.x;
-    for (; i + stride < n_vec; i += 2 * stride) {
-        float v0[16], v1[16];
-        uint32_t m0, m1;
-        L::template load<16, true>(x + i * kVec, v0, m0);
-        L::template load<16, true>(x + (i + stride) * kVec, v1, m1);
-        m_run = m0 > m_run ? m0 : m_run;
-        m_run = m1 > m_run ? m1 : m_run;
-        const bool n0 = L::has_nan(m0), n1 = L::has_nan(m1);
-        __builtin_nontemporal_store(encode16<kE4M3>(v0, s0, d0 || n0), reinterpret_cast<u4*>(out0 + i * kVec));
-        __builtin_nontemporal_store(encode16<kE5M2>(v0, s1, d1 || n0), reinterpret_cast<u4*>(out1 + i * kVec));
-        __builtin_nontemporal_store(encode16<kE4M3>(v1, s0, d0 || n1), reinterpret_cast<u4*>(out0 + (i + stride) * kVec));
-        __builtin_nontemporal_store(encode16<kE5M2>(v1, s1, d1 || n1), reinterpret_cast<u4*>(out1 + (i + stride) * kVec));
-    }
-    if (i < n_vec) {
-        float v0[16];
-        uint32_t m0;
-        L::template load<16, true>(x + i * kVec, v0, m0);
-        m_run = m0 > m_run ? m0 : m_run;
-        const bool n0 = L::has_nan(m0);
-        __builtin_nontemporal_store(encode16<kE4M3>(v0, s0, d0 || n0), reinterpret_cast<u4*>(out0 + i * kVec));
-        __builtin_nontemporal_store(encode16<kE5M2>(v0, s1, d1 || n0), reinterpret_cast<u4*>(out1 + i * kVec));
-    }
-    for (int64_t j = n_vec * kVec + (int64_t)blockIdx.x * kFlatThreads + threadIdx.x; j < n; j += stride) {
-        uint32_t m;
-        const float xv = L::load1(x + j, m);
-        m_run = m > m_run ? m : m_run;
-        out0[j] = encode1<kE4M3>(xv, s0);
-        out1[j] = encode1<kE5M2>(xv, s1);
-    }
+    constexpr int E = kChunk<S>;
+    for_each_chunk<S>(
+        x, n_vec, n, blockIdx.x, gridDim.x,
+        [&](const float(&v)[E], uint32_t m, int64_t at) {
+            m_run = m > m_run ? m : m_run;
+            uint32_t w[E / 4];
+            encode<kE4M3, E>(v, s0, d0 || L::has_nan(m), w);
+            store_chunk<E>(out0 + at, w);
+            encode<kE5M2, E>(v, s1, d1 || L::has_nan(m), w);
+            store_chunk<E>(out1 + at, w);
+        },
+        [&](float v, uint32_t m, int64_t j) {
+            m_run = m > m_run ? m : m_run;
+            out0[j] = encode1<kE4M3>(v, s0);
+            out1[j] = encode1<kE5M2>(v, s1);
+        });
     publish_and_finalize<kFlatThreads>(L::to_f32_bits(m_run), ws, io0, kModeDelayed, pre0, blockIdx.x, gridDim.x, &io1, &pre1);
 }
 
@@ -425,7 +500,33 @@ __device__ __forceinline__ void store_row_bytes(uint8_t* __restrict__ p, const u
     }
 }
 
-template <typename S, int F, bool kAmax, int E>
+// Eight lanes hold 128 columns of a row, lane l as Q loads of 16 / Q columns each, 128 / Q columns apart (so that one load of
+// the eight lanes is a whole line).  gather_span exchanges the loads' bytes among Q neighbouring lanes; lane l then holds the
+// 16 consecutive columns of group span_group(l).
+template <int Q>
+__device__ __forceinline__ int span_group(int l) {
+    return (l % Q) * (8 / Q) + l / Q;
+}
+template <int kPerm>
+__device__ __forceinline__ void exchange(uint32_t& a, uint32_t& b, bool upper) {   // a lower lane's b <-> its upper partner's a
+    const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)(upper ? a : b), kPerm, 0xf, 0xf, true);
+    a = upper ? r : a;
+    b = upper ? b : r;
+}
+template <int Q>
+__device__ __forceinline__ void gather_span(uint32_t (&w)[4], int l) {
+    if constexpr (Q == 2) {   // w[0..1]: the first load's words
+        exchange<0xB1>(w[0], w[2], l & 1);   // quad_perm [1, 0, 3, 2]
+        exchange<0xB1>(w[1], w[3], l & 1);
+    } else {
+        exchange<0xB1>(w[0], w[1], l & 1);
+        exchange<0xB1>(w[2], w[3], l & 1);
+        exchange<0x4E>(w[0], w[2], l & 2);   // quad_perm [2, 3, 0, 1]
+        exchange<0x4E>(w[1], w[3], l & 2);
+    }
+}
+
+template <typename S, int F, bool kAmax, int E, bool kStream>
 __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typename ElemOf<S>::type* __restrict__ x,
                                                                    int64_t rows, int64_t cols,
                                                                    uint8_t* __restrict__ out,
@@ -434,16 +535,14 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
                                                                    Workspace* ws, ScalarIO io) {
     typedef Src<S> L;
     typedef Tile<E> T;
-    // (16 fp32 values are four 16-byte loads of a lane that lie 64 bytes apart across the lanes: streaming lines do not stay
-    // for the other three.  Streaming / ordinary, us: delayed step of 2^22 to 2^23 elements 12.5 / 10.2, 2^24 to 2^25 44 / 29,
-    // 2^25 to 2^26 103 / 64)
-    constexpr bool kStream = kAmax && sizeof(*x) == 2;
+    // whole lines per load of eight lanes (not for fp32 rows that start anywhere: 36.7 against 34.8 us, 4095 x 4097)
+    constexpr bool kLines = E == 16 && (kStream || sizeof(*x) == 2);
     __shared__ __attribute__((aligned(16))) uint32_t tile[T::kT * T::kPitch];
     const float scale = *scale_ptr;
     const bool degen = degenerate_scale(scale);
     const int64_t tiles_c = (cols + T::kT - 1) / T::kT;
     const int64_t tiles = ((rows + T::kT - 1) / T::kT) * tiles_c;
-    const int cgrp = threadIdx.x % (T::kT / E), rgrp = threadIdx.x / (T::kT / E);
+    const int lane_grp = threadIdx.x % (T::kT / E), rgrp = threadIdx.x / (T::kT / E);
     EpiloguePrefetch pre = {0.0f, 1.0f};
     if constexpr (kAmax) pre = prefetch_epilogue(io, kModeDelayed);
     else record_cast_scale(io, scale, blockIdx.x);
@@ -451,36 +550,70 @@ __global__ __launch_bounds__(kTileThreads) void quant_transpose_kernel(const typ
     // persistent over tiles: the number of blocks (and so of reduction atomics) stays small
     for (int64_t tile_id = blockIdx.x; tile_id < tiles; tile_id += gridDim.x) {
         const int64_t row0 = (tile_id / tiles_c) * T::kT, col0 = (tile_id % tiles_c) * T::kT;
-        const int64_t c = col0 + cgrp * E;
-        float v[4][E];
-        uint32_t m[4];
-        if (c + E <= cols) {
+        uint32_t w[4][E / 4];
+        int cgrp = lane_grp;   // the thread's columns: E from E cgrp on
+        bool whole = false;
+        if constexpr (kLines) whole = col0 + T::kT <= cols;   // uniform
+        if (whole) {
+            if constexpr (kLines) {
+                constexpr int C = kChunk<S>, Q = E / C;   // Q loads of C elements a row, kT / Q columns apart
+                cgrp = span_group<Q>(lane_grp);
+                u4 raw[4][Q];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t row = row0 + rgrp * 4 + r;
-                L::template load<E, kStream>(x + (row < rows ? row : rows - 1) * cols + c, v[r], m[r]);
-            }
-        } else {
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = row0 + rgrp * 4 + r;
+                    const typename ElemOf<S>::type* p = x + (row < rows ? row : rows - 1) * cols + col0 + lane_grp * C;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t row = row0 + rgrp * 4 + r;
-                const typename ElemOf<S>::type* p = x + (row < rows ? row : rows - 1) * cols;
-                m[r] = 0;
+                    for (int q = 0; q < Q; ++q) raw[r][q] = load_vec<kStream, sizeof(*x), u4>(p + q * (T::kT / Q));
+                }
 #pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    uint32_t me;
-                    v[r][e] = L::load1(p + (c + e < cols ? c + e : cols - 1), me);
-                    m[r] = me > m[r] ? me : m[r];
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = row0 + rgrp * 4 + r;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        float v[C];
+                        uint32_t e[C / 4], m;
+                        L::unpack(raw[r][q], v, m);
+                        encode<F, C>(v, scale, degen || L::has_nan(m), e);
+#pragma unroll
+                        for (int i = 0; i < C / 4; ++i) w[r][q * (C / 4) + i] = e[i];
+                        if constexpr (kAmax) m_run = m > m_run ? m : m_run;
+                    }
+                    gather_span<Q>(w[r], lane_grp);
+                    if (out && row < rows) store_row_bytes<E>(out + row * cols + col0 + cgrp * E, w[r], E);
                 }
             }
-        }
-        uint32_t w[4][E / 4];
+        } else {
+            const int64_t c = col0 + cgrp * E;
+            float v[4][E];
+            uint32_t m[4];
+            if (c + E <= cols) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t row = row0 + rgrp * 4 + r;
-            if constexpr (kAmax) m_run = m[r] > m_run ? m[r] : m_run;
-            encode<F, E>(v[r], scale, degen || L::has_nan(m[r]), w[r]);
-            if (out && row < rows && c < cols) store_row_bytes<E>(out + row * cols + c, w[r], cols - c);
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = row0 + rgrp * 4 + r;
+                    L::template load<E, kStream>(x + (row < rows ? row : rows - 1) * cols + c, v[r], m[r]);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = row0 + rgrp * 4 + r;
+                    const typename ElemOf<S>::type* p = x + (row < rows ? row : rows - 1) * cols;
+                    m[r] = 0;
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        uint32_t me;
+                        v[r][e] = L::load1(p + (c + e < cols ? c + e : cols - 1), me);
+                        m[r] = me > m[r] ? me : m[r];
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = row0 + rgrp * 4 + r;
+                if constexpr (kAmax) m_run = m[r] > m_run ? m[r] : m_run;
+                encode<F, E>(v[r], scale, degen || L::has_nan(m[r]), w[r]);
+                if (out && row < rows && c < cols) store_row_bytes<E>(out + row * cols + c, w[r], cols - c);
+            }
         }
         deposit_block<E>(tile, w, cgrp, rgrp);
         __syncthreads();
@@ -799,9 +932,9 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __rest
 }
 
 // ---------------------------------------------------------------------------------------------
-// Bandwidth yardsticks: the access pattern of the flat quantise kernel (one 1024-thread workgroup per CU, two
-// 16-element groups per lane and trip, 128-bit non-temporal accesses) with the arithmetic and the reduction taken
-// out.  kProbeRead: 32 bytes read per group, nothing written.  kProbeHalf: 32 bytes read, 16 written (the traffic of
+// Bandwidth yardsticks: the access pattern of the flat quantise kernel (one 1024-thread workgroup per CU, two spans of
+// 16 bf16 elements per lane in flight, 16-byte streaming loads side by side) with the arithmetic and the reduction taken
+// out.  kProbeRead: 32 bytes read per lane and span, nothing written.  kProbeHalf: 32 bytes read, 16 written (the traffic of
 // a bf16 -> fp8 cast).  kProbeCopy: 32 read, 32 written.
 enum ProbeMode { kProbeRead = NTFP8_PROBE_READ, kProbeHalf = NTFP8_PROBE_HALF, kProbeCopy = NTFP8_PROBE_COPY };
 template <int MODE>
@@ -810,12 +943,15 @@ __global__ __launch_bounds__(kFlatThreads) void stream_probe_kernel(const u4* __
     int64_t i = (int64_t)blockIdx.x * kFlatThreads + threadIdx.x;
     u4 seen = {0u, 0u, 0u, 0u};
     auto one = [&](int64_t k) {
-        const u4 a = __builtin_nontemporal_load(src + 2 * k), b = __builtin_nontemporal_load(src + 2 * k + 1);
+        const int64_t span = k / kFlatThreads;
+        const bool whole = (span + 1) * kFlatThreads <= n_vec;
+        const int64_t ka = whole ? 2 * span * kFlatThreads + threadIdx.x : 2 * k, kb = whole ? ka + kFlatThreads : ka + 1;
+        const u4 a = __builtin_nontemporal_load(src + ka), b = __builtin_nontemporal_load(src + kb);
         if constexpr (MODE == kProbeRead) seen = seen | (a ^ b);
         else if constexpr (MODE == kProbeHalf) __builtin_nontemporal_store(a ^ b, dst + k);
         else {
-            __builtin_nontemporal_store(a, dst + 2 * k);
-            __builtin_nontemporal_store(b, dst + 2 * k + 1);
+            __builtin_nontemporal_store(a, dst + ka);
+            __builtin_nontemporal_store(b, dst + kb);
         }
     };
     for (; i + stride < n_vec; i += 2 * stride) {
@@ -851,13 +987,18 @@ static int grid_for(int64_t work_items, int threads = kThreads, int per_cu_block
 static void clear_stale_error() { (void)hipGetLastError(); }
 static int check_launch() { return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH; }
 
+// workgroups of the flat kernels: two spans each until there is one workgroup per CU
+template <typename S>
+static int flat_grid(int64_t n_vec, int64_t n) {
+    return grid_for(n_vec > 0 ? (n_vec + 2 * kVec / kChunk<S> - 1) / (2 * kVec / kChunk<S>) : n, kFlatThreads, 1);
+}
+
 template <typename S, int F>
 static int launch_flat(int mode, const void* x, int64_t n, bool vec_ok, uint8_t* out, const float* scale_ptr,
                        Workspace* ws, const ScalarIO& io, hipStream_t st) {
     typedef typename ElemOf<S>::type E;
-    const int64_t n_vec = vec_ok ? n / kVec : 0;
-    // two 16-element groups per lane per trip
-    const int grid = grid_for(n_vec > 0 ? (n_vec + 1) / 2 : n, kFlatThreads, 1);
+    const int64_t n_vec = vec_ok ? n / kChunk<S> : 0;
+    const int grid = flat_grid<S>(n_vec, n);
     const E* xp = static_cast<const E*>(x);
     if (mode == kModeAmaxOnly)
         hipLaunchKernelGGL((quant_flat_kernel<S, F, kModeAmaxOnly>), dim3(grid), dim3(kFlatThreads), 0, st, xp, n_vec, n, out,
@@ -909,11 +1050,19 @@ static int launch_transpose(const void* x, int64_t rows, int64_t cols, uint8_t* 
     // instead of 24.2, fp32 of 512 24.6 instead of 23.6)
     const int64_t cap = kAmax ? std::min<int64_t>(2 * cus, kCells) : 8 * cus;
     const int grid = (int)(tiles < cap ? tiles : cap);
-    if (e == 16)
-        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
+    // Streaming loads where rows start on lines.  us, one row of 16 elements per thread and load / whole lines, streaming: cast
+    // with copy bf16 4096 x 4096 15.9 / 14.7, fp32 22.2 / 19.9, 11008 x 4096 54.0 / 50.3; delayed step bf16 18.5 / 16.6, fp32
+    // 11008 x 4096 57.8 / 53.5.  Rows that start anywhere: bf16 4095 x 4097 whole lines, streaming 30.7, ordinary 29.2.
+    constexpr bool kSmall = kAmax && sizeof(E) == 2;
+    const bool lines = cols * (int64_t)sizeof(E) % 128 == 0 && (reinterpret_cast<uintptr_t>(x) & 127) == 0;
+    if (e == 16 && lines)
+        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16, true>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
+                           out_t, scale_ptr, ws, io);
+    else if (e == 16)
+        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 16, false>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
                            out_t, scale_ptr, ws, io);
     else
-        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 4>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
+        hipLaunchKernelGGL((quant_transpose_kernel<S, F, kAmax, 4, kSmall>), dim3(grid), dim3(kTileThreads), 0, st, xp, rows, cols, out,
                            out_t, scale_ptr, ws, io);
     return check_launch();
 }
@@ -1037,11 +1186,11 @@ static int launch_flat_multi(const QuantDesc* const* q, int count, hipStream_t s
         T.x = d.x;
         T.out = static_cast<uint8_t*>(d.out);
         T.n = n;
-        T.n_vec = vec_ok ? n / kVec : 0;
+        T.n_vec = vec_ok ? n / kChunk<S> : 0;
         T.ws = static_cast<Workspace*>(d.ws);
         T.io = d.io;
         T.first_block = blocks;
-        T.blocks = grid_for(T.n_vec > 0 ? (T.n_vec + 1) / 2 : n, kFlatThreads, 1);
+        T.blocks = flat_grid<S>(T.n_vec, n);
         blocks += T.blocks;
     }
     hipLaunchKernelGGL((quant_flat_multi_kernel<S, F>), dim3(blocks), dim3(kFlatThreads), 0, st, Q);
@@ -1091,22 +1240,16 @@ int run_quant_dual(const void* x, int x_dtype, int64_t n, uint8_t* out_e4m3, uin
                    const ScalarIO& io_e4m3, const ScalarIO& io_e5m2, hipStream_t st) {
     clear_stale_error();
     const bool vec_ok = aligned(x, 16) && aligned(out_e4m3, 16) && aligned(out_e5m2, 16);
-    const int64_t n_vec = vec_ok ? n / kVec : 0;
-    const int grid = grid_for(n_vec > 0 ? (n_vec + 1) / 2 : n, kFlatThreads, 1);
-    switch (x_dtype) {
-        case NTFP8_F32:
-            hipLaunchKernelGGL((quant_flat_dual_kernel<float>), dim3(grid), dim3(kFlatThreads), 0, st,
-                               static_cast<const float*>(x), n_vec, n, out_e4m3, out_e5m2, ws, io_e4m3, io_e5m2);
-            break;
-        case NTFP8_F16:
-            hipLaunchKernelGGL((quant_flat_dual_kernel<f16_tag>), dim3(grid), dim3(kFlatThreads), 0, st,
-                               static_cast<const uint16_t*>(x), n_vec, n, out_e4m3, out_e5m2, ws, io_e4m3, io_e5m2);
-            break;
-        default:
-            hipLaunchKernelGGL((quant_flat_dual_kernel<bf16_tag>), dim3(grid), dim3(kFlatThreads), 0, st,
-                               static_cast<const uint16_t*>(x), n_vec, n, out_e4m3, out_e5m2, ws, io_e4m3, io_e5m2);
-            break;
-    }
+#define NT_DUAL(S) \
+    do { \
+        const int64_t n_vec = vec_ok ? n / kChunk<S> : 0; \
+        hipLaunchKernelGGL((quant_flat_dual_kernel<S>), dim3(flat_grid<S>(n_vec, n)), dim3(kFlatThreads), 0, st, \
+                           static_cast<const ElemOf<S>::type*>(x), n_vec, n, out_e4m3, out_e5m2, ws, io_e4m3, io_e5m2); \
+    } while (0)
+    if (x_dtype == NTFP8_F32) NT_DUAL(float);
+    else if (x_dtype == NTFP8_F16) NT_DUAL(f16_tag);
+    else NT_DUAL(bf16_tag);
+#undef NT_DUAL
     return check_launch();
 }
 
