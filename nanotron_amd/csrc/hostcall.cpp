@@ -181,34 +181,53 @@ PyObject* quantised(at::Tensor out, at::Tensor out_t, const Scalars& s) {
     return Py_BuildValue("(NNNN)", wrap(std::move(out)), wrap_or_none(std::move(out_t)), wrap(s.element(0)), wrap(s.element(1)));
 }
 
-// quantize(x, fmt, margin, state | None, flag | None, history_len, with_transpose) -> (bytes, bytes^T | None, amax, scale)
-// state None: current scaling; flag given: the role may not hold a scale yet; otherwise the fused delayed-scaling step
-PyObject* quantize(PyObject* const* a) {
-    const at::Tensor x = operand(a[0]);
-    const int fmt = (int)number(a[1]), margin = (int)number(a[2]), hist = (int)number(a[5]);
-    const bool with_t = truth(a[6]);
+struct Quantised {
+    at::Tensor out, out_t;
+    Scalars s;
+};
+PyObject* quantised(Quantised&& q) { return quantised(std::move(q.out), std::move(q.out_t), q.s); }
+
+// A dense tensor on a CUDA device.  buf [scale, hist[0..H-1]] null: current scaling; flag given: the role may not hold a scale
+// yet; otherwise the fused delayed-scaling step
+Quantised quantise(const at::Tensor& x, int fmt, int margin, float* buf, float* flag, int hist, bool with_t) {
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
-    float* const buf = none(a[3]) ? nullptr : values(a[3], x.device(), 1 + hist);   // [scale, hist[0..H-1]]
-    float* const flag = none(a[4]) ? nullptr : values(a[4], x.device());
-    at::Tensor out = bytes_like(x, x.sizes()), out_t;
-    if (with_t) out_t = bytes_like(x, {cols, rows});
-    const Scalars s(x);
+    Quantised q{bytes_like(x, x.sizes()), at::Tensor(), Scalars(x)};
+    if (with_t) q.out_t = bytes_like(x, {cols, rows});
     void* st = stream_of(x);
     void* ws = workspace_of(x, st);
-    void* tp = with_t ? out_t.data_ptr() : nullptr;
+    void* out = q.out.data_ptr();
+    void* tp = with_t ? q.out_t.data_ptr() : nullptr;
     const int xd = code_of(x.scalar_type());
+    float* const p = q.s.p;
     if (buf == nullptr)
-        call(ntfp8_quantize_current(x.data_ptr(), xd, rows, cols, fmt, margin, s.p, s.p + 1, out.data_ptr(), tp, nullptr, 0, nullptr, ws, st),
-             "ntfp8_quantize_current");
+        call(ntfp8_quantize_current(x.data_ptr(), xd, rows, cols, fmt, margin, p, p + 1, out, tp, nullptr, 0, nullptr, ws, st), "ntfp8_quantize_current");
     else if (flag != nullptr)
-        call(ntfp8_quantize_first_use(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, flag, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
-             "ntfp8_quantize_first_use");
+        call(ntfp8_quantize_first_use(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, flag, p, p + 1, out, tp, ws, st), "ntfp8_quantize_first_use");
     else
-        call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, s.p, s.p + 1, out.data_ptr(), tp, ws, st),
-             "ntfp8_quantize_delayed");
-    return quantised(std::move(out), std::move(out_t), s);
+        call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, p, p + 1, out, tp, ws, st), "ntfp8_quantize_delayed");
+    return q;
+}
+Quantised cast_held(const at::Tensor& x, const float* scale, int fmt, bool with_t) {
+    int64_t rows, cols;
+    rows_cols(x, &rows, &cols);
+    require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
+    Quantised q{bytes_like(x, x.sizes()), at::Tensor(), Scalars(x)};
+    if (with_t) q.out_t = bytes_like(x, {cols, rows});
+    call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, scale, fmt, q.s.p, q.s.p + 1, q.out.data_ptr(),
+                               with_t ? q.out_t.data_ptr() : nullptr, stream_of(x)),
+         "ntfp8_cast_with_scale");
+    return q;
+}
+
+// quantize(x, fmt, margin, state | None, flag | None, history_len, with_transpose) -> (bytes, bytes^T | None, amax, scale)
+PyObject* quantize(PyObject* const* a) {
+    const at::Tensor x = operand(a[0]);
+    const int hist = (int)number(a[5]);
+    float* const buf = none(a[3]) ? nullptr : values(a[3], x.device(), 1 + hist);
+    float* const flag = none(a[4]) ? nullptr : values(a[4], x.device());
+    return quantised(quantise(x, (int)number(a[1]), (int)number(a[2]), buf, flag, hist, truth(a[6])));
 }
 
 // quantize_batch([(x, state, history_len, margin, with_transpose), ...], fmt) -> [(bytes, bytes^T | None, amax, scale), ...]:
@@ -367,35 +386,25 @@ PyObject* gemm_fp8(PyObject* const* p) {
 // cast_with_scale(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None, amax = 0, scale)
 PyObject* cast_with_scale(PyObject* const* a) {
     const at::Tensor x = operand(a[0]);
-    const int fmt = (int)number(a[2]);
-    const bool with_t = truth(a[3]);
-    int64_t rows, cols;
-    rows_cols(x, &rows, &cols);
-    require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
-    const float* scale = values(a[1], x.device());
-    at::Tensor out = bytes_like(x, x.sizes()), out_t;
-    if (with_t) out_t = bytes_like(x, {cols, rows});
-    const Scalars s(x);
-    call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, scale, fmt,
-                               s.p, s.p + 1, out.data_ptr(), with_t ? out_t.data_ptr() : nullptr, stream_of(x)),
-         "ntfp8_cast_with_scale");
-    return quantised(std::move(out), std::move(out_t), s);
+    return quantised(cast_held(x, values(a[1], x.device()), (int)number(a[2]), truth(a[3])));
 }
 
+at::Tensor sum_columns(const at::Tensor& x, int out_code) {
+    const auto opt = at::TensorOptions().device(x.device());
+    at::Tensor out = at::empty({x.size(1)}, opt.dtype(type_of(out_code))), scratch;
+    const int64_t need = ntfp8_column_sum_scratch(x.size(0), x.size(1));
+    if (need > 0) scratch = at::empty({need / 4}, opt.dtype(at::kFloat));
+    void* st = stream_of(x);
+    call(ntfp8_column_sum(x.data_ptr(), code_of(x.scalar_type()), x.size(0), x.size(1), out.data_ptr(), out_code,
+                          need > 0 ? scratch.data_ptr() : nullptr, workspace_of(x, st), st),
+         "ntfp8_column_sum");
+    return out;
+}
 // column_sum([rows, cols], out_code) -> [cols]
 PyObject* column_sum(PyObject* const* a) {
     const at::Tensor x = operand(a[0]);
     require(x.dim() == 2, "a 2-D tensor is expected");
-    const long code = number(a[1]);
-    const auto opt = at::TensorOptions().device(x.device());
-    at::Tensor out = at::empty({x.size(1)}, opt.dtype(type_of(code))), scratch;
-    const int64_t need = ntfp8_column_sum_scratch(x.size(0), x.size(1));
-    if (need > 0) scratch = at::empty({need / 4}, opt.dtype(at::kFloat));
-    void* st = stream_of(x);
-    call(ntfp8_column_sum(x.data_ptr(), code_of(x.scalar_type()), x.size(0), x.size(1), out.data_ptr(), (int)code,
-                          need > 0 ? scratch.data_ptr() : nullptr, workspace_of(x, st), st),
-         "ntfp8_column_sum");
-    return wrap(std::move(out));
+    return wrap(sum_columns(x, (int)number(a[1])));
 }
 
 // cast(x, scale, fmt, with_transpose) -> (bytes, bytes^T | None)
@@ -443,27 +452,161 @@ bool reads_b(int64_t M, int64_t N, int64_t K) {
 }
 PyObject* b_transposed_supported(PyObject* const* a) { return PyBool_FromLong(reads_b(number(a[0]), number(a[1]), number(a[2]))); }
 
+bool aligned16(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }   // 16-byte loads / stores
+// What the library's A and B of D = op(mat_b) . mat_a are: 1 A is mat_b's transposed copy, 2 B is mat_a's transposed copy, 4 B
+// read as its transpose, 8 A read as its transpose.  `a_plain`: mat_a may be read as it is.
+bool readable(const at::Tensor& a, bool has_copy, bool read_b) { return read_b && !has_copy && a.dim() == 2 && a.is_contiguous() && aligned16(a); }
+int form_wgrad(bool a_plain, int64_t K, int64_t N, int64_t M, bool b_plain, bool read_a, bool b_copy_aligned) {
+    // D[cols of mat_b, cols of mat_a], reduction over the rows of both
+    if (a_plain && read_a && b_plain && M % 16 == 0 && reads_b(M, N, K)) return 4 | 8;
+    if (a_plain && b_copy_aligned && reads_b(M, N, K)) return 1 | 4;
+    return 1 | 2;
+}
+int form_dgrad(bool a_plain, int64_t K, int64_t N, int64_t M) { return a_plain && reads_b(M, N, K) ? 4 : 2; }
+
 // operand_form(mat_a, its transposed copy | None, transpose_a, mat_b, its transposed copy | None, transpose_b, accumulate_into |
-// None, allow_bt, read_b, read_a) -> bits: 1 the library's A is mat_b's transposed copy, 2 its B is mat_a's transposed copy, 4 B read as its
-// transpose, 8 A read as its transpose
+// None, allow_bt, read_b, read_a) -> bits as above
 PyObject* operand_form(PyObject* const* p) {
     const at::Tensor &a = tensor(p[0]), &b = tensor(p[3]);
     require(a.is_cuda() && b.is_cuda(), "The tensors must be on a CUDA device in order to use the FP8 kernel!!");
     const bool ta = truth(p[2]), tb = truth(p[5]);
     if (ta) return PyLong_FromLong(tb ? 1 : 0);
-    const bool read_b = truth(p[7]) && truth(p[8]), read_a = truth(p[9]);
-    auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };   // 16-byte loads / stores
-    const bool plain_a = read_b && none(p[1]) && a.dim() == 2 && a.is_contiguous() && aligned(a) && aligned(b) && (none(p[6]) || aligned(tensor(p[6])));
-    if (tb) {
-        // D[cols of mat_b, cols of mat_a], reduction over the rows of both
-        if (plain_a && read_a && none(p[4]) && b.dim() == 2 && b.is_contiguous() && b.size(1) % 16 == 0 && reads_b(b.size(1), a.size(1), a.size(0)))
-            return PyLong_FromLong(4 | 8);
-        // (a copy that has yet to be made is a fresh allocation: aligned)
-        if (plain_a && (none(p[4]) || aligned(tensor(p[4]))) && b.dim() == 2 && reads_b(b.size(1), a.size(1), a.size(0))) return PyLong_FromLong(1 | 4);
-        return PyLong_FromLong(1 | 2);
+    const bool plain_a = readable(a, !none(p[1]), truth(p[7]) && truth(p[8])) && aligned16(b) && (none(p[6]) || aligned16(tensor(p[6])));
+    if (a.dim() != 2 || b.dim() != 2) return PyLong_FromLong(tb ? 1 | 2 : 2);
+    // (a copy that has yet to be made is a fresh allocation: aligned)
+    if (tb) return PyLong_FromLong(form_wgrad(plain_a, a.size(0), a.size(1), b.size(1), none(p[4]) && b.is_contiguous(), truth(p[9]), none(p[4]) || aligned16(tensor(p[4]))));
+    return PyLong_FromLong(form_dgrad(plain_a, a.size(0), a.size(1), b.size(0)));
+}
+
+// ---- a layer's passes, one call each.  Between the pieces above a pass of a small layer spends more time in Python than the
+// pieces take.  What is not served here (None is returned, nothing launched) takes the way through the pieces.
+void gemm_desc(ntfp8_gemm_desc* d, const at::Tensor& a, int fa, const float* sa, const at::Tensor& b, int fb, const float* sb, const at::Tensor& out, int64_t M,
+              int64_t N, int64_t K, bool bt, bool at_, bool accumulate) {
+    *d = {};
+    d->A = a.data_ptr(), d->scale_a = sa, d->fmt_a = fa;
+    d->B = b.data_ptr(), d->scale_b = sb, d->fmt_b = fb;
+    d->D = out.data_ptr(), d->d_dtype = code_of(out.scalar_type()), d->accumulate = accumulate;
+    d->M = M, d->N = N, d->K = K;
+    d->b_transposed = bt, d->a_transposed = at_;
+}
+// an fp8 operand [rows, cols] beside a tensor of that device
+bool bytes_of(const at::Tensor& t, c10::Device device) {
+    return t.is_cuda() && t.device() == device && t.dim() == 2 && t.element_size() == 1 && t.is_contiguous();
+}
+
+// linear_forward(x, fmt, margin, state | None, history_len, held, wants a transposed copy unless dW's GEMM reads the input as it
+// is, read_b, weight bytes, fmt, scale, bias | None, out_code) -> (y, bytes, bytes^T | None, amax, scale) | None: quantisation of the input (current scaling, the fused
+// delayed-scaling step, or, with `held`, a cast with the state's scale that leaves the state alone) and Y = X . W^T
+PyObject* linear_forward(PyObject* const* p) {
+    const at::Tensor &input = tensor(p[0]), &w = tensor(p[8]);
+    if (!input.is_cuda() || input.dim() < 1 || input.numel() == 0 || code_of(input.scalar_type()) < 0 || !bytes_of(w, input.device()) ||
+        input.size(-1) != w.size(1))
+        Py_RETURN_NONE;
+    const int64_t K = w.size(1), N = w.size(0);
+    at::Tensor x = input.dim() == 2 ? input : input.reshape({-1, K});
+    x = dense(x);
+    const int64_t M = x.size(0);
+    const int hist = (int)number(p[4]), fmt = (int)number(p[1]);
+    const long out_code = number(p[12]);
+    if (out_code < 0 || out_code > NTFP8_BF16) Py_RETURN_NONE;
+    float* const buf = none(p[3]) ? nullptr : values(p[3], x.device(), 1 + hist);
+    const bool held = truth(p[5]), with_t = truth(p[6]) && !(truth(p[7]) && reads_b(N, K, M));
+    const float* sw = values(p[10], x.device());
+    at::Tensor bias;
+    if (!none(p[11])) {
+        bias = dense(tensor(p[11]));
+        require(bias.dim() == 1 && bias.size(0) == N && bias.device() == x.device(), "bias must hold one value per output column");
+        require(code_of(bias.scalar_type()) >= 0, "unsupported bias dtype");
     }
-    if (plain_a && b.dim() == 2 && reads_b(b.size(0), a.size(1), a.size(0))) return PyLong_FromLong(4);
-    return PyLong_FromLong(2);
+    Quantised q = held ? cast_held(x, buf, fmt, with_t) : quantise(x, fmt, (int)number(p[2]), buf, nullptr, hist, with_t);
+    std::vector<int64_t> shape(input.sizes().begin(), input.sizes().end());
+    shape.back() = N;
+    at::Tensor y = at::empty(shape, at::TensorOptions().dtype(type_of(out_code)).device(x.device()));
+    ntfp8_gemm_desc d;
+    gemm_desc(&d, q.out, fmt, q.s.p + 1, w, (int)number(p[9]), sw, y, M, N, K, false, false, false);
+    if (bias.defined()) d.bias = bias.data_ptr(), d.bias_dtype = code_of(bias.scalar_type());
+    call(ntfp8_gemm_batch(&d, 1, stream_of(x)), "ntfp8_gemm_batch");
+    return Py_BuildValue("(NNNNN)", wrap(std::move(y)), wrap(std::move(q.out)), wrap_or_none(std::move(q.out_t)), wrap(q.s.element(0)), wrap(q.s.element(1)));
+}
+
+// linear_backward(dY, its scale where it is fp8 bytes | None, input bytes, their transposed copy | None, fmt, scale, weight bytes, their
+// transposed copy | None, fmt, scale, gradient fmt, margin, state | None, history_len, bias code | -1, dX code | -1, (state,
+// history_len, margin) of an fp8 dX | None, wants dW, dW to accumulate into | None, read_b, read_a) -> (bias gradient | None,
+// dX | None, dW | None[, amax, scale of an fp8 dX]) | None: bias gradient, quantisation of dY (current scaling or the fused
+// delayed-scaling step), dX = dY . W and dW = dY^T . X
+PyObject* linear_backward(PyObject* const* p) {
+    const at::Tensor &grad = tensor(p[0]), &x = tensor(p[2]), &w = tensor(p[6]);
+    const bool quantised_already = !none(p[1]);
+    if (!grad.is_cuda() || grad.dim() < 1 || grad.numel() == 0) Py_RETURN_NONE;
+    const c10::Device dev = grad.device();
+    if (!bytes_of(x, dev) || !bytes_of(w, dev)) Py_RETURN_NONE;
+    const int64_t N = w.size(0), K = w.size(1), T = x.size(0);
+    if (grad.size(-1) != N || grad.numel() != T * N || x.size(1) != K) Py_RETURN_NONE;
+    if (quantised_already ? !bytes_of(grad, dev) || !aligned16(grad) : code_of(grad.scalar_type()) < 0) Py_RETURN_NONE;
+    const bool has_xt = !none(p[3]), has_wt = !none(p[7]);
+    if ((has_xt && !bytes_of(tensor(p[3]), dev)) || (has_wt && !bytes_of(tensor(p[7]), dev))) Py_RETURN_NONE;
+    const bool wants_dw = truth(p[17]), read_b = truth(p[19]), read_a = truth(p[20]);
+    const long bias_code = number(p[14]), dx_code = number(p[15]);
+    const bool fp8_dx = !none(p[16]);
+    if (bias_code > NTFP8_BF16 || (bias_code >= 0 && quantised_already) || (dx_code > NTFP8_BF16) != fp8_dx) Py_RETURN_NONE;
+    at::Tensor dw;
+    const bool accumulate = !none(p[18]);
+    if (accumulate) {
+        dw = tensor(p[18]);
+        if (dw.scalar_type() != at::kFloat || dw.dim() != 2 || dw.size(0) != N || dw.size(1) != K || !dw.is_contiguous() || dw.device() != dev) Py_RETURN_NONE;
+    }
+    // the forms of the two GEMMs (bytes that are yet to be made are fresh allocations: aligned), before anything is launched
+    const bool with_t = !quantised_already && wants_dw && !(!has_xt && read_a && read_b && N % 16 == 0 && reads_b(N, K, T));
+    const int dform = dx_code < 0 ? 0 : form_dgrad(readable(w, has_wt, read_b && !(fp8_dx && T % 4)), N, K, T);
+    if ((dform & 2) && !has_wt) Py_RETURN_NONE;
+    const int wform = !wants_dw ? 0 : form_wgrad(readable(x, has_xt, read_b) && (!accumulate || aligned16(dw)), T, K, N, !with_t, read_a, true);
+    if (((wform & 2) && !has_xt) || ((wform & 1) && !with_t)) Py_RETURN_NONE;
+    const int hist = (int)number(p[13]), fx = (int)number(p[4]), fw = (int)number(p[8]), fg = (int)number(p[10]);
+    const float *sx = values(p[5], dev), *sw = values(p[9], dev);
+    float* const buf = none(p[12]) ? nullptr : values(p[12], dev, 1 + hist);
+
+    at::Tensor db, dx, gq, gq_t;
+    const float* sg;
+    Scalars made(grad);   // [amax, scale] of an fp8 dX
+    at::Tensor keep;      // the scale of a dY quantised here
+    if (quantised_already) {
+        gq = grad;
+        sg = values(p[1], dev);
+    } else {
+        at::Tensor g = dense(grad);
+        if (g.dim() != 2) g = g.view({T, N});
+        if (bias_code >= 0) db = sum_columns(g, (int)bias_code);
+        Quantised q = quantise(g, fg, (int)number(p[11]), buf, nullptr, hist, with_t);
+        gq = std::move(q.out), gq_t = std::move(q.out_t), keep = q.s.both;
+        sg = q.s.p + 1;
+    }
+    ntfp8_gemm_desc d[2];
+    int n = 0;
+    const auto opt = at::TensorOptions().device(dev);
+    void* const st = stream_of(gq);
+    if (dx_code >= 0) {   // dX[T, K] = dY[T, N] . W[N, K]
+        dx = at::empty({T, K}, opt.dtype(type_of(dx_code)));
+        gemm_desc(&d[0], gq, fg, sg, dform & 4 ? w : tensor(p[7]), fw, sw, dx, T, K, N, dform & 4, false, false);
+        if (fp8_dx) {
+            PyObject* const role = p[16];
+            if (!PyTuple_Check(role) || PyTuple_GET_SIZE(role) != 3) stop(PyExc_TypeError, "the role of an fp8 gradient is a tuple of 3");
+            const int h = (int)number(PyTuple_GET_ITEM(role, 1)), margin = (int)number(PyTuple_GET_ITEM(role, 2));
+            float* const state = values(PyTuple_GET_ITEM(role, 0), dev, 1 + h);
+            d[0].d_dtype = (int)dx_code;
+            d[0].scale_d = state;
+            d[0].amax_workspace = workspace_of(gq, st);
+            call(ntfp8_gemm_fp8(&d[0], margin, state, state + 1, h, made.p, made.p + 1, st), "ntfp8_gemm_fp8");
+        } else {
+            ++n;
+        }
+    }
+    if (wants_dw) {       // dW[N, K] = dY[T, N]^T . X[T, K]
+        if (!accumulate) dw = at::empty({N, K}, opt.dtype(at::kFloat));
+        gemm_desc(&d[n++], wform & 8 ? gq : gq_t, fg, sg, wform & 4 ? x : tensor(p[3]), fx, sx, dw, N, K, T, wform & 4, wform & 8, accumulate);
+    }
+    if (n) call(ntfp8_gemm_batch(d, n, st), "ntfp8_gemm_batch");
+    if (!fp8_dx) return Py_BuildValue("(NNN)", wrap_or_none(std::move(db)), wrap_or_none(std::move(dx)), wrap_or_none(std::move(dw)));
+    return Py_BuildValue("(NNNNN)", wrap_or_none(std::move(db)), wrap(std::move(dx)), wrap_or_none(std::move(dw)), wrap(made.element(0)), wrap(made.element(1)));
 }
 
 // workspace(device index) -> (workspace, stream); workspace_pool(device index, count) -> ([>= count] workspaces, stream): what
@@ -514,7 +657,8 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
-                         NT_METHOD(operand_form, 10), NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
+                         NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 13), NT_METHOD(linear_backward, 21),
+                         NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -3,14 +3,16 @@ from typing import Optional, Tuple, TypedDict, Union
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.autograd import forward_ad
 
 from nanotron_amd import _native as nt
 from nanotron_amd.fp8.constants import INITIAL_AMAX, INITIAL_SCALING_FACTOR
 from nanotron_amd.fp8.dtypes import DTypes
+from nanotron_amd.fp8 import kernel as _kernel
 from nanotron_amd.fp8.kernel import a_transposed_supported, fp8_matmul_kernel, fp8_matmul_pair, needs_transposed_copy
 from nanotron_amd.fp8.meta import FP8Meta
 from nanotron_amd.fp8.parameter import FP8Parameter
-from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, cast_with_scale, update_scaling_factor
+from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, _assemble, cast_with_scale, update_scaling_factor
 
 
 class FP8LinearMeta(TypedDict):
@@ -132,7 +134,8 @@ class FP8Linear(nn.Linear):
         state = self.scaling["weight"] if self.scaling is not None else None
         if stream is None:
             w.data = FP8Tensor(hp, dtype=DTypes.FP8E4M3, state=state, with_transpose=needs_transposed_copy(*hp.shape))
-            self._weight_ready = None
+            if self._weight_ready is not None:
+                self._weight_ready = None
             return
         cur = torch.cuda.current_stream(hp.device)
         stream.wait_stream(cur)
@@ -210,6 +213,11 @@ class FP8Linear(nn.Linear):
             torch.cuda.current_stream(input.device).wait_event(self._weight_ready)
             self._weight_ready = None
 
+        if type(input) is torch.Tensor and not torch.is_grad_enabled() and _no_transform():
+            # nothing to record: the two kernels, past autograd's machinery
+            quick = _quantise_and_multiply(self, input, weight, self.bias, False)
+            if quick is not None:
+                return quick[0]
         # phony tensor that makes autograd call our backward although the weight's gradient is
         # produced by the fp8 kernels, not by autograd (linear.py:56-60)
         phony = torch.empty(0, device=input.device, requires_grad=True)
@@ -266,6 +274,15 @@ class _FP8Matmul(torch.autograd.Function):
         ctx.set_materialize_grads(False)   # a missing gradient arrives as None, not as a tensor filled with zeros
         ctx.has_handle = input_handle is not None
         ctx.input_box = getattr(input_handle, "_grad_box", None) if input_handle is not None else None
+        quick = _quantise_and_multiply(module, input, weight, bias, needs_wgrad) if plain and module is not None else None
+        if quick is not None:
+            output = quick[0]
+            ctx.save_for_backward(_assemble(FP8Tensor, DTypes.FP8E4M3, *quick[1:]), weight, bias)
+            ctx.module = module
+            ctx.fp8_meta = fp8_meta
+            ctx.fp8_out = False
+            ctx.out_shape, ctx.out_dtype = output.shape, output.dtype
+            return output, phony
         if plain:
             x2d = input if len(in_shape) == 2 else input.reshape(-1, in_shape[-1])
             input = FP8Tensor(x2d, dtype=DTypes.FP8E4M3, state=scaling["input"] if scaling else None,
@@ -288,7 +305,8 @@ class _FP8Matmul(torch.autograd.Function):
                 out_dtype=out_dtype, out_state=state, out_with_transpose=module.fp8_output_transpose, bias=gemm_bias,
             )
             ctx.mark_non_differentiable(output)
-            ctx.grad_box = module._grad_box = _GradBox(scaling["output_grad"] if scaling else None)
+            ctx.grad_box = _GradBox(scaling["output_grad"] if scaling else None)
+            object.__setattr__(module, "_grad_box", ctx.grad_box)   # (a plain value: nn.Module's own way takes 2 us)
             hp = weight.dtype if weight.dtype in (torch.float32, torch.float16, torch.bfloat16) else torch.float32
             out_shape = output.as_subclass(torch.Tensor).shape
             handle = module._zero(hp, weight.device).expand(out_shape)
@@ -334,6 +352,17 @@ class _FP8Matmul(torch.autograd.Function):
         if type(grad_output) is torch.Tensor and not grad_output.is_contiguous():
             grad_output = grad_output.contiguous()   # once: the bias gradient and the quantisation both read it whole
 
+        wants_dx = ctx.needs_input_grad[0] or (ctx.has_handle and ctx.needs_input_grad[6])
+        box = ctx.input_box if wants_dx else None
+        if box is not None:
+            box.arrivals += 1
+        fp8_dx = (box is not None and box.consumers == 1 and box.arrivals == 1 and box.state is not None
+                  and box.state.known_initialised and module is not None and module.fp8_grad_input)
+        if module is not None and not module.keep_quantised_grad:
+            quick = _backward_passes(ctx, module, grad_output, input, weight, bias, wants_dx, box if fp8_dx else None)
+            if quick is not None:
+                return quick
+
         grad_bias = None
         if bias is not None and ctx.needs_input_grad[5]:
             # what autograd does for `output + bias` (linear.py:65): the gradient summed over the tokens (in fp32)
@@ -360,27 +389,14 @@ class _FP8Matmul(torch.autograd.Function):
         if module is not None and module.keep_quantised_grad:
             module.quantised_grad_output = grad_output   # for checkers: the e5m2 operand of dgrad and wgrad
 
-        wants_dx = ctx.needs_input_grad[0] or (ctx.has_handle and ctx.needs_input_grad[6])
         grad_input = None
-        box = ctx.input_box if wants_dx else None
-        if box is not None:
-            box.arrivals += 1
-        fp8_dx = (box is not None and box.consumers == 1 and box.arrivals == 1 and box.state is not None
-                  and box.state.known_initialised and module is not None and module.fp8_grad_input)
         # dX[M,K] = dY[M,N] . W[N,K]
         dgrad = dict(mat_a=weight.data, transpose_a=False, mat_b=grad_output, transpose_b=False, use_split_accumulator=True,
                      out_dtype=ctx.in_dtype or torch.float32)
         wgrad, slot = None, None
         if weight.requires_grad:
-            # dW[N,K] = dY[M,N]^T . X[M,K].  The gradient is fp32 (kernel.py:24).  An fp32 parameter takes it as `.grad`
-            # (side effect, as linear.py:110); a 16-bit parameter cannot hold an fp32 `.grad`, so there it is kept
-            # beside the parameter as `.main_grad`, the fp32 master-gradient buffer an optimizer reads.
-            slot = "grad" if weight.dtype == torch.float32 else "main_grad"
-            acc = None
-            if module is not None and module.accumulate_grad:
-                prev = getattr(weight, slot, None)
-                if prev is not None and prev.dtype == torch.float32:
-                    acc = prev
+            # dW[N,K] = dY[M,N]^T . X[M,K].  The gradient is fp32 (kernel.py:24).
+            slot, acc = _gradient_slot(module, weight)
             wgrad = dict(mat_a=input, transpose_a=False, mat_b=grad_output, transpose_b=True, use_split_accumulator=True,
                          accumulate_into=acc)
         grad_weight = None
@@ -409,6 +425,96 @@ class _FP8Matmul(torch.autograd.Function):
         if ctx.has_handle:   # the input was an fp8 activation: its gradient goes to the handle that stands for it
             return None, None, None, None, None, grad_bias, grad_input
         return grad_input, None, None, None, None, grad_bias, None
+
+
+def _no_transform() -> bool:
+    """No transform is active that has to see the autograd function of a layer although gradients are off: forward-mode
+    differentiation, functorch's, tracing."""
+    return (forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None)
+
+
+def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, needs_wgrad: bool):
+    """(Y, input bytes, their transposed copy, amax, scale) of a layer's forward pass through one native call, with the results
+    of FP8Tensor(x, ...) and fp8_matmul_kernel; None where it does not serve the case, nothing done."""
+    out_code = nt.TORCH_TO_NT.get(module.out_dtype or torch.float32)
+    if out_code is None or not isinstance(weight, FP8Parameter):
+        return None
+    buf, history_len, margin, held = None, 0, 0, False
+    if module.scaling is not None:
+        state = module.scaling["input"]
+        if not state.known_initialised or state.dtype is not DTypes.FP8E4M3:
+            return None
+        buf, history_len, margin, held = state._buf, state.history_len, state.margin, not module.training
+    w = weight.data
+    meta = w.fp8_meta
+    return nt.host.linear_forward(x, nt.E4M3, margin, buf, history_len, held, needs_wgrad, _kernel.READ_B_TRANSPOSED, w,
+                                  meta.dtype.code, meta.scale, bias, out_code)
+
+
+def _backward_passes(ctx, module: FP8Linear, grad_output, input: FP8Tensor, weight, bias, wants_dx: bool, box: Optional[_GradBox]):
+    """What `_FP8Matmul._backward` returns, through one native call (bias gradient, quantisation of dY, dgrad and wgrad) with the
+    results of the pieces it is put together from; None where that does not serve the case, nothing done.  `box`: dX leaves as
+    e5m2 bytes under the role of the layer that made the input."""
+    if not isinstance(weight, FP8Parameter):
+        return None
+    buf, history_len, margin, g_scale = None, 0, 0, None
+    if type(grad_output) is FP8Tensor:
+        if grad_output.__dict__.get("_transposed") is not None or grad_output.fp8_meta.dtype is not DTypes.FP8E5M2:
+            return None
+        g_scale = grad_output.fp8_meta.scale
+    elif type(grad_output) is not torch.Tensor:
+        return None
+    elif module.scaling is not None:
+        state = module.scaling["output_grad"]
+        if not state.known_initialised or state.dtype is not DTypes.FP8E5M2:
+            return None
+        buf, history_len, margin = state._buf, state.history_len, state.margin
+    bias_code, dx_code, role = -1, -1, None
+    if bias is not None and ctx.needs_input_grad[5]:
+        bias_code = nt.TORCH_TO_NT.get(bias.dtype)
+    if box is not None:
+        if box.state.dtype is not DTypes.FP8E5M2:
+            return None
+        dx_code, role = nt.OUT_E5M2, (box.state._buf, box.state.history_len, box.state.margin)
+    elif wants_dx:
+        dx_code = nt.TORCH_TO_NT.get(ctx.in_dtype or torch.float32)
+    if bias_code is None or dx_code is None:
+        return None
+    wants_dw, slot, acc = weight.requires_grad, None, None
+    if wants_dw:
+        slot, acc = _gradient_slot(module, weight)
+    w = weight.data
+    mx, mw = input.fp8_meta, w.fp8_meta
+    res = nt.host.linear_backward(grad_output, g_scale, input, getattr(input, "_transposed", None), mx.dtype.code, mx.scale, w,
+                                  getattr(w, "_transposed", None), mw.dtype.code, mw.scale, nt.E5M2, margin, buf, history_len,
+                                  bias_code, dx_code, role, wants_dw, acc, _kernel.READ_B_TRANSPOSED, _kernel.READ_A_TRANSPOSED)
+    if res is None:
+        return None
+    grad_bias, grad_input, grad_weight = res[:3]
+    if box is not None:
+        box.fp8_grad = _assemble(FP8Tensor, DTypes.FP8E5M2, grad_input, None, *res[3:])
+        grad_input = module._zero(ctx.in_dtype or torch.float32, weight.device).expand(ctx.in_shape)
+        object.__setattr__(module, "fp8_grad_inputs_sent", module.fp8_grad_inputs_sent + 1)
+    if grad_input is not None and len(ctx.in_shape) != 2:
+        grad_input = grad_input.reshape(ctx.in_shape)
+    if grad_weight is not None:
+        setattr(weight, slot, grad_weight)
+    if ctx.has_handle:   # the input was an fp8 activation: its gradient goes to the handle that stands for it
+        return None, None, None, None, None, grad_bias, grad_input
+    return grad_input, None, None, None, None, grad_bias, None
+
+
+def _gradient_slot(module: Optional[FP8Linear], weight):
+    """(attribute that holds the fp32 weight gradient, the gradient to add to or None).  An fp32 parameter takes it as `.grad`
+    (side effect, as src/nanotron/fp8/linear.py:110); a 16-bit parameter cannot hold an fp32 `.grad`, so there it is kept beside
+    the parameter as `.main_grad`, the fp32 master-gradient buffer an optimizer reads."""
+    slot = "grad" if weight.dtype == torch.float32 else "main_grad"
+    if module is not None and module.accumulate_grad:
+        prev = getattr(weight, slot, None)
+        if prev is not None and prev.dtype == torch.float32:
+            return slot, prev
+    return slot, None
 
 
 def _frozen_copy(state: DelayedScaling) -> DelayedScaling:

@@ -51,7 +51,8 @@ def requantize_fp8_weights(module_or_modules, stream: Optional[torch.cuda.Stream
                                             [needs_transposed_copy(*w.shape) for w in hp])
             for lin, q in zip(lins, qs):
                 lin.weight.data = q
-                lin._weight_ready = None
+                if lin._weight_ready is not None:
+                    lin._weight_ready = None
     for lin in rest:
         lin.requantize_weight(stream=stream)
     return len(layers)

@@ -1,0 +1,147 @@
+"""A layer's passes through one native call each against the same passes put together from their pieces: outputs, gradients,
+fp8 bytes and scaling states bit for bit, over the forms that the operands take (read as they are, transposed copies, any
+sizes), and the calls that must not take the short way."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+from nanotron_amd.fp8 import DTypes, FP8Linear, FP8Parameter
+from nanotron_amd.fp8 import linear as L
+
+
+def _run(x, gys, dtype, out, bias, delayed, accumulate, dims, pieces, monkeypatch, offset=0):
+    if pieces:
+        monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
+        monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+    K, N = x.shape[-1], gys[0].shape[-1]
+    g = torch.Generator(device="cuda").manual_seed(3)
+    lin = FP8Linear(K, N, bias, "cuda", dtype=dtype, out_dtype=out, delayed_scaling=delayed, accumulate_grad=accumulate)
+    lin.weight = FP8Parameter((torch.randn(N, K, generator=g, device="cuda") * 0.02).to(dtype), DTypes.FP8E4M3)
+    if bias:
+        lin.bias.data.copy_(torch.randn(N, generator=g, device="cuda") * 0.02)
+    got = []
+    for gy in gys:
+        xg = torch.empty(x.numel() + offset, dtype=dtype, device="cuda")[offset:].view(x.shape).copy_(x).requires_grad_(True)
+        y = lin(xg)
+        saved = y.grad_fn.saved_tensors[0]
+        got += [y.detach().clone(), saved.as_subclass(torch.Tensor).clone(), saved.fp8_meta.scale.clone()]
+        y.backward(gy)
+        torch.cuda.synchronize()
+        got += [xg.grad, (lin.weight.grad if dtype == torch.float32 else lin.weight.main_grad).clone()]
+        if bias:
+            got.append(lin.bias.grad.clone())
+            lin.bias.grad = None
+        if delayed:
+            got += [r._buf.clone() for r in lin.scaling.values()]
+    lin.eval()
+    with torch.no_grad():
+        got.append(lin(x))
+    got.append(lin(x).detach())
+    if delayed:
+        got += [r._buf.clone() for r in lin.scaling.values()]
+    monkeypatch.undo()
+    return got
+
+CASES = [
+    # tokens, K, N, dtype, out, bias, delayed, accumulate, dims
+    (128, 128, 128, torch.float32, None, True, False, False, 2),
+    (256, 144, 272, torch.bfloat16, torch.bfloat16, True, True, True, 2),
+    (512, 256, 384, torch.bfloat16, torch.float32, False, True, True, 3),
+    (1021, 256, 320, torch.float16, torch.float16, True, True, False, 2),
+    (77, 130, 91, torch.float32, torch.float32, True, True, True, 3),
+    (96, 515, 601, torch.float16, torch.float16, False, False, True, 2),
+    (1, 64, 48, torch.bfloat16, torch.bfloat16, True, False, False, 1),
+    (300, 256, 264, torch.bfloat16, torch.bfloat16, False, True, False, 2),
+]
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("tokens,K,N,dtype,out,bias,delayed,accumulate,dims", CASES)
+def test_same_as_the_pieces(tokens, K, N, dtype, out, bias, delayed, accumulate, dims, offset, monkeypatch):
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    lead = {1: (), 2: (tokens,), 3: (1, tokens)}[dims]
+    x = torch.randn(*lead, K, generator=g, device="cuda").to(dtype)
+    gys = [(torch.randn(*lead, N, generator=g, device="cuda") * 1e-3).to(out or torch.float32) for _ in range(4)]
+    if tokens == 300:   # a strided gradient
+        gys = [torch.stack([t, t], -1)[..., 0] for t in gys]
+    args = (x, gys, dtype, out, bias, delayed, accumulate, dims)
+    short = _run(*args, False, monkeypatch, offset)
+    pieces = _run(*args, True, monkeypatch, offset)
+    assert len(short) == len(pieces)
+    for i, (a, b) in enumerate(zip(short, pieces)):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
+
+@pytest.mark.gpu
+def test_frozen_weight_and_input_without_gradient(monkeypatch):
+    x = torch.randn(256, 256, device="cuda", dtype=torch.bfloat16)
+    gy = torch.randn(256, 384, device="cuda", dtype=torch.bfloat16)
+    for frozen in (False, True):
+        res = []
+        for pieces in (False, True):
+            if pieces:
+                monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+            torch.manual_seed(0)
+            lin = FP8Linear(256, 384, True, "cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16)
+            lin.weight.requires_grad_(not frozen)
+            xg = x.clone().requires_grad_(frozen)
+            lin(xg).backward(gy)
+            assert (xg.grad is None) == (not frozen) and (getattr(lin.weight, "main_grad", None) is None) == frozen
+            res.append([xg.grad if frozen else lin.weight.main_grad, lin.bias.grad])
+            monkeypatch.undo()
+        assert all(torch.equal(a, b) for a, b in zip(*res))
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,dims,bias", [(512, (256, 384, 272), False), (300, (256, 320, 272), False), (258, (272, 320, 256), True), (64, (128, 96, 112), False)])
+def test_chain_same_as_the_pieces(tokens, dims, bias, monkeypatch):
+    """fp8 activations forward and e5m2 gradients back, at sizes that are read as they are and others."""
+    res = []
+    for pieces in (False, True):
+        if pieces:
+            monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
+            monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+        g = torch.Generator(device="cuda").manual_seed(tokens)
+        lins = []
+        for i, (a, b) in enumerate(zip(dims, dims[1:])):
+            lin = FP8Linear(a, b, bias, "cuda", dtype=torch.bfloat16, out_dtype=DTypes.FP8E4M3 if i == 0 else torch.bfloat16, delayed_scaling=True)
+            lin.weight = FP8Parameter((torch.randn(b, a, generator=g, device="cuda") * 0.05).to(torch.bfloat16), DTypes.FP8E4M3)
+            if bias:
+                lin.bias.data.zero_()
+            lins.append(lin)
+        got = []
+        for step in range(3):
+            x = torch.randn(tokens, dims[0], generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True)
+            h = x
+            for lin in lins:
+                h = lin(h)
+            h.backward((torch.randn(tokens, dims[-1], generator=g, device="cuda") * 1e-3).to(torch.bfloat16))
+            torch.cuda.synchronize()
+            got += [h.detach(), x.grad] + [lin.weight.main_grad for lin in lins] + [r._buf.clone() for lin in lins for r in lin.scaling.values()]
+            if bias:
+                got += [lin.bias.grad.clone() for lin in lins]
+        got.append(torch.tensor([lin.fp8_grad_inputs_sent for lin in lins]))
+        res.append(got)
+        monkeypatch.undo()
+    for i, (a, b) in enumerate(zip(*res)):
+        assert torch.equal(a, b), i
+
+
+@pytest.mark.gpu
+def test_saved_tensor_hooks_see_what_a_layer_saves():
+    lin = FP8Linear(256, 256, False, "cuda", out_dtype=torch.float32)
+    x = torch.randn(256, 256, device="cuda", requires_grad=True)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+        y = lin(x)
+    assert any(t.dtype == torch.uint8 and t.shape == x.shape for t in packed)
+    with pytest.raises(AssertionError, match="FP8Tensors"):   # hooks hand back the weight's storage, not the parameter
+        y.sum().backward()
+
+
+def test_transforms_are_seen():
+    assert L._no_transform()
+    with forward_ad.dual_level():
+        assert not L._no_transform()
+    seen = []
+    torch.func.vmap(lambda t: seen.append(L._no_transform()) or t)(torch.zeros(2))
+    torch.jit.trace(lambda t: seen.append(L._no_transform()) or t + 1, torch.zeros(2), check_trace=False)
+    assert seen == [False, False] and L._no_transform()
