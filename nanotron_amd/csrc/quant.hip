@@ -220,7 +220,9 @@ __device__ __forceinline__ void store_chunk(uint8_t* __restrict__ p, const uint3
 
 // Streams a tensor of n elements, n_vec whole 16-byte chunks of it as vectors: `body(v, m, index)` for every chunk,
 // `one(x, m, index)` for elements past them (all of them where a pointer is misaligned).
-template <typename S, typename Body, typename One>
+// kOne: one chunk for every thread is all there is (a kernel of its own: small tensors are bound by latency, which code read
+// from memory is part of).
+template <typename S, bool kOne, typename Body, typename One>
 __device__ __forceinline__ void for_each_chunk(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n, uint32_t bid,
                                                uint32_t nblocks, Body body, One one) {
     typedef Src<S> L;
@@ -240,15 +242,20 @@ __device__ __forceinline__ void for_each_chunk(const typename ElemOf<S>::type* _
         for (int k = 0; k < G * U; ++k) body(v[k], m[k], index(k));
         g += (int64_t)G * nblocks;
     };
-    while (g + nblocks < full) spans(std::integral_constant<int, 2>{});
-    if (g < full) spans(std::integral_constant<int, 1>{});
-    if (g == full) {   // what is left of the last span: one workgroup's
-        for (int64_t c = full * kSpan<S> + threadIdx.x; c < n_vec; c += kFlatThreads) {
-            float v[E];
-            uint32_t m;
-            L::template load<E, true>(x + c * E, v, m);
-            body(v, m, c * E);
-        }
+    auto chunk = [&](int64_t c) {
+        float v[E];
+        uint32_t m;
+        L::template load<E, true>(x + c * E, v, m);
+        body(v, m, c * E);
+    };
+    if constexpr (kOne) {
+        const int64_t c = (int64_t)bid * kFlatThreads + threadIdx.x;
+        if (c < n_vec) chunk(c);
+    } else {
+        while (g + nblocks < full) spans(std::integral_constant<int, 2>{});
+        if (g < full) spans(std::integral_constant<int, 1>{});
+        if (g == full)   // what is left of the last span: one workgroup's
+            for (int64_t c = full * kSpan<S> + threadIdx.x; c < n_vec; c += kFlatThreads) chunk(c);
     }
     for (int64_t j = n_vec * E + (int64_t)bid * kFlatThreads + threadIdx.x; j < n; j += (int64_t)nblocks * kFlatThreads) {
         uint32_t m;
@@ -260,11 +267,21 @@ __device__ __forceinline__ void for_each_chunk(const typename ElemOf<S>::type* _
 // max|x| alone: 16 elements per lane in a row and ordinary loads (the first touches every line, the others find it in the
 // cache; and the pass that follows finds lines in the memory-side cache).  fp32 11008 x 4096, 16 elements in a row / side by
 // side: 32.2 / 33.1 us.
-template <typename S>
+template <typename S, bool kOne>
 __device__ __forceinline__ uint32_t flat_max(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n, uint32_t bid,
                                              uint32_t nblocks) {
     typedef Src<S> L;
     uint32_t m_run = 0;
+    if constexpr (kOne) {
+        constexpr int E = kChunk<S>;
+        const int64_t c = (int64_t)bid * kFlatThreads + threadIdx.x;
+        float v[E];
+        uint32_t m = 0;
+        if (c < n_vec) L::template load<E, false>(x + c * E, v, m);
+        const int64_t j = n_vec * E + c;   // fewer than E elements past the chunks
+        if (j < n) (void)L::load1(x + j, m_run);
+        return m > m_run ? m : m_run;
+    }
     n_vec /= kVec / kChunk<S>;
     const int64_t stride = (int64_t)nblocks * kFlatThreads;
     int64_t i = (int64_t)bid * kFlatThreads + threadIdx.x;
@@ -290,7 +307,7 @@ __device__ __forceinline__ uint32_t flat_max(const typename ElemOf<S>::type* __r
     return m_run;
 }
 
-template <typename S, int F, int MODE>
+template <typename S, int F, int MODE, bool kOne = false>
 __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* __restrict__ x, int64_t n_vec, int64_t n,
                                                 uint8_t* __restrict__ out, const float* __restrict__ scale_ptr,
                                                 Workspace* ws, const ScalarIO& io, uint32_t bid, uint32_t nblocks) {
@@ -309,9 +326,9 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     if constexpr (kAmax) pre = prefetch_epilogue(io, MODE);
     uint32_t m_run = 0;  // in source-format bits
     if constexpr (!kCast) {
-        m_run = flat_max<S>(x, n_vec, n, bid, nblocks);
+        m_run = flat_max<S, kOne>(x, n_vec, n, bid, nblocks);
     } else {
-        for_each_chunk<S>(
+        for_each_chunk<S, kOne>(
             x, n_vec, n, bid, nblocks,
             [&](const float(&v)[E], uint32_t m, int64_t at) {
                 if constexpr (kAmax) m_run = m > m_run ? m : m_run;
@@ -327,12 +344,12 @@ __device__ __forceinline__ void quant_flat_body(const typename ElemOf<S>::type* 
     if constexpr (kAmax) publish_and_finalize<kFlatThreads>(L::to_f32_bits(m_run), ws, io, MODE, pre, bid, nblocks);
 }
 
-template <typename S, int F, int MODE>
+template <typename S, int F, int MODE, bool kOne>
 __global__ __launch_bounds__(kFlatThreads) void quant_flat_kernel(const typename ElemOf<S>::type* __restrict__ x,
                                                               int64_t n_vec, int64_t n, uint8_t* __restrict__ out,
                                                               const float* __restrict__ scale_ptr, Workspace* ws,
                                                               ScalarIO io) {
-    quant_flat_body<S, F, MODE>(x, n_vec, n, out, scale_ptr, ws, io, blockIdx.x, gridDim.x);
+    quant_flat_body<S, F, MODE, kOne>(x, n_vec, n, out, scale_ptr, ws, io, blockIdx.x, gridDim.x);
 }
 
 // One source tensor, both formats, one pass: the fused delayed-scaling step of an e4m3 role and an e5m2 role that
@@ -350,7 +367,7 @@ __global__ __launch_bounds__(kFlatThreads) void quant_flat_dual_kernel(const typ
     const EpiloguePrefetch pre1 = prefetch_epilogue(io1, kModeDelayed);
     uint32_t m_run = 0;
     constexpr int E = kChunk<S>;
-    for_each_chunk<S>(
+    for_each_chunk<S, false>(
         x, n_vec, n, blockIdx.x, gridDim.x,
         [&](const float(&v)[E], uint32_t m, int64_t at) {
             m_run = m > m_run ? m : m_run;
@@ -987,29 +1004,36 @@ static int grid_for(int64_t work_items, int threads = kThreads, int per_cu_block
 static void clear_stale_error() { (void)hipGetLastError(); }
 static int check_launch() { return hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH; }
 
-// workgroups of the flat kernels: two spans each until there is one workgroup per CU
+// Workgroups of the flat kernels: two spans each until there is one workgroup per CU; for a tensor by itself one span each as
+// long as there are CUs for that.
 template <typename S>
-static int flat_grid(int64_t n_vec, int64_t n) {
-    return grid_for(n_vec > 0 ? (n_vec + 2 * kVec / kChunk<S> - 1) / (2 * kVec / kChunk<S>) : n, kFlatThreads, 1);
+static int flat_grid(int64_t n_vec, int64_t n, bool alone = false) {
+    if (n_vec == 0) return grid_for(n, kFlatThreads, 1);
+    const int64_t spans = (n_vec + kSpan<S> - 1) / kSpan<S>, cus = cu_count();
+    return (int)(alone && spans <= cus ? spans : std::min((spans + 1) / 2, cus));
 }
 
+// A chunk for every thread where that is no more than a workgroup per CU.  us, spans / chunks: bf16 16 x 4096 cast 2.9 / 2.4, delayed
+// step 5.2 / 4.0; 1024 x 2048 3.6 / 2.9 and 6.2 / 5.2; fp32 512 x 1024 3.6 / 2.4 and 6.7 / 4.7, current scaling 8.9 / 7.0.  Beyond,
+// one span a workgroup instead of two: bf16 2048 x 2048 delayed step 6.7 / 6.0, fp32 7.8 / 7.1.
+template <typename S, int F, bool kOne>
+static int launch_flat_grid(int grid, int mode, const typename ElemOf<S>::type* x, int64_t n_vec, int64_t n, uint8_t* out, const float* scale_ptr,
+                            Workspace* ws, const ScalarIO& io, hipStream_t st) {
+#define NT_FLAT(M) hipLaunchKernelGGL((quant_flat_kernel<S, F, M, kOne>), dim3(grid), dim3(kFlatThreads), 0, st, x, n_vec, n, out, scale_ptr, ws, io)
+    if (mode == kModeAmaxOnly) NT_FLAT(kModeAmaxOnly);
+    else if (mode == kModeCastOnly) NT_FLAT(kModeCastOnly);
+    else NT_FLAT(kModeDelayed);
+#undef NT_FLAT
+    return check_launch();
+}
 template <typename S, int F>
 static int launch_flat(int mode, const void* x, int64_t n, bool vec_ok, uint8_t* out, const float* scale_ptr,
                        Workspace* ws, const ScalarIO& io, hipStream_t st) {
-    typedef typename ElemOf<S>::type E;
     const int64_t n_vec = vec_ok ? n / kChunk<S> : 0;
-    const int grid = flat_grid<S>(n_vec, n);
-    const E* xp = static_cast<const E*>(x);
-    if (mode == kModeAmaxOnly)
-        hipLaunchKernelGGL((quant_flat_kernel<S, F, kModeAmaxOnly>), dim3(grid), dim3(kFlatThreads), 0, st, xp, n_vec, n, out,
-                           scale_ptr, ws, io);
-    else if (mode == kModeCastOnly)
-        hipLaunchKernelGGL((quant_flat_kernel<S, F, kModeCastOnly>), dim3(grid), dim3(kFlatThreads), 0, st, xp, n_vec, n, out,
-                           scale_ptr, ws, io);
-    else
-        hipLaunchKernelGGL((quant_flat_kernel<S, F, kModeDelayed>), dim3(grid), dim3(kFlatThreads), 0, st, xp, n_vec, n, out,
-                           scale_ptr, ws, io);
-    return check_launch();
+    const typename ElemOf<S>::type* xp = static_cast<const typename ElemOf<S>::type*>(x);
+    if (n_vec > 0 && n_vec <= (int64_t)cu_count() * kFlatThreads)
+        return launch_flat_grid<S, F, true>(grid_for(n_vec, kFlatThreads, 1), mode, xp, n_vec, n, out, scale_ptr, ws, io, st);
+    return launch_flat_grid<S, F, false>(flat_grid<S>(n_vec, n, true), mode, xp, n_vec, n, out, scale_ptr, ws, io, st);
 }
 
 // Columns per thread (16: 128-wide tiles, 4: 64-wide) of the kernels that turn tiles around, and their tile count: 128-wide

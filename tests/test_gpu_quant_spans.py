@@ -46,7 +46,7 @@ def _check(x, fmt, transpose, offset=0):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n", [4 * SPAN + 1, 5 * SPAN - 1, 7 * SPAN + 8 * 37 + 3, 2 * CUS * SPAN - 4, (2 * CUS + 1) * SPAN + 5])
+@pytest.mark.parametrize("n", [9, 1024 * 8, 1024 * 8 + 7, 66000, CUS * 4096 + 3, CUS * 8192, CUS * 8192 + 8, 4 * SPAN + 1, 5 * SPAN - 1, 7 * SPAN + 8 * 37 + 3, 2 * CUS * SPAN - 4, (2 * CUS + 1) * SPAN + 5])
 def test_flat_spans(n, dtype):
     _check(_tensor((1, n), dtype, n), "e4m3" if n % 2 else "e5m2", False)
 
