@@ -149,13 +149,14 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* 
 
 // A few rows against a weight whose columns the 64-wide tiles spread over few CUs (gemm_few.h).  The lines, us in 64-wide
 // tiles / there, weights not in a cache:
-//   16 rows, N x K:  4096 x 1024 4.7 / 4.9     1024 x 2048 5.8 / 5.4     4096 x 2048 7.5 / 6.0     5120 x 2048 7.7 / 7.7
-//                    6144 x 3072 9.7 / 9.3     8192 x 4096 13.6 / 12.2   14336 x 4096 15.3 / 16.8 (in 64 columns)
-//   32 rows:         1024 x 4096 8.3 / 8.9     2048 x 6144 15.7 / 13.4   4096 x 14336 31.9 / 24.3   5120 x 5120 14.8 / 17.2
+//   16 rows, N x K:  4096 x 1024 4.5 / 4.6     4096 x 1536 5.2 / 4.9     5120 x 1536 5.2 / 5.7     8192 x 1536 6.5 / 6.8
+//                    4096 x 2048 7.5 / 5.0     6144 x 3072 9.7 / 7.5     8192 x 4096 13.6 / 10.0   10240 x 4096 12.5 / 15.0
+//   32 rows:         4096 x 2048 6.0 / 6.6     2048 x 3072 7.0 / 6.9     4096 x 4096 11.5 / 9.1    5120 x 4096 11.2 / 15.3
+//                    4096 x 14336 31.9 / 21.7  5120 x 14336 31.5 / 39.5
 static bool few_rows(const GemmDesc& g) {
     if (g.M > 32 || g.tb || is_fp8_out(g.d_dtype)) return false;
-    if (g.M <= 16) return g.K >= 2048 && g.N <= 32 * cu_count();
-    return g.K >= 6144 && g.N <= 16 * cu_count();
+    if (g.M <= 16) return (g.K >= 2048 && g.N <= 32 * cu_count()) || (g.K >= 1024 && g.N <= 16 * cu_count());
+    return g.K >= 3072 && g.N <= 16 * cu_count();
 }
 
 // Bookkeeping of an fp8 output by the workgroup that finishes last, where the launch is one round of workgroups; behind more
