@@ -434,13 +434,15 @@ def _no_transform() -> bool:
             and torch._C._get_tracing_state() is None)
 
 
-_FP8TENSOR_NEW = FP8Tensor.__new__
+_PIECES = (FP8Tensor.__new__, _kernel._gemm_nt, _kernel._gemm_nt_batch, _kernel._gemm_nt_fp8)
 
 
 def _watched() -> bool:
-    """FP8Tensor's constructor has been replaced, by something that watches or changes quantisations: the passes have to go
-    through it."""
-    return FP8Tensor.__new__ is not _FP8TENSOR_NEW
+    """One of the pieces that quantise or multiply has been replaced, by something that watches, times or changes it: the
+    passes have to go through them."""
+    new, one, batch, fp8 = _PIECES
+    return (FP8Tensor.__new__ is not new or _kernel._gemm_nt is not one or _kernel._gemm_nt_batch is not batch
+            or _kernel._gemm_nt_fp8 is not fp8)
 
 
 def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, needs_wgrad: bool):
