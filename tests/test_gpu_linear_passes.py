@@ -145,3 +145,21 @@ def test_transforms_are_seen():
     torch.func.vmap(lambda t: seen.append(L._no_transform()) or t)(torch.zeros(2))
     torch.jit.trace(lambda t: seen.append(L._no_transform()) or t + 1, torch.zeros(2), check_trace=False)
     assert seen == [False, False] and L._no_transform()
+
+
+@pytest.mark.parametrize("name", ["_gemm_nt", "_gemm_nt_batch", "_gemm_nt_fp8"])
+def test_replaced_pieces_are_seen(name, monkeypatch):
+    from nanotron_amd.fp8 import kernel as K
+    from nanotron_amd.fp8 import FP8Tensor
+
+    assert not L._watched()
+    monkeypatch.setattr(K, name, lambda *a, **k: None)
+    assert L._watched()
+    monkeypatch.undo()
+    orig = FP8Tensor.__new__
+    FP8Tensor.__new__ = lambda *a, **k: orig(*a, **k)
+    try:
+        assert L._watched()
+    finally:
+        FP8Tensor.__new__ = orig
+    assert not L._watched()
