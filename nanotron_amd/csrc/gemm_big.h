@@ -638,15 +638,18 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             back_w(No{}, No{}, f);
         } else {
         // ---- half tiles ------------------------------------------------------------------------------
-        //   front(kt): entered with fa[] = the tile's A fragments and fb[0], fb[1] = its first two B fragments; streams B
-        //              fragments 2..7; ends with the barrier that publishes tile kt + 1 and releases the stage of tile kt.
+        //   front(kt): entered with fa[] = the tile's A fragments and fb[0], fb[1] = its first two B fragments; reads B
+        //              fragments 2..7 three groups ahead of their use; ends with the barrier that publishes tile kt + 1 and
+        //              releases the stage of tile kt.
         //   back(kt):  refills fa[] / fb[0], fb[1] from tile kt + 1.
-        // The stage released by the barrier of tile kt is refilled with tile kt + NS between that barrier and the next:
-        // half of the loads under back(kt), the rest under groups 0-1 of front(kt + 1).
+        // The stage released by the barrier of tile kt is refilled with tile kt + NS between that barrier and the next, the
+        // loads spread over back(kt) and front(kt + 1): twelve of them within 16 MFMAs, and fragment 7 read behind the last group
+        // but one, cost 3 % (us, 4096 x 2048 x 4096 in 256 half tiles 29.4 / 28.4; backward of 4096 tokens, 1024 -> 4096,
+        // 36.9 / 35.8).
         v4i fb[4][2];
-        constexpr int kBackLoads = NL / 2;
-        constexpr int kFrontLoads = NL - kBackLoads;   // half under group 0, half under group 1
-        // loads: queue the second half of tile kt + NS - 1; WAIT (>= 0): barrier, after all but the newest WAIT
+        constexpr int kBackLoads = NL / 3;
+        constexpr int kFrontLoads = NL - kBackLoads;
+        // loads: queue the rest of tile kt + NS - 1; WAIT (>= 0): barrier, after all but the newest WAIT
         // loads of this wave have landed (-1: no barrier)
         auto front = [&](auto loads_tag, auto wait_tag, int kt) {
             constexpr bool loads = decltype(loads_tag)::value;
@@ -655,16 +658,17 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             sched_fence();
 #pragma unroll
             for (int j = 0; j < 6; ++j) {
-                int l = kBackLoads + j * (kFrontLoads / 2);           // next load to queue
-                const int lend = (loads && j < 2) ? l + kFrontLoads / 2 : l;
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
                     mma(i, j, frag(fb[j & 3]), frag(fa[i]));
-                    if (i == 0) fb[(j + 2) & 3][0] = rd_b(s, j + 2, 0);
-                    else if (i == 2) fb[(j + 2) & 3][1] = rd_b(s, j + 2, 1);
-                    else if (l < lend) issue(kt + NS - 1, l++);
-                    if (i == MI - 1) {   // whatever did not get a slot of its own
-                        for (; l < lend; ++l) issue(kt + NS - 1, l);
+                    // B fragment j + 3 (behind group 0 fragments 2 and 3), so that none is on its way at the barrier
+                    if (i < 2 && j < 5) fb[(j + (j ? 3 : 2)) & 3][i] = rd_b(s, j + (j ? 3 : 2), i);
+                    else if (j == 0) fb[3][i - 2] = rd_b(s, 3, i - 2);
+                    if (loads && j > 0 && i >= 2) {   // slot x of n
+                        constexpr int n = 5 * (MI - 2);
+                        const int x = (j - 1) * (MI - 2) + i - 2;
+#pragma unroll
+                        for (int l = kBackLoads + x * kFrontLoads / n; l < kBackLoads + (x + 1) * kFrontLoads / n; ++l) issue(kt + NS - 1, l);
                     }
                     sched_fence();
                 }
