@@ -58,8 +58,10 @@ __global__ __launch_bounds__(kFewThreads) void gemm_few_kernel(const BigProblem 
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < kAhead; ++s) request(s, wave + s * kFewWaves);
-    sched_fence();
+    for (int s = 0; s < kAhead; ++s) {
+        request(s, wave + s * kFewWaves);
+        sched_fence();   // the wait below counts loads: those of a slot have to be older than the next slot's
+    }
     const float alpha = descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);   // (behind the first requests)
     const int rd0 = lds_off16(row, q), rd1 = lds_off16(row, q + 4);
     for (int kt = wave; kt < KT; kt += kAhead * kFewWaves) {
