@@ -437,13 +437,16 @@ PyObject* dequantize(PyObject* const* a) {
     return wrap(std::move(out));
 }
 
+at::Tensor turned(const at::Tensor& q) {   // contiguous bytes [rows, cols] -> [cols, rows]
+    at::Tensor out = bytes_like(q, {q.size(1), q.size(0)});
+    if (q.numel()) call(ntfp8_transpose(q.data_ptr(), q.size(0), q.size(1), out.data_ptr(), stream_of(q)), "ntfp8_transpose");
+    return out;
+}
 // transpose([rows, cols] bytes) -> contiguous [cols, rows] bytes
 PyObject* transpose(PyObject* const* a) {
     const at::Tensor q = codes(operand(a[0]));
     require(q.dim() == 2, "a 2-D tensor is expected");
-    at::Tensor out = bytes_like(q, {q.size(1), q.size(0)});
-    if (q.numel()) call(ntfp8_transpose(q.data_ptr(), q.size(0), q.size(1), out.data_ptr(), stream_of(q)), "ntfp8_transpose");
-    return wrap(std::move(out));
+    return wrap(turned(q));
 }
 
 // Whether the library reads B [K, N] (and, in the second form, A [K, M] as well) from its transpose: include/ntfp8.h
@@ -532,8 +535,10 @@ PyObject* linear_forward(PyObject* const* p) {
 // linear_backward(dY, its scale where it is fp8 bytes | None, input bytes, their transposed copy | None, fmt, scale, weight bytes, their
 // transposed copy | None, fmt, scale, gradient fmt, margin, state | None, history_len, bias code | -1, dX code | -1, (state,
 // history_len, margin) of an fp8 dX | None, wants dW, dW to accumulate into | None, read_b, read_a) -> (bias gradient | None,
-// dX | None, dW | None[, amax, scale of an fp8 dX]) | None: bias gradient, quantisation of dY (current scaling or the fused
-// delayed-scaling step), dX = dY . W and dW = dY^T . X
+// dX | None, dW | None, input bytes^T | None, weight bytes^T | None[, amax, scale of an fp8 dX]) | None: bias gradient,
+// quantisation of dY (current scaling or the fused delayed-scaling step), dX = dY . W and dW = dY^T . X.  Transposed copies that
+// a GEMM needs and nobody has made (a weight that more tokens would read as it is) are made here, and the caller is
+// given those of the input and the weight, to keep beside them.
 PyObject* linear_backward(PyObject* const* p) {
     const at::Tensor &grad = tensor(p[0]), &x = tensor(p[2]), &w = tensor(p[6]);
     const bool quantised_already = !none(p[1]);
@@ -558,9 +563,7 @@ PyObject* linear_backward(PyObject* const* p) {
     // the forms of the two GEMMs (bytes that are yet to be made are fresh allocations: aligned), before anything is launched
     const bool with_t = !quantised_already && wants_dw && !(!has_xt && read_a && read_b && N % 16 == 0 && reads_b(N, K, T));
     const int dform = dx_code < 0 ? 0 : form_dgrad(readable(w, has_wt, read_b && !(fp8_dx && T % 4)), N, K, T);
-    if ((dform & 2) && !has_wt) Py_RETURN_NONE;
     const int wform = !wants_dw ? 0 : form_wgrad(readable(x, has_xt, read_b) && (!accumulate || aligned16(dw)), T, K, N, !with_t, read_a, true);
-    if (((wform & 2) && !has_xt) || ((wform & 1) && !with_t)) Py_RETURN_NONE;
     const int hist = (int)number(p[13]), fx = (int)number(p[4]), fw = (int)number(p[8]), fg = (int)number(p[10]);
     const float *sx = values(p[5], dev), *sw = values(p[9], dev);
     float* const buf = none(p[12]) ? nullptr : values(p[12], dev, 1 + hist);
@@ -580,13 +583,17 @@ PyObject* linear_backward(PyObject* const* p) {
         gq = std::move(q.out), gq_t = std::move(q.out_t), keep = q.s.both;
         sg = q.s.p + 1;
     }
+    at::Tensor xt, wt;    // copies made here
+    if ((dform & 2) && !has_wt) wt = turned(w);
+    if ((wform & 2) && !has_xt) xt = turned(x);
+    if ((wform & 1) && !with_t) gq_t = turned(gq);
     ntfp8_gemm_desc d[2];
     int n = 0;
     const auto opt = at::TensorOptions().device(dev);
     void* const st = stream_of(gq);
     if (dx_code >= 0) {   // dX[T, K] = dY[T, N] . W[N, K]
         dx = at::empty({T, K}, opt.dtype(type_of(dx_code)));
-        gemm_desc(&d[0], gq, fg, sg, dform & 4 ? w : tensor(p[7]), fw, sw, dx, T, K, N, dform & 4, false, false);
+        gemm_desc(&d[0], gq, fg, sg, dform & 4 ? w : has_wt ? tensor(p[7]) : wt, fw, sw, dx, T, K, N, dform & 4, false, false);
         if (fp8_dx) {
             PyObject* const role = p[16];
             if (!PyTuple_Check(role) || PyTuple_GET_SIZE(role) != 3) stop(PyExc_TypeError, "the role of an fp8 gradient is a tuple of 3");
@@ -602,11 +609,12 @@ PyObject* linear_backward(PyObject* const* p) {
     }
     if (wants_dw) {       // dW[N, K] = dY[T, N]^T . X[T, K]
         if (!accumulate) dw = at::empty({N, K}, opt.dtype(at::kFloat));
-        gemm_desc(&d[n++], wform & 8 ? gq : gq_t, fg, sg, wform & 4 ? x : tensor(p[3]), fx, sx, dw, N, K, T, wform & 4, wform & 8, accumulate);
+        gemm_desc(&d[n++], wform & 8 ? gq : gq_t, fg, sg, wform & 4 ? x : has_xt ? tensor(p[3]) : xt, fx, sx, dw, N, K, T, wform & 4, wform & 8, accumulate);
     }
     if (n) call(ntfp8_gemm_batch(d, n, st), "ntfp8_gemm_batch");
-    if (!fp8_dx) return Py_BuildValue("(NNN)", wrap_or_none(std::move(db)), wrap_or_none(std::move(dx)), wrap_or_none(std::move(dw)));
-    return Py_BuildValue("(NNNNN)", wrap_or_none(std::move(db)), wrap(std::move(dx)), wrap_or_none(std::move(dw)), wrap(made.element(0)), wrap(made.element(1)));
+    PyObject* const results[] = {wrap_or_none(std::move(db)), wrap_or_none(std::move(dx)), wrap_or_none(std::move(dw)), wrap_or_none(std::move(xt)), wrap_or_none(std::move(wt))};
+    if (!fp8_dx) return Py_BuildValue("(NNNNN)", results[0], results[1], results[2], results[3], results[4]);
+    return Py_BuildValue("(NNNNNNN)", results[0], results[1], results[2], results[3], results[4], wrap(made.element(0)), wrap(made.element(1)));
 }
 
 // workspace(device index) -> (workspace, stream); workspace_pool(device index, count) -> ([>= count] workspaces, stream): what

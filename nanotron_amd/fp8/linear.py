@@ -12,7 +12,7 @@ from nanotron_amd.fp8 import kernel as _kernel
 from nanotron_amd.fp8.kernel import a_transposed_supported, fp8_matmul_kernel, fp8_matmul_pair, needs_transposed_copy
 from nanotron_amd.fp8.meta import FP8Meta
 from nanotron_amd.fp8.parameter import FP8Parameter
-from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, _assemble, cast_with_scale, update_scaling_factor
+from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, _assemble, _keep_transposed, cast_with_scale, update_scaling_factor
 
 
 class FP8LinearMeta(TypedDict):
@@ -502,9 +502,13 @@ def _backward_passes(ctx, module: FP8Linear, grad_output, input: FP8Tensor, weig
                                   bias_code, dx_code, role, wants_dw, acc, _kernel.READ_B_TRANSPOSED, _kernel.READ_A_TRANSPOSED)
     if res is None:
         return None
-    grad_bias, grad_input, grad_weight = res[:3]
+    grad_bias, grad_input, grad_weight, input_t, w_t = res[:5]
+    if input_t is not None:
+        _keep_transposed(input, input_t)
+    if w_t is not None:
+        _keep_transposed(w, w_t)
     if box is not None:
-        box.fp8_grad = _assemble(FP8Tensor, DTypes.FP8E5M2, grad_input, None, *res[3:])
+        box.fp8_grad = _assemble(FP8Tensor, DTypes.FP8E5M2, grad_input, None, *res[5:])
         grad_input = module._zero(ctx.in_dtype or torch.float32, weight.device).expand(ctx.in_shape)
         object.__setattr__(module, "fp8_grad_inputs_sent", module.fp8_grad_inputs_sent + 1)
     if grad_input is not None and len(ctx.in_shape) != 2:

@@ -133,9 +133,7 @@ class FP8Tensor(torch.Tensor):
         t = getattr(self, "_transposed", None)
         if t is None:
             assert self.dim() == 2, "transposed() needs a 2-D FP8Tensor"
-            t = torch.Tensor._make_subclass(FP8Tensor, nt.host.transpose(self))
-            t.fp8_meta = self.fp8_meta
-            self._transposed = t
+            t = _keep_transposed(self, nt.host.transpose(self))
         return t
 
     def __repr__(self) -> str:
@@ -171,12 +169,18 @@ def _assemble(cls, dtype: DTypes, out: torch.Tensor, out_t: Optional[torch.Tenso
               scale: torch.Tensor) -> FP8Tensor:
     """The FP8Tensor of quantised bytes (and their transposed copy) with its metadata."""
     obj = torch.Tensor._make_subclass(cls, out)
-    obj.fp8_meta = meta = FP8Meta(amax, scale, dtype)
+    obj.fp8_meta = FP8Meta(amax, scale, dtype)
     if out_t is not None:
-        t = torch.Tensor._make_subclass(FP8Tensor, out_t)
-        t.fp8_meta = meta
-        obj._transposed = t
+        _keep_transposed(obj, out_t)
     return obj
+
+
+def _keep_transposed(q: FP8Tensor, transposed: torch.Tensor) -> FP8Tensor:
+    """The transposed bytes of an FP8Tensor as one that shares its meta, kept beside it."""
+    t = torch.Tensor._make_subclass(FP8Tensor, transposed)
+    t.fp8_meta = q.fp8_meta
+    q._transposed = t
+    return t
 
 
 @torch.no_grad()

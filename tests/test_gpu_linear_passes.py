@@ -71,6 +71,98 @@ def test_same_as_the_pieces(tokens, K, N, dtype, out, bias, delayed, accumulate,
     for i, (a, b) in enumerate(zip(short, pieces)):
         assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
 
+class _Spy:
+    """Which calls of a layer's native passes were served: (pass, fp8 gradient back?) -> [True, False, ...] in order."""
+
+    def __init__(self, monkeypatch):
+        self.forward, self.backward, self.fp8 = [], [], []
+        fwd, bwd = L._quantise_and_multiply, L._backward_passes
+
+        def forward(*a):
+            res = fwd(*a)
+            self.forward.append(res is not None)
+            return res
+
+        def backward(*a):
+            res = bwd(*a)
+            self.backward.append(res is not None)
+            self.fp8.append(a[-1] is not None)
+            return res
+
+        monkeypatch.setattr(L, "_quantise_and_multiply", forward)
+        monkeypatch.setattr(L, "_backward_passes", backward)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,K,N", [(1, 1024, 1024), (16, 1024, 1024), (100, 1024, 1024), (128, 1024, 2304), (112, 144, 256), (129, 144, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_few_tokens(tokens, K, N, bias, monkeypatch):
+    """A weight that more than 128 tokens read as it is: its transposed copy, gone with every re-quantisation, is made inside
+    the native pass."""
+    res = []
+    for pieces in (False, True):
+        g = torch.Generator(device="cuda").manual_seed(tokens)
+        torch.manual_seed(3)   # (the bias)
+        lin = FP8Linear(K, N, bias, "cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16, delayed_scaling=True)
+        lin.weight = FP8Parameter((torch.randn(N, K, generator=g, device="cuda") * 0.02).to(torch.bfloat16), DTypes.FP8E4M3)
+        assert getattr(lin.weight.data, "_transposed", None) is None
+        got = []
+        for step in range(3):
+            if pieces:
+                monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
+                monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+            spy = _Spy(monkeypatch)
+            lin.requantize_weight()
+            assert getattr(lin.weight.data, "_transposed", None) is None
+            x = torch.randn(tokens, K, generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True)
+            y = lin(x)
+            y.backward((torch.randn(tokens, N, generator=g, device="cuda") * 1e-3).to(torch.bfloat16))
+            torch.cuda.synchronize()
+            monkeypatch.undo()
+            assert spy.backward == [step > 0 and not pieces]
+            assert (getattr(lin.weight.data, "_transposed", None) is not None) == (tokens <= 128)
+            if tokens <= 128:
+                got.append(lin.weight.data._transposed.as_subclass(torch.Tensor))
+                assert torch.equal(got[-1], lin.weight.data.as_subclass(torch.Tensor).t())
+                assert lin.weight.data._transposed.fp8_meta is lin.weight.data.fp8_meta
+            got += [y.detach(), x.grad, lin.weight.main_grad] + [r._buf.clone() for r in lin.scaling.values()]
+        res.append(got)
+    for i, (a, b) in enumerate(zip(*res)):
+        assert torch.equal(a, b), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [258, 301, 100, 77])
+def test_ragged_chain_is_served(tokens, monkeypatch):
+    """An fp8 gradient of a token count that is no multiple of 4 or 16: copies of the weight, of the fp8 input and of the fp8
+    gradient are made inside the native passes, with the results of the pieces."""
+    res = []
+    for pieces in (False, True):
+        g = torch.Generator(device="cuda").manual_seed(tokens)
+        lins = [FP8Linear(a, b, False, "cuda", dtype=torch.bfloat16, out_dtype=o, delayed_scaling=True)
+                for a, b, o in ((256, 384, DTypes.FP8E4M3), (384, 272, torch.bfloat16))]
+        for lin in lins:
+            lin.weight = FP8Parameter((torch.randn(lin.weight.shape, generator=g, device="cuda") * 0.05).to(torch.bfloat16), DTypes.FP8E4M3)
+        got = []
+        for step in range(3):
+            if pieces:
+                monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
+                monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+            spy = _Spy(monkeypatch)
+            for lin in lins:
+                lin.requantize_weight()
+            x = torch.randn(tokens, 256, generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True)
+            y = lins[1](lins[0](x))
+            y.backward((torch.randn(tokens, 272, generator=g, device="cuda") * 1e-3).to(torch.bfloat16))
+            torch.cuda.synchronize()
+            monkeypatch.undo()
+            assert spy.fp8 == [step > 0, False] and spy.backward == [step > 0 and not pieces] * 2
+            got += [y.detach(), x.grad] + [lin.weight.main_grad for lin in lins] + [r._buf.clone() for lin in lins for r in lin.scaling.values()]
+        res.append(got)
+    for i, (a, b) in enumerate(zip(*res)):
+        assert torch.equal(a, b), i
+
+
 @pytest.mark.gpu
 def test_frozen_weight_and_input_without_gradient(monkeypatch):
     x = torch.randn(256, 256, device="cuda", dtype=torch.bfloat16)
