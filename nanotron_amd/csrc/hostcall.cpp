@@ -423,18 +423,18 @@ PyObject* cast(PyObject* const* a) {
     return Py_BuildValue("(NN)", wrap(std::move(out)), wrap_or_none(std::move(out_t)));
 }
 
+at::Tensor widened(const at::Tensor& q, int fmt, const float* scale, long code, bool inverse) {   // contiguous bytes
+    at::Tensor out = at::empty(q.sizes(), at::TensorOptions().dtype(type_of(code)).device(q.device()));
+    if (q.numel()) {
+        if (inverse) call(ntfp8_cast_from_fp8_scale_inv(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "cast_from_fp8");
+        else call(ntfp8_cast_from_fp8(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "ntfp8_cast_from_fp8");
+    }
+    return out;
+}
 // dequantize(bytes, fmt, scale, out_code, inverse) -> tensor
 PyObject* dequantize(PyObject* const* a) {
     const at::Tensor q = codes(operand(a[0]));
-    const int fmt = (int)number(a[1]);
-    const float* scale = values(a[2], q.device());
-    const long code = number(a[3]);
-    at::Tensor out = at::empty(q.sizes(), at::TensorOptions().dtype(type_of(code)).device(q.device()));
-    if (q.numel()) {
-        if (truth(a[4])) call(ntfp8_cast_from_fp8_scale_inv(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "cast_from_fp8");
-        else call(ntfp8_cast_from_fp8(q.data_ptr(), fmt, scale, q.numel(), out.data_ptr(), (int)code, stream_of(q)), "ntfp8_cast_from_fp8");
-    }
-    return wrap(std::move(out));
+    return wrap(widened(q, (int)number(a[1]), values(a[2], q.device()), number(a[3]), truth(a[4])));
 }
 
 at::Tensor turned(const at::Tensor& q) {   // contiguous bytes [rows, cols] -> [cols, rows]
@@ -553,7 +553,7 @@ PyObject* linear_backward(PyObject* const* p) {
     const bool wants_dw = truth(p[17]), read_b = truth(p[19]), read_a = truth(p[20]);
     const long bias_code = number(p[14]), dx_code = number(p[15]);
     const bool fp8_dx = !none(p[16]);
-    if (bias_code > NTFP8_BF16 || (bias_code >= 0 && quantised_already) || (dx_code > NTFP8_BF16) != fp8_dx) Py_RETURN_NONE;
+    if (bias_code > NTFP8_BF16 || (dx_code > NTFP8_BF16) != fp8_dx) Py_RETURN_NONE;
     at::Tensor dw;
     const bool accumulate = !none(p[18]);
     if (accumulate) {
@@ -575,6 +575,7 @@ PyObject* linear_backward(PyObject* const* p) {
     if (quantised_already) {
         gq = grad;
         sg = values(p[1], dev);
+        if (bias_code >= 0) db = sum_columns(widened(gq, fg, sg, bias_code, false), (int)bias_code);   // the values of the bytes
     } else {
         at::Tensor g = dense(grad);
         if (g.dim() != 2) g = g.view({T, N});

@@ -132,17 +132,19 @@ def test_few_tokens(tokens, K, N, bias, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [258, 301, 100, 77])
-def test_ragged_chain_is_served(tokens, monkeypatch):
+@pytest.mark.parametrize("tokens,bias", [(258, False), (301, False), (100, False), (77, False), (256, True), (301, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_ragged_chain_is_served(tokens, bias, dtype, monkeypatch):
     """An fp8 gradient of a token count that is no multiple of 4 or 16: copies of the weight, of the fp8 input and of the fp8
-    gradient are made inside the native passes, with the results of the pieces."""
+    gradient are made inside the native passes; a bias gradient summed from fp8 values.  With the results of the pieces."""
     res = []
     for pieces in (False, True):
         g = torch.Generator(device="cuda").manual_seed(tokens)
-        lins = [FP8Linear(a, b, False, "cuda", dtype=torch.bfloat16, out_dtype=o, delayed_scaling=True)
+        torch.manual_seed(3)   # (the biases)
+        lins = [FP8Linear(a, b, bias, "cuda", dtype=dtype, out_dtype=o, delayed_scaling=True)
                 for a, b, o in ((256, 384, DTypes.FP8E4M3), (384, 272, torch.bfloat16))]
         for lin in lins:
-            lin.weight = FP8Parameter((torch.randn(lin.weight.shape, generator=g, device="cuda") * 0.05).to(torch.bfloat16), DTypes.FP8E4M3)
+            lin.weight = FP8Parameter((torch.randn(lin.weight.shape, generator=g, device="cuda") * 0.05).to(dtype), DTypes.FP8E4M3)
         got = []
         for step in range(3):
             if pieces:
@@ -157,7 +159,9 @@ def test_ragged_chain_is_served(tokens, monkeypatch):
             torch.cuda.synchronize()
             monkeypatch.undo()
             assert spy.fp8 == [step > 0, False] and spy.backward == [step > 0 and not pieces] * 2
-            got += [y.detach(), x.grad] + [lin.weight.main_grad for lin in lins] + [r._buf.clone() for lin in lins for r in lin.scaling.values()]
+            got += [y.detach(), x.grad] + [lin.weight.grad if dtype == torch.float32 else lin.weight.main_grad for lin in lins] + [r._buf.clone() for lin in lins for r in lin.scaling.values()]
+            if bias:
+                got += [lin.bias.grad.clone() for lin in lins]
         res.append(got)
     for i, (a, b) in enumerate(zip(*res)):
         assert torch.equal(a, b), i
