@@ -13,6 +13,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <optional>
 #include <unordered_map>
 
 #include "../../include/ntfp8.h"
@@ -534,8 +535,9 @@ PyObject* linear_forward(PyObject* const* p) {
 
 // linear_backward(dY, its scale where it is fp8 bytes | None, input bytes, their transposed copy | None, fmt, scale, weight bytes, their
 // transposed copy | None, fmt, scale, gradient fmt, margin, state | None, history_len, bias code | -1, dX code | -1, (state,
-// history_len, margin) of an fp8 dX | None, wants dW, dW to accumulate into | None, read_b, read_a) -> (bias gradient | None,
-// dX | None, dW | None, input bytes^T | None, weight bytes^T | None[, amax, scale of an fp8 dX]) | None: bias gradient,
+// history_len, margin) of an fp8 dX | None, wants dW, dW to accumulate into | None, read_b, read_a, wants the fp8 dY) -> (bias
+// gradient | None, dX | None, dW | None, input bytes^T | None, weight bytes^T | None, (amax, scale) of an fp8 dX | None, (bytes,
+// bytes^T | None, amax, scale) of dY, of which a dY that came as bytes has only the second, | None) | None: bias gradient,
 // quantisation of dY (current scaling or the fused delayed-scaling step), dX = dY . W and dW = dY^T . X.  Transposed copies that
 // a GEMM needs and nobody has made (a weight that more tokens would read as it is) are made here, and the caller is
 // given those of the input and the weight, to keep beside them.
@@ -567,11 +569,18 @@ PyObject* linear_backward(PyObject* const* p) {
     const int hist = (int)number(p[13]), fx = (int)number(p[4]), fw = (int)number(p[8]), fg = (int)number(p[10]);
     const float *sx = values(p[5], dev), *sw = values(p[9], dev);
     float* const buf = none(p[12]) ? nullptr : values(p[12], dev, 1 + hist);
+    int dx_hist = 0, dx_margin = 0;
+    float* state = nullptr;   // of the role of an fp8 dX
+    if (fp8_dx) {
+        PyObject* const role = p[16];
+        if (!PyTuple_Check(role) || PyTuple_GET_SIZE(role) != 3) stop(PyExc_TypeError, "the role of an fp8 gradient is a tuple of 3");
+        dx_hist = (int)number(PyTuple_GET_ITEM(role, 1)), dx_margin = (int)number(PyTuple_GET_ITEM(role, 2));
+        state = values(PyTuple_GET_ITEM(role, 0), dev, 1 + dx_hist);
+    }
 
     at::Tensor db, dx, gq, gq_t;
     const float* sg;
-    Scalars made(grad);   // [amax, scale] of an fp8 dX
-    at::Tensor keep;      // the scale of a dY quantised here
+    std::optional<Scalars> made, own;   // [amax, scale] of an fp8 dX, of a dY quantised here
     if (quantised_already) {
         gq = grad;
         sg = values(p[1], dev);
@@ -581,8 +590,8 @@ PyObject* linear_backward(PyObject* const* p) {
         if (g.dim() != 2) g = g.view({T, N});
         if (bias_code >= 0) db = sum_columns(g, (int)bias_code);
         Quantised q = quantise(g, fg, (int)number(p[11]), buf, nullptr, hist, with_t);
-        gq = std::move(q.out), gq_t = std::move(q.out_t), keep = q.s.both;
-        sg = q.s.p + 1;
+        gq = std::move(q.out), gq_t = std::move(q.out_t), own = std::move(q.s);
+        sg = own->p + 1;
     }
     at::Tensor xt, wt;    // copies made here
     if ((dform & 2) && !has_wt) wt = turned(w);
@@ -596,14 +605,11 @@ PyObject* linear_backward(PyObject* const* p) {
         dx = at::empty({T, K}, opt.dtype(type_of(dx_code)));
         gemm_desc(&d[0], gq, fg, sg, dform & 4 ? w : has_wt ? tensor(p[7]) : wt, fw, sw, dx, T, K, N, dform & 4, false, false);
         if (fp8_dx) {
-            PyObject* const role = p[16];
-            if (!PyTuple_Check(role) || PyTuple_GET_SIZE(role) != 3) stop(PyExc_TypeError, "the role of an fp8 gradient is a tuple of 3");
-            const int h = (int)number(PyTuple_GET_ITEM(role, 1)), margin = (int)number(PyTuple_GET_ITEM(role, 2));
-            float* const state = values(PyTuple_GET_ITEM(role, 0), dev, 1 + h);
+            made.emplace(gq);
             d[0].d_dtype = (int)dx_code;
             d[0].scale_d = state;
             d[0].amax_workspace = workspace_of(gq, st);
-            call(ntfp8_gemm_fp8(&d[0], margin, state, state + 1, h, made.p, made.p + 1, st), "ntfp8_gemm_fp8");
+            call(ntfp8_gemm_fp8(&d[0], dx_margin, state, state + 1, dx_hist, made->p, made->p + 1, st), "ntfp8_gemm_fp8");
         } else {
             ++n;
         }
@@ -613,9 +619,14 @@ PyObject* linear_backward(PyObject* const* p) {
         gemm_desc(&d[n++], wform & 8 ? gq : gq_t, fg, sg, wform & 4 ? x : has_xt ? tensor(p[3]) : xt, fx, sx, dw, N, K, T, wform & 4, wform & 8, accumulate);
     }
     if (n) call(ntfp8_gemm_batch(d, n, st), "ntfp8_gemm_batch");
-    PyObject* const results[] = {wrap_or_none(std::move(db)), wrap_or_none(std::move(dx)), wrap_or_none(std::move(dw)), wrap_or_none(std::move(xt)), wrap_or_none(std::move(wt))};
-    if (!fp8_dx) return Py_BuildValue("(NNNNN)", results[0], results[1], results[2], results[3], results[4]);
-    return Py_BuildValue("(NNNNNNN)", results[0], results[1], results[2], results[3], results[4], wrap(made.element(0)), wrap(made.element(1)));
+    auto pair = [](const std::optional<Scalars>& v) { return v ? Py_BuildValue("(NN)", wrap(v->element(0)), wrap(v->element(1))) : Py_NewRef(Py_None); };
+    PyObject* kept = Py_NewRef(Py_None);
+    if (truth(p[21])) {
+        Py_DECREF(kept);
+        kept = own ? quantised(std::move(gq), std::move(gq_t), *own) : Py_BuildValue("(ONOO)", Py_None, wrap_or_none(std::move(gq_t)), Py_None, Py_None);
+    }
+    return Py_BuildValue("(NNNNNNN)", wrap_or_none(std::move(db)), wrap_or_none(std::move(dx)), wrap_or_none(std::move(dw)), wrap_or_none(std::move(xt)),
+                         wrap_or_none(std::move(wt)), pair(made), kept);
 }
 
 // workspace(device index) -> (workspace, stream); workspace_pool(device index, count) -> ([>= count] workspaces, stream): what
@@ -666,7 +677,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
-                         NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 13), NT_METHOD(linear_backward, 21),
+                         NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 13), NT_METHOD(linear_backward, 22),
                          NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

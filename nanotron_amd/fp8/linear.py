@@ -358,7 +358,7 @@ class _FP8Matmul(torch.autograd.Function):
             box.arrivals += 1
         fp8_dx = (box is not None and box.consumers == 1 and box.arrivals == 1 and box.state is not None
                   and box.state.known_initialised and module is not None and module.fp8_grad_input)
-        if module is not None and not module.keep_quantised_grad:
+        if module is not None:
             quick = _backward_passes(ctx, module, grad_output, input, weight, bias, wants_dx, box if fp8_dx else None)
             if quick is not None:
                 return quick
@@ -499,16 +499,23 @@ def _backward_passes(ctx, module: FP8Linear, grad_output, input: FP8Tensor, weig
     mx, mw = input.fp8_meta, w.fp8_meta
     res = nt.host.linear_backward(grad_output, g_scale, input, getattr(input, "_transposed", None), mx.dtype.code, mx.scale, w,
                                   getattr(w, "_transposed", None), mw.dtype.code, mw.scale, nt.E5M2, margin, buf, history_len,
-                                  bias_code, dx_code, role, wants_dw, acc, _kernel.READ_B_TRANSPOSED, _kernel.READ_A_TRANSPOSED)
+                                  bias_code, dx_code, role, wants_dw, acc, _kernel.READ_B_TRANSPOSED, _kernel.READ_A_TRANSPOSED,
+                                  module.keep_quantised_grad)
     if res is None:
         return None
-    grad_bias, grad_input, grad_weight, input_t, w_t = res[:5]
+    grad_bias, grad_input, grad_weight, input_t, w_t, dx_scalars, kept = res
     if input_t is not None:
         _keep_transposed(input, input_t)
     if w_t is not None:
         _keep_transposed(w, w_t)
+    if kept is not None:   # for checkers: the e5m2 operand of dgrad and wgrad
+        if g_scale is None:
+            grad_output = _assemble(FP8Tensor, DTypes.FP8E5M2, *kept)
+        elif kept[1] is not None:
+            _keep_transposed(grad_output, kept[1])
+        module.quantised_grad_output = grad_output
     if box is not None:
-        box.fp8_grad = _assemble(FP8Tensor, DTypes.FP8E5M2, grad_input, None, *res[5:])
+        box.fp8_grad = _assemble(FP8Tensor, DTypes.FP8E5M2, grad_input, None, *dx_scalars)
         grad_input = module._zero(ctx.in_dtype or torch.float32, weight.device).expand(ctx.in_shape)
         object.__setattr__(module, "fp8_grad_inputs_sent", module.fp8_grad_inputs_sent + 1)
     if grad_input is not None and len(ctx.in_shape) != 2:

@@ -168,6 +168,46 @@ def test_ragged_chain_is_served(tokens, bias, dtype, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens,dims,delayed", [(512, (256, 384), True), (300, (256, 384), False), (77, (130, 91), True), (258, (256, 384, 272), True), (256, (256, 384, 272), True)])
+def test_quantised_gradient_kept_on_request(tokens, dims, delayed, monkeypatch):
+    """The e5m2 output gradient that a checker asks for is the one that the native passes multiply."""
+    res = []
+    for pieces in (False, True):
+        g = torch.Generator(device="cuda").manual_seed(tokens)
+        lins = []
+        for i, (a, b) in enumerate(zip(dims, dims[1:])):
+            out = torch.bfloat16 if i == len(dims) - 2 else DTypes.FP8E4M3
+            lin = FP8Linear(a, b, False, "cuda", dtype=torch.bfloat16, out_dtype=out, delayed_scaling=delayed)
+            lin.weight = FP8Parameter((torch.randn(b, a, generator=g, device="cuda") * 0.05).to(torch.bfloat16), DTypes.FP8E4M3)
+            lin.keep_quantised_grad = True
+            lins.append(lin)
+        got = []
+        for step in range(2):
+            if pieces:
+                monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+            spy = _Spy(monkeypatch)
+            h = torch.randn(tokens, dims[0], generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True)
+            for lin in lins:
+                h = lin(h)
+            h.backward((torch.randn(tokens, dims[-1], generator=g, device="cuda") * 1e-3).to(torch.bfloat16))
+            torch.cuda.synchronize()
+            monkeypatch.undo()
+            assert spy.backward == [not pieces and (step > 0 or not delayed)] * len(lins)
+            for lin in lins:
+                q, lin.quantised_grad_output = lin.quantised_grad_output, None
+                assert q.fp8_meta.dtype is DTypes.FP8E5M2 and q.shape == (tokens, lin.weight.shape[0])
+                t = getattr(q, "_transposed", None)
+                got += [q.as_subclass(torch.Tensor), q.fp8_meta.amax, q.fp8_meta.scale, torch.tensor(t is not None)]
+                if t is not None:
+                    got.append(t.as_subclass(torch.Tensor))
+                    assert torch.equal(got[-1], got[-5].t())
+        res.append(got)
+    assert len(res[0]) == len(res[1])
+    for i, (a, b) in enumerate(zip(*res)):
+        assert a.shape == b.shape and torch.equal(a, b), i
+
+
+@pytest.mark.gpu
 def test_frozen_weight_and_input_without_gradient(monkeypatch):
     x = torch.randn(256, 256, device="cuda", dtype=torch.bfloat16)
     gy = torch.randn(256, 384, device="cuda", dtype=torch.bfloat16)
