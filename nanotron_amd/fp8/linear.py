@@ -427,11 +427,17 @@ class _FP8Matmul(torch.autograd.Function):
         return grad_input, None, None, None, None, grad_bias, None
 
 
+# What tells whether a functorch transform or a tracer is active (None: no).  These are no public names of torch: where one is
+# missing nobody can tell, and the answer is never None.
+_unknown = lambda: "unknown"   # noqa: E731
+_functorch_active = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", _unknown)
+_tracing_state = getattr(torch._C, "_get_tracing_state", _unknown)
+
+
 def _no_transform() -> bool:
     """No transform is active that has to see the autograd function of a layer although gradients are off: forward-mode
-    differentiation, functorch's, tracing."""
-    return (forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._get_tracing_state() is None)
+    differentiation, functorch's, tracing.  False as well where torch does not say."""
+    return getattr(forward_ad, "_current_level", 0) < 0 and _functorch_active() is None and _tracing_state() is None
 
 
 _PIECES = (FP8Tensor.__new__, _kernel._gemm_nt, _kernel._gemm_nt_batch, _kernel._gemm_nt_fp8)

@@ -283,6 +283,21 @@ def test_transforms_are_seen():
     assert seen == [False, False] and L._no_transform()
 
 
+@pytest.mark.parametrize("owner,name", [(forward_ad, "_current_level"), (torch._C._functorch, "peek_interpreter_stack"), (torch._C, "_get_tracing_state"),
+                                        (torch._C, "_functorch")])
+def test_a_torch_that_does_not_tell_of_transforms(owner, name, monkeypatch):
+    """Without one of the private names the way past autograd is not taken; nothing raises."""
+    import importlib.util
+
+    spec = importlib.util.spec_from_file_location("linear_elsewhere", L.__file__)
+    module = importlib.util.module_from_spec(spec)
+    monkeypatch.delattr(owner, name)
+    spec.loader.exec_module(module)
+    assert not module._no_transform()
+    monkeypatch.undo()
+    assert L._no_transform()
+
+
 @pytest.mark.parametrize("name", ["_gemm_nt", "_gemm_nt_batch", "_gemm_nt_fp8"])
 def test_replaced_pieces_are_seen(name, monkeypatch):
     from nanotron_amd.fp8 import kernel as K
