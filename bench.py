@@ -304,48 +304,31 @@ def gemm_algorithmic_bytes():
 
 
 def gemm_in_step_timing(step, first_index, steps):
-    """Times every GEMM call where it runs: `steps` further steps of the same workload with a HIP event
-    recorded on the launch stream before and after each call of the GEMM entry points (a backward issues
-    its dgrad and wgrad as one batched call).  Returns (flops, milliseconds) summed over one step and the
+    """Times every GEMM call where it runs: `steps` further steps of the same workload, on the path they always take,
+    with a HIP event recorded on the launch stream before and after each GEMM call of the library (a backward
+    issues its dgrad and wgrad as one batched call).  Returns (flops, milliseconds) summed over one step and the
     per-call averages in call order."""
     import torch
 
-    from nanotron_amd.fp8 import kernel as K
+    from nanotron_amd import _native as nt
 
-    orig_one, orig_batch, orig_fp8 = K._gemm_nt, K._gemm_nt_batch, K._gemm_nt_fp8
-    log = []
+    log, begun = [], []
 
-    def bracket(fn, shapes):
-        e0 = torch.cuda.Event(enable_timing=True)
-        e1 = torch.cuda.Event(enable_timing=True)
-        e0.record()
-        out = fn()
-        e1.record()
-        log.append((shapes, e0, e1))
-        return out
+    def observe(issued, shapes):
+        e = torch.cuda.Event(enable_timing=True)
+        e.record()
+        if issued:
+            log.append((shapes, begun.pop(), e))
+        else:
+            begun.append(e)
 
-    def timed_one(a, b, out_dtype, accumulate_into, bias=None):
-        return bracket(lambda: orig_one(a, b, out_dtype, accumulate_into, bias), [(a.shape[0], b.shape[0], a.shape[1])])
-
-    def timed_fp8(a, b, dtype, state, with_transpose, bias=None, bt=False, at=False):
-        mnk = (a.shape[1 if at else 0], b.shape[1 if bt else 0], a.shape[0 if at else 1])
-        return bracket(lambda: orig_fp8(a, b, dtype, state, with_transpose, bias, bt, at), [mnk])
-
-    def timed_batch(problems):
-        # elements 5 and 7 of a problem mark operands handed over as their transposes ([K, N] / [K, M])
-        def mnk(p):
-            bt = len(p) > 4 and p[4]
-            at = len(p) > 6 and p[6]
-            return (p[0].shape[1 if at else 0], p[1].shape[1 if bt else 0], p[0].shape[0 if at else 1])
-        return bracket(lambda: orig_batch(problems), [mnk(p) for p in problems])
-
-    K._gemm_nt, K._gemm_nt_batch, K._gemm_nt_fp8 = timed_one, timed_batch, timed_fp8
+    before = nt.host.set_gemm_observer(observe)
     try:
         for i in range(steps):
             step(first_index + i)
         torch.cuda.synchronize()
     finally:
-        K._gemm_nt, K._gemm_nt_batch, K._gemm_nt_fp8 = orig_one, orig_batch, orig_fp8
+        nt.host.set_gemm_observer(before)
     per_step = len(log) // steps
     names = [f"{n}.{t}" for n, _, _ in LINEARS for t in ("fwd", "dgrad+wgrad")]
     assert per_step == len(names), (per_step, len(names))

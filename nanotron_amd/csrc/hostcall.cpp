@@ -22,6 +22,8 @@ namespace {
 
 PyObject* g_check = nullptr;   // nanotron_amd._native.check: raises RuntimeError, has the workspaces dropped after a failed launch
 
+PyObject* g_observer = nullptr;   // of the GEMM calls, see set_gemm_observer
+
 struct Stop {};   // a Python error is set
 
 [[noreturn]] void stop(PyObject* type, const char* msg) {
@@ -172,6 +174,30 @@ struct Scalars {
         return v;
     }
 };
+
+// Every GEMM call of this file, on the calling thread's stream, between the two calls of an observer if there is one
+void tell(const ntfp8_gemm_desc* d, int n, bool issued) {
+    PyObject* shapes = PyTuple_New(n);
+    if (shapes == nullptr) throw Stop{};
+    for (int i = 0; i < n; ++i) PyTuple_SET_ITEM(shapes, i, Py_BuildValue("(LLL)", (long long)d[i].M, (long long)d[i].N, (long long)d[i].K));
+    PyObject* const observer = Py_NewRef(g_observer);
+    PyObject* r = PyObject_CallFunction(observer, "ON", issued ? Py_True : Py_False, shapes);
+    Py_DECREF(observer);
+    if (r == nullptr) throw Stop{};
+    Py_DECREF(r);
+}
+void multiply(const ntfp8_gemm_desc* d, int n, void* stream) {
+    const bool observed = g_observer != nullptr;
+    if (observed) tell(d, n, false);
+    call(ntfp8_gemm_batch(d, n, stream), "ntfp8_gemm_batch");
+    if (observed && g_observer != nullptr) tell(d, n, true);
+}
+void multiply_fp8(const ntfp8_gemm_desc& d, int margin, float* state, int hist, const Scalars& s, void* stream) {
+    const bool observed = g_observer != nullptr;
+    if (observed) tell(&d, 1, false);
+    call(ntfp8_gemm_fp8(&d, margin, state, state + 1, hist, s.p, s.p + 1, stream), "ntfp8_gemm_fp8");
+    if (observed && g_observer != nullptr) tell(&d, 1, true);
+}
 
 void rows_cols(const at::Tensor& x, int64_t* rows, int64_t* cols) {
     *cols = x.dim() >= 2 ? x.size(-1) : x.numel();
@@ -338,7 +364,7 @@ PyObject* gemm(PyObject* const* p) {
     ntfp8_gemm_desc d = {};
     Problem k;
     fill(p, &d, &k);
-    call(ntfp8_gemm_batch(&d, 1, stream_of(k.a)), "ntfp8_gemm_batch");
+    multiply(&d, 1, stream_of(k.a));
     return wrap(std::move(k.out));
 }
 
@@ -357,7 +383,7 @@ PyObject* gemm_batch(PyObject* const* args) {
         fill(&PyTuple_GET_ITEM(t, 0), &d[i], &k[i]);
         require(k[i].a.device() == k[0].a.device(), "all problems of a batch are on one device");
     }
-    call(ntfp8_gemm_batch(d.data(), (int)n, stream_of(k[0].a)), "ntfp8_gemm_batch");
+    multiply(d.data(), (int)n, stream_of(k[0].a));
     PyObject* out = PyList_New(n);
     if (out == nullptr) throw Stop{};
     for (Py_ssize_t i = 0; i < n; ++i) PyList_SET_ITEM(out, i, wrap(std::move(k[i].out)));
@@ -380,7 +406,7 @@ PyObject* gemm_fp8(PyObject* const* p) {
     d.scale_d = buf;
     d.D_t = out_t.defined() ? out_t.data_ptr() : nullptr;
     d.amax_workspace = ws;
-    call(ntfp8_gemm_fp8(&d, margin, buf, buf + 1, hist, s.p, s.p + 1, st), "ntfp8_gemm_fp8");
+    multiply_fp8(d, margin, buf, hist, s, st);
     return quantised(std::move(k.out), std::move(out_t), s);
 }
 
@@ -529,7 +555,7 @@ PyObject* linear_forward(PyObject* const* p) {
     ntfp8_gemm_desc d;
     gemm_desc(&d, q.out, fmt, q.s.p + 1, w, (int)number(p[9]), sw, y, M, N, K, false, false, false);
     if (bias.defined()) d.bias = bias.data_ptr(), d.bias_dtype = code_of(bias.scalar_type());
-    call(ntfp8_gemm_batch(&d, 1, stream_of(x)), "ntfp8_gemm_batch");
+    multiply(&d, 1, stream_of(x));
     return Py_BuildValue("(NNNNN)", wrap(std::move(y)), wrap(std::move(q.out)), wrap_or_none(std::move(q.out_t)), wrap(q.s.element(0)), wrap(q.s.element(1)));
 }
 
@@ -609,7 +635,7 @@ PyObject* linear_backward(PyObject* const* p) {
             d[0].d_dtype = (int)dx_code;
             d[0].scale_d = state;
             d[0].amax_workspace = workspace_of(gq, st);
-            call(ntfp8_gemm_fp8(&d[0], dx_margin, state, state + 1, dx_hist, made->p, made->p + 1, st), "ntfp8_gemm_fp8");
+            multiply_fp8(d[0], dx_margin, state, dx_hist, *made, st);
         } else {
             ++n;
         }
@@ -618,7 +644,7 @@ PyObject* linear_backward(PyObject* const* p) {
         if (!accumulate) dw = at::empty({N, K}, opt.dtype(at::kFloat));
         gemm_desc(&d[n++], wform & 8 ? gq : gq_t, fg, sg, wform & 4 ? x : has_xt ? tensor(p[3]) : xt, fx, sx, dw, N, K, T, wform & 4, wform & 8, accumulate);
     }
-    if (n) call(ntfp8_gemm_batch(d, n, st), "ntfp8_gemm_batch");
+    if (n) multiply(d, n, st);
     auto pair = [](const std::optional<Scalars>& v) { return v ? Py_BuildValue("(NN)", wrap(v->element(0)), wrap(v->element(1))) : Py_NewRef(Py_None); };
     PyObject* kept = Py_NewRef(Py_None);
     if (truth(p[21])) {
@@ -651,6 +677,16 @@ PyObject* drop_workspaces(PyObject* const*) {
     Py_RETURN_NONE;
 }
 
+// set_gemm_observer(callable | None) -> the one before: called as f(issued, ((M, N, K), ...)) right before (issued False) and right
+// behind (True) every GEMM call of the library that these functions make, on the thread and the stream that makes it, so that
+// whoever times a step can put events there.  It changes nothing about the calls; what it raises, the call raises.
+PyObject* set_gemm_observer(PyObject* const* a) {
+    if (!none(a[0]) && !PyCallable_Check(a[0])) stop(PyExc_TypeError, "a callable or None is expected");
+    PyObject* const before = g_observer == nullptr ? Py_NewRef(Py_None) : g_observer;
+    g_observer = none(a[0]) ? nullptr : Py_NewRef(a[0]);
+    return before;
+}
+
 PyObject* set_check(PyObject* const* a) {
     Py_INCREF(a[0]);
     Py_XSETREF(g_check, a[0]);
@@ -678,7 +714,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
                          NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 13), NT_METHOD(linear_backward, 22),
-                         NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), {nullptr, nullptr, 0, nullptr}};
+                         NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), NT_METHOD(set_gemm_observer, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -440,22 +440,11 @@ def _no_transform() -> bool:
     return getattr(forward_ad, "_current_level", 0) < 0 and _functorch_active() is None and _tracing_state() is None
 
 
-_PIECES = (FP8Tensor.__new__, _kernel._gemm_nt, _kernel._gemm_nt_batch, _kernel._gemm_nt_fp8)
-
-
-def _watched() -> bool:
-    """One of the pieces that quantise or multiply has been replaced, by something that watches, times or changes it: the
-    passes have to go through them."""
-    new, one, batch, fp8 = _PIECES
-    return (FP8Tensor.__new__ is not new or _kernel._gemm_nt is not one or _kernel._gemm_nt_batch is not batch
-            or _kernel._gemm_nt_fp8 is not fp8)
-
-
 def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, needs_wgrad: bool):
     """(Y, input bytes, their transposed copy, amax, scale) of a layer's forward pass through one native call, with the results
     of FP8Tensor(x, ...) and fp8_matmul_kernel; None where it does not serve the case, nothing done."""
     out_code = nt.TORCH_TO_NT.get(module.out_dtype or torch.float32)
-    if out_code is None or not isinstance(weight, FP8Parameter) or _watched():
+    if out_code is None or not isinstance(weight, FP8Parameter):
         return None
     buf, history_len, margin, held = None, 0, 0, False
     if module.scaling is not None:
@@ -473,7 +462,7 @@ def _backward_passes(ctx, module: FP8Linear, grad_output, input: FP8Tensor, weig
     """What `_FP8Matmul._backward` returns, through one native call (bias gradient, quantisation of dY, dgrad and wgrad) with the
     results of the pieces it is put together from; None where that does not serve the case, nothing done.  `box`: dX leaves as
     e5m2 bytes under the role of the layer that made the input."""
-    if not isinstance(weight, FP8Parameter) or _watched():
+    if not isinstance(weight, FP8Parameter):
         return None
     buf, history_len, margin, g_scale = None, 0, 0, None
     if type(grad_output) is FP8Tensor:

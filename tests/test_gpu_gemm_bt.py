@@ -301,37 +301,38 @@ def test_a_transposed_requests_the_kernels_do_not_serve_are_refused():
         assert call(M, N, K) == -5, (M, N, K)
 
 
-def test_linear_backward_reads_the_output_gradient_as_it_is():
+def test_linear_backward_reads_the_output_gradient_as_it_is(monkeypatch):
     """FP8Linear's wgrad takes dY without a transposed copy when the shape allows it, and gives the bits of the path on
     transposed copies."""
     import nanotron_amd.fp8.kernel as K
-    from nanotron_amd.fp8 import DTypes, FP8Linear, FP8Parameter, FP8Tensor
+    import nanotron_amd.fp8.linear as L
+    from nanotron_amd.fp8 import DTypes, FP8Linear, FP8Parameter
 
     T, H, I = 384, 512, 768
     w = O.normal_tensor(1, (I, H), 0.05, torch.bfloat16)
-    seen, results = [], []
-    orig = FP8Tensor.__new__
+    copies, native, results = [], [], []
+    passes = L._backward_passes
 
-    def spy(cls, tensor, dtype, **kw):
-        if dtype == DTypes.FP8E5M2:
-            seen.append(bool(kw.get("with_transpose")))
-        return orig(cls, tensor, dtype, **kw)
+    def spy(*a):
+        res = passes(*a)
+        native.append(res is not None)
+        return res
 
+    monkeypatch.setattr(L, "_backward_passes", spy)
     for direct in (True, False):
-        K.READ_A_TRANSPOSED = direct
-        FP8Tensor.__new__ = spy
-        try:
-            lin = FP8Linear(H, I, bias=False, device="cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16, delayed_scaling=True)
-            lin.weight = FP8Parameter(w.cuda(), DTypes.FP8E4M3)
-            outs = []
-            for step in range(3):
-                x = O.normal_tensor(10 + step, (T, H), 1.0, torch.bfloat16).cuda().requires_grad_(True)
-                lin(x).backward(O.normal_tensor(20 + step, (T, I), 1e-2, torch.bfloat16).cuda())
-                outs += [x.grad.clone(), lin.weight.main_grad.clone()]
-            results.append(outs)
-        finally:
-            K.READ_A_TRANSPOSED = True
-            FP8Tensor.__new__ = orig
-    assert seen == [False] * 3 + [True] * 3
+        monkeypatch.setattr(K, "READ_A_TRANSPOSED", direct)
+        lin = FP8Linear(H, I, bias=False, device="cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16, delayed_scaling=True)
+        lin.weight = FP8Parameter(w.cuda(), DTypes.FP8E4M3)
+        lin.keep_quantised_grad = True
+        outs = []
+        for step in range(3):
+            x = O.normal_tensor(10 + step, (T, H), 1.0, torch.bfloat16).cuda().requires_grad_(True)
+            lin(x).backward(O.normal_tensor(20 + step, (T, I), 1e-2, torch.bfloat16).cuda())
+            torch.cuda.synchronize()
+            copies.append(getattr(lin.quantised_grad_output, "_transposed", None) is not None)
+            outs += [x.grad.clone(), lin.weight.main_grad.clone(), lin.quantised_grad_output.as_subclass(torch.Tensor)]
+        results.append(outs)
+    assert copies == [False] * 3 + [True] * 3
+    assert native == [False, True, True] * 2   # (the first use of a role takes the pieces)
     for a, b in zip(*results):
         assert torch.equal(_bits(a), _bits(b))

@@ -298,19 +298,40 @@ def test_a_torch_that_does_not_tell_of_transforms(owner, name, monkeypatch):
     assert L._no_transform()
 
 
-@pytest.mark.parametrize("name", ["_gemm_nt", "_gemm_nt_batch", "_gemm_nt_fp8"])
-def test_replaced_pieces_are_seen(name, monkeypatch):
-    from nanotron_amd.fp8 import kernel as K
-    from nanotron_amd.fp8 import FP8Tensor
+@pytest.mark.gpu
+def test_gemm_observer_sees_the_calls_of_the_native_passes(monkeypatch):
+    from nanotron_amd import _native as nt
 
-    assert not L._watched()
-    monkeypatch.setattr(K, name, lambda *a, **k: None)
-    assert L._watched()
-    monkeypatch.undo()
-    orig = FP8Tensor.__new__
-    FP8Tensor.__new__ = lambda *a, **k: orig(*a, **k)
+    T, K, N = 256, 384, 272
+    x = torch.randn(T, K, device="cuda", dtype=torch.bfloat16)
+    gy = torch.randn(T, N, device="cuda", dtype=torch.bfloat16)
+    res, seen = [], []
+    for watch in (False, True):
+        torch.manual_seed(0)
+        lin = FP8Linear(K, N, False, "cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16)
+        spy = _Spy(monkeypatch)
+        assert nt.host.set_gemm_observer((lambda *a: seen.append(a)) if watch else None) is None
+        xg = x.clone().requires_grad_(True)
+        y = lin(xg)
+        y.backward(gy)
+        assert (nt.host.set_gemm_observer(None) is not None) == watch
+        monkeypatch.undo()
+        assert spy.forward == [True] and spy.backward == [True]
+        res.append([y.detach(), xg.grad, lin.weight.main_grad])
+    forward, backward = ((T, N, K),), ((T, K, N), (N, K, T))
+    assert seen == [(False, forward), (True, forward), (False, backward), (True, backward)]
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+    def refuse(*a):
+        raise ValueError("no")
+
+    nt.host.set_gemm_observer(refuse)
     try:
-        assert L._watched()
+        with pytest.raises(ValueError, match="no"):
+            lin(x)
     finally:
-        FP8Tensor.__new__ = orig
-    assert not L._watched()
+        nt.host.set_gemm_observer(None)
+    with torch.no_grad():
+        assert torch.equal(lin(x), res[0][0])
+    with pytest.raises(TypeError):
+        nt.host.set_gemm_observer(3)
