@@ -9,10 +9,33 @@ from nanotron_amd.fp8 import DTypes, FP8Linear, FP8Parameter
 from nanotron_amd.fp8 import linear as L
 
 
+class _Spy:
+    """Which calls of the native forward and backward were served, in order, and which of the latter were to send an fp8 dX."""
+
+    def __init__(self, monkeypatch):
+        self.forward, self.backward, self.fp8 = [], [], []
+        fwd, bwd = L._quantise_and_multiply, L._backward_passes
+
+        def forward(*a):
+            res = fwd(*a)
+            self.forward.append(res is not None)
+            return res
+
+        def backward(*a):
+            res = bwd(*a)
+            self.backward.append(res is not None)
+            self.fp8.append(a[-1] is not None)
+            return res
+
+        monkeypatch.setattr(L, "_quantise_and_multiply", forward)
+        monkeypatch.setattr(L, "_backward_passes", backward)
+
+
 def _run(x, gys, dtype, out, bias, delayed, accumulate, dims, pieces, monkeypatch, offset=0):
     if pieces:
         monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
         monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+    spy = _Spy(monkeypatch)
     K, N = x.shape[-1], gys[0].shape[-1]
     g = torch.Generator(device="cuda").manual_seed(3)
     lin = FP8Linear(K, N, bias, "cuda", dtype=dtype, out_dtype=out, delayed_scaling=delayed, accumulate_grad=accumulate)
@@ -40,7 +63,12 @@ def _run(x, gys, dtype, out, bias, delayed, accumulate, dims, pieces, monkeypatc
     if delayed:
         got += [r._buf.clone() for r in lin.scaling.values()]
     monkeypatch.undo()
+    # the first use of a scaling role takes the pieces, every other pass is served; without gradients a pass that is not
+    # served asks once more inside autograd's function
+    steps = [not pieces and (i > 0 or not delayed) for i in range(len(gys))]
+    assert spy.backward == steps and spy.forward == steps + ([False] * 3 if pieces else [True] * 2)
     return got
+
 
 CASES = [
     # tokens, K, N, dtype, out, bias, delayed, accumulate, dims
@@ -53,6 +81,7 @@ CASES = [
     (1, 64, 48, torch.bfloat16, torch.bfloat16, True, False, False, 1),
     (300, 256, 264, torch.bfloat16, torch.bfloat16, False, True, False, 2),
 ]
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("offset", [0, 1])
@@ -70,27 +99,6 @@ def test_same_as_the_pieces(tokens, K, N, dtype, out, bias, delayed, accumulate,
     assert len(short) == len(pieces)
     for i, (a, b) in enumerate(zip(short, pieces)):
         assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
-
-class _Spy:
-    """Which calls of a layer's native passes were served: (pass, fp8 gradient back?) -> [True, False, ...] in order."""
-
-    def __init__(self, monkeypatch):
-        self.forward, self.backward, self.fp8 = [], [], []
-        fwd, bwd = L._quantise_and_multiply, L._backward_passes
-
-        def forward(*a):
-            res = fwd(*a)
-            self.forward.append(res is not None)
-            return res
-
-        def backward(*a):
-            res = bwd(*a)
-            self.backward.append(res is not None)
-            self.fp8.append(a[-1] is not None)
-            return res
-
-        monkeypatch.setattr(L, "_quantise_and_multiply", forward)
-        monkeypatch.setattr(L, "_backward_passes", backward)
 
 
 @pytest.mark.gpu
@@ -220,11 +228,14 @@ def test_frozen_weight_and_input_without_gradient(monkeypatch):
             lin = FP8Linear(256, 384, True, "cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16)
             lin.weight.requires_grad_(not frozen)
             xg = x.clone().requires_grad_(frozen)
+            spy = _Spy(monkeypatch)
             lin(xg).backward(gy)
+            assert spy.forward == [True] and spy.backward == [not pieces]
             assert (xg.grad is None) == (not frozen) and (getattr(lin.weight, "main_grad", None) is None) == frozen
             res.append([xg.grad if frozen else lin.weight.main_grad, lin.bias.grad])
             monkeypatch.undo()
         assert all(torch.equal(a, b) for a, b in zip(*res))
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens,dims,bias", [(512, (256, 384, 272), False), (300, (256, 320, 272), False), (258, (272, 320, 256), True), (64, (128, 96, 112), False)])
@@ -235,6 +246,7 @@ def test_chain_same_as_the_pieces(tokens, dims, bias, monkeypatch):
         if pieces:
             monkeypatch.setattr(L, "_quantise_and_multiply", lambda *a: None)
             monkeypatch.setattr(L, "_backward_passes", lambda *a: None)
+        spy = _Spy(monkeypatch)
         g = torch.Generator(device="cuda").manual_seed(tokens)
         lins = []
         for i, (a, b) in enumerate(zip(dims, dims[1:])):
@@ -257,6 +269,9 @@ def test_chain_same_as_the_pieces(tokens, dims, bias, monkeypatch):
         got.append(torch.tensor([lin.fp8_grad_inputs_sent for lin in lins]))
         res.append(got)
         monkeypatch.undo()
+        # the last layer first; an fp8 output is not the native forward's, nor is the pass over an fp8 input
+        assert spy.fp8 == [False, False, True, False, True, False] and spy.forward == [False] * 3
+        assert spy.backward == [False] * 2 + [not pieces] * 4
     for i, (a, b) in enumerate(zip(*res)):
         assert torch.equal(a, b), i
 
