@@ -6,7 +6,7 @@
 //
 // Data movement per K-tile: every wave brings a quarter of the A and B tiles from global memory into
 // LDS (16 bytes per lane, XOR-swizzled), reads its MI A fragments from LDS once and keeps them in
-// registers, and streams its 8 B fragments from LDS two MFMA groups ahead of their use.  One MFMA
+// registers, and reads its 8 B fragments ahead of their use (below).  One MFMA
 // group = the MI MFMAs that share one B fragment.
 //
 // Loads go straight from memory into LDS.  Whole tiles (MI = 8): two LDS stages and two workgroup barriers per K-tile.
@@ -20,7 +20,8 @@
 // byte passes through a register on its way to LDS.  us, loads kept in registers for a K-tile / straight into LDS:
 // 4096 x 4096 x 4096 50.6 / 48.5, 4096 x 14336 x 4096 179 / 173, 4096 x 4096 x 14336 165 / 160; both operands transposed
 // beside dgrad, 4096 tokens: 4096 -> 4096 110 / 104, 4096 -> 14336 384 / 362, 14336 -> 4096 387 / 372.
-// Half tiles (MI = 4): three stages, one barrier behind group 5 that releases the stage of tile kt and publishes tile kt + 1.
+// Half tiles (MI = 4): three stages, one barrier behind group 5 that releases the stage of tile kt and publishes tile kt + 1;
+// B fragments in a ring of four, read three groups ahead.
 //
 // Instantiations beside the operand formats and MI: kFp8Out (the outputs are fp8 bytes, cast in the
 // epilogue, with an optional transposed copy and the amax of the results) and kBT (the B operands are
@@ -391,7 +392,6 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     constexpr int LA = MI * 2 * 16 / 8 / kBigWaves;  // wave-level loads of the A tile per wave per stage
     constexpr int LB = kBigLB;
     constexpr int NL = LA + LB;                      // loads per wave per K-tile
-    static_assert(NL % 4 == 0, "the loads are queued in four equal portions");
     const int wm = (wave >> 1) * (MI * 16), wn = (wave & 1) * 128;
 
     v4f acc[MI][kBigNJ];
@@ -544,6 +544,9 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             constexpr int kRelease = 25;              // slot of the first barrier
             constexpr int kEvery = 3;                 // slots from load to load
             constexpr int kFront = (MI * 6 - 1 - kRelease) / kEvery;   // loads in front(), the others in back()
+            constexpr int kReads = 4 * (kBigNJ - 2);  // B fragments 2-7 are read behind every other of so many slots
+            static_assert(kRelease > kReads - 2 && kRelease < MI * 6, "the stage is released behind the last read of it, within front()");
+            static_assert(kFront > 0 && kFront <= NL, "front() requests the first loads of a tile, back() the others");
             v4i fw[kBigNJ][2];   // all B fragments of a tile
             auto front_w = [&](auto l_tag, auto b_tag, int f) {
                 constexpr bool L = decltype(l_tag)::value, B = decltype(b_tag)::value;   // L: there is a tile f + 2; B: f + 1
@@ -553,7 +556,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
                 for (int x = 0; x < MI * 6; ++x) {
                     const int j = x / MI, i = x % MI;
                     mma(i, j, frag(fw[j]), frag(fa[i]));
-                    if (x < 24 && x % 2 == 0) fw[2 + x / 4][x / 2 % 2] = rd_b(s, 2 + x / 4, x / 2 % 2);
+                    if (x < kReads && x % 2 == 0) fw[2 + x / 4][x / 2 % 2] = rd_b(s, 2 + x / 4, x / 2 % 2);
                     if constexpr (L) {
                         if (x == kRelease) {
                             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every fragment of tile f is in registers
@@ -649,6 +652,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         v4i fb[4][2];
         constexpr int kBackLoads = NL / 3;
         constexpr int kFrontLoads = NL - kBackLoads;
+        static_assert(kBackLoads > 0 && kFrontLoads > 0, "every load of a tile is requested once, in back() or in front()");
         // loads: queue the rest of tile kt + NS - 1; WAIT (>= 0): barrier, after all but the newest WAIT
         // loads of this wave have landed (-1: no barrier)
         auto front = [&](auto loads_tag, auto wait_tag, int kt) {
