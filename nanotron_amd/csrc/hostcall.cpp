@@ -539,8 +539,10 @@ PyObject* linear_forward(PyObject* const* p) {
     const int hist = (int)number(p[4]), fmt = (int)number(p[1]);
     const long out_code = number(p[12]);
     if (out_code < 0 || out_code > NTFP8_BF16) Py_RETURN_NONE;
+    const bool held = truth(p[5]);
+    if (held && tensor(p[3]).device() != x.device()) Py_RETURN_NONE;   // the pieces bring a held scale over
     float* const buf = none(p[3]) ? nullptr : values(p[3], x.device(), 1 + hist);
-    const bool held = truth(p[5]), with_t = truth(p[6]) && !(truth(p[7]) && reads_b(N, K, M));
+    const bool with_t = truth(p[6]) && !(truth(p[7]) && reads_b(N, K, M));
     const float* sw = values(p[10], x.device());
     at::Tensor bias;
     if (!none(p[11])) {

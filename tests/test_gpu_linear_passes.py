@@ -277,6 +277,23 @@ def test_chain_same_as_the_pieces(tokens, dims, bias, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_evaluation_with_a_scale_held_on_another_device():
+    """A layer whose scaling roles were kept on the host after training evaluates with the scale they hold."""
+    lin = FP8Linear(256, 384, False, "cuda", dtype=torch.bfloat16, out_dtype=torch.bfloat16, delayed_scaling=True)
+    x = torch.randn(64, 256, device="cuda", dtype=torch.bfloat16)
+    lin(x)
+    torch.cuda.synchronize()
+    lin.eval()
+    with torch.no_grad():
+        want = lin(x)
+        state = lin.scaling["input"]
+        assert state.known_initialised
+        state._buf = state._buf.cpu()
+        assert torch.equal(lin(x), want)
+    assert torch.equal(lin(x).detach(), want)
+
+
+@pytest.mark.gpu
 def test_saved_tensor_hooks_see_what_a_layer_saves():
     lin = FP8Linear(256, 256, False, "cuda", out_dtype=torch.float32)
     x = torch.randn(256, 256, device="cuda", requires_grad=True)
