@@ -192,9 +192,10 @@ void multiply(const ntfp8_gemm_desc* d, int n, void* stream) {
     call(ntfp8_gemm_batch(d, n, stream), "ntfp8_gemm_batch");
     if (observed && g_observer != nullptr) tell(d, n, true);
 }
-void multiply_fp8(const ntfp8_gemm_desc& d, int margin, float* state, int hist, const Scalars& s, void* stream) {
+void multiply_fp8(ntfp8_gemm_desc& d, int margin, float* state, int hist, const Scalars& s, void* stream) {
     const bool observed = g_observer != nullptr;
     if (observed) tell(&d, 1, false);
+    d.amax_workspace = workspace_of(s.both, stream);   // (not before the observer: while it runs, others may drop workspaces)
     call(ntfp8_gemm_fp8(&d, margin, state, state + 1, hist, s.p, s.p + 1, stream), "ntfp8_gemm_fp8");
     if (observed && g_observer != nullptr) tell(&d, 1, true);
 }
@@ -402,10 +403,8 @@ PyObject* gemm_fp8(PyObject* const* p) {
     if (truth(p[kProblem + 3])) out_t = bytes_like(k.a, {d.N, d.M});
     const Scalars s(k.a);
     void* st = stream_of(k.a);
-    void* ws = workspace_of(k.a, st);
     d.scale_d = buf;
     d.D_t = out_t.defined() ? out_t.data_ptr() : nullptr;
-    d.amax_workspace = ws;
     multiply_fp8(d, margin, buf, hist, s, st);
     return quantised(std::move(k.out), std::move(out_t), s);
 }
@@ -636,7 +635,6 @@ PyObject* linear_backward(PyObject* const* p) {
             made.emplace(gq);
             d[0].d_dtype = (int)dx_code;
             d[0].scale_d = state;
-            d[0].amax_workspace = workspace_of(gq, st);
             multiply_fp8(d[0], dx_margin, state, dx_hist, *made, st);
         } else {
             ++n;

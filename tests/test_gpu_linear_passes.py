@@ -354,6 +354,22 @@ def test_gemm_observer_sees_the_calls_of_the_native_passes(monkeypatch):
     assert seen == [(False, forward), (True, forward), (False, backward), (True, backward)]
     assert all(torch.equal(a, b) for a, b in zip(*res))
 
+    # whoever is told may drop the workspaces: an fp8 output's bookkeeping takes its own afterwards
+    fp8 = []
+    for watch in (False, True):
+        torch.manual_seed(0)
+        out = FP8Linear(K, N, False, "cuda", dtype=torch.bfloat16, out_dtype=DTypes.FP8E4M3, delayed_scaling=True)
+        out(x)
+        torch.cuda.synchronize()
+        nt.host.set_gemm_observer((lambda *a: nt.host.drop_workspaces()) if watch else None)
+        try:
+            q = out(x)
+        finally:
+            nt.host.set_gemm_observer(None)
+        fp8.append([q.as_subclass(torch.Tensor), q.fp8_meta.amax, out.scaling["output"]._buf])
+        assert float(q.fp8_meta.amax) > 0
+    assert all(torch.equal(a, b) for a, b in zip(*fp8))
+
     def refuse(*a):
         raise ValueError("no")
 
