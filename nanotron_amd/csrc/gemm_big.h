@@ -72,8 +72,9 @@ __device__ __forceinline__ void swap_rows16(uint32_t& x, uint32_t& y) {
     y = r.y;
 }
 // 16 bytes per lane from global memory into registers; offsets past the descriptor read as zero
+template <int kPolicy = 0>
 __device__ __forceinline__ v4i reg_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
-    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kPolicy));
 }
 __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
 // 16 bytes of output to global memory, written through to memory as they are issued (sc0 sc1) and marked streaming
@@ -85,6 +86,34 @@ __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0
 // of four lanes now and then).
 __device__ __forceinline__ void store16_through(void* p, v4i v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
+// 16 / 4 bytes per lane to global memory through a buffer descriptor; offsets past its size are dropped.  Cache policy
+// of the builtin's last argument on gfx950: bit 0 = sc0, bit 1 = nt, bit 4 = sc1 (written through, as store16_through).
+constexpr int kStoreThrough = 1 | 2 | 16, kStreaming = 2;
+template <int kPolicy = kStoreThrough>
+__device__ __forceinline__ void reg_store16(__amdgpu_buffer_rsrc_t r, uint32_t voff, v4i data) {
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, data), r, voff, 0, kPolicy);
+}
+__device__ __forceinline__ void reg_store4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t data) {
+    __builtin_amdgcn_raw_buffer_store_b32(data, r, voff, 0, kStoreThrough);
+}
+constexpr uint32_t kDropped = 0xfffffff0u;   // past every descriptor
+// within groups of 16 lanes: lanes 8 .. 15 of x <-> lanes 0 .. 7 of y
+__device__ __forceinline__ void swap_octets(uint32_t& x, uint32_t& y) {
+    const int a = (int)x, b = (int)y;
+    x = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false);   // row_ror:8 into banks 2, 3
+    y = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false);   // row_ror:8 into banks 0, 1
+}
+
+// `count` rows from m_base on of a row-major M x N output: rows past its end fall behind the descriptor
+constexpr int kMaxColumns = 1 << 22;   // 128 rows within reach of 32-bit offsets
+template <typename O>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(O* D, int M, int N, int m_base, int count) {
+    // (a clamp is a vector instruction, and through a descriptor in vector registers the compiler accesses in a loop)
+    const uint32_t rows = (uint32_t)__builtin_amdgcn_readfirstlane(max(0, min(M - m_base, count)));
+    return make_rsrc(D + (int64_t)m_base * N, rows * (uint32_t)N * (uint32_t)sizeof(O));
 }
 
 // Epilogue of one wave: MI x NJ accumulator blocks of 16 x 16, block (i, j) at rows m_base + 16 i,
@@ -101,7 +130,7 @@ __device__ __forceinline__ void store_wave_tile16(const v4f (&acc)[MI][NJ], void
         if constexpr (kBias) return acc[i][j][e] * alpha + bv[j][e];
         else return acc[i][j][e] * alpha;
     };
-    if constexpr (DT != NTFP8_F32) {
+    if constexpr (DT != NTFP8_F32 && NJ != 4) {
         // 16-bit outputs: a lane's 4 consecutive n are only 8 bytes.  Exchanging registers of two
         // neighbouring blocks between lane rows gives every lane 8 consecutive n (16 bytes) of one
         // block, and lane rows r / r + 2 together a full 32-byte sector per output row, which the
@@ -124,6 +153,91 @@ __device__ __forceinline__ void store_wave_tile16(const v4f (&acc)[MI][NJ], void
                         store16_through(D + (int64_t)m * N + n, (v4i){(int)x0, (int)x1, (int)y0, (int)y1});
                 }
             }
+            return;
+        }
+    }
+    if constexpr (DT != NTFP8_F32 && NJ == 4) {
+        // The same, and exchanging words between lanes l and l ^ 8 of two such pairs, a store covers 64 columns, a whole line, of 8 rows.
+        // (us, half lines of 16 rows / this: bf16 1021 x 2304 x 1024 with bias 9.5 / 8.9, 3000 x 1000 x 1024 10.7 / 9.6,
+        // most shapes the same; the 256-wide tiles the same everywhere)
+        if ((N & 7) == 0 && N < kMaxColumns) {
+            const __amdgpu_buffer_rsrc_t rd = rows_rsrc(D, M, N, m_base, 16 * MI);
+            // lane row q holds n 8 (q / 2) .. + 7 of block j + (q & 1), lanes 8 .. 15 of it those of the pair behind
+            const int col = n_base + ((mrow >> 3) * 2 + (q & 1)) * 16 + (q >> 1) * 8;
+            const uint32_t step = 8u * (uint32_t)N * 2u;
+            uint32_t at = ((uint32_t)(mrow & 7) * (uint32_t)N + (uint32_t)col) * 2u;
+#pragma unroll
+            for (int i = 0; i < MI; ++i, at += 2 * step) {
+#pragma unroll
+                for (int j0 = 0; j0 < NJ; j0 += 4) {
+                    uint32_t w[2][4];
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const int j = j0 + 2 * p;
+                        uint32_t x0 = OutT<DT>::pack2(val(i, j, 0), val(i, j, 1));
+                        uint32_t x1 = OutT<DT>::pack2(val(i, j, 2), val(i, j, 3));
+                        uint32_t y0 = OutT<DT>::pack2(val(i, j + 1, 0), val(i, j + 1, 1));
+                        uint32_t y1 = OutT<DT>::pack2(val(i, j + 1, 2), val(i, j + 1, 3));
+                        swap_rows16(x0, y0);
+                        swap_rows16(x1, y1);
+                        w[p][0] = x0, w[p][1] = x1, w[p][2] = y0, w[p][3] = y1;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) swap_octets(w[0][e], w[1][e]);
+                    const bool in = col + j0 * 16 < N;
+                    reg_store16(rd, in ? at + j0 * 32 : kDropped, (v4i){(int)w[0][0], (int)w[0][1], (int)w[0][2], (int)w[0][3]});
+                    reg_store16(rd, in ? at + step + j0 * 32 : kDropped, (v4i){(int)w[1][0], (int)w[1][1], (int)w[1][2], (int)w[1][3]});
+                }
+                sched_fence();
+            }
+            return;
+        }
+    }
+    if constexpr (DT == NTFP8_F32) {
+        // A lane's 4 consecutive n are 16 bytes, the four lane rows together 64 bytes of an output row, half a line.
+        // Exchanging words between lanes l and l ^ 8 of two neighbouring blocks, a store (or the load of the accumulator)
+        // covers 32 columns, a whole line, of 8 rows.  Rows of whole 64-byte pieces are written through as 16-bit outputs are,
+        // or, where the line has just been read for the accumulation, read and written with the streaming hint alone; others
+        // keep ordinary accesses, which put the pieces together in the L2.  us, half lines and ordinary accesses / here:
+        //   2048 x 2048 x 2048  14.3 / 12.7     14336 x 4096 x 4096, both transposed  211 / 195, accumulated  257 / 232
+        //   4096 x 4096 x 14336 with that weight gradient  369 / 358, accumulated  413 / 386
+        //   rows of 64-byte pieces  4096 x 4112 x 512  32.6 / 28.0, accumulated  57.7 / 48.0 (written through 56.8)
+        //   others  4096 x 4104 x 512  32.3 / 31.4 (written through 43.6)
+        if ((N & (NJ == 4 ? 3 : 15)) == 0 && N < kMaxColumns) {   // (NJ = 8: no registers for two kinds of accesses)
+            const __amdgpu_buffer_rsrc_t rd = rows_rsrc(D, M, N, m_base, 16 * MI);
+            const int col = n_base + (mrow >> 3) * 16 + q * 4;
+            const uint32_t step = 8u * (uint32_t)N * 4u;
+            auto rows = [&](auto policy_tag) {
+                constexpr int kPolicy = decltype(policy_tag)::value;
+                uint32_t at = ((uint32_t)(mrow & 7) * (uint32_t)N + (uint32_t)col) * 4u;
+#pragma unroll
+                for (int i = 0; i < MI; ++i, at += 2 * step) {
+                    v4f old[NJ];   // all of a row block's old values are requested before the first one is needed
+                    if constexpr (kAcc) {
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            old[j] = __builtin_bit_cast(v4f, reg_load16<kPolicy>(rd, col + (j & ~1) * 16 < N ? at + (j & 1) * step + (j & ~1) * 64 : kDropped, 0));
+                    }
+#pragma unroll
+                    for (int j = 0; j < NJ; j += 2) {
+                        v4f x, y;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            uint32_t a = __float_as_uint(val(i, j, e)), b = __float_as_uint(val(i, j + 1, e));
+                            swap_octets(a, b);
+                            x[e] = __uint_as_float(a), y[e] = __uint_as_float(b);
+                        }
+                        if constexpr (kAcc) x = x + old[j], y = y + old[j + 1];
+                        const bool in = col + j * 16 < N;
+                        reg_store16<kPolicy>(rd, in ? at + j * 64 : kDropped, __builtin_bit_cast(v4i, x));
+                        reg_store16<kPolicy>(rd, in ? at + step + j * 64 : kDropped, __builtin_bit_cast(v4i, y));
+                        sched_fence();
+                    }
+                    // (values of several row blocks at once do not fit the registers)
+                }
+            };
+            if (NJ != 4 || (N & 15) == 0) rows(std::integral_constant<int, kAcc ? kStreaming : kStoreThrough>{});   // uniform
+            else rows(std::integral_constant<int, 0>{});
             return;
         }
     }
@@ -179,17 +293,6 @@ __device__ __forceinline__ void store_wave_tile16(const v4f (&acc)[MI][NJ], void
     }
 }
 
-// 16 / 4 bytes per lane to global memory through a buffer descriptor; offsets past its size are dropped.  Cache policy
-// of the builtin's last argument on gfx950: bit 0 = sc0, bit 1 = nt, bit 4 = sc1 (written through, as store16_through).
-constexpr int kStoreThrough = 1 | 2 | 16;
-__device__ __forceinline__ void reg_store16(__amdgpu_buffer_rsrc_t r, uint32_t voff, v4i data) {
-    typedef unsigned v4u __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, data), r, voff, 0, kStoreThrough);
-}
-__device__ __forceinline__ void reg_store4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t data) {
-    __builtin_amdgcn_raw_buffer_store_b32(data, r, voff, 0, kStoreThrough);
-}
-
 // fp8 epilogue of one wave (layout as store_wave_tile16); returns the lane's max|r| as a bit pattern.
 // Shapes: N a multiple of 16, M a multiple of 4, M N < 2^32 (the launcher sends other shapes to the small kernel).
 // A lane's 4 consecutive n of a block are one word of D.  Row-major bytes: a 4 x 4 exchange of words between the
@@ -219,7 +322,6 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
     const uint32_t bytes = (uint32_t)M * (uint32_t)N;
     const __amdgpu_buffer_rsrc_t rd = make_rsrc(D, bytes);
     const __amdgpu_buffer_rsrc_t rt = make_rsrc(Dt, Dt ? bytes : 0u);
-    constexpr uint32_t kDropped = 0xfffffff0u;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int m = m_base + i * 16 + mrow;

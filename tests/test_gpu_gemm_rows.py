@@ -1,0 +1,57 @@
+"""Outputs that leave a GEMM in whole lines, rows exchanged between lanes: every column remainder (lines, 64-byte pieces, 16-byte
+chunks, none of them), row remainders of the 8 rows a store covers, the widest output, and nothing written around D.
+Operands are small integers, so every sum is exact in fp32 and results are compared bit for bit."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SMALL = [(57, 32), (64, 48), (72, 36), (9, 8), (65, 130), (200, 96)]                            # 64-wide tiles
+LARGE = [(4088, 4096), (4081, 4112), (4095, 4104), (3849, 4100), (4097, 3842)]                   # 256-wide tiles
+
+
+def _check(M, N, K, odt, acc, form="plain", full=True):
+    from nanotron_amd import _native as nt
+
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(M * 5 + N)
+    a, b = (torch.randint(-2, 3, (r, K), generator=g, device=dev, dtype=torch.int8) for r in (M, N))
+    aq, bq = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (a, b))
+    if form != "plain":
+        bq = bq.t().contiguous()
+    if form == "both":
+        aq = aq.t().contiguous()
+    guard = 64
+    out = torch.full((guard + M * N + guard,), 9.0, dtype=odt, device=dev)
+    one = torch.ones(1, device=dev)
+    d = nt.GemmDesc(A=aq.data_ptr(), scale_a=one.data_ptr(), B=bq.data_ptr(), scale_b=one.data_ptr(),
+                    D=out.data_ptr() + guard * out.element_size(), M=M, N=N, K=K, fmt_a=nt.E4M3, fmt_b=nt.E4M3,
+                    d_dtype=nt.TORCH_TO_NT[odt], accumulate=int(acc), b_transposed=int(form != "plain"), a_transposed=int(form == "both"))
+    print(f"M={M} N={N} K={K} {odt} acc={acc} {form}", flush=True)
+    st = torch.cuda.current_stream().cuda_stream
+    assert nt._lib.ntfp8_gemm_batch(ctypes.byref(d), 1, st) == 0
+    assert bool((out[:guard] == 9.0).all()) and bool((out[guard + M * N:] == 9.0).all())
+    got = out[guard:guard + M * N].view(M, N)
+    cols = slice(0, N) if full else torch.cat([torch.arange(0, 300), torch.arange(N // 2, N // 2 + 300), torch.arange(N - 300, N)]).to(dev)
+    want = a.float() @ b[cols].float().t() + (9.0 if acc else 0.0)
+    assert torch.equal(got[:, cols], want.to(odt))
+
+
+@pytest.mark.parametrize("mn", SMALL + LARGE)
+@pytest.mark.parametrize("odt,acc", [(torch.float32, False), (torch.float32, True), (torch.bfloat16, False)])
+def test_every_remainder(mn, odt, acc):
+    _check(*mn, 272, odt, acc)
+
+
+@pytest.mark.parametrize("mn", [(144, 144), (4096, 4112), (4112, 3856)])
+@pytest.mark.parametrize("acc", [False, True])
+def test_transposed_operands(mn, acc):
+    _check(*mn, 272, torch.float32, acc, "both")
+
+
+@pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
+def test_more_columns_than_32_bit_offsets_reach(odt):
+    _check(24, (1 << 22) + 16, 272, odt, False, full=False)
+    _check(24, (1 << 22) - 16, 272, odt, False, full=False)
