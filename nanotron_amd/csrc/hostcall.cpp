@@ -168,6 +168,7 @@ struct Scalars {
     float* p;
     explicit Scalars(const at::Tensor& like)
         : both(at::empty({2}, at::TensorOptions().dtype(at::kFloat).device(like.device()))), p(static_cast<float*>(both.data_ptr())) {}
+    Scalars(at::Tensor inside, float* at) : both(std::move(inside)), p(at) {}   // two values inside an allocation of something else
     at::Tensor element(int64_t i) const {
         at::Tensor v = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(both.storage()), both.key_set(), both.dtype());
         v.unsafeGetTensorImpl()->set_sizes_and_strides(c10::IntArrayRef{}, c10::IntArrayRef{}, i);
@@ -215,13 +216,22 @@ struct Quantised {
 };
 PyObject* quantised(Quantised&& q) { return quantised(std::move(q.out), std::move(q.out_t), q.s); }
 
+// Room for the bytes and the scalars of a quantisation.  `together`: one allocation, which nobody outside the call will see
+Quantised room_for(const at::Tensor& x, bool together) {
+    if (!together) return Quantised{bytes_like(x, x.sizes()), at::Tensor(), Scalars(x)};
+    const int64_t n = (x.numel() + 15) / 16 * 16;
+    at::Tensor buf = bytes_like(x, {n + 2 * (int64_t)sizeof(float)});
+    float* const p = reinterpret_cast<float*>(static_cast<char*>(buf.data_ptr()) + n);
+    return Quantised{buf, at::Tensor(), Scalars(buf, p)};
+}
+
 // A dense tensor on a CUDA device.  buf [scale, hist[0..H-1]] null: current scaling; flag given: the role may not hold a scale
 // yet; otherwise the fused delayed-scaling step
-Quantised quantise(const at::Tensor& x, int fmt, int margin, float* buf, float* flag, int hist, bool with_t) {
+Quantised quantise(const at::Tensor& x, int fmt, int margin, float* buf, float* flag, int hist, bool with_t, bool together = false) {
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
-    Quantised q{bytes_like(x, x.sizes()), at::Tensor(), Scalars(x)};
+    Quantised q = room_for(x, together);
     if (with_t) q.out_t = bytes_like(x, {cols, rows});
     void* st = stream_of(x);
     void* ws = workspace_of(x, st);
@@ -237,11 +247,11 @@ Quantised quantise(const at::Tensor& x, int fmt, int margin, float* buf, float* 
         call(ntfp8_quantize_delayed(x.data_ptr(), xd, rows, cols, fmt, margin, buf, buf + 1, hist, p, p + 1, out, tp, ws, st), "ntfp8_quantize_delayed");
     return q;
 }
-Quantised cast_held(const at::Tensor& x, const float* scale, int fmt, bool with_t) {
+Quantised cast_held(const at::Tensor& x, const float* scale, int fmt, bool with_t, bool together = false) {
     int64_t rows, cols;
     rows_cols(x, &rows, &cols);
     require(!with_t || x.dim() == 2, "with_transpose needs a 2-D tensor");
-    Quantised q{bytes_like(x, x.sizes()), at::Tensor(), Scalars(x)};
+    Quantised q = room_for(x, together);
     if (with_t) q.out_t = bytes_like(x, {cols, rows});
     call(ntfp8_cast_with_scale(x.data_ptr(), code_of(x.scalar_type()), rows, cols, scale, fmt, q.s.p, q.s.p + 1, q.out.data_ptr(),
                                with_t ? q.out_t.data_ptr() : nullptr, stream_of(x)),
@@ -524,8 +534,9 @@ bool bytes_of(const at::Tensor& t, c10::Device device) {
 }
 
 // linear_forward(x, fmt, margin, state | None, history_len, held, wants a transposed copy unless dW's GEMM reads the input as it
-// is, read_b, weight bytes, fmt, scale, bias | None, out_code) -> (y, bytes, bytes^T | None, amax, scale) | None: quantisation of the input (current scaling, the fused
-// delayed-scaling step, or, with `held`, a cast with the state's scale that leaves the state alone) and Y = X . W^T
+// is, read_b, weight bytes, fmt, scale, bias | None, out_code, only_y) -> (y, bytes, bytes^T | None, amax, scale) | None: quantisation of the input (current scaling, the fused
+// delayed-scaling step, or, with `held`, a cast with the state's scale that leaves the state alone) and Y = X . W^T.  `only_y`: (y,),
+// for a pass that nobody will look at the operands of
 PyObject* linear_forward(PyObject* const* p) {
     const at::Tensor &input = tensor(p[0]), &w = tensor(p[8]);
     if (!input.is_cuda() || input.dim() < 1 || input.numel() == 0 || code_of(input.scalar_type()) < 0 || !bytes_of(w, input.device()) ||
@@ -549,7 +560,8 @@ PyObject* linear_forward(PyObject* const* p) {
         require(bias.dim() == 1 && bias.size(0) == N && bias.device() == x.device(), "bias must hold one value per output column");
         require(code_of(bias.scalar_type()) >= 0, "unsupported bias dtype");
     }
-    Quantised q = held ? cast_held(x, buf, fmt, with_t) : quantise(x, fmt, (int)number(p[2]), buf, nullptr, hist, with_t);
+    const bool only_y = truth(p[13]);
+    Quantised q = held ? cast_held(x, buf, fmt, with_t, only_y) : quantise(x, fmt, (int)number(p[2]), buf, nullptr, hist, with_t, only_y);
     std::vector<int64_t> shape(input.sizes().begin(), input.sizes().end());
     shape.back() = N;
     at::Tensor y = at::empty(shape, at::TensorOptions().dtype(type_of(out_code)).device(x.device()));
@@ -557,7 +569,71 @@ PyObject* linear_forward(PyObject* const* p) {
     gemm_desc(&d, q.out, fmt, q.s.p + 1, w, (int)number(p[9]), sw, y, M, N, K, false, false, false);
     if (bias.defined()) d.bias = bias.data_ptr(), d.bias_dtype = code_of(bias.scalar_type());
     multiply(&d, 1, stream_of(x));
+    if (only_y) return Py_BuildValue("(N)", wrap(std::move(y)));
     return Py_BuildValue("(NNNNN)", wrap(std::move(y)), wrap(std::move(q.out)), wrap_or_none(std::move(q.out_t)), wrap(q.s.element(0)), wrap(q.s.element(1)));
+}
+
+// linear_forward_fp8(x, its scale where it is fp8 bytes | None, fmt, margin, state | None, history_len, wants a transposed copy unless dW's GEMM
+// reads the input as it is, read_b, weight bytes, fmt, scale, bias | None, out_code, (state, history_len, margin, wants a transposed
+// copy) of an fp8 output | None) -> ((y, y^T | None, amax, scale) of an fp8 output or y, (bytes, bytes^T | None, amax, scale) of an
+// input quantised here | None) | None: the forward pass of a layer that takes or hands on fp8 activations
+PyObject* linear_forward_fp8(PyObject* const* p) {
+    const at::Tensor &x = tensor(p[0]), &w = tensor(p[8]);
+    const bool quantised_already = !none(p[1]), fp8_out = !none(p[13]);
+    if (!x.is_cuda() || x.numel() == 0 || !bytes_of(w, x.device()) || x.dim() < 1 || x.size(-1) != w.size(1)) Py_RETURN_NONE;
+    if (quantised_already ? !bytes_of(x, x.device()) : code_of(x.scalar_type()) < 0) Py_RETURN_NONE;
+    const long out_code = number(p[12]);
+    if (out_code < 0 || (out_code > NTFP8_BF16) != fp8_out) Py_RETURN_NONE;
+    const int64_t K = w.size(1), N = w.size(0), M = x.numel() / K;
+    const int fmt = (int)number(p[2]), hist = (int)number(p[5]);
+    const bool with_t = truth(p[6]) && !(truth(p[7]) && reads_b(N, K, M));
+    const float *sw = values(p[10], x.device()), *sx = quantised_already ? values(p[1], x.device()) : nullptr;
+    float* const buf = quantised_already || none(p[4]) ? nullptr : values(p[4], x.device(), 1 + hist);
+    at::Tensor bias;
+    if (!none(p[11])) {
+        bias = dense(tensor(p[11]));
+        require(bias.dim() == 1 && bias.size(0) == N && bias.device() == x.device(), "bias must hold one value per output column");
+        require(code_of(bias.scalar_type()) >= 0, "unsupported bias dtype");
+    }
+    int out_hist = 0, out_margin = 0;
+    float* out_state = nullptr;
+    bool out_with_t = false;
+    if (fp8_out) {
+        PyObject* const role = p[13];
+        if (!PyTuple_Check(role) || PyTuple_GET_SIZE(role) != 4) stop(PyExc_TypeError, "the role of an fp8 output is a tuple of 4");
+        out_hist = (int)number(PyTuple_GET_ITEM(role, 1)), out_margin = (int)number(PyTuple_GET_ITEM(role, 2));
+        out_with_t = truth(PyTuple_GET_ITEM(role, 3));
+        out_state = values(PyTuple_GET_ITEM(role, 0), x.device(), 1 + out_hist);
+    }
+    std::optional<Quantised> q;
+    if (!quantised_already) {
+        at::Tensor h = dense(x);
+        if (h.dim() != 2) h = h.view({M, K});
+        q = quantise(h, fmt, (int)number(p[3]), buf, nullptr, hist, with_t);
+        sx = q->s.p + 1;
+    }
+    // (an fp8 output is [tokens, features] whatever the input's shape: what the next layer multiplies)
+    std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    if (fp8_out) shape = {M, N};
+    at::Tensor y = at::empty(shape, at::TensorOptions().dtype(type_of(out_code)).device(x.device())), y_t;
+    ntfp8_gemm_desc d;
+    gemm_desc(&d, q ? q->out : x, fmt, sx, w, (int)number(p[9]), sw, y, M, N, K, false, false, false);
+    if (bias.defined()) d.bias = bias.data_ptr(), d.bias_dtype = code_of(bias.scalar_type());
+    PyObject* res;
+    if (fp8_out) {
+        if (out_with_t) y_t = bytes_like(x, {N, M});
+        const Scalars s(x);
+        d.d_dtype = (int)out_code;
+        d.scale_d = out_state;
+        d.D_t = out_with_t ? y_t.data_ptr() : nullptr;
+        multiply_fp8(d, out_margin, out_state, out_hist, s, stream_of(x));
+        res = quantised(std::move(y), std::move(y_t), s);
+    } else {
+        multiply(&d, 1, stream_of(x));
+        res = wrap(std::move(y));
+    }
+    return Py_BuildValue("(NN)", res, q ? quantised(std::move(*q)) : Py_NewRef(Py_None));
 }
 
 // linear_backward(dY, its scale where it is fp8 bytes | None, input bytes, their transposed copy | None, fmt, scale, weight bytes, their
@@ -713,7 +789,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define NT_METHOD(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, count>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NT_METHOD(quantize, 7), NT_METHOD(quantize_batch, 2), NT_METHOD(gemm, kProblem), NT_METHOD(gemm_batch, 1), NT_METHOD(gemm_fp8, kProblem + 4),
                          NT_METHOD(cast, 4), NT_METHOD(cast_with_scale, 4), NT_METHOD(column_sum, 2), NT_METHOD(dequantize, 5), NT_METHOD(transpose, 1), NT_METHOD(b_transposed_supported, 3),
-                         NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 13), NT_METHOD(linear_backward, 22),
+                         NT_METHOD(operand_form, 10), NT_METHOD(linear_forward, 14), NT_METHOD(linear_forward_fp8, 14), NT_METHOD(linear_backward, 22),
                          NT_METHOD(workspace, 1), NT_METHOD(workspace_pool, 2), NT_METHOD(drop_workspaces, 0), NT_METHOD(set_check, 1), NT_METHOD(set_gemm_observer, 1), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

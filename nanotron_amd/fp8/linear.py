@@ -12,7 +12,15 @@ from nanotron_amd.fp8 import kernel as _kernel
 from nanotron_amd.fp8.kernel import a_transposed_supported, fp8_matmul_kernel, fp8_matmul_pair, needs_transposed_copy
 from nanotron_amd.fp8.meta import FP8Meta
 from nanotron_amd.fp8.parameter import FP8Parameter
-from nanotron_amd.fp8.tensor import DelayedScaling, FP8Tensor, _assemble, _keep_transposed, cast_with_scale, update_scaling_factor
+from nanotron_amd.fp8.tensor import (
+    DelayedScaling,
+    FP8Tensor,
+    _assemble,
+    _keep_transposed,
+    cast_with_scale,
+    quantize_delayed,
+    update_scaling_factor,
+)
 
 
 class FP8LinearMeta(TypedDict):
@@ -130,8 +138,14 @@ class FP8Linear(nn.Linear):
         on the current one, so it overlaps whatever the current stream does next (typically the
         MFMA-bound GEMMs of other layers); the next forward of this layer waits for it."""
         w = self.weight
-        hp = w.as_subclass(torch.Tensor)
         state = self.scaling["weight"] if self.scaling is not None else None
+        if (stream is None and state is not None and state.known_initialised and state.dtype is DTypes.FP8E4M3
+                and w.dtype in nt.TORCH_TO_NT and state._buf.device == w.device):
+            w.data = quantize_delayed(w, state, needs_transposed_copy(*w.shape))
+            if self._weight_ready is not None:
+                self._weight_ready = None
+            return
+        hp = w.as_subclass(torch.Tensor)
         if stream is None:
             w.data = FP8Tensor(hp, dtype=DTypes.FP8E4M3, state=state, with_transpose=needs_transposed_copy(*hp.shape))
             if self._weight_ready is not None:
@@ -215,7 +229,7 @@ class FP8Linear(nn.Linear):
 
         if type(input) is torch.Tensor and not torch.is_grad_enabled() and _no_transform():
             # nothing to record: the two kernels, past autograd's machinery
-            quick = _quantise_and_multiply(self, input, weight, self.bias, False)
+            quick = _quantise_and_multiply(self, input, weight, self.bias, False, True)
             if quick is not None:
                 return quick[0]
         # phony tensor that makes autograd call our backward although the weight's gradient is
@@ -283,6 +297,18 @@ class _FP8Matmul(torch.autograd.Function):
             ctx.fp8_out = False
             ctx.out_shape, ctx.out_dtype = output.shape, output.dtype
             return output, phony
+        if module is not None and (not plain or isinstance(module.out_dtype, DTypes)):
+            quick = _multiply_fp8(module, input, weight, bias, needs_wgrad)
+        if quick is not None:
+            output, made = quick
+            ctx.save_for_backward(_assemble(FP8Tensor, DTypes.FP8E4M3, *made) if made is not None else input, weight, bias)
+            ctx.module = module
+            ctx.fp8_meta = fp8_meta
+            if isinstance(output, tuple):
+                return _hand_on(ctx, module, weight, _assemble(FP8Tensor, module.out_dtype, *output))
+            ctx.fp8_out = False
+            ctx.out_shape, ctx.out_dtype = output.shape, output.dtype
+            return output, phony
         if plain:
             x2d = input if len(in_shape) == 2 else input.reshape(-1, in_shape[-1])
             input = FP8Tensor(x2d, dtype=DTypes.FP8E4M3, state=scaling["input"] if scaling else None,
@@ -304,15 +330,7 @@ class _FP8Matmul(torch.autograd.Function):
                 mat_a=weight.data, transpose_a=True, mat_b=input, transpose_b=False, use_split_accumulator=False,
                 out_dtype=out_dtype, out_state=state, out_with_transpose=module.fp8_output_transpose, bias=gemm_bias,
             )
-            ctx.mark_non_differentiable(output)
-            ctx.grad_box = _GradBox(scaling["output_grad"] if scaling else None)
-            object.__setattr__(module, "_grad_box", ctx.grad_box)   # (a plain value: nn.Module's own way takes 2 us)
-            hp = weight.dtype if weight.dtype in (torch.float32, torch.float16, torch.bfloat16) else torch.float32
-            out_shape = output.as_subclass(torch.Tensor).shape
-            handle = module._zero(hp, weight.device).expand(out_shape)
-            ctx.fp8_out = True
-            ctx.out_shape, ctx.out_dtype = out_shape, hp
-            return output, handle
+            return _hand_on(ctx, module, weight, output)
         ctx.fp8_out = False
         output = fp8_matmul_kernel(
             mat_a=weight.data, transpose_a=True, mat_b=input, transpose_b=False, use_split_accumulator=False,
@@ -427,6 +445,19 @@ class _FP8Matmul(torch.autograd.Function):
         return grad_input, None, None, None, None, grad_bias, None
 
 
+def _hand_on(ctx, module: FP8Linear, weight, output: FP8Tensor):
+    """The two outputs of a forward pass that returns fp8 bytes: they and the handle that their gradient travels through."""
+    ctx.mark_non_differentiable(output)
+    ctx.grad_box = _GradBox(module.scaling["output_grad"] if module.scaling else None)
+    object.__setattr__(module, "_grad_box", ctx.grad_box)   # (a plain value: nn.Module's own way takes 2 us)
+    hp = weight.dtype if weight.dtype in (torch.float32, torch.float16, torch.bfloat16) else torch.float32
+    out_shape = output.as_subclass(torch.Tensor).shape
+    handle = module._zero(hp, weight.device).expand(out_shape)
+    ctx.fp8_out = True
+    ctx.out_shape, ctx.out_dtype = out_shape, hp
+    return output, handle
+
+
 # What tells whether a functorch transform or a tracer is active (None: no).  These are no public names of torch: where one is
 # missing nobody can tell, and the answer is never None.
 _unknown = lambda: "unknown"   # noqa: E731
@@ -440,9 +471,10 @@ def _no_transform() -> bool:
     return getattr(forward_ad, "_current_level", 0) < 0 and _functorch_active() is None and _tracing_state() is None
 
 
-def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, needs_wgrad: bool):
+def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, needs_wgrad: bool, only_y: bool = False):
     """(Y, input bytes, their transposed copy, amax, scale) of a layer's forward pass through one native call, with the results
-    of FP8Tensor(x, ...) and fp8_matmul_kernel; None where it does not serve the case, nothing done."""
+    of FP8Tensor(x, ...) and fp8_matmul_kernel, or (Y,) where nobody will see the others; None where it does not serve the case,
+    nothing done."""
     out_code = nt.TORCH_TO_NT.get(module.out_dtype or torch.float32)
     if out_code is None or not isinstance(weight, FP8Parameter):
         return None
@@ -455,7 +487,44 @@ def _quantise_and_multiply(module: FP8Linear, x: torch.Tensor, weight, bias, nee
     w = weight.data
     meta = w.fp8_meta
     return nt.host.linear_forward(x, nt.E4M3, margin, buf, history_len, held, needs_wgrad, _kernel.READ_B_TRANSPOSED, w,
-                                  meta.dtype.code, meta.scale, bias, out_code)
+                                  meta.dtype.code, meta.scale, bias, out_code, only_y)
+
+
+def _multiply_fp8(module: FP8Linear, x, weight, bias, needs_wgrad: bool):
+    """((bytes, transposed copy, amax, scale) of an fp8 output or Y, the same of an input quantised on the way or None) of the forward
+    pass of a layer that takes or hands on fp8 activations, through one native call, with the results of FP8Tensor(x, ...)
+    and fp8_matmul_kernel; None where it does not serve the case, nothing done."""
+    if not isinstance(weight, FP8Parameter):
+        return None
+    scaling = module.scaling
+    x_scale, x_fmt, buf, history_len, margin, role = None, nt.E4M3, None, 0, 0, None
+    if type(x) is FP8Tensor:
+        meta = getattr(x, "fp8_meta", None)
+        if meta is None or not isinstance(meta.scale, torch.Tensor):
+            return None
+        x_scale, x_fmt = meta.scale, meta.dtype.code
+    elif type(x) is not torch.Tensor or scaling is None or not module.training:
+        return None
+    else:
+        state = scaling["input"]
+        if not state.known_initialised or state.dtype is not DTypes.FP8E4M3:
+            return None
+        buf, history_len, margin = state._buf, state.history_len, state.margin
+    out_dtype = module.out_dtype
+    if isinstance(out_dtype, DTypes):
+        # (an evaluation pass casts with a copy of the role, a role without a scale goes the long way)
+        state = scaling["output"] if scaling is not None and module.training else None
+        if state is None or not state.known_initialised or state.dtype is not out_dtype:
+            return None
+        out_code, role = out_dtype.out_code, (state._buf, state.history_len, state.margin, module.fp8_output_transpose)
+    else:
+        out_code = nt.TORCH_TO_NT.get(out_dtype or torch.float32)
+    if out_code is None or x_fmt is None:
+        return None
+    w = weight.data
+    meta = w.fp8_meta
+    return nt.host.linear_forward_fp8(x, x_scale, x_fmt, margin, buf, history_len, needs_wgrad, _kernel.READ_B_TRANSPOSED, w,
+                                      meta.dtype.code, meta.scale, bias, out_code, role)
 
 
 def _backward_passes(ctx, module: FP8Linear, grad_output, input: FP8Tensor, weight, bias, wants_dx: bool, box: Optional[_GradBox]):

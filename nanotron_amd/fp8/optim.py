@@ -5,6 +5,7 @@ and never again; its optimizers update the high-precision storage only
 (src/nanotron/optim/gradient_accumulator.py:257-267 copies the fp32 master back into the half-precision
 parameter after each step).  A training loop therefore has to refresh the fp8 copy, and the transposed copy the
 dgrad GEMM reads, after every optimizer step; these helpers do that."""
+from contextlib import nullcontext
 from typing import Iterable, Optional, Union
 
 import torch
@@ -45,8 +46,8 @@ def requantize_fp8_weights(module_or_modules, stream: Optional[torch.cuda.Stream
             if len(lins) < 2:
                 rest += lins
                 continue
-            with torch.cuda.device(dev):
-                hp = [lin.weight.as_subclass(torch.Tensor) for lin in lins]
+            with torch.cuda.device(dev) if dev.index != torch.cuda.current_device() else nullcontext():
+                hp = [lin.weight for lin in lins]   # (the extension reads a parameter as the tensor that it is)
                 qs = quantize_delayed_batch(hp, DTypes.FP8E4M3, [lin.scaling["weight"] for lin in lins],
                                             [needs_transposed_copy(*w.shape) for w in hp])
             for lin, q in zip(lins, qs):

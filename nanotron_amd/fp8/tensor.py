@@ -183,6 +183,13 @@ def _keep_transposed(q: FP8Tensor, transposed: torch.Tensor) -> FP8Tensor:
     return t
 
 
+def quantize_delayed(tensor: torch.Tensor, state: DelayedScaling, with_transpose: bool) -> FP8Tensor:
+    """FP8Tensor(tensor, state.dtype, state=state, with_transpose=with_transpose) of a tensor that can be quantised, for a
+    state of its device that already holds a scale."""
+    return _assemble(FP8Tensor, state.dtype, *nt.host.quantize(tensor, state.dtype.code, state.margin, state._buf, None,
+                                                               state.history_len, with_transpose))
+
+
 @torch.no_grad()
 def quantize_delayed_batch(tensors, dtype: DTypes, states, with_transpose) -> list:
     """[FP8Tensor(t, dtype, state=s, with_transpose=w) for t, s, w in zip(tensors, states, with_transpose)] for
