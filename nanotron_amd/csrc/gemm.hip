@@ -9,7 +9,7 @@
 //   gemm_nt_big_kernel    (gemm_big.h) 256 x 256 x 128 tiles, 4 waves of 128 x 128 with 16x16x128 MFMAs,
 //                         loads straight into LDS, two stages.  The partial last round of tiles over the CUs is
 //                         cut into 128-row half tiles.
-//   gemm_mid_kernel       (gemm_mid.h) 128 x 128 and 64 x 64 tiles of the same instruction, loads straight into four LDS
+//   gemm_mid_kernel       (gemm_mid.h) 128 x 128, 128 x 64 and 64 x 64 tiles of the same instruction, loads straight into four LDS
 //                         stages: shapes that have too few 256-wide tiles, and operands beyond the 2 GiB reach of a
 //                         buffer descriptor's 32-bit offsets.
 //   gemm_few_kernel       (gemm_few.h) up to 32 rows against a full-size weight: 16 or 32 columns per workgroup, K
@@ -29,7 +29,7 @@ namespace ntfp8 {
 constexpr int kMinTransposed = 128;   // rows and columns of a result whose B is given as its transpose: more than this
 enum GemmPath { kPathNone = -1, kPathAny = 0, kPathPlain = 1, kPathTiles = 2 };
 
-int launch_mid(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
+int launch_mid(const BigLaunch& L, int fa, int fb, int tile_m, int tile_n, bool fp8_out, int tiles, hipStream_t st);
 int launch_few(const BigProblem& p, int fa, int fb, hipStream_t st);
 int launch_any(const BigLaunch& L, int fa, int fb, int tile, bool fp8_out, int tiles, hipStream_t st);
 int launch_plain(const GemmDesc& g, hipStream_t st);
@@ -77,31 +77,37 @@ static int path_of(const GemmDesc& g) {
     return (int64_t)g.K * 128 < (1LL << 31) ? kPathTiles : kPathAny;   // (a tile's rows within reach of 32-bit offsets)
 }
 
-// What a launch of `n` problems takes in tiles of edge 256, 128 or 64, in nanoseconds: rounds of workgroups times what a
+// What a launch of `n` problems takes in tiles of 256 x 256, 128 x 128, 128 x 64 or 64 x 64, in nanoseconds: rounds of workgroups times what a
 // workgroup takes for its K-tiles and for everything else.  The constants are fits to launches of one problem with
 // bf16 output (plain / B transposed / both transposed), warm operands; what matters is where the lines cross.
 //   us, 256 / 128 / 64 wide:  1024 x 1024 x 1024  10.1 / 7.5 / 4.8     2048 x 1024 x 4096  26.5 / 16.3 / 15.3
 //   2048 x 2048 x 2048  16.7 / 11.8 / 16.9      both transposed  19.6 / 12.6 / 24.3
 //   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101
+//   128 x 128 / 128 x 64 / 64 x 64:  2048 x 1024 x 1024 7.6 / 5.9 / 6.6, x 4096 15.6 / 12.9 / 15.2; B transposed 8.0 / 6.6 / 8.0 and
+//   16.9 / 16.3 / 20.2; both transposed x 2048 12.1 / 10.4 / 13.6; 1021 x 2304 x 1024 (288 tiles of 128 x 64) 7.8 / 10.4 / 9.0
 //   at equal estimates:   3696 x 1088 x 944 (bf16) 10.6 / - / 11.8     1072 x 3600 x 320 (fp8 output) 12.5 / - / 17.6,
 //                         528 x 2528 x 1008 with its weight gradient 19.5 / - / 14.8
 // Several problems: by their average depth.  (The end of the list as the CUs work it off, longest tile first, predicts
 // single launches no better and chose worse for one pair in twenty, up to 10.7 -> 18.1 us, though 4 % better on average.)
-static int64_t launch_cost(const GemmDesc* const* g, int n, int edge, int64_t cus) {
+struct Edge {
+    int m, n;
+};
+static int64_t launch_cost(const GemmDesc* const* g, int n, Edge edge, int64_t cus) {
     int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
     int form = 0;
     for (int i = 0; i < n; ++i) {
-        const int64_t t = (((int64_t)g[i]->M + edge - 1) / edge) * (((int64_t)g[i]->N + edge - 1) / edge);
+        const int64_t t = (((int64_t)g[i]->M + edge.m - 1) / edge.m) * (((int64_t)g[i]->N + edge.n - 1) / edge.n);
         tiles += t;
         kt += t * ((g[i]->K + kBK - 1) / kBK);
         form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
     }
     const int64_t k = kt / tiles;   // K-tiles of an average tile
-    if (edge == 256) {
+    if (edge.m == 256) {
         const int64_t rem = tiles % cus, full = tiles / cus;
         return full * (1400 * k + 7000) + (rem == 0 ? 0 : 2 * rem <= cus ? 700 * k + 7000 : 1400 * k + 7000);
     }
-    if (edge == 128) return ((tiles + cus - 1) / cus) * (390 * k + 5200);
+    if (edge.n == 128) return ((tiles + cus - 1) / cus) * (390 * k + 5200);
+    if (edge.m == 128) return ((tiles + cus - 1) / cus) * ((form ? 400 : 290) * k + 3600);
     // two workgroups per CU
     static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
     const int64_t rem = tiles % (2 * cus), full = tiles / (2 * cus);
@@ -110,7 +116,7 @@ static int64_t launch_cost(const GemmDesc* const* g, int n, int edge, int64_t cu
 
 // The tile list of a launch, problem by problem, longest K first: the long tiles start together and the shorter ones fill
 // the rounds behind them.  Returns the number of tiles.
-static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* L) {
+static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch* L) {
     int order[kBigMaxProblems];
     for (int i = 0; i < n; ++i) order[i] = i;
     for (int i = 1; i < n; ++i)   // insertion sort, stable, K descending
@@ -133,8 +139,8 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, int edge, BigLaunch* 
         p.M = d.M;
         p.N = d.N;
         p.K = d.K;
-        p.tiles_m = (d.M - 1) / edge + 1;
-        p.tiles_n = (d.N - 1) / edge + 1;
+        p.tiles_m = (d.M - 1) / edge.m + 1;
+        p.tiles_n = (d.N - 1) / edge.n + 1;
         p.tile_begin = (int)tiles;
         p.d_dtype = d.d_dtype;
         p.accumulate = d.accumulate;
@@ -178,14 +184,15 @@ static int finish_behind(const GemmDesc& g, int rc, hipStream_t st) {
 template <int FA, int FB>
 static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     const int cus = cu_count();   // (asked once: the question goes to the runtime)
-    int edge = 128;
+    Edge edge{128, 128};
     {
         bool big = true;
         for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
-        int64_t best = launch_cost(g, n, 128, cus);
+        int64_t best = launch_cost(g, n, edge, cus);
         // (where the lines meet, the wider tiles for one problem, the narrower for several)
-        for (const int e : {n == 1 ? 256 : 64, n == 1 ? 64 : 256}) {
-            if (e == 256 && !big) continue;
+        const int first = n == 1 ? 256 : 64;
+        for (const Edge e : {Edge{first, first}, Edge{320 - first, 320 - first}, Edge{128, 64}}) {
+            if (e.m == 256 && !big) continue;
             const int64_t c = launch_cost(g, n, e, cus);
             if (c < best) best = c, edge = e;
         }
@@ -194,10 +201,10 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     const int64_t tiles = list_tiles(g, n, edge, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     const bool fp8_out = is_fp8_out(g[0]->d_dtype);
-    L.round_size = cus * (edge == 64 ? 2 : 1);
+    L.round_size = cus * (edge.m == 64 ? 2 : 1);
     finish_inside(g, n, tiles, &L);
-    if (edge != 256) {
-        const int rc = launch_mid(L, FA, FB, edge, fp8_out, (int)tiles, st);
+    if (edge.m != 256) {
+        const int rc = launch_mid(L, FA, FB, edge.m, edge.n, fp8_out, (int)tiles, st);
         return L.fin_blocks ? rc : finish_behind(*g[0], rc, st);
     }
     const int rem = (int)(tiles % cus);
@@ -234,8 +241,8 @@ static int launch_any_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     BigLaunch L;
     int edge = 128;
     const int cus = cu_count();
-    int64_t tiles = list_tiles(g, n, edge, &L);
-    if (tiles < cus) tiles = list_tiles(g, n, edge = 64, &L);
+    int64_t tiles = list_tiles(g, n, Edge{edge, edge}, &L);
+    if (tiles < cus) edge = 64, tiles = list_tiles(g, n, Edge{edge, edge}, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     L.round_size = 2 * cus;   // (LDS: two workgroups of 128-wide tiles on a CU, more of the others)
     finish_inside(g, n, tiles, &L);
@@ -262,14 +269,14 @@ static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
 #else
     if (path == kPathAny && n == 1 && tiny(*g[0])) {
         BigLaunch L;
-        list_tiles(g, 1, 64, &L);
+        list_tiles(g, 1, Edge{64, 64}, &L);
         return finish_behind(*g[0], launch_tiny(L.p[0], fa, fb, st), st);
     }
     if (path == kPathAny) return launch_any_tiles(g, n, st);
     if (path == kPathPlain || (n == 1 && short_k(*g[0]))) return finish_behind(*g[0], launch_plain(*g[0], st), st);
     if (n == 1 && few_rows(*g[0])) {
         BigLaunch L;
-        list_tiles(g, 1, 64, &L);
+        list_tiles(g, 1, Edge{64, 64}, &L);
         return launch_few(L.p[0], fa, fb, st);
     }
     if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, st) : launch_tiles<kE4M3, kE5M2>(g, n, st);

@@ -1,4 +1,4 @@
-"""Outputs that leave a GEMM in whole lines, rows exchanged between lanes: every column remainder (lines, 64-byte pieces, 16-byte
+"""Edges of the tiles that leave a GEMM in whole lines (256, 128 x 64 and 64 wide), rows exchanged between lanes: every column remainder (lines, 64-byte pieces, 16-byte
 chunks, none of them), row remainders of the 8 rows a store covers, the widest output, and nothing written around D.
 Operands are small integers, so every sum is exact in fp32 and results are compared bit for bit."""
 import ctypes
@@ -9,6 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SMALL = [(57, 32), (64, 48), (72, 36), (9, 8), (65, 130), (200, 96)]                            # 64-wide tiles
+NARROW = [(2048, 1024), (1921, 1024), (2048, 961), (1935, 1000), (2045, 964)]                     # 128 x 64 tiles: one round of workgroups
 LARGE = [(4088, 4096), (4081, 4112), (4095, 4104), (3849, 4100), (4097, 3842)]                   # 256-wide tiles
 
 
@@ -39,16 +40,42 @@ def _check(M, N, K, odt, acc, form="plain", full=True):
     assert torch.equal(got[:, cols], want.to(odt))
 
 
-@pytest.mark.parametrize("mn", SMALL + LARGE)
+@pytest.mark.parametrize("mn", SMALL + NARROW + LARGE)
 @pytest.mark.parametrize("odt,acc", [(torch.float32, False), (torch.float32, True), (torch.bfloat16, False)])
 def test_every_remainder(mn, odt, acc):
     _check(*mn, 272, odt, acc)
 
 
-@pytest.mark.parametrize("mn", [(144, 144), (4096, 4112), (4112, 3856)])
+@pytest.mark.parametrize("mn", [(144, 144), (4096, 4112), (4112, 3856), (2048, 1024), (1936, 976), (2032, 1008)])
 @pytest.mark.parametrize("acc", [False, True])
 def test_transposed_operands(mn, acc):
     _check(*mn, 272, torch.float32, acc, "both")
+
+
+@pytest.mark.parametrize("mn", NARROW)
+@pytest.mark.parametrize("K", [16, 128, 256, 400, 528, 656])
+def test_narrow_tiles_with_every_number_of_k_tiles(mn, K):
+    _check(*mn, K, torch.float32, False)
+    if K >= 256 and mn[1] % 16 == 0:
+        _check(*mn, K, torch.bfloat16, False, "b")
+
+
+@pytest.mark.parametrize("mn", [(2048, 1024), (1924, 976), (2044, 1008)])
+@pytest.mark.parametrize("form", ["plain", "b"])
+def test_narrow_tiles_with_fp8_outputs(mn, form):
+    from nanotron_amd import _native as nt
+
+    (M, N), K = mn, 272
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    a, b = (torch.randint(-2, 3, (r, K), generator=g, device=dev).float() for r in (M, N))
+    aq, bq = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (a, b if form == "plain" else b.t().contiguous()))
+    one, state = torch.ones(1, device=dev), torch.tensor([0.25, 0.0], device=dev)
+    print(f"{mn} {form}", flush=True)
+    y, y_t, amax, scale = nt.host.gemm_fp8(aq, nt.E4M3, one, bq, nt.E4M3, one, nt.OUT_E4M3, None, form == "b", None, False, state, 1, 0, True)
+    r = a @ b.t()
+    want = (r * 0.25).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(y, want) and torch.equal(y_t, want.t()) and float(amax) == float(r.abs().max()) and float(scale) == 0.25
 
 
 @pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
