@@ -141,6 +141,7 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch*
         p.K = d.K;
         p.tiles_m = (d.M - 1) / edge.m + 1;
         p.tiles_n = (d.N - 1) / edge.n + 1;
+        p.magic = magic_of((uint32_t)kGroupM * (uint32_t)p.tiles_n);
         p.tile_begin = (int)tiles;
         p.d_dtype = d.d_dtype;
         p.accumulate = d.accumulate;
@@ -202,6 +203,7 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
     const bool fp8_out = is_fp8_out(g[0]->d_dtype);
     L.round_size = cus * (edge.m == 64 ? 2 : 1);
+    L.round_magic = magic_of((uint32_t)L.round_size);
     finish_inside(g, n, tiles, &L);
     if (edge.m != 256) {
         const int rc = launch_mid(L, FA, FB, edge.m, edge.n, fp8_out, (int)tiles, st);

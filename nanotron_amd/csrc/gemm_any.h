@@ -78,17 +78,14 @@ __global__ __launch_bounds__(kAnyThreads) void gemm_any_kernel(const BigLaunch L
 
     int pid = blockIdx.x;
     if (gridDim.x % kXcds == 0) pid = (pid % kXcds) * (gridDim.x / kXcds) + pid / kXcds;   // an XCD works on a run of tiles
-    int which = 0;
-#pragma unroll
-    for (int i = 1; i < kBigMaxProblems; ++i)
-        if (i < L.count && pid >= L.p[i].tile_begin) which = i;
-    const BigProblem& P = L.p[which];
-    const uint8_t* __restrict__ A = P.A;
-    const uint8_t* __restrict__ B = P.B;
-    const int M = P.M, N = P.N, K = P.K;
-    pid -= P.tile_begin;
+    const Picked G = pick_problem(L, pid);
+    const BigProblem& P = L.p[G.which];
+    const uint8_t* __restrict__ A = G.A;
+    const uint8_t* __restrict__ B = G.B;
+    const int M = G.M, N = G.N, K = G.K;
+    pid -= G.tile_begin;
     int pid_m, pid_n;
-    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
+    tile_in_group(pid, G.tiles_m, G.tiles_n, G.magic, pid_m, pid_n);
     const int m0 = pid_m * kT, n0 = pid_n * kT;
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;

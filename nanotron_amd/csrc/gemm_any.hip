@@ -85,12 +85,12 @@ __global__ __launch_bounds__(kGemmThreads, 3) void gemm_nt_kernel(const uint8_t*
                                                                void* __restrict__ Dv, const float* __restrict__ scale_a,
                                                                const float* __restrict__ scale_b, int M, int N, int K,
                                                                int tiles_m, int tiles_n, Fp8Out fp8, GemmExtras ex,
-                                                               int d_dtype, int accumulate) {
+                                                               int d_dtype, int accumulate, uint32_t magic) {
     __shared__ __attribute__((aligned(16))) uint8_t sA[kBM * kBK];
     __shared__ __attribute__((aligned(16))) uint8_t sB[kBN * kBK];
 
     int pid_m, pid_n;
-    tile_of_block(tiles_m, tiles_n, pid_m, pid_n);
+    tile_of_block(tiles_m, tiles_n, magic, pid_m, pid_n);
     const int m0 = pid_m * kBM, n0 = pid_n * kBN;
 
     const int t = threadIdx.x;
@@ -197,7 +197,7 @@ static void launch_plain_fmt(const GemmDesc& g, hipStream_t st) {
     const GemmExtras ex = {g.bias, g.bias_dtype, g.scale_inv};
     auto go = [&](auto dt) {
         hipLaunchKernelGGL((gemm_nt_kernel<FA, FB, decltype(dt)::value>), dim3(tm * tn), dim3(kGemmThreads), 0, st, a, b, g.D, g.sa, g.sb,
-                           g.M, g.N, g.K, tm, tn, fp8, ex, g.d_dtype, g.accumulate);
+                           g.M, g.N, g.K, tm, tn, fp8, ex, g.d_dtype, g.accumulate, magic_of((uint32_t)kGroupM * (uint32_t)tn));
     };
     if (g.d_dtype == NTFP8_OUT_E4M3) go(std::integral_constant<int, NTFP8_OUT_E4M3>{});
     else if (g.d_dtype == NTFP8_OUT_E5M2) go(std::integral_constant<int, NTFP8_OUT_E5M2>{});

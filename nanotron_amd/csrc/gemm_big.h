@@ -367,20 +367,23 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
 // layer, say): their tiles form one list, longest K first, so that the rounds of one problem fill up
 // with tiles of the next instead of ending in a partial round and a kernel boundary each.
 struct BigProblem {
+    // what a workgroup needs before its first load (pick_problem)
     const uint8_t* A;
     const uint8_t* B;
-    void* D;
     const float* scale_a;
     const float* scale_b;
     int M, N, K;
-    int tiles_m, tiles_n;   // 256 x 256 tiles
+    int tiles_m, tiles_n;   // in the launch's tile size
+    uint32_t magic;         // magic_of(kGroupM tiles_n)
     int tile_begin;         // position of this problem's first tile in the launch's tile list
-    int d_dtype;            // NTFP8_F32 / NTFP8_F16 / NTFP8_BF16 / NTFP8_OUT_E4M3 / NTFP8_OUT_E5M2
-    int accumulate;         // fp32 outputs only: D += result
-    Fp8Out fp8;             // fp8 outputs only
-    GemmExtras ex;          // bias, inverse-scale flag
     int at;                 // A is given as [K, M] row-major (its transpose); only together with bt
     int bt;                 // B is given as [K, N] row-major (its transpose)
+    // and behind its K loop
+    int d_dtype;            // NTFP8_F32 / NTFP8_F16 / NTFP8_BF16 / NTFP8_OUT_E4M3 / NTFP8_OUT_E5M2
+    int accumulate;         // fp32 outputs only: D += result
+    void* D;
+    Fp8Out fp8;             // fp8 outputs only
+    GemmExtras ex;          // bias, inverse-scale flag
 };
 constexpr int kBigMaxProblems = 4;
 struct BigLaunch {
@@ -389,11 +392,42 @@ struct BigLaunch {
     int full_blocks;        // tiles (of the whole list) computed whole
     int tail_tiles;         // tiles at the end of the list computed as two halves
     int round_size;         // workgroups resident at once
+    uint32_t round_magic;   // magic_of(round_size)
     // a launch of one problem with fp8 outputs: the workgroup that finishes last (of fin_blocks, over both launches of a
     // call with a tail) turns the collected maxima into the output role's bookkeeping (0: left in the workspace)
     int fin_blocks;
     ScalarIO fin;
 };
+
+// The problem that tile `pid` of the launch's list belongs to, as far as a workgroup needs it before its first load.  The fields
+// of the first two problems are read at once and chosen from: looked up by number they come in three dependent trips (which
+// problem, its sizes, its pointers) to a launch's arguments, which are in no cache.  us, looked up and tiles found by
+// divisions / here: 512 x 512 x 512 3.97 / 3.65, 2048 x 1024 x 1024 5.89 / 5.56, 1021 x 2304 x 1024 7.78 / 7.40, 4096 x 4096 x 4096
+// 47.5 / 46.8, dgrad and wgrad of 256 x 256 x 256 4.05 / 3.68.
+struct Picked {
+    const uint8_t *A, *B;
+    const float *scale_a, *scale_b;
+    int M, N, K, tiles_m, tiles_n, tile_begin, at, bt, which;
+    uint32_t magic;
+};
+__device__ __forceinline__ Picked pick_problem(const BigLaunch& L, int pid) {
+    Picked r = {};
+    auto look = [&](int i, bool take) {
+        const BigProblem& p = L.p[i];
+        r.A = take ? p.A : r.A, r.B = take ? p.B : r.B;
+        r.scale_a = take ? p.scale_a : r.scale_a, r.scale_b = take ? p.scale_b : r.scale_b;
+        r.M = take ? p.M : r.M, r.N = take ? p.N : r.N, r.K = take ? p.K : r.K;
+        r.tiles_m = take ? p.tiles_m : r.tiles_m, r.tiles_n = take ? p.tiles_n : r.tiles_n;
+        r.magic = take ? p.magic : r.magic, r.tile_begin = take ? p.tile_begin : r.tile_begin;
+        r.at = take ? p.at : r.at, r.bt = take ? p.bt : r.bt;
+        r.which = take ? i : r.which;
+    };
+    look(0, true);
+    look(1, L.count > 1 && pid >= L.p[1].tile_begin);
+    if (L.count > 2)   // (no registers for the fields of all of them at once)
+        for (int i = 2; i < L.count; ++i) look(i, pid >= L.p[i].tile_begin);
+    return r;
+}
 
 // End of a workgroup with fp8 outputs, its maxima published: `bid` of L.fin_blocks.  Replaces a one-wave kernel behind the
 // GEMM (4.3 us of GPU and 3 us of host time).
@@ -440,7 +474,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         // Workgroups are dealt to the XCDs round robin.  Within each round of `round_size` workgroups (one per
         // CU) an XCD gets a contiguous run of the tile list, so its L2 sees few operand panels; across rounds
         // the list is walked in order, so that the long tiles at its head start together on the whole chip.
-        const int round0 = (pid / L.round_size) * L.round_size;
+        const int round0 = quotient(pid, L.round_size, L.round_magic) * L.round_size;
         const int in_round = min(L.round_size, L.full_blocks - round0);
         const int local = pid - round0;
 #ifdef NTFP8_STAMPS
@@ -454,18 +488,15 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         half = pid & 1;
         pid = L.full_blocks + (pid >> 1);
     }
-    int which = 0;
-#pragma unroll
-    for (int i = 1; i < kBigMaxProblems; ++i)
-        if (i < L.count && pid >= L.p[i].tile_begin) which = i;
-    const BigProblem& P = L.p[which];
-    const uint8_t* __restrict__ A = P.A;
-    const uint8_t* __restrict__ B = P.B;
-    void* __restrict__ Dv = P.D;
-    const int M = P.M, N = P.N, K = P.K;
-    pid -= P.tile_begin;
+    const Picked G = pick_problem(L, pid);
+    const BigProblem& P = L.p[G.which];
+    const uint8_t* __restrict__ A = G.A;
+    const uint8_t* __restrict__ B = G.B;
+    const int M = G.M, N = G.N, K = G.K;
+    const float scale_a = *G.scale_a, scale_b = *G.scale_b;
+    pid -= G.tile_begin;
     int pid_m, pid_n;
-    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
+    tile_in_group(pid, G.tiles_m, G.tiles_n, G.magic, pid_m, pid_n);
     const int n0 = pid_n * kBigN;
     const int m0 = pid_m * 256 + half * 128;
     // this workgroup's place among all of the call
@@ -489,7 +520,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     const int ld_kc = ((lane & 7) ^ (lane >> 3) ^ (wave & 1)) << 4;
     // chunks of the last K-tile at k >= K must read as zero, not as the start of the next row
     const bool tail_dead = (KT - 1) * kBK + ld_kc >= K;
-    const float alpha = descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);
+    float alpha = 0.0f;
 
     constexpr int LA = MI * 2 * 16 / 8 / kBigWaves;  // wave-level loads of the A tile per wave per stage
     constexpr int LB = kBigLB;
@@ -706,6 +737,8 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             if (KT == 2) poison_tail();
 #pragma unroll
             for (int l = 0; l < NL; ++l) issue(1, l);
+            // (behind the first requests: the scales were written by the kernel before, a trip of their own to memory)
+            alpha = descale_factor(scale_a, scale_b, P.ex.scale_inv);
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");   // tile 0 has landed, tile 1 may still be in flight
             wg_barrier();
             NTFP8_STAMP(st_first);
@@ -830,6 +863,9 @@ void gemm_nt_big_kernel(const BigLaunch L) {
             if (KT == 3) poison_tail();
 #pragma unroll
             for (int l = 0; l < NL; ++l) issue(2, l);
+        }
+        alpha = descale_factor(scale_a, scale_b, P.ex.scale_inv);   // (as for whole tiles)
+        if (KT > 2) {
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL) : "memory");
         } else {
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
@@ -865,7 +901,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         }
     };
     if constexpr (kBT) {
-        if (P.at) kloop(std::true_type{});   // uniform for the workgroup
+        if (G.at) kloop(std::true_type{});   // uniform for the workgroup
         else kloop(std::false_type{});
     } else {
         kloop(std::false_type{});
@@ -874,6 +910,7 @@ void gemm_nt_big_kernel(const BigLaunch L) {
     NTFP8_STAMP(st_loop);
     NTFP8_CYCLES(cy_loop);
     {
+        void* const Dv = P.D;
         // output type, accumulation and bias are properties of the problem, not of the kernel (fp8 outputs apart)
         auto epilogue = [&](auto bias_tag, const float (*bv)[4]) {
             constexpr bool kBias = decltype(bias_tag)::value;

@@ -98,9 +98,12 @@ __device__ __forceinline__ v16f mfma_32x32x64(v8i b_frag, v8i a_frag, v16f c) {
 
 // scale product applied to the accumulated sum: the operands' scales divide it; inverse scales (the form
 // tex.te_gemm is handed, src/nanotron/fp8/kernel.py:48,52) multiply it
-__device__ __forceinline__ float descale_factor(const float* scale_a, const float* scale_b, int scale_inv) {
-    const float sa = *scale_a, sb = *scale_b;
+__device__ __forceinline__ float descale_factor(float sa, float sb, int scale_inv) {
     return scale_inv ? sa * sb : (1.0f / sa) * (1.0f / sb);
+}
+
+__device__ __forceinline__ float descale_factor(const float* scale_a, const float* scale_b, int scale_inv) {
+    return descale_factor(*scale_a, *scale_b, scale_inv);
 }
 
 // element n of a bias vector of any supported type, as fp32 (exact)
@@ -154,21 +157,31 @@ struct GemmExtras {
     int scale_inv;      // the scale pointers hold inverse scales
 };
 
-// tile `pid` of a problem: kGroupM row-tiles are swept before moving along N
-__device__ __forceinline__ void tile_in_group(int pid, int tiles_m, int tiles_n, int& pid_m, int& pid_n) {
+// n / d for a d >= 2 that the host knows: multiplied by magic_of(d), which is too large by less than one for any n, instead
+// of a division, some forty dependent instructions in front of a workgroup's first load.
+__host__ __device__ constexpr uint32_t magic_of(uint32_t d) { return (uint32_t)((1ull << 32) / d) + 1u; }
+__device__ __forceinline__ int quotient(int n, int d, uint32_t magic) {
+    const uint32_t q = __umulhi((uint32_t)n, magic);
+    return (int)(q * (uint32_t)d > (uint32_t)n ? q - 1 : q);
+}
+
+// tile `pid` of a problem: kGroupM row-tiles are swept before moving along N.  `magic`: of kGroupM tiles_n.
+__device__ __forceinline__ void tile_in_group(int pid, int tiles_m, int tiles_n, uint32_t magic, int& pid_m, int& pid_n) {
+    static_assert(kGroupM == 4, "");
     const int in_group = kGroupM * tiles_n;
-    const int group = pid / in_group;
+    const int group = quotient(pid, in_group, magic);
     const int first_m = group * kGroupM;
-    const int gsz = min(tiles_m - first_m, kGroupM);
-    pid_m = first_m + (pid % in_group) % gsz;
-    pid_n = (pid % in_group) / gsz;
+    const int gsz = min(tiles_m - first_m, kGroupM), r = pid - group * in_group;
+    // r / gsz, exact for any r
+    pid_n = gsz == 4 ? r >> 2 : gsz == 2 ? r >> 1 : gsz == 1 ? r : (int)__umulhi((uint32_t)r, 0x55555556u);
+    pid_m = first_m + r - pid_n * gsz;
 }
 // the same with the workgroups of an XCD on a contiguous run of tiles
-__device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int& pid_m, int& pid_n) {
+__device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, uint32_t magic, int& pid_m, int& pid_n) {
     int pid = blockIdx.x;
     const int nwg = gridDim.x;
     if (nwg % kXcds == 0) pid = (pid % kXcds) * (nwg / kXcds) + pid / kXcds;
-    tile_in_group(pid, tiles_m, tiles_n, pid_m, pid_n);
+    tile_in_group(pid, tiles_m, tiles_n, magic, pid_m, pid_n);
 }
 
 // Epilogue of one wave: MI x NJ accumulator blocks of 32 x 32, block (i, j) at rows m_base + 32 i,

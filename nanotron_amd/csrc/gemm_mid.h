@@ -36,26 +36,24 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
     // within a round of workgroups an XCD works on a contiguous run of the tile list (workgroups are dealt round robin)
     int pid;
     {
-        const int round0 = ((int)blockIdx.x / L.round_size) * L.round_size, local = blockIdx.x - round0;
+        const int round0 = quotient((int)blockIdx.x, L.round_size, L.round_magic) * L.round_size, local = blockIdx.x - round0;
         const int in_round = min(L.round_size, (int)gridDim.x - round0);
         const int xcd = local % kXcds, q = in_round / kXcds, r = in_round % kXcds;
         pid = round0 + xcd * q + min(xcd, r) + local / kXcds;
     }
-    int which = 0;
-#pragma unroll
-    for (int i = 1; i < kBigMaxProblems; ++i)
-        if (i < L.count && pid >= L.p[i].tile_begin) which = i;
-    const BigProblem& P = L.p[which];
-    const int M = P.M, N = P.N, K = P.K;
-    pid -= P.tile_begin;
+    const Picked G = pick_problem(L, pid);
+    const BigProblem& P = L.p[G.which];
+    const int M = G.M, N = G.N, K = G.K;
+    const float scale_a = *G.scale_a, scale_b = *G.scale_b;
+    pid -= G.tile_begin;
     int pid_m, pid_n;
-    tile_in_group(pid, P.tiles_m, P.tiles_n, pid_m, pid_n);
+    tile_in_group(pid, G.tiles_m, G.tiles_n, G.magic, pid_m, pid_n);
     const int m0 = pid_m * TM, n0 = pid_n * TN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WN * (16 * MI), wn = wave % WN * 64;
     const int KT = (K + kBK - 1) / kBK;
-    const float alpha = descale_factor(P.scale_a, P.scale_b, P.ex.scale_inv);
+    float alpha = 0.0f;
 
     v4f acc[MI][NJ];
 #pragma unroll
@@ -68,10 +66,10 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
         // A K-contiguous operand is addressed from its tile's first row (any tensor size); rows past the end fall
         // behind the descriptor and read as zeros.  A transposed one is addressed from its first element (< 2 GiB): rows
         // k >= K fall behind the descriptor, columns past the end wrap into the next row and reach no stored output.
-        const __amdgpu_buffer_rsrc_t ra = kAT ? make_rsrc(P.A, (uint32_t)((int64_t)M * K))
-                                              : make_rsrc(P.A + (int64_t)m0 * K, (uint32_t)(min(M - m0, TM) * (int64_t)K));
-        const __amdgpu_buffer_rsrc_t rb = kBT ? make_rsrc(P.B, (uint32_t)((int64_t)N * K))
-                                              : make_rsrc(P.B + (int64_t)n0 * K, (uint32_t)(min(N - n0, TN) * (int64_t)K));
+        const __amdgpu_buffer_rsrc_t ra = kAT ? make_rsrc(G.A, (uint32_t)((int64_t)M * K))
+                                              : make_rsrc(G.A + (int64_t)m0 * K, (uint32_t)(min(M - m0, TM) * (int64_t)K));
+        const __amdgpu_buffer_rsrc_t rb = kBT ? make_rsrc(G.B, (uint32_t)((int64_t)N * K))
+                                              : make_rsrc(G.B + (int64_t)n0 * K, (uint32_t)(min(N - n0, TN) * (int64_t)K));
         constexpr uint32_t kNowhere = 0xfffffff0u;
         // offset of this lane's 16 bytes of load i of K-tile 0; position p of row r receives chunk p ^ swizzle(r)
         const int ld_kc = ((lane & 7) ^ (lane >> 3) ^ (wave & 1)) << 4;   // K-contiguous: 8 rows per load, swz16
@@ -186,6 +184,8 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
 #pragma unroll
             for (int l = 0; l < kLoads; ++l) request(l);
         }
+        // (behind the first requests: the scales were written by the kernel before, a trip of their own to memory)
+        alpha = descale_factor(scale_a, scale_b, P.ex.scale_inv);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kLoads) : "memory");
         wg_barrier();
 #pragma unroll
@@ -210,8 +210,8 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
         // (loads still in flight write zeros into stages nobody reads again; they are waited for before the wave ends)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
-    if (P.at) kloop(std::true_type{}, std::true_type{});   // uniform for the workgroup
-    else if (P.bt) kloop(std::false_type{}, std::true_type{});
+    if (G.at) kloop(std::true_type{}, std::true_type{});   // uniform for the workgroup
+    else if (G.bt) kloop(std::false_type{}, std::true_type{});
     else kloop(std::false_type{}, std::false_type{});
 
     auto epilogue = [&](auto bias_tag, const float (*bv)[4]) {
