@@ -87,44 +87,99 @@ static int path_of(const GemmDesc& g) {
 //   16.9 / 16.3 / 20.2; both transposed x 2048 12.1 / 10.4 / 13.6; 1021 x 2304 x 1024 (288 tiles of 128 x 64) 7.8 / 10.4 / 9.0
 //   at equal estimates:   3696 x 1088 x 944 (bf16) 10.6 / - / 11.8     1072 x 3600 x 320 (fp8 output) 12.5 / - / 17.6,
 //                         528 x 2528 x 1008 with its weight gradient 19.5 / - / 14.8
-// Several problems: by their average depth.  (The end of the list as the CUs work it off, longest tile first, predicts
-// single launches no better and chose worse for one pair in twenty, up to 10.7 -> 18.1 us, though 4 % better on average.)
+// Several problems: the mean of what their average depth gives and of the end of the list as the CUs work it off, longest tile
+// first.  Over 273 drawn forward and backward launches of 256 to 4096 tokens the choice then costs 0.9 % more than the best tile
+// size on average; by the average depth alone 2.6 % (a dgrad of a few deep tiles beside a wgrad of many shallow ones looks as
+// if the deep ones could be shared out: 1280 tokens, 2560 -> 6912, 82 us in 256-wide tiles, 62 in 128-wide), by the end of the
+// list alone 1.8 %.
 struct Edge {
     int m, n;
 };
-static int64_t launch_cost(const GemmDesc* const* g, int n, Edge edge, int64_t cus) {
+struct TileTime {   // a tile: per_k ns for a K-tile and `rest`; half of a 256-wide one: half_k
+    int64_t per_k, half_k, rest;
+    int64_t slots;   // workgroups at once
+};
+// `alone`: 64-wide tiles, of which no more than one goes to a CU
+static TileTime tile_time(Edge e, int form, bool alone, int64_t cus) {
+    static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
+    if (e.m == 256) return {1400, 700, 7000, cus};
+    if (e.n == 128) return {390, 0, 5200, cus};
+    if (e.m == 128) return {form ? 400 : 290, 0, 3600, cus};
+    return {alone ? kAlone[form] : kPair[form], 0, alone ? 3000 : 3500, 2 * cus};
+}
+static int64_t tiles_of(const GemmDesc& g, Edge e) { return (((int64_t)g.M + e.m - 1) / e.m) * (((int64_t)g.N + e.n - 1) / e.n); }
+static int64_t k_tiles(const GemmDesc& g) { return (g.K + kBK - 1) / kBK; }
+
+// `order`: the problems, longest K first
+static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Edge edge, int64_t cus) {
     int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
     int form = 0;
     for (int i = 0; i < n; ++i) {
-        const int64_t t = (((int64_t)g[i]->M + edge.m - 1) / edge.m) * (((int64_t)g[i]->N + edge.n - 1) / edge.n);
+        const int64_t t = tiles_of(*g[i], edge);
         tiles += t;
-        kt += t * ((g[i]->K + kBK - 1) / kBK);
+        kt += t * k_tiles(*g[i]);
         form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
     }
     const int64_t k = kt / tiles;   // K-tiles of an average tile
-    if (edge.m == 256) {
-        const int64_t rem = tiles % cus, full = tiles / cus;
-        return full * (1400 * k + 7000) + (rem == 0 ? 0 : 2 * rem <= cus ? 700 * k + 7000 : 1400 * k + 7000);
+    const TileTime whole = tile_time(edge, form, false, cus), last = tile_time(edge, form, true, cus);
+    const int64_t slots = whole.slots, rem = tiles % slots;
+    const bool halves = edge.m == 256 && rem != 0 && 2 * rem <= cus;
+    const TileTime& end = edge.m == 64 && rem <= cus ? last : whole;
+    const int64_t average =
+        tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : (halves ? end.half_k : end.per_k) * k + end.rest);
+    if (n == 1 || tiles > 64 * slots) return average;
+
+    // groups of CUs that are busy for equally long: the next tiles go to those that are free first
+    struct {
+        int64_t until, count;
+    } at[4 * kBigMaxProblems + 2] = {{0, slots}};
+    int groups = 1;
+    const TileTime& tt = edge.m == 64 && tiles <= cus ? last : whole;
+    int64_t left = halves ? tiles - rem : tiles, tail_k = 0;
+    for (int i = 0; i < n; ++i) {
+        const GemmDesc& d = *g[order[i]];
+        int64_t t = tiles_of(d, edge);
+        if (t > left && tail_k == 0) tail_k = k_tiles(d);
+        t = std::min(t, left);
+        left -= t;
+        const int64_t takes = tt.per_k * k_tiles(d) + tt.rest;
+        while (t > 0) {
+            int first = 0;
+            for (int j = 1; j < groups; ++j)
+                if (at[j].until < at[first].until) first = j;
+            const int64_t now = at[first].until, c = std::min(t, at[first].count);
+            t -= c;
+            at[first].count -= c;
+            int to = 0;
+            while (to < groups && at[to].until != now + takes) ++to;
+            if (to < groups) {
+                at[to].count += c;
+                if (at[first].count == 0) at[first] = at[--groups];
+            } else if (at[first].count == 0) {
+                at[first] = {now + takes, c};
+            } else if (groups < (int)(sizeof(at) / sizeof(at[0]))) {
+                at[groups++] = {now + takes, c};
+            } else {
+                return average;
+            }
+        }
     }
-    if (edge.n == 128) return ((tiles + cus - 1) / cus) * (390 * k + 5200);
-    if (edge.m == 128) return ((tiles + cus - 1) / cus) * ((form ? 400 : 290) * k + 3600);
-    // two workgroups per CU
-    static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
-    const int64_t rem = tiles % (2 * cus), full = tiles / (2 * cus);
-    return full * (kPair[form] * k + 3500) + (rem == 0 ? 0 : rem <= cus ? kAlone[form] * k + 3000 : kPair[form] * k + 3500);
+    int64_t busy = 0;
+    for (int j = 0; j < groups; ++j) busy = std::max(busy, at[j].until);
+    if (halves) busy += whole.half_k * tail_k + whole.rest;
+    return (average + busy) / 2;
 }
 
 // The tile list of a launch, problem by problem, longest K first: the long tiles start together and the shorter ones fill
 // the rounds behind them.  Returns the number of tiles.
-static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch* L) {
-    int order[kBigMaxProblems];
+static void by_depth(const GemmDesc* const* g, int n, int* order) {
     for (int i = 0; i < n; ++i) order[i] = i;
     for (int i = 1; i < n; ++i)   // insertion sort, stable, K descending
-        for (int j = i; j > 0 && g[order[j]]->K > g[order[j - 1]]->K; --j) {
-            const int t = order[j];
-            order[j] = order[j - 1];
-            order[j - 1] = t;
-        }
+        for (int j = i; j > 0 && g[order[j]]->K > g[order[j - 1]]->K; --j) std::swap(order[j], order[j - 1]);
+}
+static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch* L) {
+    int order[kBigMaxProblems];
+    by_depth(g, n, order);
     *L = {};
     L->count = n;
     int64_t tiles = 0;
@@ -189,12 +244,14 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     {
         bool big = true;
         for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
-        int64_t best = launch_cost(g, n, edge, cus);
+        int order[kBigMaxProblems];
+        by_depth(g, n, order);
+        int64_t best = launch_cost(g, n, order, edge, cus);
         // (where the lines meet, the wider tiles for one problem, the narrower for several)
         const int first = n == 1 ? 256 : 64;
         for (const Edge e : {Edge{first, first}, Edge{320 - first, 320 - first}, Edge{128, 64}}) {
             if (e.m == 256 && !big) continue;
-            const int64_t c = launch_cost(g, n, e, cus);
+            const int64_t c = launch_cost(g, n, order, e, cus);
             if (c < best) best = c, edge = e;
         }
     }
