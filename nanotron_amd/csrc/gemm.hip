@@ -95,54 +95,49 @@ static int path_of(const GemmDesc& g) {
 struct Edge {
     int m, n;
 };
-struct TileTime {   // a tile: per_k ns for a K-tile and `rest`; half of a 256-wide one: half_k
-    int64_t per_k, half_k, rest;
+struct TileTime {   // a tile: per_k ns for a K-tile and `rest`
+    int64_t per_k, rest;
     int64_t slots;   // workgroups at once
 };
 // `alone`: 64-wide tiles, of which no more than one goes to a CU
 static TileTime tile_time(Edge e, int form, bool alone, int64_t cus) {
     static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
-    if (e.m == 256) return {1400, 700, 7000, cus};
-    if (e.n == 128) return {390, 0, 5200, cus};
-    if (e.m == 128) return {form ? 400 : 290, 0, 3600, cus};
-    return {alone ? kAlone[form] : kPair[form], 0, alone ? 3000 : 3500, 2 * cus};
+    if (e.m == 256) return {1400, 7000, cus};
+    if (e.n == 128) return {390, 5200, cus};
+    if (e.m == 128) return {form ? 400 : 290, 3600, cus};
+    return {alone ? kAlone[form] : kPair[form], alone ? 3000 : 3500, 2 * cus};
+}
+// The partial last round of 256-wide tiles is computed in parts if there is a CU for each: in how many (1: whole), unless all of
+// the list in one launch ends earlier (shallow tiles beside a few deep ones).  Halves are the 256-wide kernel's own; behind full
+// rounds quarters (128 x 128) and eighths (128 x 64) are quicker yet.  Backward launches with 1 to 64 tiles in the last round, us,
+// halves / these: 2912 tokens, 2544 -> 3520, 77.0 / 67.1; 3152, 2464 -> 3712, 72.3 / 59.3; 1888, 3232 -> 3872, 67.8 / 63.3.
+static int tail_parts(int64_t tiles, int64_t cus) {
+    const int64_t rem = tiles % cus;
+    if (rem == 0 || 2 * rem > cus) return 1;
+    return tiles < cus || 4 * rem > cus ? 2 : 8 * rem > cus ? 4 : 8;
+}
+static TileTime tail_time(int parts, int form, int64_t cus) {
+    if (parts == 2) return {700, 7000, cus};
+    return tile_time(parts == 4 ? Edge{128, 128} : Edge{128, 64}, form, false, cus);
 }
 static int64_t tiles_of(const GemmDesc& g, Edge e) { return (((int64_t)g.M + e.m - 1) / e.m) * (((int64_t)g.N + e.n - 1) / e.n); }
 static int64_t k_tiles(const GemmDesc& g) { return (g.K + kBK - 1) / kBK; }
 
-// `order`: the problems, longest K first
-static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Edge edge, int64_t cus) {
-    int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
-    int form = 0;
-    for (int i = 0; i < n; ++i) {
-        const int64_t t = tiles_of(*g[i], edge);
-        tiles += t;
-        kt += t * k_tiles(*g[i]);
-        form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
-    }
-    const int64_t k = kt / tiles;   // K-tiles of an average tile
-    const TileTime whole = tile_time(edge, form, false, cus), last = tile_time(edge, form, true, cus);
-    const int64_t slots = whole.slots, rem = tiles % slots;
-    const bool halves = edge.m == 256 && rem != 0 && 2 * rem <= cus;
-    const TileTime& end = edge.m == 64 && rem <= cus ? last : whole;
-    const int64_t average =
-        tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : (halves ? end.half_k : end.per_k) * k + end.rest);
-    if (n == 1 || tiles > 64 * slots) return average;
-
-    // groups of CUs that are busy for equally long: the next tiles go to those that are free first
+// When the last of `left` tiles ends, the first of the list (problems by `order`, longest K first): groups of CUs that are busy for
+// equally long, the next tiles go to those that are free first.  -1: too many groups.  *next_k: depth of the tile behind them.
+static int64_t list_end(const GemmDesc* const* g, int n, const int* order, Edge edge, const TileTime& time, int64_t left, int64_t* next_k) {
     struct {
         int64_t until, count;
-    } at[4 * kBigMaxProblems + 2] = {{0, slots}};
+    } at[4 * kBigMaxProblems + 2] = {{0, time.slots}};
     int groups = 1;
-    const TileTime& tt = edge.m == 64 && tiles <= cus ? last : whole;
-    int64_t left = halves ? tiles - rem : tiles, tail_k = 0;
+    *next_k = 0;
     for (int i = 0; i < n; ++i) {
         const GemmDesc& d = *g[order[i]];
         int64_t t = tiles_of(d, edge);
-        if (t > left && tail_k == 0) tail_k = k_tiles(d);
+        if (t > left && *next_k == 0) *next_k = k_tiles(d);
         t = std::min(t, left);
         left -= t;
-        const int64_t takes = tt.per_k * k_tiles(d) + tt.rest;
+        const int64_t takes = time.per_k * k_tiles(d) + time.rest;
         while (t > 0) {
             int first = 0;
             for (int j = 1; j < groups; ++j)
@@ -160,14 +155,43 @@ static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Ed
             } else if (groups < (int)(sizeof(at) / sizeof(at[0]))) {
                 at[groups++] = {now + takes, c};
             } else {
-                return average;
+                return -1;
             }
         }
     }
     int64_t busy = 0;
     for (int j = 0; j < groups; ++j) busy = std::max(busy, at[j].until);
-    if (halves) busy += whole.half_k * tail_k + whole.rest;
-    return (average + busy) / 2;
+    return busy;
+}
+
+// `order`: the problems, longest K first.  *parts: of the tiles of a partial last round of 256-wide ones
+static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Edge edge, int64_t cus, int* parts) {
+    int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
+    int form = 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t t = tiles_of(*g[i], edge);
+        tiles += t;
+        kt += t * k_tiles(*g[i]);
+        form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
+    }
+    const int64_t k = kt / tiles;   // K-tiles of an average tile
+    const TileTime whole = tile_time(edge, form, false, cus), few = tile_time(edge, form, true, cus);
+    const int64_t slots = whole.slots, rem = tiles % slots;
+    auto cost = [&](int split) -> int64_t {
+        const TileTime end = split > 1 ? tail_time(split, form, cus) : edge.m == 64 && rem <= cus ? few : whole;
+        const int64_t average = tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : end.per_k * k + end.rest);
+        if (n == 1 || tiles > 64 * slots) return average;
+        int64_t next_k;
+        const int64_t busy = list_end(g, n, order, edge, edge.m == 64 && tiles <= cus ? few : whole, split > 1 ? tiles - rem : tiles, &next_k);
+        if (busy < 0) return average;
+        return (average + busy + (split > 1 ? end.per_k * next_k + end.rest : 0)) / 2;
+    };
+    const int64_t as_is = cost(*parts = 1);
+    const int split = edge.m == 256 ? tail_parts(tiles, cus) : 1;
+    if (split == 1) return as_is;
+    const int64_t cut = cost(split);
+    if (cut < as_is) *parts = split;
+    return std::min(cut, as_is);
 }
 
 // The tile list of a launch, problem by problem, longest K first: the long tiles start together and the shorter ones fill
@@ -241,18 +265,20 @@ template <int FA, int FB>
 static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
     const int cus = cu_count();   // (asked once: the question goes to the runtime)
     Edge edge{128, 128};
+    int parts = 1;
     {
         bool big = true;
         for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
         int order[kBigMaxProblems];
         by_depth(g, n, order);
-        int64_t best = launch_cost(g, n, order, edge, cus);
+        int64_t best = launch_cost(g, n, order, edge, cus, &parts);
         // (where the lines meet, the wider tiles for one problem, the narrower for several)
         const int first = n == 1 ? 256 : 64;
         for (const Edge e : {Edge{first, first}, Edge{320 - first, 320 - first}, Edge{128, 64}}) {
             if (e.m == 256 && !big) continue;
-            const int64_t c = launch_cost(g, n, order, e, cus);
-            if (c < best) best = c, edge = e;
+            int p;
+            const int64_t c = launch_cost(g, n, order, e, cus, &p);
+            if (c < best) best = c, edge = e, parts = p;
         }
     }
     BigLaunch L;
@@ -266,8 +292,7 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
         const int rc = launch_mid(L, FA, FB, edge.m, edge.n, fp8_out, (int)tiles, st);
         return L.fin_blocks ? rc : finish_behind(*g[0], rc, st);
     }
-    const int rem = (int)(tiles % cus);
-    L.tail_tiles = (rem != 0 && 2 * rem <= cus) ? rem : 0;
+    L.tail_tiles = parts > 1 ? (int)(tiles % cus) : 0;
     L.full_blocks = (int)tiles - L.tail_tiles;
     if (L.fin_blocks) L.fin_blocks = L.full_blocks + 2 * L.tail_tiles;
     (void)hipGetLastError();   // an error left behind by an unrelated earlier call is not this launch's
@@ -275,7 +300,7 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
         constexpr bool kFp8Out = decltype(fp8_tag)::value, kBT = decltype(bt_tag)::value;
         if (L.full_blocks > 0)
             hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 8, kFp8Out, kBT>), dim3(L.full_blocks), dim3(kBigThreads), 0, st, L);
-        if (L.tail_tiles > 0)
+        if (parts == 2)
             hipLaunchKernelGGL((gemm_nt_big_kernel<FA, FB, 4, kFp8Out, kBT>), dim3(2 * L.tail_tiles), dim3(kBigThreads), 0, st, L);
     };
 #ifdef NTFP8_PROFILE_NARROW
@@ -289,7 +314,8 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
         else go(std::false_type{}, std::false_type{});
     }
 #endif
-    const int rc = hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+    int rc = hipGetLastError() == hipSuccess ? NTFP8_OK : NTFP8_ERR_LAUNCH;
+    if (parts > 2 && rc == NTFP8_OK) rc = launch_mid(L, FA, FB, 128, parts == 4 ? 128 : 64, fp8_out, parts * L.tail_tiles, st);
     return L.fin_blocks ? rc : finish_behind(*g[0], rc, st);
 }
 

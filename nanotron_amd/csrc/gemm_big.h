@@ -481,10 +481,10 @@ void gemm_nt_big_kernel(const BigLaunch L) {
         if (g_plain_tile_order) {
         } else
 #endif
-        if (in_round % kXcds == 0) pid = round0 + (local % kXcds) * (in_round / kXcds) + local / kXcds;
+        pid = round0 + run_of_xcd(local, in_round);
     } else {
         const int nb = 2 * L.tail_tiles;
-        if (nb % kXcds == 0) pid = (pid % kXcds) * (nb / kXcds) + pid / kXcds;
+        pid = run_of_xcd(pid, nb);
         half = pid & 1;
         pid = L.full_blocks + (pid >> 1);
     }

@@ -157,6 +157,12 @@ struct GemmExtras {
     int scale_inv;      // the scale pointers hold inverse scales
 };
 
+// Place of workgroup `local` of `count` that are dealt to the XCDs round robin, when each XCD takes a contiguous run
+__device__ __forceinline__ int run_of_xcd(int local, int count) {
+    const int xcd = local % kXcds;
+    return xcd * (count / kXcds) + min(xcd, count % kXcds) + local / kXcds;
+}
+
 // n / d for a d >= 2 that the host knows: multiplied by magic_of(d), which is too large by less than one for any n, instead
 // of a division, some forty dependent instructions in front of a workgroup's first load.
 __host__ __device__ constexpr uint32_t magic_of(uint32_t d) { return (uint32_t)((1ull << 32) / d) + 1u; }

@@ -38,9 +38,13 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
     {
         const int round0 = quotient((int)blockIdx.x, L.round_size, L.round_magic) * L.round_size, local = blockIdx.x - round0;
         const int in_round = min(L.round_size, (int)gridDim.x - round0);
-        const int xcd = local % kXcds, q = in_round / kXcds, r = in_round % kXcds;
-        pid = round0 + xcd * q + min(xcd, r) + local / kXcds;
+        pid = round0 + run_of_xcd(local, in_round);
     }
+    // (uniform) the tail of a launch of 256-wide tiles: parts of the tiles from full_blocks on
+    const bool tail = L.tail_tiles != 0;
+    constexpr int kAcross = 256 / TN, kParts = 256 / TM * kAcross;
+    const int part = tail ? pid % kParts : 0;
+    if (tail) pid = L.full_blocks + pid / kParts;
     const Picked G = pick_problem(L, pid);
     const BigProblem& P = L.p[G.which];
     const int M = G.M, N = G.N, K = G.K;
@@ -48,7 +52,8 @@ __global__ __launch_bounds__(kBigThreads, TM == 64 ? 2 : 1) void gemm_mid_kernel
     pid -= G.tile_begin;
     int pid_m, pid_n;
     tile_in_group(pid, G.tiles_m, G.tiles_n, G.magic, pid_m, pid_n);
-    const int m0 = pid_m * TM, n0 = pid_n * TN;
+    const int m0 = pid_m * (tail ? 256 : TM) + part / kAcross * TM, n0 = pid_n * (tail ? 256 : TN) + part % kAcross * TN;
+    if (m0 >= M || n0 >= N) return;   // a part of an edge tile with nothing in it (no bookkeeping inside such launches)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WN * (16 * MI), wn = wave % WN * 64;

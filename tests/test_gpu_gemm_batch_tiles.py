@@ -5,7 +5,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-BACKWARD = [(1024, 2048, 4864), (512, 1280, 4096), (768, 2048, 6912), (3856, 1856, 832), (336, 816, 3936), (2048, 1024, 1024), (272, 144, 4096)]
+BACKWARD = [(1024, 2048, 4864), (512, 1280, 4096), (768, 2048, 6912), (3856, 1856, 832), (336, 816, 3936), (2048, 1024, 1024), (272, 144, 4096),
+            (2912, 2544, 3520), (1040, 3664, 3920), (3152, 2464, 3712)]   # ... with a few 256-wide tiles behind a round of them
 
 
 def _operand(g, rows, cols):

@@ -10,6 +10,7 @@ pytestmark = pytest.mark.gpu
 
 SMALL = [(57, 32), (64, 48), (72, 36), (9, 8), (65, 130), (200, 96)]                            # 64-wide tiles
 NARROW = [(2048, 1024), (1921, 1024), (2048, 961), (1935, 1000), (2045, 964)]                     # 128 x 64 tiles: one round of workgroups
+TAILS = [(4400, 3900), (4361, 4100), (4352, 3856), (4097, 4352)]   # a round of 256-wide tiles and a few more, computed in quarters or eighths
 LARGE = [(4088, 4096), (4081, 4112), (4095, 4104), (3849, 4100), (4097, 3842)]                   # 256-wide tiles
 
 
@@ -40,13 +41,14 @@ def _check(M, N, K, odt, acc, form="plain", full=True):
     assert torch.equal(got[:, cols], want.to(odt))
 
 
-@pytest.mark.parametrize("mn", SMALL + NARROW + LARGE)
+@pytest.mark.parametrize("mn", SMALL + NARROW + TAILS + LARGE)
 @pytest.mark.parametrize("odt,acc", [(torch.float32, False), (torch.float32, True), (torch.bfloat16, False)])
 def test_every_remainder(mn, odt, acc):
     _check(*mn, 272, odt, acc)
 
 
-@pytest.mark.parametrize("mn", [(144, 144), (4096, 4112), (4112, 3856), (2048, 1024), (1936, 976), (2032, 1008)])
+@pytest.mark.parametrize("mn", [(144, 144), (4096, 4112), (4112, 3856), (2048, 1024), (1936, 976), (2032, 1008),
+                                (4400, 3904), (4368, 4112)])
 @pytest.mark.parametrize("acc", [False, True])
 def test_transposed_operands(mn, acc):
     _check(*mn, 272, torch.float32, acc, "both")
@@ -60,9 +62,9 @@ def test_narrow_tiles_with_every_number_of_k_tiles(mn, K):
         _check(*mn, K, torch.bfloat16, False, "b")
 
 
-@pytest.mark.parametrize("mn", [(2048, 1024), (1924, 976), (2044, 1008)])
+@pytest.mark.parametrize("mn", [(2048, 1024), (1924, 976), (2044, 1008), (4404, 3904), (4364, 4112)])
 @pytest.mark.parametrize("form", ["plain", "b"])
-def test_narrow_tiles_with_fp8_outputs(mn, form):
+def test_fp8_outputs(mn, form):
     from nanotron_amd import _native as nt
 
     (M, N), K = mn, 272
