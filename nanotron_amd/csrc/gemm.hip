@@ -8,7 +8,7 @@
 // Kernels:
 //   gemm_nt_big_kernel    (gemm_big.h) 256 x 256 x 128 tiles, 4 waves of 128 x 128 with 16x16x128 MFMAs,
 //                         loads straight into LDS, two stages.  The partial last round of tiles over the CUs is
-//                         cut into 128-row half tiles.
+//                         computed in parts: 128-row half tiles, or tiles of the next kernel.
 //   gemm_mid_kernel       (gemm_mid.h) 128 x 128, 128 x 64 and 64 x 64 tiles of the same instruction, loads straight into four LDS
 //                         stages: shapes that have too few 256-wide tiles, and operands beyond the 2 GiB reach of a
 //                         buffer descriptor's 32-bit offsets.

@@ -360,8 +360,8 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
 
 // Launch geometry, computed on the host.  The first `full_blocks` tiles (in grouped order) are computed
 // whole by the MI = 8 kernel.  If the tile count leaves a partial last round over the CUs, the
-// remaining `tail_tiles` tiles are cut into two 128-row halves and computed by a second launch of
-// the MI = 4 kernel with 2 tail_tiles workgroups, so that the last round is half as long.
+// remaining `tail_tiles` tiles are computed in parts by a second launch, so that the last round is shorter: two 128-row halves
+// each by the MI = 4 kernel, or four or eight parts by the tiles of gemm_mid.h.
 //
 // One launch can carry several independent GEMMs of the same operand formats (the dgrad and wgrad of a
 // layer, say): their tiles form one list, longest K first, so that the rounds of one problem fill up
@@ -390,7 +390,7 @@ struct BigLaunch {
     BigProblem p[kBigMaxProblems];
     int count;
     int full_blocks;        // tiles (of the whole list) computed whole
-    int tail_tiles;         // tiles at the end of the list computed as two halves
+    int tail_tiles;         // tiles at the end of the list computed in parts
     int round_size;         // workgroups resident at once
     uint32_t round_magic;   // magic_of(round_size)
     // a launch of one problem with fp8 outputs: the workgroup that finishes last (of fin_blocks, over both launches of a
