@@ -175,7 +175,11 @@ static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Ed
         form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
     }
     const int64_t k = kt / tiles;   // K-tiles of an average tile
-    const TileTime whole = tile_time(edge, form, false, cus), few = tile_time(edge, form, true, cus);
+    TileTime whole = tile_time(edge, form, false, cus);
+    const TileTime few = tile_time(edge, form, true, cus);
+    // One problem on part of the CUs: the chip is clocked higher (140 to 210 tiles 1050 to 1180 ns a K-tile).  us, 128 / 256 wide:
+    // 3584 x 2560 x 5888 (140 tiles) 62 / 54, 168 tiles of K = 8700 91 / 80; 130 to 135 tiles, K 2048 to 4096, 21 to 37 / 25 to 44
+    if (n == 1 && edge.m == 256 && tiles < cus) whole.per_k = 1150;
     const int64_t slots = whole.slots, rem = tiles % slots;
     auto cost = [&](int split) -> int64_t {
         const TileTime end = split > 1 ? tail_time(split, form, cus) : edge.m == 64 && rem <= cus ? few : whole;

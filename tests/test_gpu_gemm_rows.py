@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 SMALL = [(57, 32), (64, 48), (72, 36), (9, 8), (65, 130), (200, 96)]                            # 64-wide tiles
 NARROW = [(2048, 1024), (1921, 1024), (2048, 961), (1935, 1000), (2045, 964)]                     # 128 x 64 tiles: one round of workgroups
 TAILS = [(4400, 3900), (4361, 4100), (4352, 3856), (4097, 4352)]   # a round of 256-wide tiles and a few more, computed in quarters or eighths
-LARGE = [(4088, 4096), (4081, 4112), (4095, 4104), (3849, 4100), (4097, 3842)]                   # 256-wide tiles
+LARGE = [(4088, 4096), (4081, 4112), (4095, 4104), (3849, 4100), (4097, 3842), (2560, 3584)]     # 256-wide tiles
 
 
 def _check(M, N, K, odt, acc, form="plain", full=True):
