@@ -299,9 +299,10 @@ __device__ __forceinline__ void store_wave_tile16(const v4f (&acc)[MI][NJ], void
 // four lane rows and four neighbouring blocks gives lane row q the 16 consecutive n of block j0 + q, one 16-byte
 // store per lane and 64 contiguous bytes per output row and instruction.  Transposed bytes: a 4 x 4 byte transpose
 // inside each quad of lanes (4 consecutive m) turns the word into 4 consecutive m of one n.
-// All stores go through buffer descriptors of M N bytes: rows past the end fall outside and are dropped, columns
-// past the end get an offset that does; nothing is predicated, which keeps the scalar registers of the epilogue
-// (and with them the register budget of the K loop before it) small.
+// All stores go through buffer descriptors of M N bytes: rows and columns past the end get an offset that falls outside
+// and are dropped.  (Their own offsets would not do: they run past M N by up to 255 rows, and past 2^32, to the first rows
+// again, where M N is close to it.)  Nothing is predicated, which keeps the scalar registers of the epilogue (and with
+// them the register budget of the K loop before it) small.
 // Accumulators past M and past N stay out of the amax: they hold zeros times whatever the other operand holds (NaN
 // against an infinite code), plus the bias, or, where an operand is read through the transposing loads and wraps
 // into its next row, arbitrary values.  N is a multiple of 16, so a block's columns are in or out together, uniformly
@@ -339,8 +340,7 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
             for (int j = 0; j < NJ; ++j) {
                 const uint32_t t = quad_transpose_bytes(w[j], lane);
                 const int nt = n_base + j * 16 + q * 4 + (lane & 3);
-                // nt >= N lies past the end of the [N, M] bytes by itself
-                reg_store4(rt, mq < M ? (uint32_t)nt * (uint32_t)M + (uint32_t)mq : kDropped, t);
+                reg_store4(rt, m < M && n_base + j * 16 < N ? (uint32_t)nt * (uint32_t)M + (uint32_t)mq : kDropped, t);
             }
         }
 #pragma unroll
@@ -350,9 +350,9 @@ __device__ __forceinline__ uint32_t store_wave_tile16_fp8(const v4f (&acc)[MI][N
             swap_rows16(x2, x3);
             swap_halves(x0, x2);   // lane rows 2, 3 <-> rows 0, 1 two blocks further on
             swap_halves(x1, x3);
-            // lane row q now holds n 0-3, 4-7, 8-11, 12-15 of block j0 + q; m >= M lies past the end by itself
+            // lane row q now holds n 0-3, 4-7, 8-11, 12-15 of block j0 + q
             const int n = n_base + (j0 + q) * 16;
-            reg_store16(rd, n < N ? (uint32_t)m * (uint32_t)N + (uint32_t)n : kDropped, (v4i){(int)x0, (int)x1, (int)x2, (int)x3});
+            reg_store16(rd, m < M && n < N ? (uint32_t)m * (uint32_t)N + (uint32_t)n : kDropped, (v4i){(int)x0, (int)x1, (int)x2, (int)x3});
         }
     }
     return amax;
