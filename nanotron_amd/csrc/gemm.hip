@@ -22,6 +22,7 @@
 //                         fewer than two K-tiles.
 #include "gemm_common.h"
 #include "gemm_big.h"
+#include "gemm_choice.h"
 
 namespace ntfp8 {
 
@@ -36,13 +37,6 @@ int launch_plain(const GemmDesc& g, hipStream_t st);
 int launch_tiny(const BigProblem& p, int fa, int fb, hipStream_t st);
 int run_amax_finalize(Workspace* ws, const ScalarIO& io, hipStream_t st);
 
-// operands within reach of 32-bit buffer offsets: what the 256-wide tiles and transposed operands need
-static bool fits32(const GemmDesc& g) {
-    return (int64_t)(g.M + 256) * g.K < (1LL << 31) && (int64_t)(g.N + kBigN) * g.K < (1LL << 31);
-}
-// the 256-wide tiles' pipeline starts with two K-tiles
-static bool big_ok(const GemmDesc& g) { return fits32(g) && g.K >= 2 * kBK; }
-
 // A launch of one problem of fewer than two K-tiles (the 256-wide tiles cannot take it) and more 64-wide tiles than the
 // chip works on at once: nothing hides the prologue and epilogue of the one or two workgroups per CU of the smaller tiles,
 // and 16- and 32-bit rows that end inside a 64-byte piece of memory make their streaming stores partial writes (for fp8
@@ -51,12 +45,12 @@ static bool big_ok(const GemmDesc& g) { return fits32(g) && g.K >= 2 * kBK; }
 //   bf16, others:         up to 256 tiles 4.0 / 4.8, 257 to 512 5.7 / 5.3, 513 to 1024 8.0 / 6.1, more 18.5 / 10.1
 //   fp8:                  257 to 512 tiles 9.3 / 11.3, 513 to 1024 10.7 / 12.2, 1025 to 1536 16.0 / 13.4
 //   fp8 with its copy, N % 64 != 0:  257 to 512 11.7 / 12.5, 513 to 768 14.2 / 13.2, more 38.7 / 22.1
-static bool short_k(const GemmDesc& g) {
+static bool short_k(const GemmDesc& g, int cus) {
     if (g.K >= 2 * kBK || g.tb) return false;
     const int64_t tiles = (((int64_t)g.M + 63) / 64) * (((int64_t)g.N + 63) / 64);
     const bool whole = (int64_t)g.N * (g.d_dtype == NTFP8_F32 ? 4 : is_fp8_out(g.d_dtype) ? 1 : 2) % 64 == 0;
     const int per_cu = whole ? 4 : !is_fp8_out(g.d_dtype) ? 1 : g.Dt ? 2 : 4;
-    return tiles > per_cu * cu_count();
+    return tiles > per_cu * cus;
 }
 
 // which kernels serve a problem
@@ -77,134 +71,8 @@ static int path_of(const GemmDesc& g) {
     return (int64_t)g.K * 128 < (1LL << 31) ? kPathTiles : kPathAny;   // (a tile's rows within reach of 32-bit offsets)
 }
 
-// What a launch of `n` problems takes in tiles of 256 x 256, 128 x 128, 128 x 64 or 64 x 64, in nanoseconds: rounds of workgroups times what a
-// workgroup takes for its K-tiles and for everything else.  The constants are fits to launches of one problem with
-// bf16 output (plain / B transposed / both transposed), warm operands; what matters is where the lines cross.
-//   us, 256 / 128 / 64 wide:  1024 x 1024 x 1024  10.1 / 7.5 / 4.8     2048 x 1024 x 4096  26.5 / 16.3 / 15.3
-//   2048 x 2048 x 2048  16.7 / 11.8 / 16.9      both transposed  19.6 / 12.6 / 24.3
-//   2048 x 4096 x 4096  32.5 / 40.4 / 55.8      4096 x 4096 x 4096  51.9 / 73.5 / 101
-//   128 x 128 / 128 x 64 / 64 x 64:  2048 x 1024 x 1024 7.6 / 5.9 / 6.6, x 4096 15.6 / 12.9 / 15.2; B transposed 8.0 / 6.6 / 8.0 and
-//   16.9 / 16.3 / 20.2; both transposed x 2048 12.1 / 10.4 / 13.6; 1021 x 2304 x 1024 (288 tiles of 128 x 64) 7.8 / 10.4 / 9.0
-//   at equal estimates:   3696 x 1088 x 944 (bf16) 10.6 / - / 11.8     1072 x 3600 x 320 (fp8 output) 12.5 / - / 17.6,
-//                         528 x 2528 x 1008 with its weight gradient 19.5 / - / 14.8
-// Several problems: the mean of what their average depth gives and of the end of the list as the CUs work it off, longest tile
-// first.  Over 273 drawn forward and backward launches of 256 to 4096 tokens the choice then costs 0.9 % more than the best tile
-// size on average; by the average depth alone 2.6 % (a dgrad of a few deep tiles beside a wgrad of many shallow ones looks as
-// if the deep ones could be shared out: 1280 tokens, 2560 -> 6912, 82 us in 256-wide tiles, 62 in 128-wide), by the end of the
-// list alone 1.8 %.
-struct Edge {
-    int m, n;
-};
-struct TileTime {   // a tile: per_k ns for a K-tile and `rest`
-    int64_t per_k, rest;
-    int64_t slots;   // workgroups at once
-};
-// `alone`: 64-wide tiles, of which no more than one goes to a CU
-static TileTime tile_time(Edge e, int form, bool alone, int64_t cus) {
-    static constexpr int kAlone[3] = {185, 260, 280}, kPair[3] = {350, 530, 620};
-    if (e.m == 256) return {1400, 7000, cus};
-    if (e.n == 128) return {390, 5200, cus};
-    if (e.m == 128) return {form ? 400 : 290, 3600, cus};
-    return {alone ? kAlone[form] : kPair[form], alone ? 3000 : 3500, 2 * cus};
-}
-// The partial last round of 256-wide tiles is computed in parts if there is a CU for each: in how many (1: whole), unless all of
-// the list in one launch ends earlier (shallow tiles beside a few deep ones).  Halves are the 256-wide kernel's own; behind full
-// rounds quarters (128 x 128) and eighths (128 x 64) are quicker yet.  Backward launches with 1 to 64 tiles in the last round, us,
-// halves / these: 2912 tokens, 2544 -> 3520, 77.0 / 67.1; 3152, 2464 -> 3712, 72.3 / 59.3; 1888, 3232 -> 3872, 67.8 / 63.3.
-static int tail_parts(int64_t tiles, int64_t cus) {
-    const int64_t rem = tiles % cus;
-    if (rem == 0 || 2 * rem > cus) return 1;
-    return tiles < cus || 4 * rem > cus ? 2 : 8 * rem > cus ? 4 : 8;
-}
-static TileTime tail_time(int parts, int form, int64_t cus) {
-    if (parts == 2) return {700, 7000, cus};
-    return tile_time(parts == 4 ? Edge{128, 128} : Edge{128, 64}, form, false, cus);
-}
-static int64_t tiles_of(const GemmDesc& g, Edge e) { return (((int64_t)g.M + e.m - 1) / e.m) * (((int64_t)g.N + e.n - 1) / e.n); }
-static int64_t k_tiles(const GemmDesc& g) { return (g.K + kBK - 1) / kBK; }
-
-// When the last of `left` tiles ends, the first of the list (problems by `order`, longest K first): groups of CUs that are busy for
-// equally long, the next tiles go to those that are free first.  -1: too many groups.  *next_k: depth of the tile behind them.
-static int64_t list_end(const GemmDesc* const* g, int n, const int* order, Edge edge, const TileTime& time, int64_t left, int64_t* next_k) {
-    struct {
-        int64_t until, count;
-    } at[4 * kBigMaxProblems + 2] = {{0, time.slots}};
-    int groups = 1;
-    *next_k = 0;
-    for (int i = 0; i < n; ++i) {
-        const GemmDesc& d = *g[order[i]];
-        int64_t t = tiles_of(d, edge);
-        if (t > left && *next_k == 0) *next_k = k_tiles(d);
-        t = std::min(t, left);
-        left -= t;
-        const int64_t takes = time.per_k * k_tiles(d) + time.rest;
-        while (t > 0) {
-            int first = 0;
-            for (int j = 1; j < groups; ++j)
-                if (at[j].until < at[first].until) first = j;
-            const int64_t now = at[first].until, c = std::min(t, at[first].count);
-            t -= c;
-            at[first].count -= c;
-            int to = 0;
-            while (to < groups && at[to].until != now + takes) ++to;
-            if (to < groups) {
-                at[to].count += c;
-                if (at[first].count == 0) at[first] = at[--groups];
-            } else if (at[first].count == 0) {
-                at[first] = {now + takes, c};
-            } else if (groups < (int)(sizeof(at) / sizeof(at[0]))) {
-                at[groups++] = {now + takes, c};
-            } else {
-                return -1;
-            }
-        }
-    }
-    int64_t busy = 0;
-    for (int j = 0; j < groups; ++j) busy = std::max(busy, at[j].until);
-    return busy;
-}
-
-// `order`: the problems, longest K first.  *parts: of the tiles of a partial last round of 256-wide ones
-static int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Edge edge, int64_t cus, int* parts) {
-    int64_t tiles = 0, kt = 0;   // kt: summed over the tiles
-    int form = 0;
-    for (int i = 0; i < n; ++i) {
-        const int64_t t = tiles_of(*g[i], edge);
-        tiles += t;
-        kt += t * k_tiles(*g[i]);
-        form = g[i]->ta ? 2 : (g[i]->tb && form < 1 ? 1 : form);
-    }
-    const int64_t k = kt / tiles;   // K-tiles of an average tile
-    TileTime whole = tile_time(edge, form, false, cus);
-    const TileTime few = tile_time(edge, form, true, cus);
-    // One problem on part of the CUs: the chip is clocked higher (140 to 210 tiles 1050 to 1180 ns a K-tile).  us, 128 / 256 wide:
-    // 3584 x 2560 x 5888 (140 tiles) 62 / 54, 168 tiles of K = 8700 91 / 80; 130 to 135 tiles, K 2048 to 4096, 21 to 37 / 25 to 44
-    if (n == 1 && edge.m == 256 && tiles < cus) whole.per_k = 1150;
-    const int64_t slots = whole.slots, rem = tiles % slots;
-    auto cost = [&](int split) -> int64_t {
-        const TileTime end = split > 1 ? tail_time(split, form, cus) : edge.m == 64 && rem <= cus ? few : whole;
-        const int64_t average = tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : end.per_k * k + end.rest);
-        if (n == 1 || tiles > 64 * slots) return average;
-        int64_t next_k;
-        const int64_t busy = list_end(g, n, order, edge, edge.m == 64 && tiles <= cus ? few : whole, split > 1 ? tiles - rem : tiles, &next_k);
-        if (busy < 0) return average;
-        return (average + busy + (split > 1 ? end.per_k * next_k + end.rest : 0)) / 2;
-    };
-    const int64_t as_is = cost(*parts = 1);
-    const int split = edge.m == 256 ? tail_parts(tiles, cus) : 1;
-    if (split == 1) return as_is;
-    const int64_t cut = cost(split);
-    if (cut < as_is) *parts = split;
-    return std::min(cut, as_is);
-}
-
 // The tile list of a launch, problem by problem, longest K first: the long tiles start together and the shorter ones fill
 // the rounds behind them.  Returns the number of tiles.
-static void by_depth(const GemmDesc* const* g, int n, int* order) {
-    for (int i = 0; i < n; ++i) order[i] = i;
-    for (int i = 1; i < n; ++i)   // insertion sort, stable, K descending
-        for (int j = i; j > 0 && g[order[j]]->K > g[order[j - 1]]->K; --j) std::swap(order[j], order[j - 1]);
-}
 static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch* L) {
     int order[kBigMaxProblems];
     by_depth(g, n, order);
@@ -243,10 +111,10 @@ static int64_t list_tiles(const GemmDesc* const* g, int n, Edge edge, BigLaunch*
 //                    4096 x 2048 7.5 / 5.0     6144 x 3072 9.7 / 7.5     8192 x 4096 13.6 / 10.0   10240 x 4096 12.5 / 15.0
 //   32 rows:         4096 x 2048 6.0 / 6.6     2048 x 3072 7.0 / 6.9     4096 x 4096 11.5 / 9.1    5120 x 4096 11.2 / 15.3
 //                    4096 x 14336 31.9 / 21.7  5120 x 14336 31.5 / 39.5
-static bool few_rows(const GemmDesc& g) {
+static bool few_rows(const GemmDesc& g, int cus) {
     if (g.M > 32 || g.tb || is_fp8_out(g.d_dtype)) return false;
-    if (g.M <= 16) return (g.K >= 2048 && g.N <= 32 * cu_count()) || (g.K >= 1024 && g.N <= 16 * cu_count());
-    return g.K >= 3072 && g.N <= 16 * cu_count();
+    if (g.M <= 16) return (g.K >= 2048 && g.N <= 32 * cus) || (g.K >= 1024 && g.N <= 16 * cus);
+    return g.K >= 3072 && g.N <= 16 * cus;
 }
 
 // Bookkeeping of an fp8 output by the workgroup that finishes last, where the launch is one round of workgroups; behind more
@@ -264,27 +132,12 @@ static int finish_behind(const GemmDesc& g, int rc, hipStream_t st) {
 }
 
 // One launch over up to kBigMaxProblems problems of the same operand formats, in the tile size that takes least (256-wide
-// tiles: one more launch for a half-tile tail).
+// tiles: one more launch for a tail in parts).
 template <int FA, int FB>
-static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
-    const int cus = cu_count();   // (asked once: the question goes to the runtime)
-    Edge edge{128, 128};
-    int parts = 1;
-    {
-        bool big = true;
-        for (int i = 0; i < n; ++i) big = big && big_ok(*g[i]);
-        int order[kBigMaxProblems];
-        by_depth(g, n, order);
-        int64_t best = launch_cost(g, n, order, edge, cus, &parts);
-        // (where the lines meet, the wider tiles for one problem, the narrower for several)
-        const int first = n == 1 ? 256 : 64;
-        for (const Edge e : {Edge{first, first}, Edge{320 - first, 320 - first}, Edge{128, 64}}) {
-            if (e.m == 256 && !big) continue;
-            int p;
-            const int64_t c = launch_cost(g, n, order, e, cus, &p);
-            if (c < best) best = c, edge = e, parts = p;
-        }
-    }
+static int launch_tiles(const GemmDesc* const* g, int n, int cus, hipStream_t st) {
+    const TileChoice choice = choose_tiles(g, n, cus);
+    const Edge edge = choice.edge;
+    const int parts = choice.parts;
     BigLaunch L;
     const int64_t tiles = list_tiles(g, n, edge, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
@@ -326,10 +179,9 @@ static int launch_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
 // Problems no 16-byte chunk of which lies in one piece: 128-wide tiles once there is one for every CU, 64-wide below
 // (us, 64 / 128 wide: 1536 x 1536 x 1021, 144 tiles of 128, 18.4 / 20.4; 2048 x 2048 x 1021, 256 tiles, 23.4 / 21.6;
 // 4096 x 4096 x 4095 262 / 179)
-static int launch_any_tiles(const GemmDesc* const* g, int n, hipStream_t st) {
+static int launch_any_tiles(const GemmDesc* const* g, int n, int cus, hipStream_t st) {
     BigLaunch L;
     int edge = 128;
-    const int cus = cu_count();
     int64_t tiles = list_tiles(g, n, Edge{edge, edge}, &L);
     if (tiles < cus) edge = 64, tiles = list_tiles(g, n, Edge{edge, edge}, &L);
     if (tiles > 0x7fffffff) return NTFP8_ERR_SIZE;
@@ -348,28 +200,28 @@ static bool tiny(const GemmDesc& g) {
 }
 
 static int dispatch(const GemmDesc* const* g, int n, int path, hipStream_t st) {
-    const int fa = g[0]->fmt_a, fb = g[0]->fmt_b;
+    const int fa = g[0]->fmt_a, fb = g[0]->fmt_b, cus = cu_count();   // (asked once: the question goes to the runtime)
     if (path == kPathNone) return NTFP8_ERR_UNSUPPORTED;
 #ifdef NTFP8_PROFILE_NARROW
     // experiment builds of the profiling library carry one instantiation only: e4m3 x e4m3, K-contiguous operands,
     // 16-bit or fp32 output (what the loop experiments launch); everything else is refused
     if (fa != kE4M3 || fb != kE4M3 || path != kPathTiles || g[0]->tb || is_fp8_out(g[0]->d_dtype)) return NTFP8_ERR_UNSUPPORTED;
-    return launch_tiles<kE4M3, kE4M3>(g, n, st);
+    return launch_tiles<kE4M3, kE4M3>(g, n, cus, st);
 #else
     if (path == kPathAny && n == 1 && tiny(*g[0])) {
         BigLaunch L;
         list_tiles(g, 1, Edge{64, 64}, &L);
         return finish_behind(*g[0], launch_tiny(L.p[0], fa, fb, st), st);
     }
-    if (path == kPathAny) return launch_any_tiles(g, n, st);
-    if (path == kPathPlain || (n == 1 && short_k(*g[0]))) return finish_behind(*g[0], launch_plain(*g[0], st), st);
-    if (n == 1 && few_rows(*g[0])) {
+    if (path == kPathAny) return launch_any_tiles(g, n, cus, st);
+    if (path == kPathPlain || (n == 1 && short_k(*g[0], cus))) return finish_behind(*g[0], launch_plain(*g[0], st), st);
+    if (n == 1 && few_rows(*g[0], cus)) {
         BigLaunch L;
         list_tiles(g, 1, Edge{64, 64}, &L);
         return launch_few(L.p[0], fa, fb, st);
     }
-    if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, st) : launch_tiles<kE4M3, kE5M2>(g, n, st);
-    return fb == kE4M3 ? launch_tiles<kE5M2, kE4M3>(g, n, st) : launch_tiles<kE5M2, kE5M2>(g, n, st);
+    if (fa == kE4M3) return fb == kE4M3 ? launch_tiles<kE4M3, kE4M3>(g, n, cus, st) : launch_tiles<kE4M3, kE5M2>(g, n, cus, st);
+    return fb == kE4M3 ? launch_tiles<kE5M2, kE4M3>(g, n, cus, st) : launch_tiles<kE5M2, kE5M2>(g, n, cus, st);
 #endif
 }
 
@@ -407,6 +259,30 @@ int run_gemm_batch(const GemmDesc* g, int n, hipStream_t st) {
 }
 
 }  // namespace ntfp8
+
+// The tile size of a launch of these problems on a GPU of `cus` CUs, and in how many parts the tiles of a partial last round of
+// 256-wide ones are computed; for tests, which have to know what they reach.  Nothing is launched and no pointer of a
+// problem is followed.  NTFP8_ERR_UNSUPPORTED where they do not share a launch of the tile kernels.
+extern "C" __attribute__((visibility("default"))) int ntfp8_debug_gemm_tiles(const ntfp8_gemm_desc* p, int n, int cus, int* tile_m, int* tile_n, int* parts) {
+    using namespace ntfp8;
+    if (!p || !tile_m || !tile_n || !parts) return NTFP8_ERR_NULL;
+    if (n < 1 || n > kBigMaxProblems || cus < 1) return NTFP8_ERR_SIZE;
+    GemmDesc g[kBigMaxProblems] = {};
+    const GemmDesc* all[kBigMaxProblems];
+    for (int i = 0; i < n; ++i) {
+        if (p[i].M < 1 || p[i].N < 1 || p[i].K < 1 || p[i].M > 0x7fffffff || p[i].N > 0x7fffffff || p[i].K > 0x7fffffff) return NTFP8_ERR_SIZE;
+        g[i].A = p[i].A, g[i].B = p[i].B, g[i].D = p[i].D, g[i].Dt = p[i].D_t;
+        g[i].M = (int)p[i].M, g[i].N = (int)p[i].N, g[i].K = (int)p[i].K;
+        g[i].d_dtype = p[i].d_dtype, g[i].accumulate = p[i].accumulate;
+        g[i].tb = p[i].b_transposed, g[i].ta = p[i].a_transposed;
+        all[i] = &g[i];
+        if (path_of(g[i]) != kPathTiles || g[i].tb != g[0].tb || is_fp8_out(g[i].d_dtype) != is_fp8_out(g[0].d_dtype)) return NTFP8_ERR_UNSUPPORTED;
+    }
+    if (n == 1 && (short_k(g[0], cus) || few_rows(g[0], cus))) return NTFP8_ERR_UNSUPPORTED;
+    const TileChoice c = choose_tiles(all, n, cus);
+    *tile_m = c.edge.m, *tile_n = c.edge.n, *parts = c.parts;
+    return NTFP8_OK;
+}
 
 #ifdef NTFP8_STAMPS
 // Profiling build only: copies the per-workgroup time stamps of the last gemm_nt_big_kernel launches to host memory
