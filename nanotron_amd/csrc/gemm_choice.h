@@ -111,9 +111,12 @@ inline int64_t launch_cost(const GemmDesc* const* g, int n, const int* order, Ed
     const int64_t k = kt / tiles;   // K-tiles of an average tile
     TileTime whole = tile_time(edge, form, false, cus);
     const TileTime few = tile_time(edge, form, true, cus);
-    // One problem on part of the CUs: the chip is clocked higher (140 to 210 tiles 1050 to 1180 ns a K-tile).  us, 128 / 256 wide:
-    // 3584 x 2560 x 5888 (140 tiles) 62 / 54, 168 tiles of K = 8700 91 / 80; 130 to 135 tiles, K 2048 to 4096, 21 to 37 / 25 to 44
-    if (n == 1 && edge.m == 256 && tiles < cus) whole.per_k = 1150;
+    // One problem on part of the CUs: the chip is clocked higher (129 to 255 tiles 950 to 1200 ns a K-tile), and the 256-wide tiles
+    // are the fastest wherever 128-wide ones need more than two rounds (129 to 255 tiles, K 512 to 8192, every form, 16-bit, fp32
+    // and accumulated: 1.08 to 1.95 times).  Two rounds of those are faster from a K of about 700 on, which is where the ordinary
+    // price has the line: 504 of them against 132 tiles, us, 128 / 256 wide: K = 1024 bf16 14.2 / 15.9, fp32 16.5 / 19.7, both
+    // transposed 18.4 / 20.2; K = 512 11.5 / 11.9, 13.6 / 15.7, 15.0 / 16.0; K = 4096 bf16 32.0 / 39.0.
+    if (n == 1 && edge.m == 256 && tiles < cus && tiles_of(*g[0], Edge{128, 128}) > 2 * cus) whole.per_k = 1150;
     const int64_t slots = whole.slots, rem = tiles % slots;
     auto cost = [&](int split) -> int64_t {
         const TileTime end = split > 1 ? tail_time(split, form, cus) : edge.m == 64 && rem <= cus ? few : whole;

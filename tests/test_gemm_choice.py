@@ -16,6 +16,20 @@ def test_one_problem(problem, want):
     assert tiles(problem) == want
 
 
+@pytest.mark.parametrize("mn", [(2656, 3072), (1888, 4352), (2688, 2864)])   # 132 to 136 tiles of 256, two rounds of 128-wide ones
+@pytest.mark.parametrize("K", [768, 1024, 1152, 4096])
+@pytest.mark.parametrize("out,form", [(BF16, 0), (F32, 0), (BF16, 1), (F32, 2)])
+def test_two_rounds_of_128_wide_tiles(mn, K, out, form):
+    assert tiles((*mn, K, out, form)) == (128, 128, 1)
+
+
+@pytest.mark.parametrize("mn", [(2560, 3328), (2400, 3840), (3584, 2560), (3840, 4352)])   # 130 to 255 tiles of 256, more rounds of 128-wide ones
+@pytest.mark.parametrize("K", [1024, 4096, 5120, 8192])
+@pytest.mark.parametrize("out,form", [(BF16, 0), (F32, 0), (BF16, 1), (F32, 2)])
+def test_part_of_the_chip_in_256_wide_tiles(mn, K, out, form):
+    assert tiles((*mn, K, out, form)) == (256, 256, 1)
+
+
 def test_what_other_kernels_serve():
     assert tiles((16, 4096, 4096, BF16, 0)) is None             # a few rows
     assert tiles((4096, 4096, 128, BF16, 0)) is None            # one K-tile, more tiles than the chip works on at once
