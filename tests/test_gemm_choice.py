@@ -30,6 +30,34 @@ def test_part_of_the_chip_in_256_wide_tiles(mn, K, out, form):
     assert tiles((*mn, K, out, form)) == (256, 256, 1)
 
 
+@pytest.mark.parametrize("layer,out,acc,want", [   # (tokens, in features, out features); us in the tiles wanted / others
+    ((256, 256, 7760), BF16, False, (64, 64)),      # 20.4 / 128 x 64 27.4
+    ((288, 256, 3840), BF16, False, (64, 64)),      # 9.4 / 128 x 64 12.6
+    ((432, 256, 3824), F32, False, (64, 64)),       # 11.6 / 128 x 64 15.9
+    ((256, 448, 4416), BF16, True, (64, 64)),       # 13.8 / 128 x 128 19.9
+    ((768, 1056, 3184), BF16, True, (256, 256)),    # 22.9 / 128 x 128 28.3
+    ((976, 1136, 3664), F32, True, (256, 256)),     # 28.2 / 128 x 128 34.0
+    ((2304, 1520, 3584), BF16, False, (256, 256)),  # 40.3 / 128 x 128 44.1
+    ((1280, 2560, 6912), BF16, False, (128, 128)),  # 62 / 256 x 256 82
+])
+def test_input_and_weight_gradient_in_one_launch(layer, out, acc, want):
+    tokens, fin, fout = layer
+    assert tiles((tokens, fin, fout, out, 1), (fout, fin, tokens, F32, 2, acc))[:2] == want
+
+
+@pytest.mark.parametrize("a,b", [((3904, 256, 384, BF16, 0), (224, 352, 7152, BF16, 0)),       # 13.9 / 128 x 64 22.1
+                                 ((1280, 768, 2016, BF16, 0), (160, 400, 3984, BF16, 0))])     # 10.3 / 128 x 64 14.3
+def test_deep_tiles_beside_shallow_ones(a, b):
+    assert tiles(a, b)[:2] == tiles(b, a)[:2] == (64, 64)
+
+
+@pytest.mark.parametrize("cus", [1, 7, 64, 256, 304])
+def test_any_list_on_any_gpu(cus):
+    for a, b in [((304, 304, 256, F32, 2), (70000, 4096, 512, F32, 2, True)), ((272, 272, 8192, F32, 2), (272, 272, 256, F32, 2)),
+                 ((100000, 8192, 256, F32, 2), (100000, 8192, 512, F32, 2))]:
+        assert tiles(a, b, cus=cus) is not None and tiles(a, b, a, b, cus=cus) is not None
+
+
 def test_what_other_kernels_serve():
     assert tiles((16, 4096, 4096, BF16, 0)) is None             # a few rows
     assert tiles((4096, 4096, 128, BF16, 0)) is None            # one K-tile, more tiles than the chip works on at once
