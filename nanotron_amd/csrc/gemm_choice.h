@@ -55,6 +55,18 @@ inline int64_t tiles_of(const GemmDesc& g, Edge e) {
 inline int form_of(const GemmDesc& g) { return g.ta ? 2 : g.tb ? 1 : 0; }
 inline int64_t k_tiles(const GemmDesc& g) { return (g.K + kBK - 1) / kBK; }
 
+// A second round of 128 x 64 tiles, both operands K-contiguous: nothing of its start or of the first round's stores is hidden, the more so the
+// narrower the output's rows are in a tile.  The other way there are halves of 256-wide tiles (up to 128 of them).  us, those / two rounds
+// (387 to 507 tiles of 128 x 64):
+//   K               256          512          1024         1536         2048         3072         4096         6144
+//   16-bit       6.1 /  7.5   7.4 /  8.4   9.7 / 10.1  12.1 / 13.0  14.3 / 14.2  19.0 / 20.0  23.2 / 22.3  32.5 / 32.3
+//   fp32         8.1 /  8.4   9.5 /  9.5  11.8 / 11.2  14.3 / 14.1  16.4 / 15.1  21.1 / 21.0  25.5 / 23.1  34.4 / 33.2
+//   fp8          8.1 / 10.1   9.5 / 11.3  11.8 / 12.9  14.3 / 15.6  16.5 / 16.7  21.3 / 22.5  25.6 / 25.2  34.7 / 34.9
+//   and copy    11.1 / 14.4  12.8 / 15.6  15.2 / 17.4  17.3 / 19.5  19.9 / 20.8  24.4 / 26.5  28.5 / 28.6  37.7 / 38.2
+inline int64_t narrow_again(const GemmDesc& g) {
+    return is_fp8_out(g.d_dtype) ? (g.Dt ? 3700 : 2700) : g.d_dtype == NTFP8_F32 ? 400 : 1500;
+}
+
 // *parts: of the tiles of a partial last round of 256-wide ones
 inline int64_t cost_of_one(const GemmDesc& g, Edge edge, int64_t cus, int* parts) {
     const int64_t tiles = tiles_of(g, edge), k = k_tiles(g);
@@ -69,7 +81,8 @@ inline int64_t cost_of_one(const GemmDesc& g, Edge edge, int64_t cus, int* parts
     const int64_t slots = whole.slots, rem = tiles % slots;
     auto cost = [&](int split) -> int64_t {
         const TileTime end = split > 1 ? tail_time(split, form, cus) : edge.m == 64 && rem <= cus ? tile_time(edge, form, true, cus) : whole;
-        return tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : end.per_k * k + end.rest);
+        const int64_t more = edge.m == 128 && edge.n == 64 && form == 0 ? (tiles - 1) / slots * narrow_again(g) : 0;
+        return tiles / slots * (whole.per_k * k + whole.rest) + (rem == 0 ? 0 : end.per_k * k + end.rest) + more;
     };
     const int64_t as_is = cost(*parts = 1);
     const int split = edge.m == 256 ? tail_parts(tiles, cus) : 1;

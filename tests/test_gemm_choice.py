@@ -30,6 +30,17 @@ def test_part_of_the_chip_in_256_wide_tiles(mn, K, out, form):
     assert tiles((*mn, K, out, form)) == (256, 256, 1)
 
 
+@pytest.mark.parametrize("mn", [(3632, 1088), (1568, 2496), (5400, 704), (16500, 192)])   # 387 to 507 tiles of 128 x 64, up to 75 of 256
+@pytest.mark.parametrize("out,copy,K,want", [
+    (BF16, 0, 256, (256, 256, 2)), (BF16, 0, 512, (256, 256, 2)), (BF16, 0, 1536, (256, 256, 2)), (BF16, 0, 4096, (128, 64, 1)),
+    (F32, 0, 256, (256, 256, 2)), (F32, 0, 1024, (128, 64, 1)), (F32, 0, 4096, (128, 64, 1)),
+    (OUT_E4M3, 0, 256, (256, 256, 2)), (OUT_E4M3, 0, 1536, (256, 256, 2)), (OUT_E4M3, 0, 4096, (128, 64, 1)),
+    (OUT_E4M3, 1, 256, (256, 256, 2)), (OUT_E4M3, 1, 3072, (256, 256, 2)),
+])
+def test_second_round_of_128_x_64_tiles(mn, out, copy, K, want):
+    assert tiles((*mn, K, out, 0), copy=copy) == want
+
+
 @pytest.mark.parametrize("layer,out,acc,want", [   # (tokens, in features, out features); us in the tiles wanted / others
     ((256, 256, 7760), BF16, False, (64, 64)),      # 20.4 / 128 x 64 27.4
     ((288, 256, 3840), BF16, False, (64, 64)),      # 9.4 / 128 x 64 12.6
