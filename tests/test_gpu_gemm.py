@@ -70,7 +70,7 @@ def test_integer_operands_bit_exact(fa, fb, mnk):
 @pytest.mark.parametrize("mnk,fa,fb", [
     ((4096, 4096, 272), O.E4M3, O.E4M3),    # 256 whole 256x256 tiles (one per CU), K tail of 16
     ((4096, 6144, 256), O.E5M2, O.E4M3),    # 384 tiles: one whole round + 128 tiles as 128-row halves; two K-tiles
-    ((4000, 4136, 400), O.E4M3, O.E5M2),    # 272 tiles with ragged bottom / right edges, odd K-tile count
+    ((4000, 4136, 400), O.E4M3, O.E5M2),    # 272 tiles with ragged bottom / right edges, odd K-tile count: the last 16 in eighths
     ((2304, 2048, 1024), O.E4M3, O.E4M3),   # 72 tiles: every tile computed as halves
 ])
 def test_large_grid_bit_exact(mnk, fa, fb):

@@ -36,7 +36,7 @@ def test_integer_operands_ragged_sweep_singly_and_batched():
 
     rng = torch.Generator().manual_seed(31415)
     one = torch.tensor(1.0)
-    shapes = [(2304, 2048, 400), (4096, 4352, 256), (129, 144, 256), (1000, 272, 1040)]   # half tiles only; whole + half; minimal
+    shapes = [(2304, 2048, 400), (4096, 4352, 256), (129, 144, 256), (1000, 272, 1040)]   # half tiles only; whole tiles and a tail in eighths; minimal
     for _ in range(10):
         shapes.append((int(torch.randint(129, 1400, (1,), generator=rng)), 16 * int(torch.randint(9, 88, (1,), generator=rng)),
                        16 * int(torch.randint(16, 130, (1,), generator=rng))))
