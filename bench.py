@@ -23,6 +23,7 @@ One JSON line is printed.  `roofline` describes the dominant kernel (the fp8 MFM
 `cpu_baseline` is the CPU oracle (a port of the reference's arithmetic) timed on this host.
 """
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -35,9 +36,10 @@ if ROOT not in sys.path:
 PEAK_FP8_TFLOPS = 5000.0  # MI355X dense fp8 MFMA peak
 PEAK_HBM_GBPS = 8000.0    # MI355X HBM3E peak
 # HBM-side traffic is not measurable from inside this process: it comes from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
-# runs of this same script, whose summary (figures, commands, the commit and flags they were taken at) is the text
-# file below.  Its "bench-readable" block is parsed here and handed on with its provenance.
+# runs of this same script, whose summary (figures, commands, the commit, kernels and flags they were taken at) is the
+# text file below.  Its "bench-readable" block is parsed here and handed on with its provenance.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_counters.txt")
+KERNEL_DIR = os.path.join(ROOT, "nanotron_amd", "csrc")
 
 TOKENS = 4096
 LINEARS = [  # name, in_features (K), out_features (N): benchmark configuration 5 (the parity test uses the same list)
@@ -105,9 +107,20 @@ def flags_of(args):
     return "default" if not on else ",".join(on)
 
 
+def kernel_digest():
+    """What the kernels are, as recorded next to counter figures: a digest of their sources."""
+    h = hashlib.sha256()
+    for name in sorted(os.listdir(KERNEL_DIR)):
+        if name.endswith((".h", ".hip")):
+            with open(os.path.join(KERNEL_DIR, name), "rb") as f:
+                h.update(name.encode() + b"\0" + f.read() + b"\0")
+    return h.hexdigest()[:16]
+
+
 def read_traffic(args):
     """{"gemm": bytes per step | None, "quant": bytes per launch | None, "source": {...}} from the bench-readable
-    block of the counter summary under profiles/.  A figure taken with other flags than this run's is not used."""
+    block of the counter summary under profiles/.  A figure taken with other flags than this run's, or of other kernels, is
+    not used."""
     out = {"gemm": None, "quant": None, "source": {"file": os.path.relpath(TRAFFIC_FILE, ROOT)}}
     try:
         text = open(TRAFFIC_FILE).read()
@@ -126,6 +139,9 @@ def read_traffic(args):
     out["source"].update({"commit": kv.get("commit"), "flags": kv.get("flags"), "workload": kv.get("workload")})
     if kv.get("flags") != flags_of(args):
         out["source"]["note"] = f"counters were taken with flags '{kv.get('flags')}', this run uses '{flags_of(args)}': not used"
+        return out
+    if kv.get("kernels") != kernel_digest():
+        out["source"]["note"] = "counters were taken of other kernels than this tree's: not used"
         return out
     try:
         out["gemm"] = float(kv["gemm_fetch_bytes_per_step"]) + float(kv["gemm_write_bytes_per_step"])

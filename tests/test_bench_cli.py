@@ -1,5 +1,6 @@
 """bench.py from the command line: the refusals that need no GPU, and on the GPU the switches that change which kernels
 a step launches (each must still produce one JSON line with the contract's fields)."""
+import argparse
 import json
 import os
 import subprocess
@@ -19,6 +20,22 @@ def test_more_than_one_gpu_is_refused_with_a_message():
     r = _bench("--gpus", "2")
     assert r.returncode == 2
     assert "one GPU" in r.stderr and r.stdout.strip() == ""
+
+
+def test_counter_figures_of_other_kernels_are_not_used(tmp_path, monkeypatch):
+    monkeypatch.syspath_prepend(ROOT)
+    import bench
+
+    args = argparse.Namespace(weight_stream=False, transposed_copies=False, grad_transposed_copy=False, fp8_activations=False)
+    summary = tmp_path / "counters.txt"
+    monkeypatch.setattr(bench, "TRAFFIC_FILE", str(summary))
+    for kernels, flags, used in ((bench.kernel_digest(), "default", True), ("0" * 16, "default", False), (None, "default", False),
+                                 (bench.kernel_digest(), "weight_stream", False)):
+        summary.write_text("[bench-readable]\nflags = %s\n%sgemm_fetch_bytes_per_step = 4e9\ngemm_write_bytes_per_step = 1e9\n"
+                           "quant_fetch_bytes_per_launch = 3e7\nquant_write_bytes_per_launch = 2e7\n" % (flags, f"kernels = {kernels}\n" if kernels else ""))
+        got = bench.read_traffic(args)
+        assert (got["gemm"], got["quant"]) == ((5e9, 5e7) if used else (None, None))
+        assert ("note" in got["source"]) != used
 
 
 @pytest.mark.gpu
