@@ -270,7 +270,7 @@ __device__ __forceinline__ void store_wave_tile16(const v4f (&acc)[MI][NJ], void
                 if constexpr (DT == NTFP8_F32) {
                     v4f o = {v[0], v[1], v[2], v[3]};
                     if constexpr (kAcc) o = o + old[j];
-                    // (fp32 outputs keep the ordinary store: written through they measured the same or slower)
+                    // (rows that end inside a 64-byte piece, and rows too wide for the descriptors above: ordinary stores, as there)
                     *reinterpret_cast<v4f*>(dp) = o;
                 } else {
                     *reinterpret_cast<uint2*>(dp) = make_uint2(OutT<DT>::pack2(v[0], v[1]), OutT<DT>::pack2(v[2], v[3]));
